@@ -691,14 +691,15 @@ int enqueue_prep(clm_ctx* c, const Plan& pl) {
             continue;
         }
         if ((rc = enqueue_fill(c, B.nrm.p, g.K, 0))) return rc;
-        const long long lines = (long long)g.K * g.Lp;
-        const unsigned nb = (unsigned)((lines + 255) / 256);
+        const int pl_lines = prep_lines(g.n_r);
+        const unsigned nb = (unsigned)((long long)g.K * ((g.Lp + pl_lines - 1) / pl_lines));
+        const size_t plds = prep_lds_bytes(g.n_r);
         if (j.p.pf_dtype == CLM_C128)
-            hipLaunchKernelGGL(prep_kernel<double>, dim3(nb), dim3(256), 0, c->stream, (const double*)j.io.pf, g,
+            hipLaunchKernelGGL(prep_kernel<double>, dim3(nb), dim3(PREP_T), plds, c->stream, (const double*)j.io.pf, g,
                                (const double*)B.H.p, (double2*)B.P64.p, (float2*)B.P32.p, B.Bop.p, j.opk,
                                (unsigned*)B.nrm.p, ctr + 0, j.lsh);
         else
-            hipLaunchKernelGGL(prep_kernel<float>, dim3(nb), dim3(256), 0, c->stream, (const float*)j.io.pf, g,
+            hipLaunchKernelGGL(prep_kernel<float>, dim3(nb), dim3(PREP_T), plds, c->stream, (const float*)j.io.pf, g,
                                (const double*)B.H.p, (double2*)B.P64.p, (float2*)B.P32.p, B.Bop.p, j.opk,
                                (unsigned*)B.nrm.p, ctr + 0, j.lsh);
         HIPCHK(c, hipGetLastError());

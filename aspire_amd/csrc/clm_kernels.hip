@@ -27,10 +27,29 @@
 namespace clm {
 
 // -------------------------------------------------------------- preprocess
-// One thread per line (k,l).  Sequential FP64 arithmetic in the oracle's
-// order so P64 is bit-identical to the CPU restatement.
+// Lines (k, l): one workgroup per image and PREP_NL consecutive lines.  The
+// two blocks of pf columns that these lines are assembled from (l.. and
+// L + l..) are contiguous, so they come in as whole cache lines; everything
+// but the two sums over a line is done one element per thread.  The sums run
+// in one thread per line, over terms left in LDS, in the oracle's order, so
+// P64 is bit-identical to the CPU restatement.
+// HBM bound: 103 us at K = 1000, n_r = 45 (0.49 GB read and written, 4.8
+// TB/s; a plain device copy reaches 5.1 here) and 264 us at K = 1500,
+// n_r = 65, complex128.  One thread per line, with every load and store a
+// stride of a whole line apart, took 784 and 1830 us.
+constexpr int PREP_T = 256;
+
+// Lines per workgroup: as many as keep the terms and rays of a workgroup
+// within 40 KB of LDS, so that four workgroups share a CU.
+__host__ __device__ inline int prep_lines(int n_r) { return n_r <= 66 ? 16 : 8; }
+// per line: 2 n_r - 1 terms (the row padded to an odd number of doubles, for
+// the banks of the threads that walk the rows) and R complex values
+__host__ __device__ inline size_t prep_lds_bytes(int n_r) {
+    return (size_t)prep_lines(n_r) * ((size_t)(2 * n_r + 1) * 8 + (size_t)n_r * 16) + 2 * 16 * sizeof(double);
+}
+
 template <typename InT>
-__global__ void prep_kernel(const InT* __restrict__ pf, Geom g,
+__global__ __launch_bounds__(PREP_T) void prep_kernel(const InT* __restrict__ pf, Geom g,
                             const double* __restrict__ H,  // 2n_r-1, zeroed band
                             double2* __restrict__ P64,     // [K][L][R] or null
                             float2* __restrict__ P32,      // [K][L][Rp]
@@ -39,70 +58,92 @@ __global__ void prep_kernel(const InT* __restrict__ pf, Geom g,
                             unsigned* __restrict__ nrm_bits,  // [K] float bits
                             unsigned long long* __restrict__ n_small,
                             const double* __restrict__ lsh) { // [K][L] per-line shift (px) or null
+    extern __shared__ __align__(16) char s_prep[];
+    const int n_r = g.n_r, R = g.R, L = g.L, T = g.T, Rp = g.Rp, Lp = g.Lp;
+    const int NL = prep_lines(n_r);
+    const int ldt = 2 * n_r + 1;
+    double2* s_z = (double2*)s_prep;                  // [NL][n_r] filtered half rays
+    double* s_t = (double*)(s_z + (size_t)NL * n_r);  // [NL][ldt] terms of the sums
+    double* s_nr = s_t + (size_t)NL * ldt;            // [NL] line norms
+    const int tid = threadIdx.x;
     // lines run over the padded range l < Lp so padding rows of the operand
     // planes are written (zeros) by the same launch
-    const long line = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (line >= (long)g.K * g.Lp) return;
-    const int k = (int)(line / g.Lp), l = (int)(line % g.Lp);
-    const int n_r = g.n_r, R = g.R, L = g.L, T = g.T, Rp = g.Rp, Lp = g.Lp;
+    const int nblk = (Lp + NL - 1) / NL;
+    const int k = blockIdx.x / nblk, l0 = (blockIdx.x % nblk) * NL;
+    const int nl = min(NL, L - l0);    // lines with rays (may be <= 0)
+    const int nlp = min(NL, Lp - l0);  // lines of the operand planes
     auto put = [&](size_t idx, float v) {
         if (op_kind == 0) ((float*)Bop)[idx] = v;
         else if (op_kind == 1) ((__bf16*)Bop)[idx] = (__bf16)v;
         else ((_Float16*)Bop)[idx] = (_Float16)v;
     };
-    const size_t pre0 = (((size_t)k * 2 + 0) * Lp + l) * Rp;
-    const size_t pim0 = (((size_t)k * 2 + 1) * Lp + l) * Rp;
-    if (l >= L) {
-        for (int r = 0; r < Rp; r++) { put(pre0 + r, 0.f); put(pim0 + r, 0.f); }
-        return;
-    }
-    const InT* base = pf + 2 * (size_t)k * T * n_r;
-    double ss = 0.0;
-    for (int i = 0; i < 2 * n_r - 1; i++) {
-        int rr, tt;
-        if (i < n_r - 1) { rr = n_r - 1 - i; tt = L + l; }
-        else             { rr = i - (n_r - 1); tt = l; }
-        const InT* z = base + 2 * ((size_t)tt * n_r + rr);
-        double re = (double)z[0] * H[i], im = (double)z[1] * H[i];
-        ss += re * re + im * im;
-    }
-    const double nr = sqrt(ss);
-    if (nr < 1.0e-13) atomicAdd(n_small, 1ull);
-    const InT* zc = base + 2 * ((size_t)(L + l) * n_r);
-    double2* o64 = P64 ? P64 + ((size_t)k * L + l) * R : nullptr;
-    float2* o32 = P32 + ((size_t)k * L + l) * Rp;
-    double hn = 0.0;
-    const double a = lsh ? lsh[(size_t)k * L + l] : 0.0;
-    for (int r = 0; r < R; r++) {
-        const int rr = n_r - 1 - r;
-        double re = ((double)zc[2 * rr] * H[r]) / nr;
-        double im = ((double)zc[2 * rr + 1] * H[r]) / nr;
-        if (lsh) {
-            // line moved by a px: times exp(-2*pi*i*rk*a/(2R+1)), rk = r - R,
-            // the phase the shift search applies for shift a
-            const double th = ((-2.0 * M_PI * (double)(r - R)) * a) / (double)(2 * R + 1);
-            const double c = cos(th), sn = sin(th);
-            const double xr = re * c - im * sn, xi = re * sn + im * c;
-            re = xr;
-            im = xi;
+    const int nv = max(nl, 0) * n_r;
+    // element i of a line (i = 0..2 n_r - 2) is column L + l at n_r - 1 - i
+    // below the middle, column l at i - (n_r - 1) from there on
+    for (int half = 0; half < 2; half++) {
+        const InT* base = pf + 2 * ((size_t)k * T + (half ? 0 : L) + l0) * n_r;
+        for (int x = tid; x < nv; x += PREP_T) {
+            const int j = x / n_r, rr = x - j * n_r;
+            if (!half && rr == 0) continue;
+            const int i = half ? n_r - 1 + rr : n_r - 1 - rr;
+            const double re = (double)base[2 * x] * H[i], im = (double)base[2 * x + 1] * H[i];
+            s_t[j * ldt + i] = re * re + im * im;
+            if (!half) s_z[j * n_r + i] = make_double2(re, im);
         }
-        if (o64) o64[r] = make_double2(re, im);
-        float fr = (float)re, fi = (float)im;
-        o32[r] = make_float2(fr, fi);
-        hn += re * re + im * im;
-        put(pre0 + r, fr);
-        put(pim0 + r, fi);
     }
-    for (int r = R; r < Rp; r++) {
-        o32[r] = make_float2(0.f, 0.f);
-        put(pre0 + r, 0.f);
-        put(pim0 + r, 0.f);
+    __syncthreads();
+    if (tid < nl) {
+        const double* t = s_t + tid * ldt;
+        double ss = 0.0;
+        for (int i = 0; i < 2 * n_r - 1; i++) ss += t[i];
+        const double nr = sqrt(ss);
+        if (nr < 1.0e-13) atomicAdd(n_small, 1ull);
+        s_nr[tid] = nr;
     }
+    __syncthreads();
+    for (int x = tid; x < nlp * Rp; x += PREP_T) {
+        const int j = x / Rp, r = x - j * Rp, l = l0 + j;
+        float fr = 0.f, fi = 0.f;
+        if (j < nl && r < R) {
+            const double nr = s_nr[j];
+            const double2 z = s_z[j * n_r + r];
+            double re = z.x / nr, im = z.y / nr;
+            if (lsh) {
+                // line moved by a px: times exp(-2*pi*i*rk*a/(2R+1)), rk = r - R,
+                // the phase the shift search applies for shift a
+                const double a = lsh[(size_t)k * L + l];
+                const double th = ((-2.0 * M_PI * (double)(r - R)) * a) / (double)(2 * R + 1);
+                const double c = cos(th), sn = sin(th);
+                const double xr = re * c - im * sn, xi = re * sn + im * c;
+                re = xr;
+                im = xi;
+            }
+            if (P64) P64[((size_t)k * L + l) * R + r] = make_double2(re, im);
+            fr = (float)re;
+            fi = (float)im;
+            s_t[j * ldt + r] = re * re + im * im;
+        }
+        if (j < nl) P32[((size_t)k * L + l) * Rp + r] = make_float2(fr, fi);
+        put((((size_t)k * 2 + 0) * Lp + l) * Rp + r, fr);
+        put((((size_t)k * 2 + 1) * Lp + l) * Rp + r, fi);
+    }
+    __syncthreads();
     // max half-line norm of the image, rounded up (bound input of the
     // certified threshold).  Non-finite norms are left out: their lines
     // give NaN correlations, which every max below ignores.
-    float hf = (float)(sqrt(hn) * (1.0 + 1.0e-6));
-    if (isfinite(hf)) atomicMax(nrm_bits + k, __float_as_uint(hf));
+    if (tid < 16) {
+        float hf = 0.f;
+        if (tid < nl) {
+            const double* t = s_t + tid * ldt;
+            double hn = 0.0;
+            for (int r = 0; r < R; r++) hn += t[r];
+            hf = (float)(sqrt(hn) * (1.0 + 1.0e-6));
+            if (!isfinite(hf)) hf = 0.f;
+        }
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) hf = fmaxf(hf, __shfl_xor(hf, o, 16));
+        if (tid == 0 && nl > 0) atomicMax(nrm_bits + k, __float_as_uint(hf));
+    }
 }
 
 // ------------------------------------------------------------ re-scoring
