@@ -53,11 +53,11 @@ struct clm_ctx {
     clmh::DevBuf ex_v, ex_k;
     // shift network: activations and gradients of the last batch
     clmh::DevBuf sn_h1, sn_h2, sn_z, sn_y, sn_dy, sn_dz, sn_dz2, sn_dz1;
-    // polar Fourier transform: per-axis tables, staged images, host-form buffers;
+    // polar Fourier transform: per-axis tables, folded images, host-form buffers;
     // the NUFFT method's oversampled grids, windows, kernel weights and
     // deconvolution factors, and its hipFFT plans (opaque handles) with their
     // grid side and batch
-    clmh::DevBuf pft_ax, pft_ay, pft_xt, pft_img, pft_out;
+    clmh::DevBuf pft_ax, pft_xt, pft_img, pft_out;
     clmh::DevBuf pft_grid, pft_base, pft_wt, pft_dec;
     void* fft_plan[2] = {nullptr, nullptr};
     int fft_side[2] = {0, 0}, fft_batch[2] = {0, 0};

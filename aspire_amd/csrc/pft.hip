@@ -14,13 +14,17 @@
 // u is the first (row) index of an image, paired with fx = r*sin(theta); v is
 // the second, paired with fy = r*cos(theta).
 //
-// On the device this is a contraction over the n*n pixels of a complex weight
-// matrix E (M x n^2, M = n_r*n_theta/2) with the real image stack (n^2 x K):
-// FP64 MFMA (v_mfma_f64_16x16x4f64).  E is never stored: the exponential
-// factors per axis, E(m,(u,v)) = ax(u,m) * ay(v,m), come from two small tables
-// and a per-point rotation, and each lane forms its operand with complex
-// products in registers.  Images are first staged pixel-major (pixel rows of Kp images,
-// FP64) so the B fragments load as 128-byte rows.
+// On the device this is a contraction over the pixels on FP64 MFMA
+// (v_mfma_f64_16x16x4f64).  The images are real and the points come in
+// quadruples of frequencies (+-fx, +-fy) (ray j, its mirror n_theta/2 - j and
+// their conjugates), so the pixels are first folded over both axes into four
+// planes, even or odd in u and in v, a = |g(u)|, b = |g(v)|:
+//   Scc = sum cos(fx a) cos(fy b) pee(a, b)    Sss = sum sin sin poo
+//   Ssc = sum sin(fx a) cos(fy b) poe(a, b)    Scs = sum cos sin peo
+//   pf(j) = Scc - Sss + i (Ssc + Scs)          pf(n_theta/2 - j) = Scc + Sss + i (Ssc - Scs)
+// Four real products over a quarter of the pixels serve two rays: a quarter
+// of the multiplications of the sums as written.  The weights are never
+// stored: a lane forms its operand as one product of two table entries.
 //
 // CLM_PFT_NUFFT: the same sums by a type-2 non-uniform FFT, the method the
 // reference's nufft2 uses when a NUFFT library is installed
@@ -49,64 +53,73 @@ namespace pft {
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 
-constexpr int MB = 128;  // polar points per workgroup (4 waves x 32)
-constexpr int KB = 64;   // images per workgroup (4 column tiles of 16)
 constexpr int KCHUNK = 8192;  // images per staged chunk
+constexpr int FA = 32;        // folded columns per staging workgroup
 
 struct Geo {
-    int n, n_r, n_theta, M, Mp;  // M = n_r * n_theta/2 polar points, Mp = roundup(M, MB)
-    int nup;                     // roundup(n, 4): pixel rows per image column in the staged stack
-    int Kc, Kp;                  // images in this chunk, roundup(Kc, KB)
+    int n, n_r, n_theta;
+    int M, Mp;       // quadrant points n_r * (n_theta/4 + 1), rows of the tables (padded for the row tiles)
+    int c;           // pixel index of the origin: g(c) = 0
+    int nh, nab;     // folded side floor(n/2) + 1, blocks of 4 of it
+    int Kc, nct;     // images in this chunk, column tiles of 16
 };
 
-// ax[u*Mp + m] = exp(+1i*fx(m)*g(u)) (u < 4; the first four rows),
-// ay[v*Mp + m] = exp(+1i*fy(m)*g(v)) (v < n), and
-// ax[4*Mp + m] = exp(+4i*fx(m)), the step from pixel u to u + 4 (zero for
-// m >= M).  grid: (Mp/256, 5 + n).
-__global__ void tables_kernel(Geo g, double2* ax, double2* ay) {
+// tab[0][a*Mp + m] = cos(fx(m) a), tab[1] sin; then cos(fy(m) b) and
+// sin(fy(m) b), 4 nab rows each (zero for m >= M).  grid: (Mp/256, 8 nab).
+__global__ void tables_kernel(Geo g, double* tab) {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    const int t = blockIdx.y;
     if (m >= g.Mp) return;
-    const bool is_x = t < 5;
-    const int idx = is_x ? t : t - 5;
-    double2 out = make_double2(0.0, 0.0);
+    const int na = 4 * g.nab;
+    const bool is_x = (int)blockIdx.y < na;
+    const int idx = is_x ? blockIdx.y : blockIdx.y - na;
+    double s = 0.0, c = 0.0;
     if (m < g.M) {
         const int k = m % g.n_r, j = m / g.n_r;
         const double omega0 = 2.0 * M_PI / (2.0 * g.n_r - 1.0);  // cryo_pft.m:49
         const double dtheta = 2.0 * M_PI / g.n_theta;             // cryo_pft.m:50
         const double f = is_x ? (k * omega0) * sin(j * dtheta) : (k * omega0) * cos(j * dtheta);
-        const double gt = idx == 4 && is_x ? 4.0 : ceil(-0.5 * g.n + idx);  // nudft2.m:40
-        double s, c;
-        sincos(f * gt, &s, &c);
-        out = make_double2(c, s);
+        sincos(f * idx, &s, &c);
     }
-    (is_x ? ax : ay)[(size_t)idx * g.Mp + m] = out;
+    double* t = tab + (size_t)(is_x ? 0 : 2) * na * g.Mp + (size_t)idx * g.Mp + m;
+    t[0] = c;
+    t[(size_t)na * g.Mp] = s;
 }
 
-// Staged stack: xt[(v*nup + u)*Kp + i] = p(u, v, k0 + i), zero-padded in u and
-// i.  One workgroup moves 64 pixel rows x 64 images through LDS so that both
-// the reads (along u) and the writes (along i) are contiguous.
+// Folded images, one 512-byte block per (column tile of 16 images, plane,
+// 4 values of a, b), the operand of one MFMA:
+//   xt[(((ct*4 + plane)*nab + a/4)*nh + b)*64 + (a%4)*16 + image%16],
+// planes ee, oo, oe (odd in u), eo; zero past nh and past the last image.
+// One workgroup folds FA columns a of the two rows +-b of 16 images: the rows
+// are read along u (contiguous) into LDS and written along the images.
 template <typename T>
-__global__ __launch_bounds__(256) void stage_kernel(Geo g, const T* __restrict__ img, long long k0, int K,
-                                                    double* __restrict__ xt) {
-    __shared__ double tile[64][65];
-    const int q0 = blockIdx.x * 64;  // staged pixel row
-    const int i0 = blockIdx.y * 64;  // image within the chunk
-    const int npix = g.n * g.nup;
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    for (int r = ty; r < 64; r += 4) {
-        const int i = i0 + r, q = q0 + tx;
-        double val = 0.0;
-        if (q < npix && i < g.Kc && k0 + i < K) {
-            const int v = q / g.nup, u = q - v * g.nup;
-            if (u < g.n) val = (double)img[(size_t)(k0 + i) * g.n * g.n + (size_t)v * g.n + u];
-        }
-        tile[r][tx] = val;
+__global__ __launch_bounds__(256) void fold_kernel(Geo g, const T* __restrict__ img, long long k0,
+                                                   double* __restrict__ xt) {
+    __shared__ double s_p[4][16][FA + 1];  // p(+a,+b), p(-a,+b), p(+a,-b), p(-a,-b), zero where not a pixel
+    const int a0 = blockIdx.x * FA, b = blockIdx.y, ct = blockIdx.z;
+    const int tid = threadIdx.x;
+    for (int x = tid; x < 4 * 16 * FA; x += 256) {
+        const int da = x % FA, i = (x / FA) % 16, q = x / (16 * FA);
+        const int a = a0 + da;
+        // the axes' own pixels count once
+        const int u = q & 1 ? g.c - a : g.c + a, v = q & 2 ? g.c - b : g.c + b;
+        const bool ok = u >= 0 && u < g.n && v >= 0 && v < g.n && 16 * ct + i < g.Kc && !((q & 1) && a == 0) &&
+                        !((q & 2) && b == 0);
+        s_p[q][i][da] = ok ? (double)img[((size_t)(k0 + 16 * ct + i) * g.n + v) * g.n + u] : 0.0;
     }
     __syncthreads();
-    for (int r = ty; r < 64; r += 4) {
-        const int q = q0 + r, i = i0 + tx;
-        if (q < npix && i < g.Kp) xt[(size_t)q * g.Kp + i] = tile[tx][r];
+    for (int x = tid; x < 16 * FA; x += 256) {
+        const int i = x % 16, da = x / 16;
+        const int a = a0 + da;
+        if (a >= 4 * g.nab) break;
+        const double pp = s_p[0][i][da], np = s_p[1][i][da], pn = s_p[2][i][da], nn = s_p[3][i][da];
+        const double ep = pp + np, op = pp - np, en = pn + nn, on = pn - nn;
+        const bool oa = a != 0, ob = b != 0;  // odd planes vanish on their axis
+        double* o = xt + (((size_t)ct * 4 * g.nab + (a >> 2)) * g.nh + b) * 64 + (a & 3) * 16 + i;
+        const size_t pl = (size_t)g.nab * g.nh * 64;
+        o[0] = ep + en;
+        o[pl] = oa && ob ? op - on : 0.0;
+        o[2 * pl] = oa ? op + on : 0.0;
+        o[3 * pl] = ob ? ep - en : 0.0;
     }
 }
 
@@ -121,80 +134,116 @@ __device__ inline void put<float2>(float2* pf, size_t at, double re, double im) 
     pf[at] = make_float2((float)re, (float)im);
 }
 
-// One workgroup: MB polar points x KB images (tile t of a 1-D grid; the tiles
-// a workgroup's XCD runs are contiguous, polar-point blocks fastest, so they
-// stream the same images through that XCD's L2); wave w takes points
-// [32w, 32w + 32) of the block as two 16-row tiles, each split into its real
-// and imaginary weight rows, against 4 column tiles of 16 images: 16
-// accumulator tiles (16 x 16 FP64 each).  Each step contracts 4 pixels (one
-// MFMA k-block): lane l holds pixel u0 + l/16 for point (l % 16) of a row
-// tile (A) and image (l % 16) of a column tile (B).  Along u the lane's
-// exponential factor advances by the rotation exp(+4i*fx(m)) (one complex
-// product); it restarts from the table at every v.  Staged pixels u >= n
-// are zero, so the factor's value there does not matter.
-template <typename OutT>
+// One workgroup: 16 RT quadrant points x 16 CT images; wave w contracts plane
+// w.  Each step is 4 folded pixels (4 values of a, one b): lane l holds pixel
+// a = l/16 of point l%16 of a row tile (A, the product of a table entry along
+// a, kept over the loop of b, and one along b) and of image l%16 of a column
+// tile (B, one contiguous 512-byte block); the next step's loads are issued
+// before this step's MFMAs.  RT x CT accumulator tiles of 16 x 16 FP64.  At
+// the end the four planes meet in LDS and every quadrant point gives its two
+// rays and their conjugate rays, written along the ray.
+// The 1-D grid gives each XCD (dispatch goes round-robin over 8) a contiguous
+// range of tiles, points fastest, so that its workgroups stream the same
+// images through its L2.
+// Bound: FP64 MFMA.  3.33 ms for 1000 images of 129 x 129, n_r = 65,
+// n_theta = 360: 63 TFLOP/s of the folded work (a large FP64 matrix product
+// reaches 72 here).  The unfolded contraction, 3.9 times the work, took 13.7 ms
+// at 57 TFLOP/s.  Smaller tiles than 4 x 4 only where they leave fewer MFMA
+// cycles on the busiest CU (few images or points).
+template <typename OutT, int RT, int CT>
 __global__ __launch_bounds__(256, 2) void pft_kernel(Geo g, const double* __restrict__ xt,
-                                                  const double2* __restrict__ ax, const double2* __restrict__ ay,
-                                                  OutT* __restrict__ pf, long long k0, int nmb, int ntiles,
-                                                  int per_xcd) {
-    const int b = blockIdx.x;
-    const int t = (b % 8) * per_xcd + b / 8;  // dispatch goes round-robin over the 8 XCDs
+                                                     const double* __restrict__ tab, OutT* __restrict__ pf,
+                                                     long long k0, int nmb, int ntiles, int per_xcd) {
+    __shared__ double s_s[4][16][16 * CT + 1];
+    const int t = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
     if (t >= ntiles) return;
     const int mb = t % nmb, kb = t / nmb;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    const int plane = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int r16 = lane & 15, kq = lane >> 4;
-    const int mA = mb * MB + wave * 32 + r16, mB = mA + 16;
-    const int ib = kb * KB;
-    d4 acc[2][2][4];
+    const int na = 4 * g.nab;
+    const double* tx = tab + (size_t)(plane == 1 || plane == 2) * na * g.Mp + (size_t)kq * g.Mp + mb * 16 * RT + r16;
+    const double* ty = tab + (size_t)(2 + (plane & 1)) * na * g.Mp + mb * 16 * RT + r16;
+    const double* bp[CT];
 #pragma unroll
-    for (int a = 0; a < 2; a++)
+    for (int c = 0; c < CT; c++) {
+        const int ct = min(kb * CT + c, g.nct - 1);  // past the last tile: that tile again, not stored
+        bp[c] = xt + ((size_t)ct * 4 + plane) * g.nab * g.nh * 64 + lane;
+    }
+    d4 acc[RT][CT];
 #pragma unroll
-        for (int b = 0; b < 2; b++)
+    for (int r = 0; r < RT; r++)
 #pragma unroll
-            for (int c = 0; c < 4; c++) acc[a][b][c] = d4{0.0, 0.0, 0.0, 0.0};
-    const double2 rA = ax[(size_t)4 * g.Mp + mA], rB = ax[(size_t)4 * g.Mp + mB];
-    const double2 x0A = ax[(size_t)kq * g.Mp + mA], x0B = ax[(size_t)kq * g.Mp + mB];
-    auto cmul = [](double2 p, double2 q) { return make_double2(p.x * q.x - p.y * q.y, p.x * q.y + p.y * q.x); };
-    for (int v = 0; v < g.n; v++) {
-        const double2 yA = ay[(size_t)v * g.Mp + mA], yB = ay[(size_t)v * g.Mp + mB];
-        double2 xA = x0A, xB = x0B;
-        const double* xr = xt + ((size_t)v * g.nup + kq) * g.Kp + ib + r16;
-        for (int u0 = 0; u0 < g.nup; u0 += 4) {
-            double bx[4];
+        for (int c = 0; c < CT; c++) acc[r][c] = d4{0.0, 0.0, 0.0, 0.0};
+    double y[RT], x[RT], bx[CT];
 #pragma unroll
-            for (int c = 0; c < 4; c++) bx[c] = xr[(size_t)u0 * g.Kp + 16 * c];
-            const double2 eA = cmul(xA, yA), eB = cmul(xB, yB);  // E = ax * ay
+    for (int c = 0; c < CT; c++) bx[c] = bp[c][0];
 #pragma unroll
-            for (int c = 0; c < 4; c++) {
-                acc[0][0][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(eA.x, bx[c], acc[0][0][c], 0, 0, 0);
-                acc[0][1][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(eA.y, bx[c], acc[0][1][c], 0, 0, 0);
-                acc[1][0][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(eB.x, bx[c], acc[1][0][c], 0, 0, 0);
-                acc[1][1][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(eB.y, bx[c], acc[1][1][c], 0, 0, 0);
+    for (int r = 0; r < RT; r++) y[r] = ty[16 * r];
+    const int steps = g.nab * g.nh;
+    int at = 0;
+    for (int ab = 0; ab < g.nab; ab++) {
+#pragma unroll
+        for (int r = 0; r < RT; r++) x[r] = tx[(size_t)4 * ab * g.Mp + 16 * r];
+        for (int b = 0; b < g.nh; b++) {
+            at++;
+            const size_t nx = at < steps ? (size_t)at * 64 : 0;
+            const int nb = b + 1 < g.nh ? b + 1 : 0;
+            double yn[RT], bn[CT];
+#pragma unroll
+            for (int c = 0; c < CT; c++) bn[c] = bp[c][nx];
+#pragma unroll
+            for (int r = 0; r < RT; r++) yn[r] = ty[(size_t)nb * g.Mp + 16 * r];
+#pragma unroll
+            for (int r = 0; r < RT; r++) {
+                const double w = x[r] * y[r];
+#pragma unroll
+                for (int c = 0; c < CT; c++)
+                    acc[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(w, bx[c], acc[r][c], 0, 0, 0);
             }
-            xA = cmul(xA, rA);
-            xB = cmul(xB, rB);
+#pragma unroll
+            for (int c = 0; c < CT; c++) bx[c] = bn[c];
+#pragma unroll
+            for (int r = 0; r < RT; r++) y[r] = yn[r];
         }
     }
-    // D tile layout of the FP64 16x16x4 MFMA: lane l, element t holds row
-    // 4*t + l/16, column l % 16 (one row per element, unlike the FP32 tiles).
+    // D tile layout of the FP64 16x16x4 MFMA: lane l, element e holds row
+    // 4*e + l/16, column l % 16 (one row per element, unlike the FP32 tiles).
     const int L = g.n_theta / 2;
 #pragma unroll
-    for (int a = 0; a < 2; a++)
+    for (int r = 0; r < RT; r++) {
+        __syncthreads();
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int m = mb * MB + wave * 32 + a * 16 + 4 * e + kq;
-            if (m >= g.M) continue;
+        for (int c = 0; c < CT; c++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) s_s[plane][4 * e + kq][16 * c + r16] = acc[r][c][e];
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < CT; q++) {
+            const int row = threadIdx.x & 15, col = (threadIdx.x >> 4) + 16 * q;
+            const int m = (mb * RT + r) * 16 + row, i = kb * 16 * CT + col;
+            if (m >= g.M || i >= g.Kc) continue;
             const int k = m % g.n_r, j = m / g.n_r;
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                const int i = ib + 16 * c + r16;
-                if (i >= g.Kc) continue;
-                const size_t img = (size_t)(k0 + i) * g.n_theta;
-                const double re = acc[a][0][c][e], im = acc[a][1][c][e];
-                put<OutT>(pf, (img + j) * g.n_r + k, re, im);
-                put<OutT>(pf, (img + j + L) * g.n_r + k, re, -im);
+            const double cc = s_s[0][row][col], ss = s_s[1][row][col], sc = s_s[2][row][col], cs = s_s[3][row][col];
+            const size_t ray = (size_t)(k0 + i) * g.n_theta;
+            put<OutT>(pf, (ray + j) * g.n_r + k, cc - ss, sc + cs);
+            put<OutT>(pf, (ray + j + L) * g.n_r + k, cc - ss, -(sc + cs));
+            if (j > 0 && 2 * j < L) {
+                put<OutT>(pf, (ray + L - j) * g.n_r + k, cc + ss, sc - cs);
+                put<OutT>(pf, (ray + 2 * L - j) * g.n_r + k, cc + ss, -(sc - cs));
             }
         }
+    }
+}
+
+template <int RT, int CT>
+void pft_launch(hipStream_t st, const Geo& g, bool c128, const double* xt, const double* tab, void* pf, long long k0) {
+    const int nmb = (g.M + 16 * RT - 1) / (16 * RT), ntiles = nmb * ((g.nct + CT - 1) / CT);
+    const int per = (ntiles + 7) / 8;
+    if (c128)
+        pft_kernel<double2, RT, CT><<<8 * per, 256, 0, st>>>(g, xt, tab, (double2*)pf, k0, nmb, ntiles, per);
+    else
+        pft_kernel<float2, RT, CT><<<8 * per, 256, 0, st>>>(g, xt, tab, (float2*)pf, k0, nmb, ntiles, per);
 }
 
 // ------------------------------------------------------------ type-2 NUFFT
@@ -359,48 +408,55 @@ int pft_run(clm_ctx* c, const clm_pft_params* p, const void* d_img, void* d_pf, 
     g.n = p->n;
     g.n_r = p->n_r;
     g.n_theta = p->n_theta;
-    g.M = p->n_r * (p->n_theta / 2);
-    g.Mp = (g.M + MB - 1) / MB * MB;
-    g.nup = (p->n + 3) / 4 * 4;
+    g.M = p->n_r * (p->n_theta / 4 + 1);
+    g.Mp = (g.M + 63) / 64 * 64;  // whole blocks of the tallest tile
+    g.c = p->n / 2;
+    g.nh = p->n / 2 + 1;
+    g.nab = (g.nh + 3) / 4;
     const int K = p->K;
     const int kc = K < KCHUNK ? K : KCHUNK;
-    const int kcp = (kc + KB - 1) / KB * KB;
     int rc;
-    if ((rc = ensure(c, c->pft_ax, (size_t)5 * g.Mp * sizeof(double2))) ||
-        (rc = ensure(c, c->pft_ay, (size_t)g.n * g.Mp * sizeof(double2))) ||
-        (rc = ensure(c, c->pft_xt, (size_t)g.n * g.nup * (size_t)kcp * sizeof(double))))
+    if ((rc = ensure(c, c->pft_ax, (size_t)16 * g.nab * g.Mp * sizeof(double))) ||
+        (rc = ensure(c, c->pft_xt, (size_t)((kc + 15) / 16) * 4 * g.nab * g.nh * 64 * sizeof(double))))
         return rc;
     hipEvent_t* ev = c->ev;
+    double* tab = (double*)c->pft_ax.p;
+    double* xt = (double*)c->pft_xt.p;
     HIPCHK(c, hipEventRecord(ev[0], c->stream));
-    tables_kernel<<<dim3(g.Mp / 256 + (g.Mp % 256 != 0), 5 + g.n), 256, 0, c->stream>>>(
-        g, (double2*)c->pft_ax.p, (double2*)c->pft_ay.p);
+    tables_kernel<<<dim3((g.Mp + 255) / 256, 8 * g.nab), 256, 0, c->stream>>>(g, tab);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipEventRecord(ev[1], c->stream));
     float ms_stage = 0.f, ms_pft = 0.f;
     int chunks = 0;
     for (long long k0 = 0; k0 < K; k0 += KCHUNK) {
         g.Kc = (int)((K - k0) < KCHUNK ? (K - k0) : KCHUNK);
-        g.Kp = (g.Kc + KB - 1) / KB * KB;
-        const int npix = g.n * g.nup;
-        dim3 sgrid((npix + 63) / 64, g.Kp / 64);
+        g.nct = (g.Kc + 15) / 16;
+        dim3 fgrid((4 * g.nab + FA - 1) / FA, g.nh, g.nct);
         HIPCHK(c, hipEventRecord(ev[2], c->stream));
         if (p->img_dtype == CLM_R64)
-            stage_kernel<double><<<sgrid, 256, 0, c->stream>>>(g, (const double*)d_img, k0, K, (double*)c->pft_xt.p);
+            fold_kernel<double><<<fgrid, 256, 0, c->stream>>>(g, (const double*)d_img, k0, xt);
         else
-            stage_kernel<float><<<sgrid, 256, 0, c->stream>>>(g, (const float*)d_img, k0, K, (double*)c->pft_xt.p);
+            fold_kernel<float><<<fgrid, 256, 0, c->stream>>>(g, (const float*)d_img, k0, xt);
         HIPCHK(c, hipGetLastError());
         HIPCHK(c, hipEventRecord(ev[3], c->stream));
-        const int nmb = g.Mp / MB, ntiles = nmb * (g.Kp / KB);
-        const int per = (ntiles + 7) / 8;
-        const dim3 grid(8 * per);
-        if (p->pf_dtype == CLM_C128)
-            pft_kernel<double2><<<grid, 256, 0, c->stream>>>(g, (const double*)c->pft_xt.p, (const double2*)c->pft_ax.p,
-                                                               (const double2*)c->pft_ay.p, (double2*)d_pf, k0, nmb,
-                                                               ntiles, per);
-        else
-            pft_kernel<float2><<<grid, 256, 0, c->stream>>>(g, (const double*)c->pft_xt.p, (const double2*)c->pft_ax.p,
-                                                              (const double2*)c->pft_ay.p, (float2*)d_pf, k0, nmb,
-                                                              ntiles, per);
+        // the tile whose busiest CU has the fewest cycles: 64 per MFMA, and
+        // about 24 per operand load of a step
+        const bool c128 = p->pf_dtype == CLM_C128;
+        const int rts[] = {4, 2, 1, 1}, cts[] = {4, 4, 4, 1};
+        int best = 0;
+        double cost = 0;
+        for (int q = 0; q < 4; q++) {
+            const long long tiles = (long long)((g.M + 16 * rts[q] - 1) / (16 * rts[q])) * ((g.nct + cts[q] - 1) / cts[q]);
+            const double cq = (double)((tiles + c->n_cu - 1) / c->n_cu) * (64 * rts[q] * cts[q] + 24 * (rts[q] + cts[q]));
+            if (q == 0 || cq < cost) {
+                cost = cq;
+                best = q;
+            }
+        }
+        if (best == 0) pft_launch<4, 4>(c->stream, g, c128, xt, tab, d_pf, k0);
+        else if (best == 1) pft_launch<2, 4>(c->stream, g, c128, xt, tab, d_pf, k0);
+        else if (best == 2) pft_launch<1, 4>(c->stream, g, c128, xt, tab, d_pf, k0);
+        else pft_launch<1, 1>(c->stream, g, c128, xt, tab, d_pf, k0);
         HIPCHK(c, hipGetLastError());
         HIPCHK(c, hipEventRecord(ev[4], c->stream));
         HIPCHK(c, hipEventSynchronize(ev[4]));
