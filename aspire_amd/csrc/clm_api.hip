@@ -4,6 +4,7 @@
 #include "clm_ctx.h"
 #include "clm_kernels.hip"
 #include "clm_clmap.h"
+#include "clm_search64.h"
 
 #include <algorithm>
 #include <cmath>
@@ -503,6 +504,17 @@ int prepare(clm_ctx* c, Plan& pl, int n, const clm_params* ps, const clm_stack_i
         d.npairs = j.P;
         d.filt = j.filt;
         d.wts = j.filt > 0 ? (const double*)B.W.p : nullptr;
+        d.eps64 = 4.0 * (g.R + 8.0) * 0x1p-53;
+        if (j.exact && g.sym) {
+            // what the phases of the paired shifts differ from conjugates
+            double dev = 0.0;
+            for (int e = 0; e < g.S; e++)
+                for (int r = 0; r < g.R; r++) {
+                    const double2 x = j.s.ph64[(size_t)e * g.R + r], y = j.s.ph64[(size_t)(g.S - 1 - e) * g.R + r];
+                    dev = std::max({dev, std::fabs(x.x - y.x), std::fabs(x.y + y.y)});
+                }
+            d.eps64 += 2.0 * dev;
+        }
     }
     for (Group& G : pl.groups) {
         long long base = 0;
@@ -750,6 +762,47 @@ int enqueue_exact(clm_ctx* c, Exact64Args ea, long long n_upper, int S) {
     return CLM_OK;
 }
 
+// FP64 search of the pairs of stack ti (all of them, or the list of a sel
+// group): on the FP64 matrix cores, with exact64_kernel for the pairs they
+// leave open (listed in ovf_list, which holds at least the group's pairs).
+int enqueue_search64(clm_ctx* c, const Plan& pl, int ti, Exact64Args ea, int* ovf_count,
+                     SlotRef* ovf_list) {
+    const StackDev& d = pl.table[ti];
+    const Geom& g = d.g;
+    Search64Args a{};
+    a.x = ea;
+    a.x.stack0 = ti;
+    a.x.nstacks = 1;
+    if (!ea.list) {
+        a.x.item0 = d.pair_base;
+        a.x.n_all = d.pair_base + d.npairs;
+    }
+    a.x.item_cap = d.npairs;
+    // units (shifts x row blocks) of a pair over several workgroups while the
+    // pairs alone leave the chip short of eight workgroups per CU
+    const long long units = (long long)g.NE * ((g.L + S64_ROWS - 1) / S64_ROWS);
+    const long long want = (8LL * c->n_cu + d.npairs - 1) / d.npairs;
+    a.x.sj = (int)std::max(1LL, std::min({want, units, (long long)EX_SJ}));
+    if (d.npairs > EX_CAP) a.x.sj = 1;
+    a.x.sv = (double*)c->ex_v.p;
+    a.x.sk = (long long*)c->ex_k.p;
+    a.ovf_count = ovf_count;
+    a.ovf_list = ovf_list;
+    int KS = 0;
+    const Search64Fn fn = pick_search64(g.R, g.L, g.sym != 0, KS);
+    const size_t lds = search64_lds(KS);
+    HIPCHK(c, hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(fn, dim3((unsigned)std::min<long long>(d.npairs, 16LL * c->n_cu), (unsigned)a.x.sj), dim3(256), lds,
+                       c->stream, a);
+    HIPCHK(c, hipGetLastError());
+    if (a.x.sj > 1) {
+        hipLaunchKernelGGL(search64_reduce_kernel, dim3((unsigned)((d.npairs + 255) / 256)), dim3(256), 0, c->stream,
+                           a);
+        HIPCHK(c, hipGetLastError());
+    }
+    return CLM_OK;
+}
+
 int enqueue_job(clm_ctx* c, const Plan& pl, bool timed, int phases = PHASE_ALL) {
     int rc;
     unsigned long long* ctr = (unsigned long long*)c->ctr.p;
@@ -786,8 +839,17 @@ int enqueue_job(clm_ctx* c, const Plan& pl, bool timed, int phases = PHASE_ALL) 
                 HIPCHK(c, hipGetLastError());
                 continue;
             }
+            // the fallback list is free until phase B: pairs the matrix cores
+            // leave open are listed there, counted in the group's own counter
+            int* const open = (int*)(ctr + 16 + GSTRIDE * gi);
+            SlotRef* const olist = (SlotRef*)c->fblist.p;
             int S = 1;
-            for (int i : G.members) S = std::max(S, pl.jobs[i].s.g.S);
+            for (int ti = G.first; ti < G.first + (int)G.members.size(); ti++) {
+                S = std::max(S, pl.table[ti].g.S);
+                if ((rc = enqueue_search64(c, pl, ti, ea, open, olist))) return rc;
+            }
+            ea.list = olist;
+            ea.n_dev = open;
             if ((rc = enqueue_exact(c, ea, G.P, S))) return rc;
             continue;
         }
@@ -950,7 +1012,9 @@ int enqueue_job(clm_ctx* c, const Plan& pl, bool timed, int phases = PHASE_ALL) 
         HIPCHK(c, hipGetLastError());
     }
     // pairs no pass could settle: FP64 exhaustive search
-    if (pl.P > 0) {
+    bool searched = false;
+    for (const Group& G : pl.groups) searched = searched || !G.exact;
+    if (pl.P > 0 && searched) {
         Exact64Args ea{};
         ea.stacks = dtab;
         ea.list = (const SlotRef*)c->fblist.p;

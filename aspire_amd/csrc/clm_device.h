@@ -75,6 +75,7 @@ struct StackDev {
     long long npairs;
     int filt;                 // map_filter_radius d (0: no map filter)
     const double* wts;        // (2d+1)^2 filter weights, row-major
+    double eps64;             // FP64 search: error bound of an MFMA sum per n1*n2
 };
 
 // Pass-2 / fallback list entry: (stack, slot)

@@ -20,8 +20,9 @@
 //                    candidate above a certified threshold).
 //   rescore_kernel   FP32 re-score of the surviving candidates, FP64
 //                    re-score of near ties, reference tie order.
-//   exact64_kernel   FP64 exhaustive search of one pair (fallback and the
-//                    CLM_FP64_REF path); the reference's own arithmetic.
+//   exact64_kernel   FP64 exhaustive search of one pair, the reference's own
+//                    arithmetic: the fallback of the other paths and of the
+//                    FP64 search (clm_search64.h).
 #include "clm_pair.h"
 
 namespace clm {
