@@ -179,6 +179,9 @@ constexpr int UCAP = 32768;
 
 // 64-bit counters per group after the 16 globals (see enqueue_job)
 constexpr int GSTRIDE = 8;
+// areas of counts after the groups' counters (a power of two); an
+// allocation-free call counts in the globals themselves
+constexpr int NSTAT = 32;
 // pass-1 work queues, one per XCD (workgroup b runs on XCD b % 8)
 constexpr int NQ = 8;
 
@@ -265,6 +268,11 @@ struct Plan {
     bool twin_lazy = false;
     bool twins_built = false;
 };
+
+// 64-bit words of a job's counters: 16 globals, GSTRIDE per group, the areas.
+size_t ctr_words(const clm_ctx* c, const Plan& pl) {
+    return 16 + GSTRIDE * pl.groups.size() + (c->arena ? 0 : (size_t)NSTAT * ST_STRIDE);
+}
 
 int enqueue_fill(clm_ctx* c, void* p, long long n, int v) {
     if (n <= 0) return CLM_OK;
@@ -524,8 +532,8 @@ int prepare(clm_ctx* c, Plan& pl, int n, const clm_params* ps, const clm_stack_i
         }
     }
     if ((rc = upload(c, c->table, pl.table))) return rc;
-    // shared buffers: counters (16 globals + GSTRIDE per group), lists, pass-2 tiles
-    if ((rc = ensure(c, c->ctr, (16 + GSTRIDE * pl.groups.size()) * sizeof(unsigned long long)))) return rc;
+    // shared buffers: counters, lists, pass-2 tiles
+    if ((rc = ensure(c, c->ctr, ctr_words(c, pl) * sizeof(unsigned long long)))) return rc;
     if ((rc = ensure(c, c->ulist, (size_t)std::max<long long>(ubase, 1) * sizeof(SlotRef)))) return rc;
     if ((rc = ensure(c, c->fblist, (size_t)std::max<long long>(pl.P, 1) * sizeof(SlotRef)))) return rc;
     long long gmax = 0;
@@ -762,6 +770,26 @@ int enqueue_exact(clm_ctx* c, Exact64Args ea, long long n_upper, int S) {
     return CLM_OK;
 }
 
+// Longest ray of a group's stacks.
+int longest_ray(const Plan& pl, const Group& G) {
+    int R = 1;
+    for (int ti = G.first; ti < G.first + (int)G.members.size(); ti++) R = std::max(R, pl.table[ti].g.R);
+    return R;
+}
+
+int launch_rescore(clm_ctx* c, const Plan& pl, unsigned grid, RescoreArgs a, int R) {
+    a.Rmax = R;
+    a.stat = (unsigned long long*)c->ctr.p;
+    a.stat_mask = 0;
+    if (!c->arena) {
+        a.stat += 16 + GSTRIDE * pl.groups.size();
+        a.stat_mask = NSTAT - 1;
+    }
+    hipLaunchKernelGGL(rescore_kernel, dim3(grid), dim3(256), rescore_lds_bytes(a.mode, R), c->stream, a);
+    HIPCHK(c, hipGetLastError());
+    return CLM_OK;
+}
+
 // FP64 search of the pairs of stack ti (all of them, or the list of a sel
 // group): on the FP64 matrix cores, with exact64_kernel for the pairs they
 // leave open (listed in ovf_list, which holds at least the group's pairs).
@@ -812,7 +840,7 @@ int enqueue_job(clm_ctx* c, const Plan& pl, bool timed, int phases = PHASE_ALL) 
     // 6 cells re-scored, 7 second-pass candidates; per group at 16+4g:
     // 0 pass-1 tile counter (one queue), 1 uncertain count, 2 pass-2 tile counter,
     // 3 pass-2 tiles, 4-7 pass-1 tile counters of the NQ XCD queues (int each)
-    if ((rc = enqueue_fill(c, ctr, 2 * (16 + GSTRIDE * (long long)pl.groups.size()), 0))) return rc;
+    if ((rc = enqueue_fill(c, ctr, 2 * (long long)ctr_words(c, pl), 0))) return rc;
     if (timed) HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
     if ((rc = enqueue_prep(c, pl))) return rc;
     if (timed) HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
@@ -910,12 +938,8 @@ int enqueue_job(clm_ctx* c, const Plan& pl, bool timed, int phases = PHASE_ALL) 
         ra.unc_list = ul;
         ra.fb_count = (int*)(ctr + 4);
         ra.fb_list = (SlotRef*)c->fblist.p;
-        ra.n64 = ctr + 1;
-        ra.ncell = ctr + 6;
-        ra.nemit = ctr + 7;
         const unsigned rgrid = (unsigned)std::min<long long>((G.P + 3) / 4, (long long)c->n_cu * 16);
-        hipLaunchKernelGGL(rescore_kernel, dim3(rgrid), dim3(256), 0, c->stream, ra);
-        HIPCHK(c, hipGetLastError());
+        if ((rc = launch_rescore(c, pl, rgrid, ra, longest_ray(pl, G)))) return rc;
     }
     }  // phase A
     if (!(phases & PHASE_B)) return CLM_OK;
@@ -961,12 +985,8 @@ int enqueue_job(clm_ctx* c, const Plan& pl, bool timed, int phases = PHASE_ALL) 
             rt.unc_list = (SlotRef*)c->ulist.p + T.ubase;
             rt.fb_count = (int*)(ctr + 4);
             rt.fb_list = (SlotRef*)c->fblist.p;
-            rt.n64 = ctr + 1;
-            rt.ncell = ctr + 6;
-            rt.nemit = ctr + 7;
             const unsigned rg = (unsigned)std::min<long long>((G0.P + 3) / 4, (long long)c->n_cu * 16);
-            hipLaunchKernelGGL(rescore_kernel, dim3(rg), dim3(256), 0, c->stream, rt);
-            HIPCHK(c, hipGetLastError());
+            if ((rc = launch_rescore(c, pl, rg, rt, longest_ray(pl, T)))) return rc;
             gi = (size_t)G0.twin;
         }
         const Group& G = pl.groups[gi];
@@ -978,9 +998,6 @@ int enqueue_job(clm_ctx* c, const Plan& pl, bool timed, int phases = PHASE_ALL) 
         ra.nstacks = (int)G.members.size();
         ra.fb_count = (int*)(ctr + 4);
         ra.fb_list = (SlotRef*)c->fblist.p;
-        ra.n64 = ctr + 1;
-        ra.ncell = ctr + 6;
-        ra.nemit = ctr + 7;
         const int cap = (int)std::min<long long>(G.P, pl.n_unc_cap);
         hipLaunchKernelGGL(build_pass2_kernel, dim3((unsigned)std::min<long long>((G.P + 255) / 256, 1024)),
                            dim3(256), 0, c->stream, dtab, (const int*)(cg + 1), (const SlotRef*)ul, cap,
@@ -1008,8 +1025,7 @@ int enqueue_job(clm_ctx* c, const Plan& pl, bool timed, int phases = PHASE_ALL) 
         ra.ulist = ul;
         ra.erecs = (const EmitRec*)c->erecs.p;
         const unsigned rg2 = (unsigned)std::min<long long>((cap + 3) / 4, (long long)c->n_cu * 16);
-        hipLaunchKernelGGL(rescore_kernel, dim3(rg2), dim3(256), 0, c->stream, ra);
-        HIPCHK(c, hipGetLastError());
+        if ((rc = launch_rescore(c, pl, rg2, ra, longest_ray(pl, G)))) return rc;
     }
     // pairs no pass could settle: FP64 exhaustive search
     bool searched = false;
@@ -1030,13 +1046,17 @@ int enqueue_job(clm_ctx* c, const Plan& pl, bool timed, int phases = PHASE_ALL) 
 // Add a finished plan's counters to st (which the caller cleared).
 int add_stats(clm_ctx* c, const Plan& pl, clm_stats* st) {
     if (!st || pl.P == 0) return CLM_OK;
-    std::vector<unsigned long long> h(16 + GSTRIDE * pl.groups.size());
+    std::vector<unsigned long long> h(ctr_words(c, pl));
     HIPCHK(c, hipMemcpy(h.data(), c->ctr.p, h.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost));
     auto as_int = [](unsigned long long x) { return (int64_t)(int)(unsigned)(x & 0xffffffffu); };
     st->small_norm_lines += (int64_t)h[0];
-    st->fp64_candidates += (int64_t)h[1];
-    st->cells_rescored += (int64_t)h[6];
-    st->emitted += (int64_t)h[7];
+    // the globals, then the areas
+    const size_t first = 16 + GSTRIDE * pl.groups.size();
+    for (size_t o = 0; o < h.size(); o = o == 0 ? first : o + ST_STRIDE) {
+        st->fp64_candidates += (int64_t)h[o + ST_64];
+        st->cells_rescored += (int64_t)h[o + ST_CELL];
+        st->emitted += (int64_t)h[o + ST_EMIT];
+    }
     st->fallback_pairs += as_int(h[4]);
     for (size_t gi = 0; gi < pl.groups.size(); gi++) {
         const Group& G = pl.groups[gi];
@@ -1080,7 +1100,7 @@ int run_plan(clm_ctx* c, Plan& pl, bool timed, clm_stats* st) {
         bool any = false;
         for (const Group& G : pl.groups) any = any || G.twin >= 0;
         if (any) {
-            std::vector<unsigned long long> h(16 + GSTRIDE * pl.groups.size());
+            std::vector<unsigned long long> h(ctr_words(c, pl));
             HIPCHK(c, hipMemcpyAsync(h.data(), c->ctr.p, h.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost,
                                      c->stream));
             HIPCHK(c, hipStreamSynchronize(c->stream));

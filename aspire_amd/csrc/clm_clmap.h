@@ -132,7 +132,7 @@ __global__ __launch_bounds__(256) void clmap_kernel(ClmapArgs a) {
                         for (int i = 0; i < w; i++)
                             for (int jx = 0; jx < w; jx++) v = v + sd.wts[i * w + jx] * sM[oi + i][oj + jx];
                         if (isnan(v)) continue;
-                        const long long key = ((long long)j * L2 + c) * L + l1;
+                        const long long key = tie_key(j, c, l1);
                         if (better64(v, key, bv, bk)) {
                             bv = v;
                             bk = key;

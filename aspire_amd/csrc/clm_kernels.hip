@@ -163,16 +163,26 @@ struct RescoreArgs {
     SlotRef* unc_list;
     int* fb_count;            // both: pairs for the FP64 exhaustive search
     SlotRef* fb_list;
-    unsigned long long* n64;  // FP64 re-scored candidates (stats)
-    unsigned long long* ncell;  // cells re-scored (stats)
-    unsigned long long* nemit;  // second-pass candidates (stats)
+    unsigned long long* stat;  // counts, one area per workgroup & stat_mask: ST_* of it
+    int stat_mask;
+    int Rmax;                 // longest ray of the stacks served (LDS rows)
 };
 
+// Counts of a job: areas of ST_STRIDE words (a cache line), which the host
+// adds up.  An atomic on one address takes 11 ns wherever it comes from, so
+// workgroups that end together are spread over areas.
+constexpr int ST_STRIDE = 16;
+constexpr int ST_64 = 1, ST_CELL = 6, ST_EMIT = 7;  // FP64 candidates, cells, second-pass candidates
+
 // Order key of the reference's tie rule (shift index first, then the column
-// of [C1 C2], then the row): smaller key wins among equal values.
-__device__ inline long long tie_key(int j, int l2p, int l1, int L) {
-    return ((long long)j * (2 * L) + l2p) * L + l1;
+// of [C1 C2], then the row): smaller key wins among equal values.  Packed in
+// fields (S <= 4096, L <= 768), so that a key comes apart without divisions.
+__device__ inline long long tie_key(int j, int l2p, int l1) {
+    return ((long long)j << 32) | (unsigned)(l2p << 16 | l1);
 }
+__device__ inline int key_l1(long long key) { return (int)key & 0xffff; }
+__device__ inline int key_l2p(long long key) { return (int)((unsigned)key >> 16); }
+__device__ inline int key_j(long long key) { return (int)(key >> 32); }
 
 __device__ inline bool better(float v, long long k, float bv, long long bk) {
     return v > bv || (v == bv && k < bk);
@@ -209,21 +219,43 @@ __device__ inline int find_stack(const StackDev* st, int n, long long item) {
     return lo;
 }
 
+// x / d and x mod d by the reciprocal inv = 1/d, corrected: exact for
+// 0 <= x < 2^24 (rows and cells of a map are below 7 million), a third of the
+// instructions of an integer division.
+__device__ inline int div_by(int x, int d, float inv, int& rem) {
+    int q = (int)((float)x * inv);
+    int r = x - q * d;
+    if (r < 0) { q--; r += d; }
+    if (r >= d) { q++; r -= d; }
+    rem = r;
+    return q;
+}
+
+// Geometry of a stack and its reciprocals, in registers.
+struct CandGeom {
+    int L, Lp, NCT, NROWS;
+    float iL, iNCT;
+};
+__device__ inline CandGeom cand_geom(const Geom& g) {
+    return CandGeom{g.L, g.Lp, g.NCT, g.NROWS, 1.0f / g.L, 1.0f / g.NCT};
+}
+
 // Decode candidate q of a pair: pass-1 cells expand to 16 rows each,
 // pass-2 lists hold (row, col) directly.  row = -1 marks padding.
-__device__ inline void cand_rc(const Geom& g, int mode, const PairRec& rec, const EmitRec* er,
+__device__ inline void cand_rc(const CandGeom& g, int mode, const PairRec& rec, const EmitRec* er,
                                int q, int& row, int& col) {
     if (mode == 0) {
         const uint32_t c = rec.cell[q >> 4];
         const int cl = c & 63, cid = c >> 6;
-        const int at = cid / g.NCT, ct = cid % g.NCT;
+        int ct;
+        const int at = div_by(cid, g.NCT, g.iNCT, ct);
         const int ri = q & 15;
         row = at * 32 + 8 * (ri >> 2) + 4 * (cl >> 5) + (ri & 3);
         col = ct * 32 + (cl & 31);
     } else {
         const uint32_t c = er->cand[q];
-        row = (int)(c / g.Lp);
-        col = (int)(c % g.Lp);
+        row = (int)(c / (unsigned)g.Lp);
+        col = (int)(c - (unsigned)row * (unsigned)g.Lp);
     }
     if (row >= g.NROWS || col >= g.L) row = -1;
 }
@@ -234,13 +266,13 @@ __device__ inline void cand_rc(const Geom& g, int mode, const PairRec& rec, cons
 // whole wave with a wave-uniform key; the result is the same in every lane.
 __device__ inline double eval64(const StackDev& sd, int k1, int k2, long long key, int lane) {
     const Geom& g = sd.g;
-    const int l1 = (int)(key % g.L);
-    const int l2p = (int)((key / g.L) % (2 * g.L));
-    const int j = (int)(key / ((long long)g.L * 2 * g.L));
+    const int l1 = key_l1(key);
+    const int l2p = key_l2p(key);
+    const int j = key_j(key);
     const double2* P1 = sd.P64 + ((size_t)k1 * g.L + l1) * g.R;
-    const double2* P2 = sd.P64 + ((size_t)k2 * g.L + (l2p % g.L)) * g.R;
-    const double2* ph = sd.ph64 + (size_t)j * g.R;
     const bool flip = l2p >= g.L;
+    const double2* P2 = sd.P64 + ((size_t)k2 * g.L + (flip ? l2p - g.L : l2p)) * g.R;
+    const double2* ph = sd.ph64 + (size_t)j * g.R;
     double acc = 0.0;
     for (int c0 = 0; c0 < g.R; c0 += 64) {
         const int r = c0 + lane;
@@ -254,9 +286,9 @@ __device__ inline double eval64(const StackDev& sd, int k1, int k2, long long ke
 __device__ inline void write_result(const StackDev& sd, int slot, double v, long long key) {
     const Geom& g = sd.g;
     if (v > 0.0) {
-        const int l1 = (int)(key % g.L);
-        const int l2p = (int)((key / g.L) % (2 * g.L));
-        const int j = (int)(key / ((long long)g.L * 2 * g.L));
+        const int l1 = key_l1(key);
+        const int l2p = key_l2p(key);
+        const int j = key_j(key);
         if (sd.cl1) sd.cl1[slot] = l1 + 1;
         if (sd.cl2) sd.cl2[slot] = l2p + 1;
         if (sd.jidx) sd.jidx[slot] = j;
@@ -272,22 +304,40 @@ __device__ inline void write_result(const StackDev& sd, int slot, double v, long
 }
 
 constexpr int RS_MAXV = 2 * MAXE;  // FP32 values kept per pair (2 per row)
+constexpr int RS_NB = 4;           // FP64 candidates evaluated together
 
-// One wave per pair.  FP32 re-score with 4 lanes per candidate row (16 rows
+// Dynamic LDS of rescore_kernel: per wave the FP32 values of a pair (cells of
+// the first pass, or a second-pass list), then the FP64 terms and keys of
+// RS_NB candidates (R terms each, rows of an odd number of doubles).
+__host__ __device__ inline int rescore_nval(int mode) { return mode == 1 ? RS_MAXV : 2 * 16 * MAXC; }
+__host__ __device__ inline size_t rescore_lds_bytes(int mode, int R) {
+    return 4 * ((size_t)rescore_nval(mode) * 4 + (size_t)RS_NB * (R | 1) * 8 + RS_NB * 8);
+}
+
+// One wave per pair.  FP32 re-score with 4 lanes per candidate row (32 rows
 // per step, the row's lanes reading adjacent 16-byte pieces), values kept in
 // LDS; then FP64 re-score of every candidate within tau of the FP32 best,
-// the whole wave on one candidate (one lane per term, the terms added in
-// the oracle's order).
-__global__ __launch_bounds__(256) void rescore_kernel(RescoreArgs a) {
-    __shared__ float s_val[4][RS_MAXV];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// RS_NB at a time: a lane per term, all their loads in flight together, and
+// the terms of each added by one lane in the oracle's order.
+// Bound by the L1 accesses of the row loads where there are many pairs (3.1 ms
+// for 499,500 pairs with 6.8 cells each at n_r = 45; 3.4 with one candidate
+// per step in FP64, divisions to take a tie key apart and one counter for
+// all), by latency where there are few (54 us for 780 pairs, was 69).
+__global__ __launch_bounds__(256, 4) void rescore_kernel(RescoreArgs a) {
+    extern __shared__ __align__(16) char s_rs[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int W = blockDim.x >> 6;
-    float* sval = s_val[wave];
-    const int q = lane & 3, rl = lane >> 2;  // k-quarter, row within the step
+    const int nvmax = rescore_nval(a.mode);
+    const int ldt = a.Rmax | 1;
+    double* const sterm = (double*)s_rs + (size_t)wave * RS_NB * ldt;
+    long long* const skey = (long long*)((double*)s_rs + (size_t)4 * RS_NB * ldt) + wave * RS_NB;
+    float* const sval = (float*)((long long*)((double*)s_rs + (size_t)4 * RS_NB * ldt) + 4 * RS_NB) + (size_t)wave * nvmax;
+    const int q = lane & 3, rl = lane >> 2;  // k-quarter, row within a set of 16
     const bool listed = a.mode != 0, emit = a.mode == 1;
     const long long n_items = listed ? (long long)min(*a.n_items_dev, a.item_cap) : a.n_items;
-    // statistics, summed in lane 0 over the wave's items and added once at
-    // the end: an atomic per pair on one address serialises across the chip
+    // counts, summed over the workgroup's items and added once at the end
+    __shared__ unsigned long long s_cnt[3][4];
     unsigned long long c_cell = 0, c_emit = 0, c_64 = 0;
     for (long long item = (long long)blockIdx.x * W + wave; item < n_items; item += (long long)gridDim.x * W) {
         int stk, slot;
@@ -302,6 +352,7 @@ __global__ __launch_bounds__(256) void rescore_kernel(RescoreArgs a) {
         // through sd, so references into it would be re-read on every row
         const StackDev& sd = a.stacks[__builtin_amdgcn_readfirstlane(stk)];
         const Geom g = sd.g;
+        const CandGeom cg = cand_geom(g);
         const float2* const P32 = sd.P32;
         const float2* const ph32 = sd.ph32;
         const int kq = g.Rp / 4;  // multiple of 4
@@ -332,57 +383,71 @@ __global__ __launch_bounds__(256) void rescore_kernel(RescoreArgs a) {
         // ---- FP32 re-score
         float bv = -INFINITY;
         long long bk = 0x7fffffffffffffffLL;
-        for (int base = 0; base < nrows; base += 16) {
-            const int r = base + rl;
-            int row = -1, col = 0;
-            if (r < nrows) cand_rc(g, cmode, rec, er, r, row, col);
-            float X = 0.f, Y = 0.f;
-            int e = 0, l1 = 0;
-            if (row >= 0) {
-                e = row / g.L;
-                l1 = row - e * g.L;
+        for (int base = 0; base < nrows; base += 32) {
+            int row[2], col[2], e[2], l1[2];
+            const float4 *p[2], *bb[2], *ph[2];
+            float X[2] = {0.f, 0.f}, Y[2] = {0.f, 0.f};
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const int r = base + 16 * u + rl;
+                row[u] = -1;
+                col[u] = 0;
+                if (r < nrows) cand_rc(cg, cmode, rec, er, r, row[u], col[u]);
+                const int rc = row[u] < 0 ? 0 : row[u];  // rows without a candidate read row 0, unused
+                if (row[u] < 0) col[u] = 0;
+                e[u] = div_by(rc, cg.L, cg.iL, l1[u]);
                 // the 4 lanes of a row read 4 adjacent 16-byte pieces per
                 // load (lane q: pieces q, q + 4, ...), so one load touches
                 // 16 half cache lines instead of 64 lines
-                const float4* p = (const float4*)(P32 + ((size_t)k1 * g.L + l1) * g.Rp) + q;
-                const float4* bb = (const float4*)(P32 + ((size_t)k2 * g.L + col) * g.Rp) + q;
-                const float4* ph = (const float4*)(ph32 + (size_t)e * g.Rp) + q;
-#pragma unroll 4
-                for (int i = 0; i < kq / 2; i++) {
-                    const float4 pv = p[4 * i], qv = ph[4 * i], b4 = bb[4 * i];
+                p[u] = (const float4*)(P32 + ((size_t)k1 * g.L + l1[u]) * g.Rp) + q;
+                bb[u] = (const float4*)(P32 + ((size_t)k2 * g.L + col[u]) * g.Rp) + q;
+                ph[u] = (const float4*)(ph32 + (size_t)e[u] * g.Rp) + q;
+            }
+            const int nu = base + 16 < nrows ? 2 : 1;
+#pragma unroll 2
+            for (int i = 0; i < kq / 2; i++) {
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    if (u >= nu) break;
+                    const float4 pv = p[u][4 * i], qv = ph[u][4 * i], b4 = bb[u][4 * i];
                     const float ar0 = fmaf(pv.x, qv.x, -pv.y * qv.y);
                     const float ai0 = fmaf(pv.x, qv.y, pv.y * qv.x);
                     const float ar1 = fmaf(pv.z, qv.z, -pv.w * qv.w);
                     const float ai1 = fmaf(pv.z, qv.w, pv.w * qv.z);
-                    X = fmaf(ar0, b4.x, X);
-                    Y = fmaf(ai0, b4.y, Y);
-                    X = fmaf(ar1, b4.z, X);
-                    Y = fmaf(ai1, b4.w, Y);
+                    X[u] = fmaf(ar0, b4.x, X[u]);
+                    Y[u] = fmaf(ai0, b4.y, Y[u]);
+                    X[u] = fmaf(ar1, b4.z, X[u]);
+                    Y[u] = fmaf(ai1, b4.w, Y[u]);
                 }
             }
-            X += __shfl_xor(X, 1, 64);
-            Y += __shfl_xor(Y, 1, 64);
-            X += __shfl_xor(X, 2, 64);
-            Y += __shfl_xor(Y, 2, 64);
-            float v1 = -INFINITY, v2 = -INFINITY;
-            long long q1 = 0x7fffffffffffffffLL, q2 = 0x7fffffffffffffffLL;
-            if (row >= 0) {
-                if (g.sym) {
-                    v1 = 2.f * (X + Y); q1 = tie_key(e, col, l1, g.L);
-                    v2 = 2.f * (X - Y); q2 = tie_key(g.S - 1 - e, g.L + col, l1, g.L);
-                } else if (e < g.S) {
-                    v1 = 2.f * (X + Y); q1 = tie_key(e, col, l1, g.L);
-                } else {
-                    // rows e >= S carry the phase of -s_{e-S}: C2(s_{e-S}) = 2(X - Y)
-                    v2 = 2.f * (X - Y); q2 = tie_key(e - g.S, g.L + col, l1, g.L);
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                if (u >= nu) break;
+                X[u] += __shfl_xor(X[u], 1, 64);
+                Y[u] += __shfl_xor(Y[u], 1, 64);
+                X[u] += __shfl_xor(X[u], 2, 64);
+                Y[u] += __shfl_xor(Y[u], 2, 64);
+                float v1 = -INFINITY, v2 = -INFINITY;
+                long long q1 = 0x7fffffffffffffffLL, q2 = 0x7fffffffffffffffLL;
+                if (row[u] >= 0) {
+                    if (g.sym) {
+                        v1 = 2.f * (X[u] + Y[u]); q1 = tie_key(e[u], col[u], l1[u]);
+                        v2 = 2.f * (X[u] - Y[u]); q2 = tie_key(g.S - 1 - e[u], g.L + col[u], l1[u]);
+                    } else if (e[u] < g.S) {
+                        v1 = 2.f * (X[u] + Y[u]); q1 = tie_key(e[u], col[u], l1[u]);
+                    } else {
+                        // rows e >= S carry the phase of -s_{e-S}: C2(s_{e-S}) = 2(X - Y)
+                        v2 = 2.f * (X[u] - Y[u]); q2 = tie_key(e[u] - g.S, g.L + col[u], l1[u]);
+                    }
                 }
+                const int r = base + 16 * u + rl;
+                if (q == 0 && r < nrows && 2 * r + 1 < nvmax) {
+                    sval[2 * r] = v1;
+                    sval[2 * r + 1] = v2;
+                }
+                if (better(v1, q1, bv, bk)) { bv = v1; bk = q1; }
+                if (better(v2, q2, bv, bk)) { bv = v2; bk = q2; }
             }
-            if (q == 0 && r < nrows && 2 * r + 1 < RS_MAXV) {
-                sval[2 * r] = v1;
-                sval[2 * r + 1] = v2;
-            }
-            if (better(v1, q1, bv, bk)) { bv = v1; bk = q1; }
-            if (better(v2, q2, bv, bk)) { bv = v2; bk = q2; }
         }
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) {
@@ -395,31 +460,67 @@ __global__ __launch_bounds__(256) void rescore_kernel(RescoreArgs a) {
         if (sd.fp64 && bv > -INFINITY) {
             __builtin_amdgcn_wave_barrier();
             // ---- FP64 re-score of every candidate within tau of the FP32
-            // best, one candidate at a time across the wave (the best by
-            // value, then tie key, does not depend on the visiting order)
+            // best (the best by value, then tie key, does not depend on the
+            // visiting order)
             const float lim = bv - sd.tau;
             double b64 = -INFINITY;
             long long k64 = 0x7fffffffffffffffLL;
-            int n64 = 0;
-            const int nv = min(2 * nrows, RS_MAXV);
+            const int nv = min(2 * nrows, nvmax);
+            const double2* const P1 = sd.P64 + (size_t)k1 * g.L * g.R;
+            const double2* const P2 = sd.P64 + (size_t)k2 * g.L * g.R;
+            const double2* const ph64 = sd.ph64;
             for (int base = 0; base < nv; base += 64) {
-                const int iv = base + lane;
-                unsigned long long mask = __ballot(iv < nv && sval[iv] >= lim);
-                while (mask) {
-                    const int ic = base + __builtin_ctzll(mask);
-                    mask &= mask - 1;
-                    int row, col;
-                    cand_rc(g, cmode, rec, er, ic >> 1, row, col);
-                    const int e = row / g.L, l1 = row - e * g.L;
-                    long long key;
-                    if (g.sym) key = (ic & 1) ? tie_key(g.S - 1 - e, g.L + col, l1, g.L) : tie_key(e, col, l1, g.L);
-                    else key = e < g.S ? tie_key(e, col, l1, g.L) : tie_key(e - g.S, g.L + col, l1, g.L);
-                    const double v = eval64(sd, k1, k2, key, lane);
-                    n64++;
-                    if (!isnan(v) && better64(v, key, b64, k64)) { b64 = v; k64 = key; }
+                const int ic = base + lane;
+                const bool on = ic < nv && sval[ic] >= lim;
+                const unsigned long long mask = __ballot(on);
+                const int n = __popcll(mask);
+                c_64 += (unsigned long long)n;
+                const int pos = __popcll(mask & lanemask_lt());
+                for (int c0 = 0; c0 < n; c0 += RS_NB) {
+                    if (on && pos >= c0 && pos < c0 + RS_NB) {
+                        int row, col;
+                        cand_rc(cg, cmode, rec, er, ic >> 1, row, col);
+                        int l1;
+                        const int e = div_by(row, cg.L, cg.iL, l1);
+                        long long key;
+                        if (g.sym) key = (ic & 1) ? tie_key(g.S - 1 - e, g.L + col, l1) : tie_key(e, col, l1);
+                        else key = e < g.S ? tie_key(e, col, l1) : tie_key(e - g.S, g.L + col, l1);
+                        skey[pos - c0] = key;
+                    }
+                    __builtin_amdgcn_wave_barrier();
+                    const int nb = min(RS_NB, n - c0);
+#pragma unroll
+                    for (int c = 0; c < RS_NB; c++) {
+                        if (c >= nb) break;
+                        const long long key = skey[c];
+                        const int l1 = key_l1(key);
+                        const int l2p = key_l2p(key);
+                        const int j = key_j(key);
+                        const bool flip = l2p >= g.L;
+                        const double2* a1 = P1 + (size_t)l1 * g.R;
+                        const double2* a2 = P2 + (size_t)(flip ? l2p - g.L : l2p) * g.R;
+                        const double2* aq = ph64 + (size_t)j * g.R;
+                        for (int r = lane; r < g.R; r += 64) sterm[c * ldt + r] = term64(a1[r], aq[r], a2[r], flip);
+                    }
+                    __builtin_amdgcn_wave_barrier();
+                    if (lane < nb) {
+                        double acc = 0.0;
+                        const double* t = sterm + lane * ldt;
+                        for (int r = 0; r < g.R; r++) acc = acc + t[r];
+                        const double v = 2.0 * acc;
+                        const long long key = skey[lane];
+                        if (!isnan(v) && better64(v, key, b64, k64)) { b64 = v; k64 = key; }
+                    }
+                    __builtin_amdgcn_wave_barrier();
                 }
             }
-            c_64 += (unsigned long long)n64;
+            // lanes 0..RS_NB-1 hold the bests of their candidates
+#pragma unroll
+            for (int o = RS_NB / 2; o > 0; o >>= 1) {
+                const double ov = __shfl_xor(b64, o, 64);
+                const long long ok = __shfl_xor(k64, o, 64);
+                if (better64(ov, ok, b64, k64)) { b64 = ov; k64 = ok; }
+            }
             fv = b64;
             fk = k64;
         }
@@ -427,9 +528,16 @@ __global__ __launch_bounds__(256) void rescore_kernel(RescoreArgs a) {
         __builtin_amdgcn_wave_barrier();
     }
     if (lane == 0) {
-        if (a.ncell && c_cell) atomicAdd(a.ncell, c_cell);
-        if (a.nemit && c_emit) atomicAdd(a.nemit, c_emit);
-        if (a.n64 && c_64) atomicAdd(a.n64, c_64);
+        s_cnt[0][wave] = c_64;
+        s_cnt[1][wave] = c_cell;
+        s_cnt[2][wave] = c_emit;
+    }
+    __syncthreads();
+    if (threadIdx.x < 3) {
+        unsigned long long n = 0;
+        for (int w = 0; w < W; w++) n += s_cnt[threadIdx.x][w];
+        const int at = threadIdx.x == 0 ? ST_64 : threadIdx.x == 1 ? ST_CELL : ST_EMIT;
+        if (n) atomicAdd(a.stat + (size_t)(blockIdx.x & a.stat_mask) * ST_STRIDE + at, n);
     }
 }
 
@@ -465,7 +573,7 @@ __global__ void build_pass2_kernel(const StackDev* stacks, const int* n_unc, con
 // is bit-identical to the oracle's.  Computed as 64 x 64 output tiles (rows
 // l1, columns l2 of one map) with 16 outputs per thread and the operands of
 // 32 consecutive r staged in LDS.  The best (value, tie key) wins; the key
-// q = (j*2L + l2p)*L + l1 is the reference's first-max order.
+// is the reference's first-max order.
 struct Exact64Args {
     const StackDev* stacks;   // the whole table (SlotRef.stack indexes it)
     int stack0, nstacks;      // without a list: stacks [stack0, stack0 + nstacks)
@@ -570,7 +678,7 @@ __global__ __launch_bounds__(256) void exact64_kernel(Exact64Args a) {
                                 const int l1 = rt * 64 + ty + 16 * i, l2 = ct * 64 + tx + 16 * k;
                                 if (l1 < L && l2 < L) {
                                     const double v = 2.0 * acc[i][k];
-                                    const long long key = tie_key(j, l2 + m * L, l1, L);
+                                    const long long key = tie_key(j, l2 + m * L, l1);
                                     if (!isnan(v) && better64(v, key, bv, bk)) { bv = v; bk = key; }
                                 }
                             }

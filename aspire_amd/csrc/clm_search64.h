@@ -203,7 +203,7 @@ __global__ __launch_bounds__(256, (KS * CT * 4 + CT * 16 <= 200 ? 2 : 1)) void s
                                     const int j = SYM ? (minus ? S - 1 - e : e) : (flip ? e - S : e);
                                     if (pos < S64_LIST) {
                                         lv[pos] = v;
-                                        lk[pos] = tie_key(j, minus ? L + l2 : l2, l1, L);
+                                        lk[pos] = tie_key(j, minus ? L + l2 : l2, l1);
                                     }
                                 }
                                 if (wc + cnt > S64_LIST) lost = true;
