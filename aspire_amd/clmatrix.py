@@ -88,11 +88,11 @@ def clmatrix_records(pf, max_shift=15, shift_step=1.0, precision="fp16", device=
         base, dt, n_r, n_theta, K = _device_view(pf)
         P = max(K * (K - 1) // 2, 0)
         dev = base.device
-        out = dict(cl1=torch.zeros(P, dtype=torch.int32, device=dev),
-                   cl2=torch.zeros(P, dtype=torch.int32, device=dev),
-                   j=torch.zeros(P, dtype=torch.int32, device=dev),
-                   corr=torch.zeros(P, dtype=torch.float64, device=dev),
-                   shift=torch.zeros(P, dtype=torch.float64, device=dev))
+        out = dict(cl1=torch.empty(P, dtype=torch.int32, device=dev),
+                   cl2=torch.empty(P, dtype=torch.int32, device=dev),
+                   j=torch.empty(P, dtype=torch.int32, device=dev),
+                   corr=torch.empty(P, dtype=torch.float64, device=dev),
+                   shift=torch.empty(P, dtype=torch.float64, device=dev))
         p = _params(n_r, n_theta, K, dt, max_shift, shift_step, precision, verbose, tie_margin, variant,
                     flags)
         # torch's own queue must be done with pf before libclm's stream reads it
@@ -185,11 +185,11 @@ def clmatrix_grouped(pfs, max_shift=15, shift_step=1.0, precision="fp16", device
         P = max(K * (K - 1) // 2, 0)
         dev = base.device
         o = out[i] if out is not None else dict(
-            cl1=torch.zeros(P, dtype=torch.int32, device=dev),
-            cl2=torch.zeros(P, dtype=torch.int32, device=dev),
-            j=torch.zeros(P, dtype=torch.int32, device=dev),
-            corr=torch.zeros(P, dtype=torch.float64, device=dev),
-            shift=torch.zeros(P, dtype=torch.float64, device=dev))
+            cl1=torch.empty(P, dtype=torch.int32, device=dev),
+            cl2=torch.empty(P, dtype=torch.int32, device=dev),
+            j=torch.empty(P, dtype=torch.int32, device=dev),
+            corr=torch.empty(P, dtype=torch.float64, device=dev),
+            shift=torch.empty(P, dtype=torch.float64, device=dev))
         outs.append(o)
         params[i] = _params(n_r, n_theta, K, dt, ms[i], ss[i], pr[i], 0, tie_margin, variant, flags)
         ios[i] = _lib.ClmStackIO(base.data_ptr(), o["cl1"].data_ptr(), o["cl2"].data_ptr(),

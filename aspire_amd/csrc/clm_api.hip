@@ -148,13 +148,12 @@ int setup(clm_ctx* c, const clm_params* p, Setup& s) {
         }
     if (g.Rp > 0) {
         s.ph32.assign((size_t)(g.NE + 1) * g.Rp, make_float2(0.f, 0.f));  // row NE stays zero
-        for (int e = 0; e < g.NE; e++) {
-            const double sh = e < g.S ? s.shifts[e] : -s.shifts[e - g.S];
+        // the evaluation shifts e >= S are -s_{e-S}: conjugate phases
+        for (int e = 0; e < g.NE; e++)
             for (int r = 0; r < R; r++) {
-                const double th = theta(r, sh);
-                s.ph32[(size_t)e * g.Rp + r] = make_float2((float)std::cos(th), (float)std::sin(th));
+                const double2 q = s.ph64[(size_t)(e < g.S ? e : e - g.S) * R + r];
+                s.ph32[(size_t)e * g.Rp + r] = make_float2((float)q.x, (float)(e < g.S ? q.y : -q.y));
             }
-        }
     }
     return CLM_OK;
 }
@@ -443,6 +442,36 @@ int prepare(clm_ctx* c, Plan& pl, int n, const clm_params* ps, const clm_stack_i
     const int nt = (int)pl.order.size();
     if (c->sb.size() < (size_t)(sb_base + nt)) c->sb.resize(sb_base + nt);
     pl.table.assign(nt, StackDev{});
+    // the table and every stack's constants in one buffer and one copy: the
+    // copies of a small job cost more than its kernels
+    std::vector<char> consts((size_t)nt * sizeof(StackDev));
+    std::vector<size_t> off((size_t)nt * 5, 0);
+    auto place = [&](const void* v, size_t bytes) {
+        const size_t at = (consts.size() + 255) & ~(size_t)255;
+        consts.resize(at + bytes);
+        if (bytes) std::memcpy(consts.data() + at, v, bytes);
+        return at;
+    };
+    for (int ti = 0; ti < nt; ti++) {
+        const StackJob& j = pl.jobs[pl.order[ti]];
+        if (j.twin_src >= 0) continue;
+        size_t* o = &off[(size_t)ti * 5];
+        o[0] = place(j.s.ph32.data(), j.s.ph32.size() * sizeof(float2));
+        o[1] = place(j.s.ph64.data(), j.s.ph64.size() * sizeof(double2));
+        o[2] = place(j.s.shifts.data(), j.s.shifts.size() * sizeof(double));
+        o[3] = place(j.s.H.data(), j.s.H.size() * sizeof(double));
+        if (j.filt > 0) {
+            // W0 = 1.25.^(21:-1:1); W(i,j) = W0(1 + |i-d| + |j-d|)  (cryo_average_clmap.m:24-26)
+            const int w = 2 * j.filt + 1;
+            std::vector<double> wv((size_t)w * w);
+            for (int a = 0; a < w; a++)
+                for (int b = 0; b < w; b++)
+                    wv[(size_t)a * w + b] = std::pow(1.25, (double)(21 - (std::abs(a - j.filt) + std::abs(b - j.filt))));
+            o[4] = place(wv.data(), wv.size() * sizeof(double));
+        }
+    }
+    if ((rc = ensure(c, c->table, consts.size()))) return rc;
+    const char* const dconst = (const char*)c->table.p;
     for (int ti = 0; ti < nt; ti++) {
         StackJob& j = pl.jobs[pl.order[ti]];
         StackBufs& B = c->sb[pl.sb_base + ti];
@@ -477,19 +506,6 @@ int prepare(clm_ctx* c, Plan& pl, int n, const clm_params* ps, const clm_stack_i
             if ((rc = ensure(c, B.astk, (size_t)K * g.NAT * tile_bytes))) return rc;
             if ((rc = ensure(c, B.recs, (size_t)j.P * sizeof(PairRec)))) return rc;
         }
-        if ((rc = upload(c, B.ph32, j.s.ph32))) return rc;
-        if ((rc = upload(c, B.ph64, j.s.ph64))) return rc;
-        if ((rc = upload(c, B.shiftv, j.s.shifts))) return rc;
-        if ((rc = upload(c, B.H, j.s.H))) return rc;
-        if (j.filt > 0) {
-            // W0 = 1.25.^(21:-1:1); W(i,j) = W0(1 + |i-d| + |j-d|)  (cryo_average_clmap.m:24-26)
-            const int w = 2 * j.filt + 1;
-            std::vector<double> wv((size_t)w * w);
-            for (int a = 0; a < w; a++)
-                for (int b = 0; b < w; b++)
-                    wv[(size_t)a * w + b] = std::pow(1.25, (double)(21 - (std::abs(a - j.filt) + std::abs(b - j.filt))));
-            if ((rc = upload(c, B.W, wv))) return rc;
-        }
         StackDev& d = pl.table[ti];
         d.g = g;
         d.astk = B.astk.p;
@@ -498,9 +514,11 @@ int prepare(clm_ctx* c, Plan& pl, int n, const clm_params* ps, const clm_stack_i
         d.recs = (PairRec*)B.recs.p;
         d.P32 = (const float2*)B.P32.p;
         d.P64 = (const double2*)B.P64.p;
-        d.ph32 = (const float2*)B.ph32.p;
-        d.ph64 = (const double2*)B.ph64.p;
-        d.shiftv = (const double*)B.shiftv.p;
+        const size_t* o = &off[(size_t)ti * 5];
+        d.ph32 = (const float2*)(dconst + o[0]);
+        d.ph64 = (const double2*)(dconst + o[1]);
+        d.shiftv = (const double*)(dconst + o[2]);
+        d.H = (const double*)(dconst + o[3]);
         d.cl1 = j.io.cl1; d.cl2 = j.io.cl2; d.jidx = j.io.jidx; d.corr = j.io.corr; d.shift1d = j.io.shift1d;
         const float u = j.opk == OPK_BF16 ? 0x1p-8f : j.opk == OPK_F16 ? 0x1p-11f : 0x1p-24f;
         d.coef = (2.0f * u + u * u + (2.0f * g.Rp + 16.0f) * 0x1p-24f) * 1.01f;
@@ -511,7 +529,7 @@ int prepare(clm_ctx* c, Plan& pl, int n, const clm_params* ps, const clm_stack_i
         d.CPP = j.v.CPP;
         d.npairs = j.P;
         d.filt = j.filt;
-        d.wts = j.filt > 0 ? (const double*)B.W.p : nullptr;
+        d.wts = j.filt > 0 ? (const double*)(dconst + o[4]) : nullptr;
         d.eps64 = 4.0 * (g.R + 8.0) * 0x1p-53;
         if (j.exact && g.sym) {
             // what the phases of the paired shifts differ from conjugates
@@ -531,7 +549,8 @@ int prepare(clm_ctx* c, Plan& pl, int n, const clm_params* ps, const clm_stack_i
             base += pl.table[ti].npairs;
         }
     }
-    if ((rc = upload(c, c->table, pl.table))) return rc;
+    std::memcpy(consts.data(), pl.table.data(), (size_t)nt * sizeof(StackDev));
+    if ((rc = upload(c, c->table, consts))) return rc;
     // shared buffers: counters, lists, pass-2 tiles
     if ((rc = ensure(c, c->ctr, ctr_words(c, pl) * sizeof(unsigned long long)))) return rc;
     if ((rc = ensure(c, c->ulist, (size_t)std::max<long long>(ubase, 1) * sizeof(SlotRef)))) return rc;
@@ -556,8 +575,13 @@ int prepare(clm_ctx* c, Plan& pl, int n, const clm_params* ps, const clm_stack_i
         if (G.W < 4 || G.W > 8) return fail(c, CLM_E_UNSUP, "workgroup of %d waves", G.W);
         G.lds = pair_lds_bytes(G.W);
         G.occ = 0;
-        HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&G.occ, (const void*)G.fn, 64 * G.W, G.lds));
-        if (G.occ < 1) G.occ = 1;
+        for (const auto& e : c->occ)
+            if (e.fn == (const void*)G.fn && e.W == G.W) G.occ = e.occ;
+        if (!G.occ) {
+            HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&G.occ, (const void*)G.fn, 64 * G.W, G.lds));
+            if (G.occ < 1) G.occ = 1;
+            c->occ.push_back({(const void*)G.fn, G.W, G.occ});
+        }
         if (!build_tiles || G.sel) continue;
         const int PPW = G.W / G.CPP;
         std::vector<long long> key;
@@ -716,11 +740,11 @@ int enqueue_prep(clm_ctx* c, const Plan& pl) {
         const size_t plds = prep_lds_bytes(g.n_r);
         if (j.p.pf_dtype == CLM_C128)
             hipLaunchKernelGGL(prep_kernel<double>, dim3(nb), dim3(PREP_T), plds, c->stream, (const double*)j.io.pf, g,
-                               (const double*)B.H.p, (double2*)B.P64.p, (float2*)B.P32.p, B.Bop.p, j.opk,
+                               pl.table[ti].H, (double2*)B.P64.p, (float2*)B.P32.p, B.Bop.p, j.opk,
                                (unsigned*)B.nrm.p, ctr + 0, j.lsh);
         else
             hipLaunchKernelGGL(prep_kernel<float>, dim3(nb), dim3(PREP_T), plds, c->stream, (const float*)j.io.pf, g,
-                               (const double*)B.H.p, (double2*)B.P64.p, (float2*)B.P32.p, B.Bop.p, j.opk,
+                               pl.table[ti].H, (double2*)B.P64.p, (float2*)B.P32.p, B.Bop.p, j.opk,
                                (unsigned*)B.nrm.p, ctr + 0, j.lsh);
         HIPCHK(c, hipGetLastError());
         if (!j.exact) {
@@ -729,7 +753,7 @@ int enqueue_prep(clm_ctx* c, const Plan& pl) {
             AstkFn af = pick_astk(j.opk, g.Rp, g.sym != 0);
             if (!af) return fail(c, CLM_E_UNSUP, "no A-stack kernel for Rp=%d", g.Rp);
             hipLaunchKernelGGL(af, dim3((unsigned)((nch + 255) / 256)), dim3(256), 0, c->stream, g,
-                               (const float2*)B.P32.p, (const float2*)B.ph32.p, (int4*)B.astk.p, nullptr, g.K);
+                               (const float2*)B.P32.p, pl.table[ti].ph32, (int4*)B.astk.p, nullptr, g.K);
             HIPCHK(c, hipGetLastError());
         }
     }
@@ -1043,11 +1067,18 @@ int enqueue_job(clm_ctx* c, const Plan& pl, bool timed, int phases = PHASE_ALL) 
     return CLM_OK;
 }
 
+// The job's counters as the stream has them now (waits for it).
+int read_counters(clm_ctx* c, const Plan& pl, std::vector<unsigned long long>& h) {
+    h.resize(ctr_words(c, pl));
+    HIPCHK(c, hipMemcpyAsync(h.data(), c->ctr.p, h.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost,
+                             c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return CLM_OK;
+}
+
 // Add a finished plan's counters to st (which the caller cleared).
-int add_stats(clm_ctx* c, const Plan& pl, clm_stats* st) {
+int add_stats(const Plan& pl, const std::vector<unsigned long long>& h, clm_stats* st) {
     if (!st || pl.P == 0) return CLM_OK;
-    std::vector<unsigned long long> h(ctr_words(c, pl));
-    HIPCHK(c, hipMemcpy(h.data(), c->ctr.p, h.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost));
     auto as_int = [](unsigned long long x) { return (int64_t)(int)(unsigned)(x & 0xffffffffu); };
     st->small_norm_lines += (int64_t)h[0];
     // the globals, then the areas
@@ -1088,31 +1119,33 @@ void timed_stats(clm_ctx* c, clm_stats* st) {
     st->ms_total = event_ms(c->ev[0], c->ev[3]);
 }
 
-// Run a plan to completion (no graph).  With lazy twins the host waits
-// after the re-score: the twins are built only if a group refined by them
-// has uncertain pairs (else their refinement launches find nothing to do).
+// Run a plan to completion (no graph).  With lazy twins the host waits after
+// the re-score and reads the counters: the second phase (twins, second pass,
+// exhaustive search) is launched only if a group has uncertain pairs.
 int run_plan(clm_ctx* c, Plan& pl, bool timed, clm_stats* st) {
     int rc;
+    std::vector<unsigned long long> h;
     if (!pl.twin_lazy) {
         if ((rc = enqueue_job(c, pl, timed))) return rc;
-    } else {
-        if ((rc = enqueue_job(c, pl, timed, PHASE_A))) return rc;
-        bool any = false;
-        for (const Group& G : pl.groups) any = any || G.twin >= 0;
-        if (any) {
-            std::vector<unsigned long long> h(ctr_words(c, pl));
-            HIPCHK(c, hipMemcpyAsync(h.data(), c->ctr.p, h.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                                     c->stream));
-            HIPCHK(c, hipStreamSynchronize(c->stream));
-            bool need = false;
-            for (size_t gi = 0; gi < pl.groups.size(); gi++)
-                if (pl.groups[gi].twin >= 0 && (int)(unsigned)(h[16 + GSTRIDE * gi + 1] & 0xffffffffu) > 0) need = true;
-            if (need && (rc = build_twins(c, pl, h))) return rc;
-        }
-        if ((rc = enqueue_job(c, pl, timed, PHASE_B))) return rc;
+        if ((rc = read_counters(c, pl, h))) return rc;
+        return add_stats(pl, h, st);
     }
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return add_stats(c, pl, st);
+    if ((rc = enqueue_job(c, pl, timed, PHASE_A))) return rc;
+    if (timed) HIPCHK(c, hipEventRecord(c->ev[3], c->stream));
+    if ((rc = read_counters(c, pl, h))) return rc;
+    bool open = false, need = false;
+    for (size_t gi = 0; gi < pl.groups.size(); gi++) {
+        const Group& G = pl.groups[gi];
+        if (G.exact || G.twin_of >= 0 || (int)(unsigned)(h[16 + GSTRIDE * gi + 1] & 0xffffffffu) <= 0) continue;
+        open = true;
+        need = need || G.twin >= 0;
+    }
+    if (open) {
+        if (need && (rc = build_twins(c, pl, h))) return rc;
+        if ((rc = enqueue_job(c, pl, timed, PHASE_B))) return rc;
+        if ((rc = read_counters(c, pl, h))) return rc;
+    }
+    return add_stats(pl, h, st);
 }
 
 void drop_graph(clm_ctx* c) {
@@ -1139,8 +1172,7 @@ std::vector<unsigned long long> signature(const clm_ctx* c, const Plan& pl) {
     add(pl.table.data(), pl.table.size() * sizeof(StackDev));
     for (size_t ti = 0; ti < pl.order.size(); ti++) {
         const StackBufs& B = c->sb[pl.sb_base + ti];
-        const void* sp[] = {B.P64.p, B.P32.p, B.Bop.p, B.nrm.p, B.astk.p, B.recs.p, B.ph32.p, B.ph64.p, B.shiftv.p, B.H.p,
-                            B.W.p};
+        const void* sp[] = {B.P64.p, B.P32.p, B.Bop.p, B.nrm.p, B.astk.p, B.recs.p};
         add(sp, sizeof sp);
     }
     const void* bufs[] = {c->table.p, c->ctr.p, c->ulist.p, c->erecs.p, c->plist.p, c->tiles2.p, c->fblist.p,
@@ -1194,8 +1226,9 @@ int run_job_core(clm_ctx* c, int n, const clm_params* ps, const clm_stack_io* io
     HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
     HIPCHK(c, hipGraphLaunch(c->gexec, c->stream));
     HIPCHK(c, hipEventRecord(c->ev[3], c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    rc = add_stats(c, pl, st);
+    std::vector<unsigned long long> h;
+    if ((rc = read_counters(c, pl, h))) return rc;
+    rc = add_stats(pl, h, st);
     if (st) st->ms_total = event_ms(c->ev[0], c->ev[3]);
     return rc;
 }
@@ -1720,7 +1753,7 @@ void clm_destroy(clm_ctx* c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     drop_graph(c);
     for (StackBufs& B : c->sb) {
-        DevBuf* sbufs[] = {&B.P64, &B.P32, &B.Bop, &B.nrm, &B.astk, &B.recs, &B.ph32, &B.ph64, &B.shiftv, &B.H, &B.W,
+        DevBuf* sbufs[] = {&B.P64, &B.P32, &B.Bop, &B.nrm, &B.astk, &B.recs,
                            &B.amap};
         for (DevBuf* b : sbufs) release(*b);
     }

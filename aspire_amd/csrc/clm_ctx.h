@@ -20,7 +20,7 @@ struct DevBuf {
 };
 
 struct StackBufs {
-    DevBuf P64, P32, Bop, nrm, astk, recs, ph32, ph64, shiftv, H, W;
+    DevBuf P64, P32, Bop, nrm, astk, recs;
     DevBuf amap;  // a twin's image -> A-stack index map (K ints), then its image list
 };
 
@@ -37,6 +37,11 @@ struct clm_ctx {
     int device = 0;
     int n_cu = 0;
     int lds_max = 65536;
+    struct Occ {
+        const void* fn;
+        int W, occ;
+    };
+    std::vector<Occ> occ;                     // workgroups per CU of the pair kernels used so far
     hipStream_t stream = nullptr;
     std::string err;
     std::vector<clmh::StackBufs> sb;          // per stack of the current call

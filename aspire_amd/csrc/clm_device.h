@@ -61,6 +61,7 @@ struct StackDev {
     const float2* ph32;       // [NE+1][Rp], row NE zero
     const double2* ph64;      // [S][R]
     const double* shiftv;     // [S]
+    const double* H;          // [2 n_r - 1] ray filter, zeroed band
     int32_t* cl1;             // outputs, [P] in equation order
     int32_t* cl2;
     int32_t* jidx;

@@ -278,12 +278,12 @@ def clmatrix_windowed(pf, prop, max_shift=12.0, shift_step=0.5, window=1.0, gate
     base, dt, n_r, n_theta, K = _device_view(pf)
     P = max(K * (K - 1) // 2, 0)
     dev = base.device
-    out = dict(cl1=torch.zeros(P, dtype=torch.int32, device=dev),
-               cl2=torch.zeros(P, dtype=torch.int32, device=dev),
-               j=torch.zeros(P, dtype=torch.int32, device=dev),
-               corr=torch.zeros(P, dtype=torch.float64, device=dev),
-               shift=torch.zeros(P, dtype=torch.float64, device=dev),
-               exhaustive=torch.zeros(P, dtype=torch.uint8, device=dev))
+    out = dict(cl1=torch.empty(P, dtype=torch.int32, device=dev),
+               cl2=torch.empty(P, dtype=torch.int32, device=dev),
+               j=torch.empty(P, dtype=torch.int32, device=dev),
+               corr=torch.empty(P, dtype=torch.float64, device=dev),
+               shift=torch.empty(P, dtype=torch.float64, device=dev),
+               exhaustive=torch.empty(P, dtype=torch.uint8, device=dev))
     prop = prop.contiguous().float()
     if prop.shape != (K, 2):
         raise ValueError("proposals must be K x 2")
