@@ -3,8 +3,8 @@
 #include "clm.h"
 #include "clm_ctx.h"
 #include "clm_kernels.hip"
-#include "clm_clmap.h"
 #include "clm_search64.h"
+#include "clm_clmap.h"
 
 #include <algorithm>
 #include <cmath>
@@ -815,8 +815,9 @@ int launch_rescore(clm_ctx* c, const Plan& pl, unsigned grid, RescoreArgs a, int
 }
 
 // FP64 search of the pairs of stack ti (all of them, or the list of a sel
-// group): on the FP64 matrix cores, with exact64_kernel for the pairs they
-// leave open (listed in ovf_list, which holds at least the group's pairs).
+// group), of filtered maps if the stack asks for them: on the FP64 matrix
+// cores.  The pairs they leave open are listed in ovf_list, which holds at
+// least the group's pairs.
 int enqueue_search64(clm_ctx* c, const Plan& pl, int ti, Exact64Args ea, int* ovf_count,
                      SlotRef* ovf_list) {
     const StackDev& d = pl.table[ti];
@@ -830,9 +831,10 @@ int enqueue_search64(clm_ctx* c, const Plan& pl, int ti, Exact64Args ea, int* ov
         a.x.n_all = d.pair_base + d.npairs;
     }
     a.x.item_cap = d.npairs;
-    // units (shifts x row blocks) of a pair over several workgroups while the
-    // pairs alone leave the chip short of eight workgroups per CU
-    const long long units = (long long)g.NE * ((g.L + S64_ROWS - 1) / S64_ROWS);
+    // units (shifts x row blocks, or x tiles) of a pair over several workgroups
+    // while the pairs alone leave the chip short of eight workgroups per CU
+    const long long side = (g.L + CF_T - 2 * d.filt - 1) / (CF_T - 2 * d.filt);
+    const long long units = d.filt > 0 ? g.S * side * side : (long long)g.NE * ((g.L + S64_ROWS - 1) / S64_ROWS);
     const long long want = (8LL * c->n_cu + d.npairs - 1) / d.npairs;
     a.x.sj = (int)std::max(1LL, std::min({want, units, (long long)EX_SJ}));
     if (d.npairs > EX_CAP) a.x.sj = 1;
@@ -841,8 +843,8 @@ int enqueue_search64(clm_ctx* c, const Plan& pl, int ti, Exact64Args ea, int* ov
     a.ovf_count = ovf_count;
     a.ovf_list = ovf_list;
     int KS = 0;
-    const Search64Fn fn = pick_search64(g.R, g.L, g.sym != 0, KS);
-    const size_t lds = search64_lds(KS);
+    const Search64Fn fn = d.filt > 0 ? clmap64_kernel : pick_search64(g.R, g.L, g.sym != 0, KS);
+    const size_t lds = d.filt > 0 ? clmap64_lds() : search64_lds(KS);
     HIPCHK(c, hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL(fn, dim3((unsigned)std::min<long long>(d.npairs, 16LL * c->n_cu), (unsigned)a.x.sj), dim3(256), lds,
                        c->stream, a);
@@ -884,13 +886,6 @@ int enqueue_job(clm_ctx* c, const Plan& pl, bool timed, int phases = PHASE_ALL) 
                 ea.list = pl.jobs[G.members[0]].sel_list;
                 ea.n_dev = pl.jobs[G.members[0]].sel_count;
             }
-            if (G.filt > 0) {
-                ClmapArgs ca{dtab, G.first, (int)G.members.size(), G.P};
-                const long long nb = std::min<long long>(G.P, (long long)c->n_cu * 2);
-                hipLaunchKernelGGL(clmap_kernel, dim3((unsigned)nb), dim3(256), 0, c->stream, ca);
-                HIPCHK(c, hipGetLastError());
-                continue;
-            }
             // the fallback list is free until phase B: pairs the matrix cores
             // leave open are listed there, counted in the group's own counter
             int* const open = (int*)(ctr + 16 + GSTRIDE * gi);
@@ -899,6 +894,13 @@ int enqueue_job(clm_ctx* c, const Plan& pl, bool timed, int phases = PHASE_ALL) 
             for (int ti = G.first; ti < G.first + (int)G.members.size(); ti++) {
                 S = std::max(S, pl.table[ti].g.S);
                 if ((rc = enqueue_search64(c, pl, ti, ea, open, olist))) return rc;
+            }
+            if (G.filt > 0) {
+                ClmapArgs ca{dtab, olist, open};
+                const long long nb = std::min<long long>(G.P, (long long)c->n_cu * 2);
+                hipLaunchKernelGGL(clmap_kernel, dim3((unsigned)nb), dim3(256), 0, c->stream, ca);
+                HIPCHK(c, hipGetLastError());
+                continue;
             }
             ea.list = olist;
             ea.n_dev = open;

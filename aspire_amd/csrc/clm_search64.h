@@ -32,8 +32,103 @@ struct Search64Args {
     SlotRef* ovf_list;
 };
 
+// A wave's running maximum and the candidates within the margin of it.
+struct CandList {
+    double* v;       // LDS, S64_LIST each
+    long long* k;
+    double mg, wm, thr;  // margin, maximum, keep threshold
+    int n;
+    bool lost;
+    __device__ inline void reset(double margin) {
+        mg = margin;
+        wm = thr = -INFINITY;
+        n = 0;
+        lost = false;
+    }
+    // Raise the threshold for a new maximum (wave-uniform).
+    __device__ inline void raise(double m) {
+        wm = fmax(wm, m);
+        thr = wm - mg;
+    }
+    // Keep each lane's candidate (ok, value x, tie key) at or above the
+    // threshold; called by the whole wave.
+    __device__ inline void keep(bool ok, double x, long long key, int lane) {
+        const bool on = ok && x >= thr;
+        const unsigned long long mask = __ballot(on);
+        if (!mask) return;
+        const int cnt = __popcll(mask);
+        if (n + cnt > S64_LIST) {  // drop what fell below the threshold
+            const double ov = lane < n ? v[lane] : 0.0;
+            const long long okey = lane < n ? k[lane] : 0;
+            const bool kp = lane < n && ov >= thr;
+            const unsigned long long km = __ballot(kp);
+            __builtin_amdgcn_wave_barrier();
+            if (kp) {
+                const int pos = __popcll(km & lanemask_lt());
+                v[pos] = ov;
+                k[pos] = okey;
+            }
+            n = __popcll(km);
+            __builtin_amdgcn_wave_barrier();
+        }
+        if (on) {
+            const int pos = n + __popcll(mask & lanemask_lt());
+            if (pos < S64_LIST) {
+                v[pos] = x;
+                k[pos] = key;
+            }
+        }
+        if (n + cnt > S64_LIST) lost = true;
+        n = min(n + cnt, S64_LIST);
+        __builtin_amdgcn_wave_barrier();
+    }
+    // The workgroup's maximum M; true if a list lost entries that the margin
+    // may hold.  Called by the four waves of the workgroup.
+    __device__ inline bool finish(double* s_rv, int* s_lost, int wave, int lane, double& M) {
+        if (lane == 0) {
+            s_rv[wave] = wm;
+            s_lost[wave] = lost;
+        }
+        __syncthreads();
+        M = s_rv[0];
+#pragma unroll
+        for (int w = 1; w < 4; w++) M = fmax(M, s_rv[w]);
+        bool over = false;
+#pragma unroll
+        for (int w = 0; w < 4; w++) over = over || (s_lost[w] && s_rv[w] >= M - mg);
+        __syncthreads();
+        return over;
+    }
+};
+
 // Key written for an item's range whose list overflowed (sj > 1).
 constexpr long long S64_LOST = -1;
+
+// An item's best of the four waves' (bv, bk): to its outputs, to its range's
+// place (sj > 1) or, where a list overflowed, to the list of open pairs.
+__device__ inline void search64_store(const Search64Args& a, const StackDev& sd, long long it, int stk, int slot,
+                                      bool over, double bv, long long bk, double* s_rv, long long* s_rk, int wave,
+                                      int lane) {
+    if (lane == 0) {
+        s_rv[wave] = bv;
+        s_rk[wave] = bk;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 4; w++)
+            if (better64(s_rv[w], s_rk[w], bv, bk)) { bv = s_rv[w]; bk = s_rk[w]; }
+        if (a.x.sj > 1) {
+            const long long o = (it - a.x.item0) * a.x.sj + blockIdx.y;
+            a.x.sv[o] = bv;
+            a.x.sk[o] = over ? S64_LOST : bk;
+        } else if (over) {
+            a.ovf_list[atomicAdd(a.ovf_count, 1)] = SlotRef{stk, slot};
+        } else {
+            write_result(sd, slot, bv, bk);
+        }
+    }
+    __syncthreads();
+}
 
 // LDS bytes: the staged rows, [r][row] with a row more than staged (the
 // threads that write a column then hit different banks), one phase row per
@@ -66,8 +161,7 @@ __global__ __launch_bounds__(256, (KS * CT * 4 + CT * 16 <= 200 ? 2 : 1)) void s
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, kq = lane >> 4;
     double2* const ph_w = s_ph + wave * 4 * KS;
-    double* const lv = s_v + wave * S64_LIST;
-    long long* const lk = s_k + wave * S64_LIST;
+    CandList cl{s_v + wave * S64_LIST, s_k + wave * S64_LIST};
     const long long n_tot = a.x.list ? (long long)*a.x.n_dev : a.x.n_all;
     const long long n = n_tot < a.x.item0 + a.x.item_cap ? n_tot : a.x.item0 + a.x.item_cap;
     for (long long it = a.x.item0 + blockIdx.x; it < n; it += gridDim.x) {
@@ -84,9 +178,7 @@ __global__ __launch_bounds__(256, (KS * CT * 4 + CT * 16 <= 200 ? 2 : 1)) void s
         const int NT = (L + 15) / 16, NRB = (L + S64_ROWS - 1) / S64_ROWS;
         const int U = NRB * NE;
         const int u0 = (int)((long long)blockIdx.y * U / a.x.sj), u1 = (int)((long long)(blockIdx.y + 1) * U / a.x.sj);
-        double wm = -INFINITY, thr = -INFINITY;  // this wave's maximum and keep threshold
-        int wc = 0;
-        bool lost = false;
+        cl.reset(mg);
         for (int cg = 0; cg < NT; cg += 4 * CT) {
             const int ct0 = cg + wave * CT;
             const bool work = ct0 < NT;
@@ -164,13 +256,12 @@ __global__ __launch_bounds__(256, (KS * CT * 4 + CT * 16 <= 200 ? 2 : 1)) void s
                             m = fmax(m, ok ? v : -INFINITY);
                         }
                     }
-                    if (!__ballot(m >= thr && m > -INFINITY)) continue;
+                    if (!__ballot(m >= cl.thr && m > -INFINITY)) continue;
                     // rare once the maximum has been seen: raise the threshold
                     // and list every candidate at or above it
 #pragma unroll
                     for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
-                    wm = fmax(wm, m);
-                    thr = wm - mg;
+                    cl.raise(m);
 #pragma unroll
                     for (int c = 0; c < CT; c++)
 #pragma unroll
@@ -180,35 +271,8 @@ __global__ __launch_bounds__(256, (KS * CT * 4 + CT * 16 <= 200 ? 2 : 1)) void s
                             for (int s = 0; s < (SYM ? 2 : 1); s++) {
                                 const bool minus = SYM ? s == 1 : flip;
                                 const double v = minus ? X[c][i] - Y[c][i] : X[c][i] + Y[c][i];
-                                const bool on = l1 < L && l2 < L && v >= thr;
-                                const unsigned long long mask = __ballot(on);
-                                if (!mask) continue;
-                                const int cnt = __popcll(mask);
-                                if (wc + cnt > S64_LIST) {  // drop what fell below the threshold
-                                    const double ov = lane < wc ? lv[lane] : 0.0;
-                                    const long long ok = lane < wc ? lk[lane] : 0;
-                                    const bool keep = lane < wc && ov >= thr;
-                                    const unsigned long long km = __ballot(keep);
-                                    __builtin_amdgcn_wave_barrier();
-                                    if (keep) {
-                                        const int pos = __popcll(km & lanemask_lt());
-                                        lv[pos] = ov;
-                                        lk[pos] = ok;
-                                    }
-                                    wc = __popcll(km);
-                                    __builtin_amdgcn_wave_barrier();
-                                }
-                                if (on) {
-                                    const int pos = wc + __popcll(mask & lanemask_lt());
-                                    const int j = SYM ? (minus ? S - 1 - e : e) : (flip ? e - S : e);
-                                    if (pos < S64_LIST) {
-                                        lv[pos] = v;
-                                        lk[pos] = tie_key(j, minus ? L + l2 : l2, l1);
-                                    }
-                                }
-                                if (wc + cnt > S64_LIST) lost = true;
-                                wc = min(wc + cnt, S64_LIST);
-                                __builtin_amdgcn_wave_barrier();
+                                const int j = SYM ? (minus ? S - 1 - e : e) : (flip ? e - S : e);
+                                cl.keep(l1 < L && l2 < L, v, tie_key(j, minus ? L + l2 : l2, l1), lane);
                             }
                         }
                 }
@@ -216,46 +280,18 @@ __global__ __launch_bounds__(256, (KS * CT * 4 + CT * 16 <= 200 ? 2 : 1)) void s
         }
         // the workgroup's maximum, then the candidates within the margin of it
         // with the oracle's arithmetic
-        if (lane == 0) {
-            s_rv[wave] = wm;
-            s_lost[wave] = lost;
-        }
-        __syncthreads();
-        double M = s_rv[0];
-#pragma unroll
-        for (int w = 1; w < 4; w++) M = fmax(M, s_rv[w]);
-        bool over = false;  // a list that lost entries which the margin may hold
-#pragma unroll
-        for (int w = 0; w < 4; w++) over = over || (s_lost[w] && s_rv[w] >= M - mg);
-        __syncthreads();
+        double M;
+        const bool over = cl.finish(s_rv, s_lost, wave, lane, M);
         double bv = -INFINITY;
         long long bk = 0x7fffffffffffffffLL;
         if (!over)
-            for (int i = 0; i < wc; i++)
-                if (lv[i] >= M - mg) {
-                    const long long key = lk[i];
+            for (int i = 0; i < cl.n; i++)
+                if (cl.v[i] >= M - mg) {
+                    const long long key = cl.k[i];
                     const double v = eval64(sd, k1, k2, key, lane);
                     if (!isnan(v) && better64(v, key, bv, bk)) { bv = v; bk = key; }
                 }
-        if (lane == 0) {
-            s_rv[wave] = bv;
-            s_rk[wave] = bk;
-        }
-        __syncthreads();
-        if (tid == 0) {
-            for (int w = 1; w < 4; w++)
-                if (better64(s_rv[w], s_rk[w], bv, bk)) { bv = s_rv[w]; bk = s_rk[w]; }
-            if (a.x.sj > 1) {
-                const long long o = (it - a.x.item0) * a.x.sj + blockIdx.y;
-                a.x.sv[o] = bv;
-                a.x.sk[o] = over ? S64_LOST : bk;
-            } else if (over) {
-                a.ovf_list[atomicAdd(a.ovf_count, 1)] = SlotRef{stk, slot};
-            } else {
-                write_result(sd, slot, bv, bk);
-            }
-        }
-        __syncthreads();
+        search64_store(a, sd, it, stk, slot, over, bv, bk, s_rv, s_rk, wave, lane);
     }
 }
 
