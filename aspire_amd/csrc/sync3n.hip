@@ -74,71 +74,68 @@ __global__ void symv_kernel(int N, int ne, const double* __restrict__ v, double*
     for (int g = 0; g < ne; g++) Vs[g * NN + t] = pr < 0 ? 0.0 : v[pr + P * g];
 }
 
-__device__ inline void mult3(double* out, const double* A, const double* B) {
+// Signs of the side pairs (ij,jk), (ik,jk), (ij,ik) in the four
+// configurations: 0 none flipped, 1 Rij flipped, 2 Rjk flipped, 3 Rik flipped.
+__device__ inline double sgn(int best, int q) {
+    // the configurations with sign -1 at q: {1, 2}, {2, 3}, {1, 3}
+    const unsigned neg = q == 0 ? 0x6u : q == 1 ? 0xcu : 0xau;
+    return (neg >> best) & 1 ? -1.0 : 1.0;
+}
+
+// The triangle (A, B, C) = (Rij, Rjk, Rik): the mismatches
+// ||Rij Rjk - Rik||^2 of the four configurations (J X J changes the sign of
+// the entries with exactly one index 3), the best configuration, its mismatch
+// and for each side pair q the smallest mismatch of the configurations that
+// differ from it in q's sign.
+// An entry of (J A J) B is s_i (x + y - z) and of A (J B J) s_j (x + y - z),
+// with x, y, z the products of A B's own entry, s = (1, 1, -1); negation is
+// exact, so the three products cost one, plus nine subtractions, with the bits
+// of the products written out.
+struct Tri {
+    int best;
+    double bv, alt[3];
+};
+__device__ inline Tri triangle(const double* A, const double* B, const double* C) {
+    double c0 = 0.0, c1 = 0.0, c2 = 0.0, c3 = 0.0;
 #pragma unroll
-    for (int i = 0; i < 3; i++)
+    for (int j = 0; j < 3; j++)
 #pragma unroll
-        for (int j = 0; j < 3; j++) {
-            const double x = __dmul_rn(A[i], B[3 * j + 0]);
-            const double y = __dmul_rn(A[3 + i], B[3 * j + 1]);
+        for (int i = 0; i < 3; i++) {
+            const double x = __dmul_rn(A[i], B[3 * j]), y = __dmul_rn(A[3 + i], B[3 * j + 1]);
             const double z = __dmul_rn(A[6 + i], B[3 * j + 2]);
-            out[3 * j + i] = __dadd_rn(__dadd_rn(x, y), z);
+            const double t = __dadd_rn(x, y), p = __dadd_rn(t, z), m = __dsub_rn(t, z);
+            const double c = C[3 * j + i], ci = i == 2 ? -c : c, cj = j == 2 ? -c : c;
+            const double d0 = __dsub_rn(p, c), d1 = __dsub_rn(m, ci);
+            const double e0 = __dmul_rn(d0, d0), e1 = __dmul_rn(d1, d1);
+            double e2 = e1, e3 = e0;
+            if ((i == 2) != (j == 2)) {
+                const double d2 = __dsub_rn(m, cj), d3 = __dadd_rn(p, c);
+                e2 = __dmul_rn(d2, d2);
+                e3 = __dmul_rn(d3, d3);
+            }
+            c0 = __dadd_rn(c0, e0);
+            c1 = __dadd_rn(c1, e1);
+            c2 = __dadd_rn(c2, e2);
+            c3 = __dadd_rn(c3, e3);
         }
+    Tri t;
+    t.best = 0;
+    t.bv = c0;
+    if (c1 < t.bv) { t.best = 1; t.bv = c1; }
+    if (c2 < t.bv) { t.best = 2; t.bv = c2; }
+    if (c3 < t.bv) { t.best = 3; t.bv = c3; }
+    const int b = t.best;
+    const double m12 = c2 < c1 ? c2 : c1, m03 = c3 < c0 ? c3 : c0;
+    const double m23 = c3 < c2 ? c3 : c2, m01 = c1 < c0 ? c1 : c0;
+    const double m13 = c3 < c1 ? c3 : c1, m02 = c2 < c0 ? c2 : c0;
+    t.alt[0] = b == 0 || b == 3 ? m12 : m03;
+    t.alt[1] = b <= 1 ? m23 : m01;
+    t.alt[2] = b == 0 || b == 2 ? m13 : m02;
+    return t;
 }
 
-__device__ inline double dnorm(const double* A, const double* B) {
-    double n = 0.0;
-#pragma unroll
-    for (int i = 0; i < 9; i++) {
-        const double d = __dsub_rn(A[i], B[i]);
-        n = __dadd_rn(n, __dmul_rn(d, d));
-    }
-    return n;
-}
-
-// J X J: the entries with exactly one index 3 change sign
-__device__ inline void jrj(const double* R, double* A) {
-    A[0] = R[0]; A[1] = R[1]; A[2] = -R[2];
-    A[3] = R[3]; A[4] = R[4]; A[5] = -R[5];
-    A[6] = -R[6]; A[7] = -R[7]; A[8] = R[8];
-}
-
-// Configurations (signs of the side pairs (ij,jk), (ik,jk), (ij,ik)): 0 none
-// flipped, 1 Rij flipped, 2 Rjk flipped, 3 Rik flipped.  For a best
-// configuration b and side pair q, the alternatives are the two
-// configurations whose sign at q differs from b's.
-__constant__ int ALT0[4][3] = {{1, 2, 1}, {0, 2, 0}, {0, 0, 1}, {1, 0, 0}};
-__constant__ int ALT1[4][3] = {{2, 3, 3}, {3, 3, 2}, {3, 1, 3}, {2, 1, 2}};
-__constant__ double SGN[4][3] = {{1, 1, 1}, {-1, 1, -1}, {-1, -1, 1}, {1, -1, -1}};
-
-// Scores of side pairs qa and qb of the triangle (Rij, Rjk, Rik); returns the
-// best configuration.
-__device__ inline int triangle2(const double* Rij, const double* Rjk, const double* Rik, int qa, int qb, double& sa,
-                                double& sb) {
-    double J[9], tmp[9], c0, c1, c2, c3;
-    mult3(tmp, Rij, Rjk);
-    c0 = dnorm(tmp, Rik);
-    jrj(Rik, J);
-    c3 = dnorm(tmp, J);
-    jrj(Rij, J);
-    mult3(tmp, J, Rjk);
-    c1 = dnorm(tmp, Rik);
-    jrj(Rjk, J);
-    mult3(tmp, Rij, J);
-    c2 = dnorm(tmp, Rik);
-    int b = 0;
-    double bv = c0;
-    if (c1 < bv) { b = 1; bv = c1; }
-    if (c2 < bv) { b = 2; bv = c2; }
-    if (c3 < bv) { b = 3; bv = c3; }
-    const double cc[4] = {c0, c1, c2, c3};
-    double alt = cc[ALT0[b][qa]];
-    if (cc[ALT1[b][qa]] < alt) alt = cc[ALT1[b][qa]];
-    sa = __dsub_rn(1.0, __dsqrt_rn(__ddiv_rn(bv, alt)));
-    alt = cc[ALT0[b][qb]];
-    if (cc[ALT1[b][qb]] < alt) alt = cc[ALT1[b][qb]];
-    sb = __dsub_rn(1.0, __dsqrt_rn(__ddiv_rn(bv, alt)));
-    return b;
+__device__ inline double score(const Tri& t, int q) {
+    return __dsub_rn(1.0, __dsqrt_rn(__ddiv_rn(t.bv, t.alt[q])));
 }
 
 struct TriArgs {
@@ -213,7 +210,7 @@ __device__ inline void f_both(double x, const double* prm, const double* lg, dou
 // the other modes' 16 at a time.  The stage size does not change the order
 // of any sum.
 template <int MODE, int NEC = 1, bool TL = false>
-__device__ __forceinline__ void tri_body(TriArgs a) {
+__device__ __forceinline__ void tri_pairs(TriArgs a) {
     constexpr int KCm = MODE == SIGNS ? 12 : KC;
     __shared__ double Lp[9][KCm][TB];
     __shared__ double Lq[9][KCm][TB];
@@ -294,8 +291,13 @@ __device__ __forceinline__ void tri_body(TriArgs a) {
                 // the histogram takes (ij,jk) from ij, (ik,jk) from jk, (ij,ik) from ik
                 const int qa = role == 2 ? 1 : 0;
                 const int qb = role == 1 ? 1 : 2;
-                double sa, sb;
-                const int best = triangle2(Rij, Rjk, Rik, qa, qb, sa, sb);
+                const Tri tr = triangle(Rij, Rjk, Rik);
+                const int best = tr.best;
+                double sa = 0.0, sb = 0.0;
+                if (MODE != SIGNS || a.entries == 1) {
+                    sa = score(tr, qa);
+                    sb = score(tr, qb);
+                }
                 if constexpr (MODE == SCORES) {
                     acc0 += sa + sb;
                     const double hs = role == 0 ? sa : (role == 1 ? sb : sb);
@@ -314,7 +316,7 @@ __device__ __forceinline__ void tri_body(TriArgs a) {
                     }
                 } else {
                     double ea, eb;
-                    const double sga = SGN[best][qa], sgb = SGN[best][qb];
+                    const double sga = sgn(best, qa), sgb = sgn(best, qb);
                     if (a.entries == 1) {
                         ea = sga * sa;
                         eb = sgb * sb;
@@ -379,10 +381,10 @@ __global__ void zero_u64_kernel(unsigned long long* p, int n) {
 // run at two; the signs product runs at three for up to four vectors (its
 // LDS and registers sized for them), at two for up to eight.
 template <bool TL>
-__global__ __launch_bounds__(256, 4) void tri_scores_kernel(TriArgs a) { tri_body<SCORES, 1, TL>(a); }
-__global__ __launch_bounds__(256) void tri_probs_kernel(TriArgs a) { tri_body<PROBS>(a); }
-__global__ __launch_bounds__(256, 3) void tri_signs4_kernel(TriArgs a) { tri_body<SIGNS, 4>(a); }
-__global__ __launch_bounds__(256) void tri_signs8_kernel(TriArgs a) { tri_body<SIGNS, MAXE>(a); }
+__global__ __launch_bounds__(256, 4) void tri_scores_kernel(TriArgs a) { tri_pairs<SCORES, 1, TL>(a); }
+__global__ __launch_bounds__(256) void tri_probs_kernel(TriArgs a) { tri_pairs<PROBS>(a); }
+__global__ __launch_bounds__(256, 3) void tri_signs4_kernel(TriArgs a) { tri_pairs<SIGNS, 4>(a); }
+__global__ __launch_bounds__(256) void tri_signs8_kernel(TriArgs a) { tri_pairs<SIGNS, MAXE>(a); }
 
 }  // namespace s3
 
