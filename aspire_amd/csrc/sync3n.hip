@@ -41,7 +41,7 @@
 namespace s3 {
 
 constexpr int TB = 16;  // pairs per tile side
-constexpr int KC = 16;  // third images per LDS stage
+constexpr int KC = 8;   // third images per LDS stage
 constexpr int MAXE = 8; // vectors of the signs product
 
 enum { SCORES = 0, PROBS = 1, SIGNS = 2 };
@@ -134,8 +134,8 @@ __device__ inline Tri triangle(const double* A, const double* B, const double* C
     return t;
 }
 
-__device__ inline double score(const Tri& t, int q) {
-    return __dsub_rn(1.0, __dsqrt_rn(__ddiv_rn(t.bv, t.alt[q])));
+__device__ inline double score(double best, double alt) {
+    return __dsub_rn(1.0, __dsqrt_rn(__ddiv_rn(best, alt)));
 }
 
 struct TriArgs {
@@ -151,9 +151,11 @@ struct TriArgs {
     double* cum;                // [P] or null
     unsigned long long* hist;   // [n_intervals] counts
     // PROBS: P2, A, a, B, b, x0; and, when lform, log A, log(P2 B),
-    // log((1 - P2) A), -b/(1 - x0)
+    // log((1 - P2) A), -b/(1 - x0); for LikeSum min(a, b), |b - a|, P2 B,
+    // (1 - P2) A
     double prm[6];
     double lg[4];
+    double lk[4];
     int lform;
     double* ind;
     double* arb;
@@ -205,145 +207,233 @@ __device__ inline void f_both(double x, const double* prm, const double* lg, dou
     ind = hi == -INFINITY ? hi : hi + log1p(exp(lo - hi));
 }
 
-// NEC: vectors the signs product stages (a.ne <= NEC); its third images are
-// staged 12 at a time (43 KB of LDS at NEC = 4: three workgroups per CU),
-// the other modes' 16 at a time.  The stage size does not change the order
-// of any sum.
-template <int MODE, int NEC = 1, bool TL = false>
-__device__ __forceinline__ void tri_pairs(TriArgs a) {
-    constexpr int KCm = MODE == SIGNS ? 12 : KC;
-    __shared__ double Lp[9][KCm][TB];
-    __shared__ double Lq[9][KCm][TB];
-    __shared__ double Vp[MODE == SIGNS ? NEC : 1][KCm][TB];
-    __shared__ double Vq[MODE == SIGNS ? NEC : 1][KCm][TB];
-    __shared__ double Sp[MODE == SIGNS ? KCm : 1][TB];
-    __shared__ double Sq[MODE == SIGNS ? KCm : 1][TB];
-    extern __shared__ unsigned int s_hist[];
-    // the thresholds after the counts, 8-byte aligned (the first stage's
-    // barrier orders these writes before any read)
+// Both log-likelihoods of a score, in the form that the parameters allow.
+__device__ inline void f_pair(const TriArgs& a, double x, double& ind, double& arb) {
+    if (a.lform) f_both(x, a.prm, a.lg, ind, arb);
+    else {
+        ind = f_ind(x, a.prm);
+        arb = f_arb(x, a.prm);
+    }
+}
+
+// Both log-likelihoods of the scores of one stage of third images with one
+// logarithm and one exponential per score, for A, B > 0, a, b > 0, 0 <= P2 < 1
+// and x0 < 1.  With u = 1 - x, mn = min(a, b) and df = |b - a|,
+//   f_ind(x) = u^mn g,   g = c_b u^(b - mn) e^(-b/(1-x0) u) + c_a u^(a - mn),
+// c_b = P2 B, c_a = (1 - P2) A (one of the two powers is 1, the other u^df),
+// so sum log f_ind = mn sum log u + log prod g: the stage's product has one
+// logarithm.  It is kept as mantissa and exponent, so it neither over- nor
+// underflows.
+struct LikeSum {
+    double lu = 0.0, mant = 1.0;
+    int ex = 0;
+    // adds the score's g to the product; returns log f_arb
+    __device__ inline double add(const TriArgs& a, double x) {
+        const double u = 1 - x, l = log(u);
+        const double pw = a.lk[1] == 0.0 ? 0.0 : a.lk[1] * l;  // u = 0: 0^0 = 1
+        double g;
+        if (a.prm[4] >= a.prm[2]) g = fma(a.lk[2], exp(fma(a.lg[3], u, pw)), a.lk[3]);  // b >= a
+        else                      g = fma(a.lk[2], exp(a.lg[3] * u), a.lk[3] * exp(pw));
+        lu += l;
+        const double m = mant * g;
+        ex += __builtin_amdgcn_frexp_exp(m);
+        mant = __builtin_amdgcn_frexp_mant(m);
+        return a.lg[0] + a.prm[2] * l;
+    }
+    // log f_ind of the scores added since the last call
+    __device__ inline double ind(const TriArgs& a) {
+        const double r = a.lk[0] * lu + (log(mant) + ex * 0.693147180559945309417);
+        *this = LikeSum();
+        return r;
+    }
+};
+
+// Staged operands of KCm third images: their rotations (and vectors, pair
+// scores) against the workgroup's 16 p- and 16 q-images.
+template <int MODE, int NEC, int KCm> struct Stage {
+    double Lp[9][KCm][TB], Lq[9][KCm][TB];
+    double Vp[MODE == SIGNS ? NEC : 1][KCm][TB], Vq[MODE == SIGNS ? NEC : 1][KCm][TB];
+    double Sp[MODE == SIGNS ? KCm : 1][TB], Sq[MODE == SIGNS ? KCm : 1][TB];
+};
+
+template <int R> struct Role {
+    static constexpr int value = R;
+};
+
+// Counts of the scores in LDS and the thresholds after them, 8-byte aligned;
+// the first stage's barrier orders these writes before any read.
+extern __shared__ unsigned int s_hist[];
+template <bool TL>
+__device__ inline const double* hist_begin(const TriArgs& a) {
     double* s_thr = (double*)(s_hist + ((a.n_intervals + 1) & ~1));
+    for (int l = threadIdx.x; l < a.n_intervals; l += blockDim.x) s_hist[l] = 0;
+    if (TL)
+        for (int l = threadIdx.x; l < a.n_intervals - 1; l += blockDim.x) s_thr[l] = a.thr[l];
+    return TL ? s_thr : a.thr;
+}
+
+// Rs (Vs, Ss) of the third images [k0, k0 + KCm) below m1 against the p- and
+// q-images, zero past the ends; every thread of the workgroup takes part.
+template <int MODE, int NEC, int KCm>
+__device__ __forceinline__ void stage(const TriArgs& a, Stage<MODE, NEC, KCm>& sm, int p0, int q0, int k0, int m1) {
     const int N = a.N;
     const long long NN = (long long)N * N;
-    const int tid = threadIdx.x;
-    if (MODE == SCORES) {
-        for (int l = tid; l < a.n_intervals; l += blockDim.x) s_hist[l] = 0;
-        if (TL)
-            for (int l = tid; l < a.n_intervals - 1; l += blockDim.x) s_thr[l] = a.thr[l];
+    const int tid = threadIdx.x, nt = blockDim.x;
+    for (int x = tid; x < 9 * KCm * TB; x += nt) {
+        const int e = x / (KCm * TB), kk = (x / TB) % KCm, j = x % TB;
+        const int k = k0 + kk;
+        const bool okp = k < m1 && p0 + j < N, okq = k < m1 && q0 + j < N;
+        sm.Lp[e][kk][j] = okp ? a.Rs[e * NN + (long long)k * N + p0 + j] : 0.0;
+        sm.Lq[e][kk][j] = okq ? a.Rs[e * NN + (long long)k * N + q0 + j] : 0.0;
     }
+    if constexpr (MODE == SIGNS) {
+        for (int x = tid; x < a.ne * KCm * TB; x += nt) {
+            const int g = x / (KCm * TB), kk = (x / TB) % KCm, j = x % TB;
+            const int k = k0 + kk;
+            sm.Vp[g][kk][j] = (k < m1 && p0 + j < N) ? a.Vs[g * NN + (long long)k * N + p0 + j] : 0.0;
+            sm.Vq[g][kk][j] = (k < m1 && q0 + j < N) ? a.Vs[g * NN + (long long)k * N + q0 + j] : 0.0;
+        }
+        if (a.entries == 2)
+            for (int x = tid; x < KCm * TB; x += nt) {
+                const int kk = x / TB, j = x % TB, k = k0 + kk;
+                sm.Sp[kk][j] = (k < m1 && p0 + j < N) ? a.Ss[(long long)k * N + p0 + j] : 0.0;
+                sm.Sq[kk][j] = (k < m1 && q0 + j < N) ? a.Ss[(long long)k * N + q0 + j] : 0.0;
+            }
+    }
+}
+
+// What third image m (staged as kk) adds to the pair (p, q): t0, t1 (scores;
+// both log-likelihoods) or tv (per vector), as the reference's single-thread
+// loop would add it.  ROLE: the pair's role where it is the same for the whole
+// workgroup and stage (0: ij, 1: jk, 2: ik), else -1; a role known at compile
+// time spares the selects of 27 matrix entries.
+template <int MODE, int NEC, int ROLE, bool OPT, int KCm>
+__device__ __forceinline__ void visit(const TriArgs& a, const Stage<MODE, NEC, KCm>& sm, const double* thr,
+                                      const double* Rpq, int p, int q, int m, int kk, double& t0, double& t1,
+                                      double* tv, LikeSum& like) {
+    const int tp = p % TB, tq = q % TB;
+    double Rpm[9], Rqm[9];
+#pragma unroll
+    for (int e = 0; e < 9; e++) {
+        Rpm[e] = sm.Lp[e][kk][tp];
+        Rqm[e] = sm.Lq[e][kk][tq];
+    }
+    // the triangle in the reference's (i, j, k) order and this pair's role in
+    // it: m > q: pair is ij, sides (p,q),(q,m),(p,m); p < m < q: pair is ik,
+    // sides (p,m),(m,q),(p,q); m < p: pair is jk, sides (m,p),(p,q),(m,q)
+    const int role = ROLE >= 0 ? ROLE : (m > q ? 0 : (m > p ? 2 : 1));
+    const double* Rij = role == 0 ? Rpq : Rpm;
+    const double* Rjk = role == 1 ? Rpq : Rqm;
+    const double* Rik = role == 0 ? Rpm : (role == 2 ? Rpq : Rqm);
+    // side pairs touching this pair: ij -> (0, 2), jk -> (0, 1), ik -> (1, 2);
+    // the histogram takes (ij,jk) from ij, (ik,jk) from jk, (ij,ik) from ik
+    const int qa = role == 2 ? 1 : 0;
+    const int qb = role == 1 ? 1 : 2;
+    const Tri tr = triangle(Rij, Rjk, Rik);
+    const double aa = qa ? tr.alt[1] : tr.alt[0], ab = qb == 1 ? tr.alt[1] : tr.alt[2];
+    double sa = 0.0, sb = 0.0;
+    if (MODE != SIGNS || a.entries == 1) {
+        sa = score(tr.bv, aa);
+        sb = score(tr.bv, ab);
+    }
+    if constexpr (MODE == SCORES) {
+        t0 = sa + sb;
+        atomicAdd(&s_hist[bin_of(role == 0 ? sa : sb, thr, a.n_intervals)], 1u);
+    } else if constexpr (MODE == PROBS) {
+        if constexpr (OPT) {
+            const double la = like.add(a, sa), lb = like.add(a, sb);
+            t1 = la + lb;
+        } else {
+            double ia, la, ib, lb;
+            f_pair(a, sa, ia, la);
+            f_pair(a, sb, ib, lb);
+            t0 = ia + ib;
+            t1 = la + lb;
+        }
+    } else {
+        double ea = sgn(tr.best, qa), eb = sgn(tr.best, qb);
+        if (a.entries == 1) {
+            ea = ea * sa;
+            eb = eb * sb;
+        } else if (a.entries == 2) {
+            // pair_scores[ij]*pair_scores[jk]*pair_scores[ik] in that order
+            const double spq = a.Ss[(long long)p * a.N + q], spm = sm.Sp[kk][tp], sqm = sm.Sq[kk][tq];
+            const double sij = role == 0 ? spq : spm, sjk = role == 1 ? spq : sqm;
+            const double sik = role == 0 ? spm : (role == 2 ? spq : sqm);
+            const double tsc = sij * sjk * sik;
+            ea = ea * tsc;
+            eb = eb * tsc;
+        }
+        // ij: v2 += e(ij,jk) v[jk] + e(ij,ik) v[ik]; jk: e(ij,jk) v[ij] + e(ik,jk) v[ik];
+        // ik: e(ij,ik) v[ij] + e(ik,jk) v[jk]
+#pragma unroll
+        for (int g = 0; g < NEC; g++) {
+            if (g >= a.ne) break;
+            const double vpm = sm.Vp[g][kk][tp], vqm = sm.Vq[g][kk][tq];
+            const double x = role == 0 ? ea * vqm : (role == 1 ? ea * vpm : eb * vpm);
+            const double y = role == 0 ? eb * vpm : (role == 1 ? eb * vqm : ea * vqm);
+            tv[g] = x + y;
+        }
+    }
+}
+
+// NEC: vectors the signs product stages (a.ne <= NEC).  Eight third images per
+// stage: 21 KB of LDS (29 with four vectors), so that four workgroups share a
+// CU (at 16 per stage three did); the stage size does not change the order of
+// any sum.
+// Bound: FP64 issue.  At N = 1000 the scores kernel issues 280 vector
+// instructions per visit (142 operations for the mismatches, the rest two
+// divisions and square roots, the bin and addresses) on 82% of the cycles.
+// OPT: the scores' thresholds are in LDS; the likelihoods are summed by LikeSum.
+template <int MODE, int NEC = 1, bool OPT = false>
+__device__ __forceinline__ void tri_pairs(TriArgs a) {
+    constexpr int KCm = KC, NV = MODE == SIGNS ? NEC : 1;
+    __shared__ Stage<MODE, NEC, KCm> sm;
+    const double* thr = nullptr;
+    if (MODE == SCORES) thr = hist_begin<OPT>(a);
+    const int N = a.N;
+    const long long NN = (long long)N * N;
     for (int t = blockIdx.x; t < a.ntiles; t += gridDim.x) {
         const int2 bt = a.tiles[t];
         const int p0 = bt.x * TB, q0 = bt.y * TB;
-        const int tp = tid / TB, tq = tid % TB;
-        const int p = p0 + tp, q = q0 + tq;
+        const int p = p0 + threadIdx.x / TB, q = q0 + threadIdx.x % TB;
         const bool act = p < q && q < N;
         double Rpq[9];
 #pragma unroll
         for (int e = 0; e < 9; e++) Rpq[e] = act ? a.Rs[e * NN + (long long)p * N + q] : 0.0;
-        double acc0 = 0.0, acc1 = 0.0;
-        double vacc[MODE == SIGNS ? NEC : 1];
+        double acc0 = 0.0, acc1 = 0.0, vacc[NV];
+        LikeSum like;
 #pragma unroll
-        for (int g = 0; g < (MODE == SIGNS ? NEC : 1); g++) vacc[g] = 0.0;
+        for (int g = 0; g < NV; g++) vacc[g] = 0.0;
         for (int k0 = 0; k0 < N; k0 += KCm) {
             __syncthreads();
-            // stage Rs[e][k][p0..p0+15] and Rs[e][k][q0..q0+15] for k in [k0, k0+KCm)
-            for (int x = tid; x < 9 * KCm * TB; x += blockDim.x) {
-                const int e = x / (KCm * TB), kk = (x / TB) % KCm, j = x % TB;
-                const int k = k0 + kk;
-                const bool okp = k < N && p0 + j < N, okq = k < N && q0 + j < N;
-                Lp[e][kk][j] = okp ? a.Rs[e * NN + (long long)k * N + p0 + j] : 0.0;
-                Lq[e][kk][j] = okq ? a.Rs[e * NN + (long long)k * N + q0 + j] : 0.0;
-            }
-            if constexpr (MODE == SIGNS) {
-                for (int x = tid; x < a.ne * KCm * TB; x += blockDim.x) {
-                    const int g = x / (KCm * TB), kk = (x / TB) % KCm, j = x % TB;
-                    const int k = k0 + kk;
-                    Vp[g][kk][j] = (k < N && p0 + j < N) ? a.Vs[g * NN + (long long)k * N + p0 + j] : 0.0;
-                    Vq[g][kk][j] = (k < N && q0 + j < N) ? a.Vs[g * NN + (long long)k * N + q0 + j] : 0.0;
-                }
-                if (a.entries == 2)
-                    for (int x = tid; x < KCm * TB; x += blockDim.x) {
-                        const int kk = x / TB, j = x % TB, k = k0 + kk;
-                        Sp[kk][j] = (k < N && p0 + j < N) ? a.Ss[(long long)k * N + p0 + j] : 0.0;
-                        Sq[kk][j] = (k < N && q0 + j < N) ? a.Ss[(long long)k * N + q0 + j] : 0.0;
-                    }
-            }
+            stage(a, sm, p0, q0, k0, N);
             __syncthreads();
             if (!act) continue;
             const int kend = min(KCm, N - k0);
-            for (int kk = 0; kk < kend; kk++) {
-                const int m = k0 + kk;
-                if (m == p || m == q) continue;
-                double Rpm[9], Rqm[9];
+            auto walk = [&](auto role) {
+                for (int kk = 0; kk < kend; kk++) {
+                    const int m = k0 + kk;
+                    if (decltype(role)::value < 0 && (m == p || m == q)) continue;
+                    double t0 = 0.0, t1 = 0.0, tv[NV];
+                    visit<MODE, NEC, decltype(role)::value, OPT>(a, sm, thr, Rpq, p, q, m, kk, t0, t1, tv, like);
+                    if constexpr (MODE == SIGNS) {
 #pragma unroll
-                for (int e = 0; e < 9; e++) {
-                    Rpm[e] = Lp[e][kk][tp];
-                    Rqm[e] = Lq[e][kk][tq];
-                }
-                // the triangle in the reference's (i, j, k) order and this
-                // pair's role in it: m > q: pair is ij, sides (p,q),(q,m),(p,m);
-                // p < m < q: pair is ik, sides (p,m),(m,q),(p,q);
-                // m < p: pair is jk, sides (m,p),(p,q),(m,q)
-                const int role = m > q ? 0 : (m > p ? 2 : 1);
-                const double* Rij = role == 0 ? Rpq : (role == 2 ? Rpm : Rpm);
-                const double* Rjk = role == 0 ? Rqm : (role == 2 ? Rqm : Rpq);
-                const double* Rik = role == 0 ? Rpm : (role == 2 ? Rpq : Rqm);
-                // side pairs touching this pair: ij -> (0, 2), jk -> (0, 1), ik -> (1, 2);
-                // the histogram takes (ij,jk) from ij, (ik,jk) from jk, (ij,ik) from ik
-                const int qa = role == 2 ? 1 : 0;
-                const int qb = role == 1 ? 1 : 2;
-                const Tri tr = triangle(Rij, Rjk, Rik);
-                const int best = tr.best;
-                double sa = 0.0, sb = 0.0;
-                if (MODE != SIGNS || a.entries == 1) {
-                    sa = score(tr, qa);
-                    sb = score(tr, qb);
-                }
-                if constexpr (MODE == SCORES) {
-                    acc0 += sa + sb;
-                    const double hs = role == 0 ? sa : (role == 1 ? sb : sb);
-                    const int bin = TL ? bin_of(hs, s_thr, a.n_intervals) : bin_of(hs, a.thr, a.n_intervals);
-                    atomicAdd(&s_hist[bin], 1u);
-                } else if constexpr (MODE == PROBS) {
-                    if (a.lform) {
-                        double ia, aa, ib, ab;
-                        f_both(sa, a.prm, a.lg, ia, aa);
-                        f_both(sb, a.prm, a.lg, ib, ab);
-                        acc0 += ia + ib;
-                        acc1 += aa + ab;
+                        for (int g = 0; g < NEC; g++)
+                            if (g < a.ne) vacc[g] += tv[g];
                     } else {
-                        acc0 += f_ind(sa, a.prm) + f_ind(sb, a.prm);
-                        acc1 += f_arb(sa, a.prm) + f_arb(sb, a.prm);
-                    }
-                } else {
-                    double ea, eb;
-                    const double sga = sgn(best, qa), sgb = sgn(best, qb);
-                    if (a.entries == 1) {
-                        ea = sga * sa;
-                        eb = sgb * sb;
-                    } else if (a.entries == 2) {
-                        // pair_scores[ij]*pair_scores[jk]*pair_scores[ik] in that order
-                        const double spq = a.Ss[(long long)p * N + q], spm = Sp[kk][tp], sqm = Sq[kk][tq];
-                        const double sij = role == 0 ? spq : spm, sjk = role == 0 ? sqm : (role == 2 ? sqm : spq);
-                        const double sik = role == 0 ? spm : (role == 2 ? spq : sqm);
-                        const double tsc = sij * sjk * sik;
-                        ea = sga * tsc;
-                        eb = sgb * tsc;
-                    } else {
-                        ea = sga;
-                        eb = sgb;
-                    }
-                    // ij: v2 += e(ij,jk) v[jk] + e(ij,ik) v[ik]; jk: e(ij,jk) v[ij] + e(ik,jk) v[ik];
-                    // ik: e(ij,ik) v[ij] + e(ik,jk) v[jk]
-#pragma unroll
-                    for (int g = 0; g < NEC; g++) {
-                        if (g >= a.ne) break;
-                        const double vpm = Vp[g][kk][tp], vqm = Vq[g][kk][tq];
-                        const double x = role == 0 ? ea * vqm : (role == 1 ? ea * vpm : eb * vpm);
-                        const double y = role == 0 ? eb * vpm : (role == 1 ? eb * vqm : ea * vqm);
-                        vacc[g] += x + y;
+                        acc0 += t0;
+                        acc1 += t1;
                     }
                 }
-            }
+            };
+            // the stage's third images all after the q-block, all before the
+            // p-block, all between, or some among the pair's own blocks
+            if (k0 >= q0 + TB) walk(Role<0>());
+            else if (k0 + KCm <= p0) walk(Role<1>());
+            else if (k0 >= p0 + TB && k0 + KCm <= q0) walk(Role<2>());
+            else walk(Role<-1>());
+            if (MODE == PROBS && OPT) acc0 += like.ind(a);
         }
         if (act) {
             const long long e = pidx(N, p, q);
@@ -361,7 +451,7 @@ __device__ __forceinline__ void tri_pairs(TriArgs a) {
     }
     if (MODE == SCORES) {
         __syncthreads();
-        for (int l = tid; l < a.n_intervals; l += blockDim.x)
+        for (int l = threadIdx.x; l < a.n_intervals; l += blockDim.x)
             if (s_hist[l]) atomicAdd(&a.hist[l], (unsigned long long)s_hist[l]);
     }
 }
@@ -376,16 +466,17 @@ __global__ void zero_u64_kernel(unsigned long long* p, int n) {
     if (l < n) p[l] = 0ull;
 }
 
-// One kernel per mode, for their own occupancy: the scores fit 128 VGPRs
-// (four waves per SIMD); the probabilities (log, exp, log1p) need more and
-// run at two; the signs product runs at three for up to four vectors (its
-// LDS and registers sized for them), at two for up to eight.
+// One kernel per mode, for their own registers: four waves per SIMD except
+// the likelihoods with a logarithm per score and the signs product of more than
+// four vectors.  N = 1000 (1.66e8 triangles): scores 5.1 ms, likelihoods 8.1,
+// signs of four vectors 4.1; with the roles of a triangle's sides selected per
+// visit, three waves per SIMD and log1p per score 5.9, 13.1 and 5.9 ms.
 template <bool TL>
 __global__ __launch_bounds__(256, 4) void tri_scores_kernel(TriArgs a) { tri_pairs<SCORES, 1, TL>(a); }
 __global__ __launch_bounds__(256) void tri_probs_kernel(TriArgs a) { tri_pairs<PROBS>(a); }
-__global__ __launch_bounds__(256, 3) void tri_signs4_kernel(TriArgs a) { tri_pairs<SIGNS, 4>(a); }
+__global__ __launch_bounds__(256, 4) void tri_like_kernel(TriArgs a) { tri_pairs<PROBS, 1, true>(a); }
+__global__ __launch_bounds__(256, 4) void tri_signs4_kernel(TriArgs a) { tri_pairs<SIGNS, 4>(a); }
 __global__ __launch_bounds__(256) void tri_signs8_kernel(TriArgs a) { tri_pairs<SIGNS, MAXE>(a); }
-
 }  // namespace s3
 
 using namespace clmh;
@@ -452,7 +543,10 @@ int s3_launch(clm_ctx* c, const s3::TriArgs& a, size_t dyn_lds) {
         else
             s3::tri_scores_kernel<false><<<grid, 256, dyn_lds, c->stream>>>(a);
     else if constexpr (MODE == s3::PROBS)
-        s3::tri_probs_kernel<<<grid, 256, dyn_lds, c->stream>>>(a);
+        if (a.lform == 2)
+            s3::tri_like_kernel<<<grid, 256, dyn_lds, c->stream>>>(a);
+        else
+            s3::tri_probs_kernel<<<grid, 256, dyn_lds, c->stream>>>(a);
     else if (a.ne <= 4)
         s3::tri_signs4_kernel<<<grid, 256, dyn_lds, c->stream>>>(a);
     else
@@ -518,6 +612,15 @@ extern "C" int clm_sync3n_pairs_probabilities(clm_ctx* c, int32_t N, const doubl
         a.lg[1] = std::log(P2 * B);
         a.lg[2] = std::log((1 - P2) * A);
         a.lg[3] = -eb / (1 - x0);
+        a.lk[0] = std::min(ea, eb);
+        a.lk[1] = std::fabs(eb - ea);
+        a.lk[2] = P2 * B;
+        a.lk[3] = (1 - P2) * A;
+        // products of the likelihoods where no factor over- or underflows:
+        // the exponential's argument at most 0, the arbitrary model present,
+        // and u^df (u >= 2^-53 or 0) far from the smallest number
+        if (a.lform && x0 < 1 && a.lk[1] <= 16 && a.lk[3] >= 1e-100 && a.lk[3] <= 1e100 && a.lk[2] <= 1e100)
+            a.lform = 2;
     }
     a.ind = d_ln_f_ind;
     a.arb = d_ln_f_arb;
