@@ -821,9 +821,7 @@ __global__ void window_merge_kernel(int K, int L, const double* __restrict__ lsh
 // Common lines of known rotations and the best 1-D shift along each: the
 // per-pair loop of cryo_estimate_shifts.m:142-223 (pair order k1 < k2; the
 // reference draws its pairs in random order, which the solution does not
-// depend on).  One wave per pair; lane s evaluates the shifts s, s + 64, ...
-// with the FP64 terms of eval64 added in order over the ray, then the wave
-// finds the first maximum of C1 and of C2 (NaN ignored, as MATLAB's max).
+// depend on).
 __device__ inline bool first_max(double v, int s, double bv, int bs) {
     return !isnan(v) && (isnan(bv) || v > bv || (v == bv && s < bs));
 }
@@ -832,29 +830,91 @@ __device__ inline bool first_max(double v, int s, double bv, int bs) {
 // wave-uniform address become scalar loads.
 typedef const double __attribute__((address_space(4)))* ConstD;
 
-// One wave takes 64 consecutive pairs at a time: each lane writes the
-// outputs of its pair if the selection leaves it out (coalesced), then the
-// wave computes the selected ones one after another (a ballot lists them).
-// With PH_LDS the shift phases are staged in LDS once per workgroup as
-// [r][s], so that the lanes (one per shift) read consecutive entries at
-// each ray index; otherwise they are read from the [s][r] table in global
-// memory.  Eight waves per workgroup share one staged table.
+// The shift index of one pair's rays p (image k1) and b (image k2) as the
+// reference finds it: lane s evaluates the shifts s, s + 64, ... with the FP64
+// terms of eval64 added in order over the ray, then the wave finds the first
+// maximum of C1 and of C2 (NaN ignored, as MATLAB's max).  Called by the whole
+// wave with uniform rays.
+__device__ inline int shift_by_terms(const Geom& g, const double2* ph64, const double2* ray1, const double2* ray2,
+                                     int lane) {
+    const ConstD ri = (ConstD)ray1, rj = (ConstD)ray2;
+    double b1 = NAN, b2 = NAN;
+    int s1 = 0, s2 = 0;
+    for (int s0 = 0; s0 < g.S; s0 += 64) {
+        const int s = s0 + lane;
+        const int sc = s < g.S ? s : g.S - 1;
+        double a1 = 0.0, a2 = 0.0;
+        for (int r = 0; r < g.R; r++) {
+            const double2 pv = make_double2(ri[2 * r], ri[2 * r + 1]);
+            const double2 bv = make_double2(rj[2 * r], rj[2 * r + 1]);
+            const double2 qv = ph64[(size_t)sc * g.R + r];
+            a1 = a1 + term64(pv, qv, bv, false);
+            a2 = a2 + term64(pv, qv, bv, true);
+        }
+        const double c1 = 2.0 * a1, c2 = 2.0 * a2;
+        if (s < g.S && first_max(c1, s, b1, s1)) { b1 = c1; s1 = s; }
+        if (s < g.S && first_max(c2, s, b2, s2)) { b2 = c2; s2 = s; }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const double v1 = __shfl_xor(b1, o, 64), v2 = __shfl_xor(b2, o, 64);
+        const int t1 = __shfl_xor(s1, o, 64), t2 = __shfl_xor(s2, o, 64);
+        if (first_max(v1, t1, b1, s1)) { b1 = v1; s1 = t1; }
+        if (first_max(v2, t2, b2, s2)) { b2 = v2; s2 = t2; }
+    }
+    // an all-NaN max is NaN at index 1 (s = 0) in MATLAB, as here
+    return b1 > b2 ? s1 : s2;
+}
 
+// Largest and second largest value, and the largest's index.
+struct Top2 {
+    double v, w;
+    int s;
+    __device__ inline void add(double x, int sx) {
+        if (x > v) { w = v; v = x; s = sx; }
+        else if (x > w) w = x;
+    }
+    __device__ inline void join(double ov, double ow, int os) {
+        if (ov > v) { w = fmax(v, ow); v = ov; s = os; }
+        else w = fmax(w, ov);
+    }
+};
+
+// One wave takes 64 consecutive pairs at a time.  Each lane finds its own
+// pair's common line (and writes the outputs of a pair that the selection
+// leaves out); the selected pairs are then correlated 16 at a time on the FP64
+// matrix cores: with z = conj(p) b and w = p b (p, b the pair's rays),
+//   C1(s) = 2 sum_r cos z.re + sin z.im,   C2(s) = 2 sum_r cos w.re + sin w.im,
+// cos + i sin = ph_s(r), a product of the pairs' rows (r, re and im) with the
+// table of phases.  Only the index of the maximum is kept, so it is certain
+// where the winning value is farther from the next one, and from the other
+// map's best, than both evaluations' rounding (eps64 of the image norms);
+// otherwise the pair is evaluated term by term.
+// Bound: the gather of the rays (2 KB per pair at n_r = 65) and FP64 MFMA
+// about equally.  0.71 ms for 1.12 M pairs, 41 shifts, n_r = 65 (3.3 TB/s of
+// rays); with a wave per pair, a lane per shift and every term in the oracle's
+// order it took 4.05 ms.
+// With PH_LDS the shift phases are staged in LDS once per workgroup as [r][s],
+// so that the lanes (one per shift) read consecutive entries at each ray
+// index; otherwise they are read from the [s][r] table in global memory.
 template <bool PH_LDS>
-__global__ __launch_bounds__(512) void rotlines_kernel(const StackDev* __restrict__ sdp,
-                                                       const double* __restrict__ rot,
-                                                       const uint8_t* __restrict__ sel, int n_theta,
-                                                       int32_t* __restrict__ cl1, int32_t* __restrict__ cl2,
-                                                       double* __restrict__ shift1d) {
+__global__ __launch_bounds__(512, 4) void rotlines_kernel(const StackDev* __restrict__ sdp,
+                                                          const double* __restrict__ rot,
+                                                          const uint8_t* __restrict__ sel, int n_theta,
+                                                          int32_t* __restrict__ cl1, int32_t* __restrict__ cl2,
+                                                          double* __restrict__ shift1d) {
+    typedef double d4 __attribute__((ext_vector_type(4)));
     extern __shared__ double2 s_ph[];  // [R][S] when PH_LDS
     const StackDev& sd = *sdp;
     const Geom g = sd.g;
+    const double2* const ph64 = sd.ph64;
+    const double2* const P64 = sd.P64;
     const long long K = g.K, P = K * (K - 1) / 2;
-    const int lane = threadIdx.x & 63;
+    const int lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
     if (PH_LDS) {
         for (int i = threadIdx.x; i < g.S * g.R; i += blockDim.x) {
             const int s = i / g.R, r = i - s * g.R;
-            s_ph[r * g.S + s] = sd.ph64[i];
+            s_ph[r * g.S + s] = ph64[i];
         }
         __syncthreads();
     }
@@ -869,22 +929,18 @@ __global__ __launch_bounds__(512) void rotlines_kernel(const StackDev* __restric
             cl2[el] = -1;
             shift1d[el] = 0.0;
         }
-        unsigned long long todo = __ballot(act);
-        while (todo) {
-            const long long e = base + __builtin_ctzll(todo);
-            todo &= todo - 1;
-            // (k1, k2) of pair e
-            long long k1 = (long long)floor(((2.0 * K - 1.0) - sqrt((2.0 * K - 1.0) * (2.0 * K - 1.0) - 8.0 * (double)e)) / 2.0);
-            if (k1 < 0) k1 = 0;
-            if (k1 > K - 2) k1 = K - 2;
-            auto first = [&](long long x) { return x * K - x * (x + 1) / 2; };
-            while (k1 > 0 && first(k1) > e) k1--;
-            while (k1 + 1 <= K - 2 && first(k1 + 1) <= e) k1++;
-            const long long k2 = e - first(k1) + k1 + 1;
+        const unsigned long long todo = __ballot(act);
+        if (!todo) continue;
+        // ---- the lane's pair: rays (image and line) of both images
+        int ray1 = 0, ray2 = 0;  // k L + line
+        double tol = 0.0;
+        if (act) {
+            int q1, q2;
+            slot_to_pair(el, (int)K, q1, q2);
             // commonline_R(R_k1.', R_k2.', n_theta): Ut = R_k2.' * R_k1, entry
             // (a, b) = sum over m of R_k2(m, a) R_k1(m, b), m in order
-            const double* Ri = rot + 9 * k1;
-            const double* Rj = rot + 9 * k2;
+            const double* Ri = rot + 9 * (size_t)q1;
+            const double* Rj = rot + 9 * (size_t)q2;
             auto ut = [&](int a, int b) {
                 return (Rj[3 * a] * Ri[3 * b] + Rj[1 + 3 * a] * Ri[1 + 3 * b]) + Rj[2 + 3 * a] * Ri[2 + 3 * b];
             };
@@ -904,53 +960,101 @@ __global__ __launch_bounds__(512) void rotlines_kernel(const StackDev* __restric
                 cji -= L2;
             }
             if (cji < 0) cji += n_theta;
-            cij += 1;
-            cji += 1;
-            // the two rays are the same for every lane: read through the
-            // constant address space, so that they come in by scalar loads
-            // (one per wave) instead of a vector load of one address per lane
-            // (values computed in vector registers from uniform inputs; read
-            // from the first lane so that the addresses are scalar)
-            const int lj = __builtin_amdgcn_readfirstlane(cji <= L2 ? cji - 1 : cji - 1 - L2);
-            const int li = __builtin_amdgcn_readfirstlane(cij - 1);
-            const int q1 = __builtin_amdgcn_readfirstlane((int)k1), q2 = __builtin_amdgcn_readfirstlane((int)k2);
-            const ConstD ri = (ConstD)(sd.P64 + ((size_t)q1 * g.L + li) * g.R);
-            const ConstD rj = (ConstD)(sd.P64 + ((size_t)q2 * g.L + lj) * g.R);
-            double b1 = NAN, b2 = NAN;
-            int s1 = 0, s2 = 0;
-            // the shift loop is uniform (lanes past the last shift compute
-            // the last one again and are ignored), so the ray loop runs
-            // outside divergent control and its ray addresses stay scalar
-            for (int s0 = 0; s0 < g.S; s0 += 64) {
-                const int s = s0 + lane;
-                const int sc = s < g.S ? s : g.S - 1;
-                double a1 = 0.0, a2 = 0.0;
-#pragma unroll 4
-                for (int r = 0; r < g.R; r++) {
-                    const double2 pv = make_double2(ri[2 * r], ri[2 * r + 1]);
-                    const double2 bv = make_double2(rj[2 * r], rj[2 * r + 1]);
-                    const double2 qv = PH_LDS ? s_ph[r * g.S + sc] : sd.ph64[(size_t)sc * g.R + r];
-                    a1 = a1 + term64(pv, qv, bv, false);
-                    a2 = a2 + term64(pv, qv, bv, true);
-                }
-                const double c1 = 2.0 * a1, c2 = 2.0 * a2;
-                if (s < g.S && first_max(c1, s, b1, s1)) { b1 = c1; s1 = s; }
-                if (s < g.S && first_max(c2, s, b2, s2)) { b2 = c2; s2 = s; }
-            }
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) {
-                const double v1 = __shfl_xor(b1, o, 64), v2 = __shfl_xor(b2, o, 64);
-                const int t1 = __shfl_xor(s1, o, 64), t2 = __shfl_xor(s2, o, 64);
-                if (first_max(v1, t1, b1, s1)) { b1 = v1; s1 = t1; }
-                if (first_max(v2, t2, b2, s2)) { b2 = v2; s2 = t2; }
-            }
-            if (lane == 0) {
-                // an all-NaN max is NaN at index 1 (s = 0) in MATLAB, as here
-                cl1[e] = cij;
-                cl2[e] = cji;
-                shift1d[e] = sd.shiftv[b1 > b2 ? s1 : s2];
+            cl1[el] = cij + 1;
+            cl2[el] = cji + 1;
+            ray1 = q1 * g.L + cij;
+            ray2 = q2 * g.L + (cji < L2 ? cji : cji - L2);
+            tol = 2.0 * sd.eps64 * (double)sd.nrm[q1] * (double)sd.nrm[q2];
+        }
+        // ---- 16 selected pairs at a time: row r16 is the (first + r16)-th
+        const int n = __popcll(todo), at = __popcll(todo & lanemask_lt());
+        // lane i of `src` holds the lane of the i-th selected pair
+        int src = 0;
+        {
+            unsigned long long m = todo;
+            for (int i = 0; i < n; i++) {
+                const int l = __builtin_ctzll(m);
+                m &= m - 1;
+                if (lane == i) src = l;
             }
         }
+        int win = -1;  // this lane's pair's shift index
+        for (int first = 0; first < n; first += 16) {
+            const int from = __shfl(src, min(first + r16, n - 1), 64);
+            const double2* p = P64 + (size_t)__shfl(ray1, from, 64) * g.R;
+            const double2* b = P64 + (size_t)__shfl(ray2, from, 64) * g.R;
+            Top2 c1[4], c2[4];  // rows 4 i + kq of the two maps
+#pragma unroll
+            for (int i = 0; i < 4; i++) c1[i] = c2[i] = Top2{-INFINITY, -INFINITY, 0};
+            for (int s0 = 0; s0 < g.S; s0 += 48) {
+                d4 X[3], Y[3];
+#pragma unroll
+                for (int c = 0; c < 3; c++) X[c] = Y[c] = d4{0.0, 0.0, 0.0, 0.0};
+                int sc[3];
+#pragma unroll
+                for (int c = 0; c < 3; c++) sc[c] = min(s0 + 16 * c + r16, g.S - 1);
+#pragma unroll 2
+                for (int r0 = 0; r0 < g.R; r0 += 4) {
+                    const int r = r0 + kq;
+                    double2 pv = make_double2(0.0, 0.0), bv = pv;
+                    if (r < g.R) {
+                        pv = p[r];
+                        bv = b[r];
+                    }
+                    const int rc = min(r, g.R - 1);
+                    const double xx = pv.x * bv.x, yy = pv.y * bv.y, xy = pv.x * bv.y, yx = pv.y * bv.x;
+                    const double zr = xx + yy, zi = xy - yx, wr = xx - yy, wi = xy + yx;
+#pragma unroll
+                    for (int c = 0; c < 3; c++) {
+                        if (s0 + 16 * c >= g.S) break;
+                        const double2 q = PH_LDS ? s_ph[rc * g.S + sc[c]] : ph64[(size_t)sc[c] * g.R + rc];
+                        X[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(zr, q.x, X[c], 0, 0, 0);
+                        Y[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(wr, q.x, Y[c], 0, 0, 0);
+                        X[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(zi, q.y, X[c], 0, 0, 0);
+                        Y[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(wi, q.y, Y[c], 0, 0, 0);
+                    }
+                }
+#pragma unroll
+                for (int c = 0; c < 3; c++) {
+                    const int s = s0 + 16 * c + r16;
+                    if (s < g.S)
+#pragma unroll
+                        for (int i = 0; i < 4; i++) {
+                            c1[i].add(X[c][i], s);
+                            c2[i].add(Y[c][i], s);
+                        }
+                }
+            }
+            // over the 16 lanes of a row, then the row's pair takes its result
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+#pragma unroll
+                for (int o = 8; o > 0; o >>= 1) {
+                    c1[i].join(__shfl_xor(c1[i].v, o, 64), __shfl_xor(c1[i].w, o, 64), __shfl_xor(c1[i].s, o, 64));
+                    c2[i].join(__shfl_xor(c2[i].v, o, 64), __shfl_xor(c2[i].w, o, 64), __shfl_xor(c2[i].s, o, 64));
+                }
+                // row 4 i + q sits in lanes 16 q..: its pair reads it there
+                const int row = at - first;
+                const int from_lane = 16 * (row & 3);
+                const double v1 = __shfl(c1[i].v, from_lane & 63, 64), w1 = __shfl(c1[i].w, from_lane & 63, 64);
+                const double v2 = __shfl(c2[i].v, from_lane & 63, 64), w2 = __shfl(c2[i].w, from_lane & 63, 64);
+                const int t1 = __shfl(c1[i].s, from_lane & 63, 64), t2 = __shfl(c2[i].s, from_lane & 63, 64);
+                if (act && row >= 0 && row < 16 && (row >> 2) == i) {
+                    if (v1 - v2 > tol && v1 - w1 > tol) win = t1;
+                    else if (v2 - v1 > tol && v2 - w2 > tol) win = t2;
+                }
+            }
+        }
+        // the pairs whose maximum is not certain
+        unsigned long long open = __ballot(act && win < 0);
+        while (open) {
+            const int l = __builtin_ctzll(open);
+            open &= open - 1;
+            const int y1 = __builtin_amdgcn_readlane(ray1, l), y2 = __builtin_amdgcn_readlane(ray2, l);
+            const int s = shift_by_terms(g, ph64, P64 + (size_t)y1 * g.R, P64 + (size_t)y2 * g.R, lane);
+            if (lane == l) win = s;
+        }
+        if (act) shift1d[el] = sd.shiftv[win];
     }
 }
 
