@@ -207,7 +207,8 @@ def autotune(pf, max_shift=15, shift_step=1.0, precision="fp16", device=0, sampl
     ``sample_pairs`` pairs of ``pf`` (device tensor, column-major as for
     :func:`clmatrix_records`); later calls with ``variant=0`` on this device
     use the fastest.  Returns one dict per variant (variant = CT*100 + waves
-    per workgroup, lag, ms, pairs, us_per_kpair) and the chosen one."""
+    per workgroup, + 50 where a wave takes a pair's column groups one after
+    another; lag, ms, pairs, us_per_kpair) and the chosen one."""
     import torch
 
     base, dt, n_r, n_theta, K = _device_view(pf)

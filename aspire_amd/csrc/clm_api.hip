@@ -24,10 +24,13 @@ namespace {
 // Operand element kinds (prep_kernel's op_kind)
 enum { OPK_F32 = 0, OPK_BF16 = 1, OPK_F16 = 2 };
 
-// Kernel variant: column tiles per wave and waves per workgroup.
+// Kernel variant: column tiles per wave and waves per workgroup.  A pair's
+// CPP column groups go to CPP waves side by side or, in the first pass with
+// ser > 0, one after another to one of ser waves (a pair per wave).
 struct Variant {
-    int ct = 0, W = 0, CPP = 0, NCTp = 0;
+    int ct = 0, W = 0, CPP = 0, NCTp = 0, ser = 0;
 };
+constexpr int SER_ID = 50;  // added to the waves in the id of such a variant
 
 // Supported padded ray lengths (k-steps of 16).
 int pad_R(int R) {
@@ -37,13 +40,29 @@ int pad_R(int R) {
     return -1;
 }
 
-Variant choose_variant(int opk, int NCT, int Rp, int want_ct, int want_W) {
-    Variant best;
-    double best_waste = 1e9;
+// Waves of a workgroup that takes a pair per wave: FP32 fits more workgroups on
+// a CU (by registers), the 16-bit operands one or two.
+int serial_waves(int opk) { return opk == OPK_F32 ? 4 : 8; }
+
+// npairs: pairs of the first pass, or 0 where they are few or unknown.
+Variant choose_variant(int opk, int NCT, int Rp, int want_ct, int want_W, long long npairs, int n_cu) {
+    Variant best, even;
+    double best_waste = 1e9, best_cost = 0, even_cost = 0;
+    const bool passes = pair_passes(opk == OPK_F32 ? 4 : 2, Rp);
+    const int sw = serial_waves(opk);
+    const int want_ser = want_W > SER_ID ? want_W - SER_ID : 0;
+    if (want_ser && (want_ser != sw || !passes)) return best;
     const int cts_mfma16[] = {3, 2, 1};
     const int cts_f32[] = {2, 1};
     const int* cts = opk == OPK_F32 ? cts_f32 : cts_mfma16;
     const int ncts = opk == OPK_F32 ? 2 : 3;
+    // Column tiles of the busiest SIMD: a workgroup's waves go to the four SIMDs
+    // in turn, so W waves cost as many as the next multiple of four, and the
+    // last round of workgroups counts whole.
+    auto cost = [&](int waves, int per_tile, int tiles_per_wave) {
+        const long long per_round = (long long)per_tile * n_cu;
+        return (double)((npairs + per_round - 1) / per_round) * ((waves + 3) / 4) * tiles_per_wave;
+    };
     for (int i = 0; i < ncts; i++) {
         const int ct = cts[i];
         if (want_ct && ct != want_ct) continue;
@@ -52,16 +71,33 @@ Variant choose_variant(int opk, int NCT, int Rp, int want_ct, int want_W) {
         const int NCTp = (NCT + ct - 1) / ct * ct;
         const int CPP = NCTp / ct;
         if (CPP > 8) continue;
-        int W = want_W ? want_W : (8 / CPP) * CPP;
-        if (opk == OPK_F32 && !want_W) W = CPP * ((4 + CPP - 1) / CPP);  // at least 4 waves
+        int W = want_W && !want_ser ? want_W : (8 / CPP) * CPP;
+        if (opk == OPK_F32 && (!want_W || want_ser)) W = CPP * ((4 + CPP - 1) / CPP);  // at least 4 waves
         if (W < CPP || W % CPP || W > 8) continue;
+        Variant v;
+        v.ct = ct; v.W = W; v.CPP = CPP; v.NCTp = NCTp; v.ser = want_ser;
+        const double side = cost(W, W / CPP, ct), one = cost(sw, sw, NCTp);
         const double waste = (double)NCTp / NCT;
         if (waste < best_waste - 1e-9) {
             best_waste = waste;
-            best.ct = ct; best.W = W; best.CPP = CPP; best.NCTp = NCTp;
+            best = v;
+            best_cost = side;
+        }
+        const bool ser = passes && CPP > 1 && one < side;
+        if (!even.ct || (ser ? one : side) < even_cost) {
+            even_cost = ser ? one : side;
+            even = v;
+            even.ser = ser ? sw : 0;
         }
     }
-    return best;
+    if (want_W || want_ct || !npairs || !best.ct) return best;
+    // The least padding, unless another split loads the SIMDs more evenly by a
+    // tenth or more.  300 rays (five column tiles), five waves a pair put two
+    // on one SIMD; FP32, 31375 pairs of n_r = 44 with one wave through the five:
+    // 19.0 -> 10.7 ms; FP16, 124750 pairs of n_r = 45 with two waves of three tiles
+    // (one of padding): 25.6 -> 8.9 ms.  360 rays, BF16, 79800 pairs of n_r = 90: three
+    // waves a pair 16.7, one through the three 13.3 ms.
+    return even_cost < 0.9 * best_cost ? even : best;
 }
 
 PairFn pick_pair_kernel(int opk, int ct, int Rp, bool sym, bool emit) {
@@ -238,6 +274,7 @@ struct StackJob {
 // Stacks that share one pair-kernel instantiation (or the FP64 kernel).
 struct Group {
     int opk = 0, exact = 0, ct = 0, Rp = 0, sym = 0, W = 0, CPP = 0, lag = 0;
+    int ser = 0;                // first pass: waves of a workgroup, a pair each (0: CPP waves a pair)
     int sel = 0;                // one stack of selected pairs (device-built tiles and list)
     int filt = 0;               // (FP64 groups) map_filter_radius of its stacks
     int norefine = 0;           // no FP32 twin: uncertain pairs take the second operand-type pass
@@ -251,6 +288,9 @@ struct Group {
     size_t lds = 0;
     int occ = 1;
     const TileCache* tc = nullptr;
+    int waves1() const { return ser ? ser : W; }            // first pass: waves of a workgroup
+    int pairs1() const { return ser ? ser : W / CPP; }      // and its pairs
+    int occ1 = 1;                                            // and workgroups per CU
 };
 
 struct Plan {
@@ -319,14 +359,14 @@ int plan_stack(clm_ctx* c, const clm_params* p, StackJob& j) {
         for (const auto& e : c->tuned)
             if (e.first == key) { want_ct = e.second.x; want_W = e.second.y; want_lag = e.second.z; }
     }
-    j.v = choose_variant(j.opk, NCT, g.Rp, want_ct, want_W);
+    j.v = choose_variant(j.opk, NCT, g.Rp, want_ct, want_W, j.P, c->n_cu);
     if (!j.v.ct) return fail(c, CLM_E_UNSUP, "no kernel variant for L=%d (variant %d)", g.L, p->variant);
     g.NCT = j.v.NCTp;
     g.Lp = 32 * j.v.NCTp;
     g.NROWS = g.NE * g.L;
     g.NAT = (g.NROWS + 31) / 32;
     if ((long long)g.NROWS * g.Lp > 0xffffffffLL) return fail(c, CLM_E_UNSUP, "map too large");
-    j.lag = (j.v.W % 2 == 0 && want_lag && !(p->reserved & 1)) ? 1 : 0;
+    j.lag = ((j.v.ser || j.v.W % 2 == 0) && want_lag && !(p->reserved & 1)) ? 1 : 0;
     return CLM_OK;
 }
 
@@ -362,13 +402,14 @@ int prepare(clm_ctx* c, Plan& pl, int n, const clm_params* ps, const clm_stack_i
         if (j.P == 0) continue;
         const Geom& g = j.s.g;
         const int lag = j.lag;
+        if (j.sel_list) j.v.ser = 0;  // the selected pairs may be few
         const int norefine = (j.p.reserved & 2) ? 1 : 0;
         int gi = -1;
         for (size_t q = 0; q < pl.groups.size() && !j.sel_list; q++) {
             const Group& G = pl.groups[q];
             if (!G.sel && G.exact == j.exact && G.filt == j.filt && G.norefine == norefine &&
                 (j.exact || (G.opk == j.opk && G.ct == j.v.ct && G.Rp == g.Rp && G.sym == g.sym && G.W == j.v.W &&
-                             G.CPP == j.v.CPP && G.lag == lag))) {
+                             G.CPP == j.v.CPP && G.ser == j.v.ser && G.lag == lag))) {
                 gi = (int)q;
                 break;
             }
@@ -376,7 +417,7 @@ int prepare(clm_ctx* c, Plan& pl, int n, const clm_params* ps, const clm_stack_i
         if (gi < 0) {
             Group G;
             G.opk = j.opk; G.exact = j.exact; G.ct = j.v.ct; G.Rp = g.Rp; G.sym = g.sym;
-            G.W = j.v.W; G.CPP = j.v.CPP; G.lag = lag;
+            G.W = j.v.W; G.CPP = j.v.CPP; G.ser = j.v.ser; G.lag = lag;
             G.sel = j.sel_list != nullptr;
             G.norefine = norefine;
             G.filt = j.filt;
@@ -395,7 +436,7 @@ int prepare(clm_ctx* c, Plan& pl, int n, const clm_params* ps, const clm_stack_i
     for (size_t gi = 0; gi < n_orig_groups && twins; gi++) {
         if (pl.groups[gi].exact || pl.groups[gi].opk == OPK_F32 || pl.groups[gi].norefine) continue;
         const StackJob& j0 = pl.jobs[pl.groups[gi].members[0]];
-        const Variant v32 = choose_variant(OPK_F32, (j0.s.g.L + 31) / 32, j0.s.g.Rp, 0, 0);
+        const Variant v32 = choose_variant(OPK_F32, (j0.s.g.L + 31) / 32, j0.s.g.Rp, 0, 0, 0, c->n_cu);
         if (!v32.ct) continue;
         Group T;
         T.opk = OPK_F32; T.ct = v32.ct; T.Rp = pl.groups[gi].Rp; T.sym = pl.groups[gi].sym;
@@ -574,16 +615,22 @@ int prepare(clm_ctx* c, Plan& pl, int n, const clm_params* ps, const clm_stack_i
         if (!G.fn || !G.fn2) return fail(c, CLM_E_UNSUP, "no kernel for ct=%d Rp=%d", G.ct, G.Rp);
         if (G.W < 4 || G.W > 8) return fail(c, CLM_E_UNSUP, "workgroup of %d waves", G.W);
         G.lds = pair_lds_bytes(G.W);
-        G.occ = 0;
-        for (const auto& e : c->occ)
-            if (e.fn == (const void*)G.fn && e.W == G.W) G.occ = e.occ;
-        if (!G.occ) {
-            HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&G.occ, (const void*)G.fn, 64 * G.W, G.lds));
-            if (G.occ < 1) G.occ = 1;
-            c->occ.push_back({(const void*)G.fn, G.W, G.occ});
-        }
+        auto workgroups = [&](int W, int* occ) {  // resident on a CU
+            *occ = 0;
+            for (const auto& e : c->occ)
+                if (e.fn == (const void*)G.fn && e.W == W) *occ = e.occ;
+            if (*occ) return hipSuccess;
+            const hipError_t r = hipOccupancyMaxActiveBlocksPerMultiprocessor(occ, (const void*)G.fn, 64 * W,
+                                                                              pair_lds_bytes(W));
+            if (r != hipSuccess) return r;
+            if (*occ < 1) *occ = 1;
+            c->occ.push_back({(const void*)G.fn, W, *occ});
+            return hipSuccess;
+        };
+        HIPCHK(c, workgroups(G.W, &G.occ));
+        HIPCHK(c, workgroups(G.waves1(), &G.occ1));
         if (!build_tiles || G.sel) continue;
-        const int PPW = G.W / G.CPP;
+        const int PPW = G.pairs1();
         std::vector<long long> key;
         for (int ti = G.first; ti < G.first + (int)G.members.size(); ti++) {
             key.push_back(ti);
@@ -617,7 +664,7 @@ int prepare(clm_ctx* c, Plan& pl, int n, const clm_params* ps, const clm_stack_i
     // tile caches can move while inserting: resolve pointers afterwards
     for (Group& G : pl.groups) {
         if (G.exact || !build_tiles || G.sel) continue;
-        const int PPW = G.W / G.CPP;
+        const int PPW = G.pairs1();
         std::vector<long long> key;
         for (int ti = G.first; ti < G.first + (int)G.members.size(); ti++) {
             key.push_back(ti);
@@ -913,7 +960,8 @@ int enqueue_job(clm_ctx* c, const Plan& pl, bool timed, int phases = PHASE_ALL) 
         pa.counter = (int*)(cg + 0);
         pa.nq = 1;
         pa.erecs = nullptr;
-        pa.CPP = G.CPP;
+        pa.CPP = G.ser ? 1 : G.CPP;
+        pa.passes = G.ser ? G.CPP : 1;
         pa.lag = G.lag;
         pa.prio = (pl.jobs[G.members[0]].p.reserved & 4) ? 0 : 1;
         long long max_tiles;
@@ -931,13 +979,13 @@ int enqueue_job(clm_ctx* c, const Plan& pl, bool timed, int phases = PHASE_ALL) 
             pa.plist = nullptr;
             max_tiles = G.tc->ntiles;
         }
-        const unsigned grid = (unsigned)std::min<long long>((long long)c->n_cu * G.occ, max_tiles);
+        const unsigned grid = (unsigned)std::min<long long>((long long)c->n_cu * G.occ1, max_tiles);
         if (!G.sel && grid >= (unsigned)NQ) {
             pa.nq = NQ;
             pa.qbeg = (const int*)(pa.tiles + pa.ntiles);
             pa.counter = (int*)(cg + 4);
         }
-        hipLaunchKernelGGL(G.fn, dim3(grid), dim3(64 * G.W), G.lds, c->stream, pa);
+        hipLaunchKernelGGL(G.fn, dim3(grid), dim3(64 * G.waves1()), pair_lds_bytes(G.waves1()), c->stream, pa);
         HIPCHK(c, hipGetLastError());
     }
     if (timed) HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
@@ -996,6 +1044,7 @@ int enqueue_job(clm_ctx* c, const Plan& pl, bool timed, int phases = PHASE_ALL) 
             pa.plist = (const int4*)c->tw_plist.p;
             pa.erecs = nullptr;
             pa.CPP = T.CPP;
+            pa.passes = 1;
             pa.lag = T.lag;
             const unsigned g1 = (unsigned)std::min<long long>((long long)c->n_cu * T.occ, G0.P);
             hipLaunchKernelGGL(T.fn, dim3(g1), dim3(64 * T.W), T.lds, c->stream, pa);
@@ -1039,6 +1088,7 @@ int enqueue_job(clm_ctx* c, const Plan& pl, bool timed, int phases = PHASE_ALL) 
         pa.plist = (const int4*)c->plist.p;
         pa.erecs = (EmitRec*)c->erecs.p;
         pa.CPP = G.CPP;
+        pa.passes = 1;
         pa.lag = G.lag;
         pa.prio = (pl.jobs[G.members[0]].p.reserved & 4) ? 0 : 1;
         const unsigned g2 = (unsigned)std::min<long long>((long long)c->n_cu * G.occ, cap);
@@ -1109,7 +1159,7 @@ void begin_stats(const Plan& pl, clm_stats* st) {
         if (j.twin_src < 0) st->pairs += j.P;
     if (!pl.jobs.empty()) {
         st->n_eval_shifts = pl.jobs[0].s.g.NE;
-        st->variant = pl.jobs[0].v.ct * 100 + pl.jobs[0].v.W;
+        st->variant = pl.jobs[0].v.ct * 100 + (pl.jobs[0].v.ser ? SER_ID + pl.jobs[0].v.ser : pl.jobs[0].v.W);
     }
 }
 
@@ -1465,6 +1515,7 @@ std::vector<std::pair<int, int>> candidate_variants(int opk, int NCT, int Rp) {
         if (CPP > 8) continue;
         for (int W = CPP; W <= 8; W += CPP)
             if (W >= 4) out.push_back({ct, W});
+        if (CPP > 1 && pair_passes(opk == OPK_F32 ? 4 : 2, Rp)) out.push_back({ct, SER_ID + serial_waves(opk)});
     }
     return out;
 }
@@ -1484,7 +1535,7 @@ int autotune(clm_ctx* c, const clm_params* p, const void* d_pf, int sample_pairs
     int4 best_v = make_int4(0, 0, 0, 0);
     int n = 0;
     for (const auto& cw : cands) {
-        for (int lag = (cw.second % 2 == 0) ? 1 : 0; lag >= 0; lag--) {
+        for (int lag = (cw.second % 2 == 0) ? 1 : 0; lag >= 0; lag--) {  // (SER_ID and its waves are even)
             clm_params q = *p;
             q.variant = cw.first * 100 + cw.second;
             q.reserved = (p->reserved & ~1) | (lag ? 0 : 1);
@@ -1493,7 +1544,7 @@ int autotune(clm_ctx* c, const clm_params* p, const void* d_pf, int sample_pairs
             if ((rc = prepare(c, pl, 1, &q, &io, false, nullptr, 0, false))) return rc;
             const Group& G = pl.groups[0];
             const long long K = g0.K;
-            const int PPW = G.W / G.CPP;
+            const int PPW = G.pairs1();
             std::vector<int4> h;
             long long taken = 0;
             for (long long k1 = 0; k1 + 1 < K && taken < Np; k1++)
@@ -1514,10 +1565,11 @@ int autotune(clm_ctx* c, const clm_params* p, const void* d_pf, int sample_pairs
             pa.ntiles = ntiles;
             pa.counter = (int*)((unsigned long long*)c->ctr.p + 16);
             pa.nq = 1;
-            pa.CPP = G.CPP;
+            pa.CPP = G.ser ? 1 : G.CPP;
+            pa.passes = G.ser ? G.CPP : 1;
             pa.lag = G.lag;
             pa.prio = (p->reserved & 4) ? 0 : 1;
-            const unsigned grid = (unsigned)std::min<long long>((long long)c->n_cu * G.occ, (long long)ntiles);
+            const unsigned grid = (unsigned)std::min<long long>((long long)c->n_cu * G.occ1, (long long)ntiles);
             if (grid >= (unsigned)NQ) {  // the same XCD queues as the measured job
                 pa.nq = NQ;
                 pa.qbeg = (const int*)(pa.tiles + ntiles);
@@ -1527,7 +1579,7 @@ int autotune(clm_ctx* c, const clm_params* p, const void* d_pf, int sample_pairs
             for (int rep = 0; rep < 2; rep++) {  // first launch warms caches and code
                 if ((rc = enqueue_fill(c, pa.counter, pa.nq, 0))) return rc;
                 HIPCHK(c, hipEventRecord(c->ev[4], c->stream));
-                hipLaunchKernelGGL(G.fn, dim3(grid), dim3(64 * G.W), G.lds, c->stream, pa);
+                hipLaunchKernelGGL(G.fn, dim3(grid), dim3(64 * G.waves1()), pair_lds_bytes(G.waves1()), c->stream, pa);
                 HIPCHK(c, hipGetLastError());
                 HIPCHK(c, hipEventRecord(c->ev[5], c->stream));
                 HIPCHK(c, hipStreamSynchronize(c->stream));

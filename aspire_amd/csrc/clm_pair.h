@@ -108,6 +108,7 @@ struct PairArgs {
     const int4* plist;     // explicit pairs {k2, slot, u, 0}
     EmitRec* erecs;        // indexed by u (second pass)
     int CPP;               // waves per pair (column chunks); same for all stacks
+    int passes;            // column chunks a wave goes through one after another (CPP = 1)
     int lag;               // 1: one wave per SIMD runs one A-tile behind
     int prio;              // 1: raised wave priority while issuing MFMAs (the other
                            // wave on the SIMD runs its epilogue meanwhile)
@@ -136,12 +137,28 @@ __device__ inline float wave_max_dpp(float v) {
 // Dynamic LDS bytes of pair_kernel (the A-tile ring is static).
 __host__ __device__ inline size_t pair_lds_bytes(int W) { return 384 + (size_t)W * WCAP * 8; }
 
+// Whether a kernel can take a pair's column chunks one after another.  The
+// 16-bit kernels of shorter rays have even loads without (and the loop costs
+// them 4%: 583 to 605 ms for 2000 images, 41 shifts, n_r = 65).
+constexpr bool pair_passes(size_t op_bytes, int Rp) { return op_bytes == 4 || Rp > 64; }
+
+// Waves per SIMD the registers are held to: FP32 operands leave them idle with
+// two (each barrier and epilogue shows).  n_r = 44, 300 rays, 31375 pairs: three
+// waves 10.7 ms, 81% of the FP32 matrix rate; four 12.9, its spilled A prefetch
+// waits on every load.  Longer rays need the registers for B.
+template <typename OpT, int CT, int NK, bool EMIT>
+constexpr int pair_min_waves() {
+    if (sizeof(OpT) != 4 || CT != 1 || EMIT) return 2;
+    return NK <= 8 ? 4 : NK <= 32 ? 3 : 2;
+}
+
 // Persistent all-pairs kernel.  A workgroup takes a tile (one image k1 and up
 // to W/CPP partner images k2).  k1's A-tiles (32 rows (e, l1) of its
 // shift-expanded rays each, precomputed by astack_kernel) stream through two
 // LDS buffers, prefetched one tile ahead through registers; each wave
 // multiplies every A-tile against its k2's columns, which stay in
-// registers.  The epilogue reduces each lane's 32x32 output tile to
+// registers (or, pass after pass, against one column group of it after the
+// other, CPP = 1).  The epilogue reduces each lane's 32x32 output tile to
 // one "cell" maximum of t = X + |Y|.
 //   EMIT = false (pass 1): each wave keeps every cell that comes within the
 //     certified margin of the pair's running maximum; at the end the cells
@@ -149,7 +166,7 @@ __host__ __device__ inline size_t pair_lds_bytes(int W) { return 384 + (size_t)W
 //   EMIT = true (pass 2): every candidate at or above the pair's threshold T
 //     from pass 1 is listed.
 template <typename OpT, int CT, int NK, bool SYM, bool EMIT>
-__global__ __launch_bounds__(512) void pair_kernel(PairArgs a) {
+__global__ __launch_bounds__(512, (pair_min_waves<OpT, CT, NK, EMIT>())) void pair_kernel(PairArgs a) {
     using O = Op<OpT>;
     using frag = typename O::frag;
     using AT = ATile<OpT, NK>;
@@ -166,7 +183,7 @@ __global__ __launch_bounds__(512) void pair_kernel(PairArgs a) {
     int* s_unc = (int*)(s_pm + 32);           // per-pair flags
     float2* s_list = (float2*)(s_unc + 32);   // [W][WCAP] (value, id bits)
     float2* wlist = s_list + wave * WCAP;
-    const int pi = wave / a.CPP, chunk = wave % a.CPP;
+    const int pi = wave / a.CPP, wchunk = wave % a.CPP;
     const int wv = __builtin_amdgcn_readfirstlane(wave);
 
     // Which waves lag: the second wave (by index) on each SIMD, from the SIMD
@@ -252,29 +269,8 @@ __global__ __launch_bounds__(512) void pair_kernel(PairArgs a) {
                 if (q < NCH) ((v4i*)buf)[q] = pre[j];
             }
         };
-        load_pre(0);
-        // ---- B operand (image k2, this wave's CT column tiles) in registers
         frag Bre[CT][NK], Bim[CT][NK];
-        {
-            const OpT* B = (const OpT*)sd.Bop;
-            const size_t plane = (size_t)g.Lp * Rp;
-#pragma unroll
-            for (int ct = 0; ct < CT; ct++) {
-                const int col = (chunk * CT + ct) * 32 + lc;
-                const OpT* br = B + ((size_t)k2 * 2 + 0) * plane + (size_t)col * Rp;
-                const OpT* bi = br + plane;
-#pragma unroll
-                for (int ks = 0; ks < NK; ks++) {
-                    if constexpr (O::KSTEP == 16) {
-                        Bre[ct][ks] = *(const frag*)(br + 16 * ks + 8 * h);
-                        Bim[ct][ks] = *(const frag*)(bi + 16 * ks + 8 * h);
-                    } else {
-                        Bre[ct][ks] = br[h * (Rp / 2) + ks];
-                        Bim[ct][ks] = bi[h * (Rp / 2) + ks];
-                    }
-                }
-            }
-        }
+        int chunk = wchunk;
         const float n1 = sd.nrm[k1], n2 = sd.nrm[k2];
         const float margin = 2.0f * (sd.coef * n1 * n2 + sd.sub * (n1 + n2)) + sd.tau_t;
         float thr = -INFINITY;
@@ -359,21 +355,16 @@ __global__ __launch_bounds__(512) void pair_kernel(PairArgs a) {
         // A fragments of k-step ks (real and imaginary halves of the row)
         auto frag_re = [&](const int4* buf, int ks) -> frag {
             const char* arow = (const char*)buf + lc * CPR * 16;
-            if constexpr (O::KSTEP == 16) {
-                return *(const frag*)(arow + AT::phys(lc, 2 * ks + h) * 16);
-            } else {
-                const int kk = h * (Rp / 2) + ks;
-                return *(const float*)(arow + AT::phys(lc, kk / 4) * 16 + (kk % 4) * 4);
-            }
+            return *(const frag*)(arow + AT::phys(lc, 2 * ks + h) * 16);
         };
         auto frag_im = [&](const int4* buf, int ks) -> frag {
             const char* arow = (const char*)buf + lc * CPR * 16;
-            if constexpr (O::KSTEP == 16) {
-                return *(const frag*)(arow + AT::phys(lc, CPR / 2 + 2 * ks + h) * 16);
-            } else {
-                const int kk = h * (Rp / 2) + ks;
-                return *(const float*)(arow + AT::phys(lc, CPR / 2 + kk / 4) * 16 + (kk % 4) * 4);
-            }
+            return *(const frag*)(arow + AT::phys(lc, CPR / 2 + 2 * ks + h) * 16);
+        };
+        // FP32: one chunk holds this lane's fragments of the four k-steps 4q..4q+3
+        auto quad = [&](const int4* buf, int half, int q) -> f32x4 {
+            const char* arow = (const char*)buf + lc * CPR * 16;
+            return *(const f32x4*)(arow + AT::phys(lc, half * (CPR / 2) + h * (NK / 4) + q) * 16);
         };
         auto step = [&](int at, const int4* cur, int4* nxt) {
             if (at + 1 < g.NAT) {
@@ -387,42 +378,73 @@ __global__ __launch_bounds__(512) void pair_kernel(PairArgs a) {
             }
             if (a.prio) __builtin_amdgcn_s_setprio(1);
             if (active) {
-                // fragments of k-steps 0 and 1 first; each fragment register
-                // is refilled two k-steps ahead as soon as the MFMAs that
-                // read it have issued, so a refill has CT + 2 CT MFMAs to
-                // arrive (the schedule is pinned below)
-                frag fa[2], fb[2];
-                fa[0] = frag_re(cur, 0);
-                fb[0] = frag_im(cur, 0);
-                if (NK > 1) {
-                    fa[1] = frag_re(cur, 1);
-                    fb[1] = frag_im(cur, 1);
-                }
-#pragma unroll
-                for (int ks = 0; ks < NK; ks++) {
-                    const int s = ks & 1;
-#pragma unroll
-                    for (int ct = 0; ct < CT; ct++) {
-                        f32x16 z = {0.f};
-                        X[ct] = O::mma(fa[s], Bre[ct][ks], ks == 0 ? z : X[ct]);
-                    }
-#pragma unroll
-                    for (int ct = 0; ct < CT; ct++) {
-                        f32x16 z = {0.f};
-                        Y[ct] = O::mma(fb[s], Bim[ct][ks], ks == 0 ? z : Y[ct]);
-                    }
-                    if (ks + 2 < NK) {
-                        fa[s] = frag_re(cur, ks + 2);
-                        fb[s] = frag_im(cur, ks + 2);
-                    }
-                }
                 if constexpr (O::KSTEP == 16) {
+                    // fragments of k-steps 0 and 1 first; each fragment register
+                    // is refilled two k-steps ahead as soon as the MFMAs that
+                    // read it have issued, so a refill has CT + 2 CT MFMAs to
+                    // arrive (the schedule is pinned below)
+                    frag fa[2], fb[2];
+                    fa[0] = frag_re(cur, 0);
+                    fb[0] = frag_im(cur, 0);
+                    if (NK > 1) {
+                        fa[1] = frag_re(cur, 1);
+                        fb[1] = frag_im(cur, 1);
+                    }
+    #pragma unroll
+                    for (int ks = 0; ks < NK; ks++) {
+                        const int s = ks & 1;
+    #pragma unroll
+                        for (int ct = 0; ct < CT; ct++) {
+                            f32x16 z = {0.f};
+                            X[ct] = O::mma(fa[s], Bre[ct][ks], ks == 0 ? z : X[ct]);
+                        }
+    #pragma unroll
+                        for (int ct = 0; ct < CT; ct++) {
+                            f32x16 z = {0.f};
+                            Y[ct] = O::mma(fb[s], Bim[ct][ks], ks == 0 ? z : Y[ct]);
+                        }
+                        if (ks + 2 < NK) {
+                            fa[s] = frag_re(cur, ks + 2);
+                            fb[s] = frag_im(cur, ks + 2);
+                        }
+                    }
                     // scheduling groups (0x100: LDS reads, 0x008: MFMAs)
                     __builtin_amdgcn_sched_group_barrier(0x100, NK > 1 ? 4 : 2, 0);
 #pragma unroll
                     for (int ks = 0; ks < NK; ks++) {
                         __builtin_amdgcn_sched_group_barrier(0x008, 2 * CT, 0);
                         if (ks + 2 < NK) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+                    }
+                } else {
+                    // four k-steps a 16-byte read (conflict-free as the 16-bit
+                    // fragments are; single words had two conflicts a read), the
+                    // next four on their way
+                    f32x4 fa = quad(cur, 0, 0), fb = quad(cur, 1, 0);
+#pragma unroll
+                    for (int q = 0; q < NK / 4; q++) {
+                        f32x4 na, nb;
+                        if (q + 1 < NK / 4) {
+                            na = quad(cur, 0, q + 1);
+                            nb = quad(cur, 1, q + 1);
+                        }
+#pragma unroll
+                        for (int u = 0; u < 4; u++) {
+                            const int ks = 4 * q + u;
+#pragma unroll
+                            for (int ct = 0; ct < CT; ct++) {
+                                f32x16 z = {0.f};
+                                X[ct] = O::mma(fa[u], Bre[ct][ks], ks == 0 ? z : X[ct]);
+                            }
+#pragma unroll
+                            for (int ct = 0; ct < CT; ct++) {
+                                f32x16 z = {0.f};
+                                Y[ct] = O::mma(fb[u], Bim[ct][ks], ks == 0 ? z : Y[ct]);
+                            }
+                        }
+                        if (q + 1 < NK / 4) {
+                            fa = na;
+                            fb = nb;
+                        }
                     }
                 }
             }
@@ -438,17 +460,46 @@ __global__ __launch_bounds__(512) void pair_kernel(PairArgs a) {
             }
         };
 
-        store_pre(sa0);
-        if (g.NAT > 1) load_pre(1);
-        __syncthreads();
-        for (int at = 0; at < g.NAT; at += 2) {
-            step(at, sa0, sa1);
-            if (at + 1 < g.NAT) step(at + 1, sa1, sa0);
-        }
-        if (lag && active) {
+        for (int pass = 1;; pass++) {
+            load_pre(0);
+            // ---- B operand (image k2, this wave's CT column tiles) in registers
+            {
+                const OpT* B = (const OpT*)sd.Bop;
+                const size_t plane = (size_t)g.Lp * Rp;
 #pragma unroll
-            for (int ct = 0; ct < CT; ct++) epi(ct, g.NAT - 1);
-            keep_cells(g.NAT - 1);
+                for (int ct = 0; ct < CT; ct++) {
+                    const int col = (chunk * CT + ct) * 32 + lc;
+                    const OpT* br = B + ((size_t)k2 * 2 + 0) * plane + (size_t)col * Rp;
+                    const OpT* bi = br + plane;
+#pragma unroll
+                    for (int ks = 0; ks < NK; ks++) {
+                        if constexpr (O::KSTEP == 16) {
+                            Bre[ct][ks] = *(const frag*)(br + 16 * ks + 8 * h);
+                            Bim[ct][ks] = *(const frag*)(bi + 16 * ks + 8 * h);
+                        } else {
+                            Bre[ct][ks] = br[h * (Rp / 2) + ks];
+                            Bim[ct][ks] = bi[h * (Rp / 2) + ks];
+                        }
+                    }
+                }
+            }
+            store_pre(sa0);
+            // every load so far has arrived (vmcnt 0): left to the first use, the
+            // wait for B lands in the loop and waits for each A prefetch as well
+            __builtin_amdgcn_s_waitcnt(0x0f70);
+            if (g.NAT > 1) load_pre(1);
+            __syncthreads();
+            for (int at = 0; at < g.NAT; at += 2) {
+                step(at, sa0, sa1);
+                if (at + 1 < g.NAT) step(at + 1, sa1, sa0);
+            }
+            if (lag && active) {
+#pragma unroll
+                for (int ct = 0; ct < CT; ct++) epi(ct, g.NAT - 1);
+                keep_cells(g.NAT - 1);
+            }
+            if (!pair_passes(sizeof(OpT), Rp) || pass == a.passes) break;
+            chunk++;
         }
         __syncthreads();
 
@@ -467,7 +518,7 @@ __global__ __launch_bounds__(512) void pair_kernel(PairArgs a) {
                 if (lost) atomicOr(&s_unc[pi], 1);
             }
             __syncthreads();
-            if (active && chunk == 0 && lane == 0) {
+            if (active && wchunk == 0 && lane == 0) {
                 float M = -INFINITY;
                 for (int c = 0; c < a.CPP; c++) M = fmaxf(M, s_pm[pi * a.CPP + c]);
                 const int n = s_i[1 + pi];
@@ -482,7 +533,7 @@ __global__ __launch_bounds__(512) void pair_kernel(PairArgs a) {
             }
         } else {
             __syncthreads();
-            if (active && chunk == 0 && lane == 0) {
+            if (active && wchunk == 0 && lane == 0) {
                 const int n = s_i[1 + pi];
                 a.erecs[uidx].n = n < MAXE ? n : MAXE;
                 a.erecs[uidx].overflow = n > MAXE;

@@ -228,7 +228,8 @@ int clm_clmatrix_grouped(clm_ctx *ctx, int32_t n, const clm_params *p,
  * Leaves the outputs of earlier calls untouched.
  */
 typedef struct clm_tune_entry {
-    int32_t variant;  /* CT*100 + waves per workgroup                */
+    int32_t variant;  /* CT*100 + waves per workgroup; + 50 where a wave
+                         takes a pair's column groups one after another */
     int32_t lag;      /* 1 = lagged wave schedule                     */
     double ms;        /* pass-1 kernel time on the sample             */
     int64_t pairs;    /* pairs in the sample                          */
