@@ -22,7 +22,7 @@
 // (K = 5000, 12.5M pairs): the packed lines (4 B/pair) and u (8 B/pair) are
 // read once and u written once, 20 B/pair, about 0.25 GB (stored tile by
 // tile, with the empty slots of the diagonal tiles), plus the 2K-long
-// partial sums of the 64 x 256-pair tiles; HBM-bound work with every
+// partial sums of the 32 x 256-pair tiles; HBM-bound work with every
 // reduction in a fixed order (results do not depend on scheduling).
 #include <hip/hip_runtime.h>
 
@@ -40,8 +40,8 @@ struct State {
     double t1, t2;      // the last scalar step's update of x and w
     double vscale;      // the current v is the stored v times vscale
     int itn, maxit, done, flag;
-    int upd;            // 1: the last scalar step's update of x and w is pending
-    int vset;           // 1: the first direction v was formed (b != 0)
+    int upd;            // 1: the last scalar step's update of x and w is pending; 0: x = 0 and w = v are
+    unsigned arrived;   // workgroups of the running step that are through
 };
 
 __device__ inline long long first(long long k1, long long K) { return k1 * K - k1 * (k1 + 1) / 2; }
@@ -78,46 +78,9 @@ __global__ void tables_kernel(int L, int by_index, double2* ta, double* tb) {
     tb[3 * c + 2] = sg;
 }
 
-// Block reduction of one double per thread (fixed order); result in thread 0.
-template <int NT>
-__device__ inline double block_sum(double v, double* sh) {
-    const int t = threadIdx.x;
-    sh[t] = v;
-    __syncthreads();
-#pragma unroll
-    for (int s = NT / 2; s > 0; s >>= 1) {
-        if (t < s) sh[t] += sh[t + s];
-        __syncthreads();
-    }
-    const double r = sh[0];
-    __syncthreads();
-    return r;
-}
-
-// Sum of p[0..n) in one fixed order whatever the block size NT >= 256:
-// thread t < 256 adds p[t], p[t + 256], ... in order, then a 256-wide tree.
-// Every block that calls it gets the same bits.
-template <int NT>
-__device__ inline double fixed_sum(const double* p, int n, double* sh) {
-    const int t = threadIdx.x;
-    double s = 0.0;
-    if (t < 256)
-        for (int i = t; i < n; i += 256) s += p[i];
-    if (t < 256) sh[t] = s;
-    __syncthreads();
-#pragma unroll
-    for (int w = 128; w > 0; w >>= 1) {
-        if (t < w) sh[t] += sh[t + w];
-        __syncthreads();
-    }
-    const double r = sh[0];
-    __syncthreads();
-    return r;
-}
-
 // Pair tiles: rows k1 in [TR*kb, TR*kb + TR), columns k2 in [TC*cb, TC*cb + TC);
 // a tile exists when it holds a pair k1 < k2 < K.
-constexpr int TR = 64, TC = 256;
+constexpr int TR = 32, TC = 256;
 
 __host__ __device__ inline bool tile_exists(int K, int kb, int cb) {
     const int kmax = min(TC * cb + TC, K) - 1;  // largest k2 of the column block
@@ -161,23 +124,33 @@ __device__ inline double wave_sum(double x) {
     x += dpp_d<0x128>(x);
     return ((readlane_d(x, 0) + readlane_d(x, 16)) + readlane_d(x, 32)) + readlane_d(x, 48);
 }
-// wave_sum of two values at once (the same order and bits as two calls),
-// the steps interleaved so each fills the other's DPP wait
-__device__ inline void wave_sum2(double& x, double& y) {
-    x += mov_dpp_d<0xb1>(x);
-    y += mov_dpp_d<0xb1>(y);
-    x += mov_dpp_d<0x4e>(x);
-    y += mov_dpp_d<0x4e>(y);
-    x += mov_dpp_d<0x124>(x);
-    y += mov_dpp_d<0x124>(y);
-    x += mov_dpp_d<0x128>(x);
-    y += mov_dpp_d<0x128>(y);
-    x = ((readlane_d(x, 0) + readlane_d(x, 16)) + readlane_d(x, 32)) + readlane_d(x, 48);
-    y = ((readlane_d(y, 0) + readlane_d(y, 16)) + readlane_d(y, 32)) + readlane_d(y, 48);
+// Sums of 8 values over each row of 16 lanes, fixed order, together: lane l of
+// a quad keeps value 4h + (l & 3) in x[h], so a step's exchange serves two
+// values (15 instructions a value, 35 with a butterfly of its own).
+__device__ inline void row_sum8(const double (&y)[8], double (&x)[2]) {
+    const int lane = threadIdx.x & 63;
+    double p[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {  // lanes l and l ^ 1: values 2q + (l & 1)
+        const bool odd = lane & 1;
+        p[q] = (odd ? y[2 * q + 1] : y[2 * q]) + mov_dpp_d<0xb1>(odd ? y[2 * q] : y[2 * q + 1]);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; h++) {  // lanes l and l ^ 2: values 4h + (l & 3)
+        const bool up = lane & 2;
+        x[h] = (up ? p[2 * h + 1] : p[2 * h]) + mov_dpp_d<0x4e>(up ? p[2 * h] : p[2 * h + 1]);
+        x[h] += mov_dpp_d<0x124>(x[h]);  // quads of the row: row_ror 4, 8
+        x[h] += mov_dpp_d<0x128>(x[h]);
+    }
 }
 // Sum of p[0..n) in one fixed order by one whole wave: lane l adds p[l],
 // p[l + 64], ... in order, then wave_sum.  Every caller gets the same bits.
+// COHERENT: the values were stored past the caches in this launch.
+template <bool COHERENT = false>
 __device__ inline double wave_fixed_sum(const double* p, int n) {
+    auto get = [&](int i) {
+        return COHERENT ? __hip_atomic_load(p + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : p[i];
+    };
     const int lane = threadIdx.x & 63;
     double s = 0.0;
     int i = lane;
@@ -185,11 +158,11 @@ __device__ inline double wave_fixed_sum(const double* p, int n) {
     for (; i + 7 * 64 < n; i += 8 * 64) {
         double a[8];
 #pragma unroll
-        for (int q = 0; q < 8; q++) a[q] = p[i + q * 64];
+        for (int q = 0; q < 8; q++) a[q] = get(i + q * 64);
 #pragma unroll
         for (int q = 0; q < 8; q++) s += a[q];
     }
-    for (; i < n; i += 64) s += p[i];
+    for (; i < n; i += 64) s += get(i);
     return wave_sum(s);
 }
 
@@ -203,8 +176,12 @@ __device__ inline double wave_fixed_sum(const double* p, int n) {
 // and, of the new u: normp[t] = sum of squares; rowp[cb][2k1 + c] = the
 // tile's row part of A'u (the k1 coefficients), colp[kb][2k2 + c] = its
 // column part (the k2 coefficients).  A thread owns one column and walks the
-// tile's rows in order; row sums go through fixed wave butterflies and then
-// the four waves in order.
+// tile's rows in order; row sums are formed over rows of 16 lanes, four tile
+// rows at a time, and the 16 partials added in order at the end.
+// Bound: memory (20 bytes a pair, which stay in the last-level cache at this
+// size) and the tables' LDS bank conflicts.  4.5 million pairs (K = 3000): 14.5 us,
+// 6.2 TB/s; with a butterfly per tile row, twice the vector instructions, 16.4;
+// with tiles of 64 rows, barely one workgroup a CU, 20.
 // LT: the two coefficient tables (5 (2L+2) doubles, ta then tb, contiguous)
 // are first copied to LDS, so the loop's table reads wait on the LDS counter
 // and not behind the next rows' HBM loads on the vector-memory counter.
@@ -215,7 +192,7 @@ __global__ __launch_bounds__(256) void pass_kernel(int K, int L, const int2* __r
                                                    const double2* __restrict__ ta, const double* __restrict__ tb,
                                                    const double* __restrict__ v, const State* S, double* u,
                                                    double* normp, double* rowp, double* colp) {
-    __shared__ double s_row[TR][4][2];
+    __shared__ double s_row[16][2 * TR + 2];  // [16-lane row of the workgroup][tile row, coefficient]
     __shared__ double s_sq[4];
     extern __shared__ double s_tab[];
     if (!INIT && S->done) return;
@@ -223,7 +200,7 @@ __global__ __launch_bounds__(256) void pass_kernel(int K, int L, const int2* __r
     __shared__ double s_v[2 * TR];
     if (!INIT && threadIdx.x < 2 * TR) {
         const int i = 2 * TR * tiles[blockIdx.x].x + threadIdx.x;
-        s_v[threadIdx.x] = i < 2 * K ? v[i] : 0.0;
+        s_v[threadIdx.x] = i < 2 * K ? v[i] * S->vscale : 0.0;
     }
     if constexpr (LT) {
         const double* src = (const double*)ta;
@@ -281,6 +258,7 @@ __global__ __launch_bounds__(256) void pass_kernel(int K, int L, const int2* __r
         }
     };
     auto finish_group = [&](int r0, const unsigned* gp, const double* gu) {
+        double rv[8];
 #pragma unroll
         for (int i = 0; i < UR; i++) {
             const int r = r0 + i;
@@ -300,28 +278,31 @@ __global__ __launch_bounds__(256) void pass_kernel(int K, int L, const int2* __r
                 B1 = B[1];
                 sg = B[2];
             }
+            const double sax = sg * A.x, say = sg * A.y;
             double un;
             if constexpr (INIT) {
                 pack[q] = gp[i];
                 un = gu[i];
             } else {
-                const double av = sg * A.x * (s_v[2 * r] * vs) + sg * A.y * (s_v[2 * r + 1] * vs) + B0 * va0 +
-                                  B1 * va1;
-                un = av - ca * gu[i];
+                const double av = fma(B1, va1, fma(B0, va0, fma(say, s_v[2 * r + 1], sax * s_v[2 * r])));
+                un = fma(-ca, gu[i], av);
             }
             u[q] = un;
-            sq += un * un;
-            double r0v = sg * A.x * un;
-            double r1v = sg * A.y * un;
-            c0 += B0 * un;
-            c1 += B1 * un;
-            wave_sum2(r0v, r1v);
-            if (lane == 0) {
-                s_row[r][wave][0] = r0v;
-                s_row[r][wave][1] = r1v;
-            }
+            sq = fma(un, un, sq);
+            rv[2 * i] = sax * un;
+            rv[2 * i + 1] = say * un;
+            c0 = fma(B0, un, c0);
+            c1 = fma(B1, un, c1);
+        }
+        double x[2];
+        row_sum8(rv, x);
+        if ((lane & 15) < 4) {
+            double* d = &s_row[t >> 4][2 * r0 + (lane & 3)];
+            d[0] = x[0];
+            d[4] = x[1];
         }
     };
+    static_assert(UR == 4, "row_sum8 takes four rows of two values");
     static_assert((TR / UR) % 2 == 0, "groups come in pairs");
     load_group(0, pk[0], ub[0]);
 #pragma unroll 1
@@ -340,33 +321,18 @@ __global__ __launch_bounds__(256) void pass_kernel(int K, int L, const int2* __r
     __syncthreads();
     if (t < 2 * TR) {
         const int r = t >> 1, c = t & 1, k1 = TR * kb + r;
+        double rs = s_row[0][t];
+#pragma unroll
+        for (int q = 1; q < 16; q++) rs += s_row[q][t];
         if (k1 < K)
-            rowp[(size_t)cb * 2 * K + 2 * k1 + c] = ((s_row[r][0][c] + s_row[r][1][c]) + s_row[r][2][c]) + s_row[r][3][c];
+            rowp[(size_t)cb * 2 * K + 2 * k1 + c] = rs;
     }
     if (t == 0) normp[blockIdx.x] = ((s_sq[0] + s_sq[1]) + s_sq[2]) + s_sq[3];
 }
 
-// Before the first iteration: beta = bnorm = |b| from the first pass's
-// tiles' sums of squares.
-__global__ __launch_bounds__(1024) void beta_kernel(int n, const double* part, State* S) {
-    __shared__ double sh[1024];
-    if (S->done) return;
-    const double beta = sqrt(fixed_sum<1024>(part, n, sh));
-    if (threadIdx.x == 0) {
-        S->beta = beta;
-        S->bnorm = beta;
-        if (beta == 0.0) {  // b = 0: x = 0 is the solution
-            S->done = 1;
-            S->flag = 0;
-        }
-    }
-}
-
-// Entries of the 2K-vector per workgroup of the element-parallel steps: 16
-// entries x 16 partial groups (256 threads); the first 16 threads finish the
-// entries.
-constexpr int VE = 16;
-constexpr int NG = 256 / VE;  // partial groups per entry
+// Entries of the 2K-vector per workgroup of the step: VE entries x NG partial
+// groups; the first wave finishes the entries.
+constexpr int VE = 64, NG = 16;
 
 // Group g's share (g = 0..NG-1) of (A'u)[i], entry i of the 2K-vector: the
 // row parts of the tiles in image i/2's row block, then the column parts of
@@ -392,20 +358,21 @@ __device__ inline double atu_part(int K, const double* rowp, const double* colp,
 }
 
 
-// One LSQR iteration after the pass is two launches:
-//  stepa_kernel (NG threads per element): the previous step's update of x
-//    and w, v <- A'u / beta - beta v, per-workgroup partial norms;
-//  stepb_kernel, one wave (scalar_step): the running
-//    Frobenius estimate of A, alpha = |v|, the damping and plane rotations,
-//    the stopping tests; the update's coefficients and the normalization
-//    1/alpha of v go to the state, applied by the next pass and stepa (or
-//    finish_kernel after the last iteration).
+// One LSQR iteration after the pass is one launch, step_kernel (NG threads per
+// element): the previous step's update of x and w, v <- A'u / beta - beta v,
+// per-workgroup partial norms; then, in one wave of the workgroup that
+// finishes last, scalar_step: the running Frobenius estimate of A, alpha =
+// |v|, the damping and plane rotations, the stopping tests; the update's
+// coefficients and the normalization 1/alpha of v go to the state, applied by
+// the next pass and step (or finish_kernel after the last iteration).  (The
+// scalar step as a launch of its own took 3.8 us and a gap each iteration.  K =
+// 3000: 5.5 us; with workgroups of 16 entries, 375 counts on one address, 9.3.)
 // beta = 0 (b in the range of A): v and alpha stay, the rotation makes the
 // last update of x and phibar becomes 0.
 // Run by one whole wave (lane 0 updates the state).
 __device__ inline void scalar_step(double beta, int nb, const double* part, State* S) {
     double alpha = S->alpha;
-    if (beta > 0.0) alpha = sqrt(wave_fixed_sum(part, nb));
+    if (beta > 0.0) alpha = sqrt(wave_fixed_sum<true>(part, nb));
     if (threadIdx.x == 0) {
         S->beta = beta;
         if (beta > 0.0) S->anorm = sqrt(S->anorm * S->anorm + S->alpha * S->alpha + beta * beta + S->damp * S->damp);
@@ -440,109 +407,103 @@ __device__ inline void scalar_step(double beta, int nb, const double* part, Stat
     }
 }
 
-// INIT (first direction, u = b/beta, beta from beta_kernel): v <- A'u / beta.
-// Else, with beta = |u| from the tiles' sums of squares (wave_fixed_sum,
-// the same bits in every workgroup) and the current v (stored v times
-// vscale):
-// the last scalar step's pending update of x and w, then v <- A'u / beta -
-// beta v (v unchanged when beta = 0).  Both with per-workgroup partial sums
-// of the squares of the new v (fixed order).
-template <bool INIT>
-__global__ __launch_bounds__(256) void stepa_kernel(int K, int ntiles, const double* normp, const double* rowp,
-                                                    const double* colp, const State* S, double* v, double* w,
-                                                    double* x, double* part) {
-    __shared__ double sh[NG][VE];
-    __shared__ double s_beta;
-    const int n2 = 2 * K;
-    if (S->done) return;
-    if (!INIT && threadIdx.x < 64) {
-        const double bb = sqrt(wave_fixed_sum(normp, ntiles));  // the bits stepb_kernel gets
-        if (threadIdx.x == 0) s_beta = bb;
-    }
-    const int j = threadIdx.x % VE, g = threadIdx.x / VE;
-    const int i = blockIdx.x * VE + j;
-    sh[g][j] = i < n2 ? atu_part(K, rowp, colp, i, g) : 0.0;  // used only when beta > 0
-    __syncthreads();
-    const double beta = INIT ? S->beta : s_beta;
-    if (threadIdx.x < 64) {
-        double t = 0.0;
-        if (threadIdx.x < VE && i < n2) {
-            double a = sh[0][j];
-#pragma unroll
-            for (int q = 1; q < NG; q++) a += sh[q][j];
-            if (INIT) {
-                t = a * (1.0 / beta);
-            } else {
-                const double vn = v[i] * S->vscale;
-                if (S->upd) {
-                    const double wi = w[i];
-                    x[i] += S->t1 * wi;
-                    w[i] = vn + S->t2 * wi;
-                }
-                t = beta > 0.0 ? a * (1.0 / beta) - beta * vn : vn;
-            }
-            v[i] = t;
-        }
-        const double sq = wave_sum(t * t);
-        if (threadIdx.x == 0) part[blockIdx.x] = sq;
-    }
-}
-
-// First direction, scalar part (one workgroup): alpha = |A'u / beta| and the
-// state of iteration 0.
-__global__ __launch_bounds__(1024) void vinit_b_kernel(int nb, const double* part, State* S) {
-    __shared__ double sh[1024];
-    if (S->done) return;
-    double s = 0.0;
-    for (int i = threadIdx.x; i < nb; i += 1024) s += part[i];
-    s = block_sum<1024>(s, sh);
+// First direction, scalar part: alpha = |A'u / beta| and the state of iteration
+// 0.  Run by one whole wave.
+__device__ inline void first_step(double beta, int nb, const double* part, State* S) {
+    const double alpha = beta == 0.0 ? 0.0 : sqrt(wave_fixed_sum<true>(part, nb));
     if (threadIdx.x == 0) {
-        const double alpha = sqrt(s);
+        S->beta = beta;
+        S->bnorm = beta;
         S->alpha = alpha;
-        S->phibar = S->beta;
+        S->phibar = beta;
         S->rhobar = alpha;
         S->anorm = 0.0;
         S->res2 = 0.0;
-        S->rnorm = S->beta;
-        S->arnorm = alpha * S->beta;
+        S->rnorm = beta;
+        S->arnorm = alpha * beta;
         S->itn = 0;
-        S->vset = 1;
-        S->vscale = 1.0;
+        S->vscale = alpha > 0.0 ? 1.0 / alpha : 0.0;
         S->upd = 0;
-        if (alpha == 0.0) {  // A'b = 0: x = 0 is a least-squares solution
+        if (alpha == 0.0) {  // b = 0 or A'b = 0: x = 0 is a least-squares solution
             S->done = 1;
             S->flag = 0;
         }
     }
 }
 
-// First direction, element part: x = 0; v <- v / alpha (0 when alpha = 0)
-// and w = v when v was formed.
-__global__ __launch_bounds__(256) void vinit_c_kernel(int n2, const State* S, double* v, double* w, double* x) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n2) return;
-    x[i] = 0.0;
-    if (S->vset) {
-        const double ia = S->alpha > 0.0 ? 1.0 / S->alpha : 0.0;
-        const double t = v[i] * ia;
-        v[i] = t;
-        w[i] = t;
+// beta = |u| from the tiles' sums of squares (wave_fixed_sum, the same bits in
+// every workgroup).  INIT (first direction, u = b): v <- A'u / beta.  Else, with
+// the current v (stored v times vscale): the last scalar step's pending update
+// of x and w (the first time: x = 0, w = v), then v <- A'u / beta - beta v (v
+// unchanged when beta = 0).  Both with per-workgroup partial sums of the squares
+// of the new v (fixed order).
+template <bool INIT>
+__global__ __launch_bounds__(VE * NG) void step_kernel(int K, int ntiles, const double* normp, const double* rowp,
+                                                   const double* colp, State* S, double* v, double* w, double* x,
+                                                   double* part) {
+    __shared__ double sh[NG][VE];
+    __shared__ double s_beta;
+    const int n2 = 2 * K;
+    if (S->done) return;
+    if (threadIdx.x < 64) {
+        const double bb = sqrt(wave_fixed_sum(normp, ntiles));
+        if (threadIdx.x == 0) s_beta = bb;
+    }
+    const int j = threadIdx.x % VE, g = threadIdx.x / VE;
+    const int i = blockIdx.x * VE + j;
+    sh[g][j] = i < n2 ? atu_part(K, rowp, colp, i, g) : 0.0;  // used only when beta > 0
+    __syncthreads();
+    const double beta = s_beta;
+    if (threadIdx.x < 64) {
+        double t = 0.0;
+        if (i < n2) {
+            double a = sh[0][j];
+#pragma unroll
+            for (int q = 1; q < NG; q++) a += sh[q][j];
+            if (INIT) {
+                t = beta == 0.0 ? 0.0 : a * (1.0 / beta);
+            } else {
+                const double vn = v[i] * S->vscale;
+                if (S->upd) {
+                    const double wi = w[i];
+                    x[i] += S->t1 * wi;
+                    w[i] = vn + S->t2 * wi;
+                } else {
+                    x[i] = 0.0;
+                    w[i] = vn;
+                }
+                t = beta > 0.0 ? a * (1.0 / beta) - beta * vn : vn;
+            }
+            v[i] = t;
+        }
+        const double sq = wave_sum(t * t);
+        // the workgroup that comes last sees every partial norm (and no other
+        // workgroup reads the state any more): it does the scalar step
+        int last = 0;
+        if (threadIdx.x == 0) {
+            // the partial norm goes past the caches and is there before the
+            // count is raised; a release would write back the whole L2
+            __hip_atomic_store(part + blockIdx.x, sq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __builtin_amdgcn_s_waitcnt(0);
+            asm volatile("" ::: "memory");
+            const unsigned n = __hip_atomic_fetch_add(&S->arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            last = n + 1 == gridDim.x;
+        }
+        if (!__builtin_amdgcn_readfirstlane(last)) return;
+        asm volatile("" ::: "memory");
+        if (threadIdx.x == 0) S->arrived = 0;
+        if (INIT)
+            first_step(beta, gridDim.x, part, S);
+        else
+            scalar_step(beta, gridDim.x, part, S);
     }
 }
 
-// The scalar step, one wave: beta = |u| (the same sum as stepa's), then
-// scalar_step on stepa's per-workgroup sums of squares.
-__global__ __launch_bounds__(64) void stepb_kernel(int ntiles, const double* normp, int nb, const double* part,
-                                                   State* S) {
-    if (S->done) return;
-    scalar_step(sqrt(wave_fixed_sum(normp, ntiles)), nb, part, S);
-}
-
-// After the last iteration: its pending update of x (x += t1 w).
+// After the last iteration: its pending update of x (x += t1 w); x = 0 if
+// there was none.
 __global__ __launch_bounds__(256) void finish_kernel(int n2, const State* S, const double* w, double* x) {
-    if (!S->upd) return;
     const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n2) x[i] += S->t1 * w[i];
+    if (i < n2) x[i] = S->upd ? x[i] + S->t1 * w[i] : 0.0;
 }
 
 }  // namespace lsq
@@ -594,7 +555,7 @@ extern "C" int clm_estimate_shifts_ex(clm_ctx* c, int32_t K, int32_t n_theta, co
     unsigned* pack = (unsigned*)c->ls_pack.p;
     double* u = (double*)c->ls_u.p;
     double* part = (double*)c->ls_part.p;  // the tiles' sums of squares of u
-    double* part2 = part + ntiles;         // stepa's per-workgroup sums of squares of v
+    double* part2 = part + ntiles;         // the steps' per-workgroup sums of squares of v
     const int2* tiles = (const int2*)c->ls_tiles.p;
     State h{};
     h.damp = damp;
@@ -626,20 +587,16 @@ extern "C" int clm_estimate_shifts_ex(clm_ctx* c, int32_t K, int32_t n_theta, co
                                                                          ta, tb, v, S, u, part, rowp, colp);
         }
     };
-    // partials of the tiles that do not exist stay zero (stepa adds every block)
+    // partials of the tiles that do not exist stay zero (step_kernel adds every block)
     HIPCHK(c, hipMemsetAsync(rowp, 0, (size_t)(ncb + nkb) * n2 * 8, c->stream));
     pass(true);
-    beta_kernel<<<1, 1024, 0, c->stream>>>(ntiles, part, S);
-    stepa_kernel<true><<<nstep, 256, 0, c->stream>>>(K, ntiles, part, rowp, colp, S, v, w, d_x, part2);
-    vinit_b_kernel<<<1, 1024, 0, c->stream>>>(nstep, part2, S);
-    vinit_c_kernel<<<nelem, 256, 0, c->stream>>>(n2, S, v, w, d_x);
+    step_kernel<true><<<nstep, VE * NG, 0, c->stream>>>(K, ntiles, part, rowp, colp, S, v, w, d_x, part2);
     HIPCHK(c, hipGetLastError());
     // launches after the stopping tests pass return at once; the done flag is
     // read back every 8 iterations so a converged solve stops issuing them
     for (int it = 0; it < maxit; it++) {
         pass(false);
-        stepa_kernel<false><<<nstep, 256, 0, c->stream>>>(K, ntiles, part, rowp, colp, S, v, w, d_x, part2);
-        stepb_kernel<<<1, 64, 0, c->stream>>>(ntiles, part, nstep, part2, S);
+        step_kernel<false><<<nstep, VE * NG, 0, c->stream>>>(K, ntiles, part, rowp, colp, S, v, w, d_x, part2);
         if (it % 8 == 7 && it + 1 < maxit) {
             int done = 0;
             HIPCHK(c, hipGetLastError());
