@@ -40,8 +40,7 @@ namespace vote {
 constexpr int NT = 60;  // histogram points (ntics)
 
 // M[i*K + j] = clstack(i, j), MT[j*K + i] = clstack(i, j) (1-based lines, 0 = none)
-__global__ void build_kernel(int K, const int* cl1, const int* cl2, unsigned short* M, unsigned short* MT) {
-    const int k1 = blockIdx.x;
+__device__ inline void build(int k1, int K, const int* cl1, const int* cl2, unsigned short* M, unsigned short* MT) {
     const long long e0 = (long long)k1 * K - (long long)k1 * (k1 + 1) / 2;
     for (int j = threadIdx.x; j < K; j += blockDim.x) {
         if (j <= k1) {
@@ -60,9 +59,8 @@ __global__ void build_kernel(int K, const int* cl1, const int* cl2, unsigned sho
     }
 }
 
-__global__ void diag_kernel(int K, double* S) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= K) return;
+// The 2 x 2 identity of image k on S's diagonal.
+__device__ inline void diag(int k, int K, double* S) {
     const size_t n2 = 2 * (size_t)K;
     S[(2 * (size_t)k) * n2 + 2 * k] = 1.0;
     S[(2 * (size_t)k + 1) * n2 + 2 * k] = 0.0;
@@ -86,8 +84,7 @@ struct Window {
 // factor 2 being exact).  ln[l] = (cos, sin) of (l - 1) * 2 * pi / n_theta - pi
 // for the lines l <= n_theta: the rotation's third Euler angle, and minus its
 // first.  win[d]: the windows.
-__global__ void trig_kernel(int n_theta, double2* cs, double2* ln, Window* win) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ inline void tables(int i, int n_theta, double2* cs, double2* ln, Window* win) {
     if (i <= 2 * n_theta) {
         const double d = (double)(i - n_theta);
         const double th = d * 2 * M_PI / (double)n_theta;
@@ -107,6 +104,17 @@ __global__ void trig_kernel(int n_theta, double2* cs, double2* ln, Window* win) 
         q.i_lo = x + (w - t) < 180 ? cosd(x + (w - t)) : -INFINITY;
         win[i] = q;
     }
+}
+
+// What the votes need, in one launch: workgroups 0..K-1 build the clstack (and
+// write the diagonal of S), the rest the tables.
+__global__ __launch_bounds__(256) void setup_kernel(int K, int n_theta, const int* cl1, const int* cl2,
+                                                    unsigned short* M, unsigned short* MT, double2* cs, double2* ln,
+                                                    Window* win, double* S) {
+    const int b = blockIdx.x;
+    if (b >= K) return tables((b - K) * 256 + threadIdx.x, n_theta, cs, ln, win);
+    if (threadIdx.x == 0) diag(b, K, S);
+    build(b, K, cl1, cl2, M, MT);
 }
 
 // Entry of line difference d (clamped to the table, so that a malformed
@@ -501,9 +509,8 @@ extern "C" int clm_syncmatrix_vote(clm_ctx* c, int32_t K, int32_t n_theta, const
     double2* ln = cs + 2 * (size_t)n_theta + 1;
     Window* win = (Window*)(ln + n_theta + 1);
     HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
-    build_kernel<<<K, 256, 0, c->stream>>>(K, d_cl1, d_cl2, M, MT);
-    trig_kernel<<<std::max(2 * n_theta + 1, NT) / 256 + 1, 256, 0, c->stream>>>(n_theta, cs, ln, win);
-    diag_kernel<<<(K + 255) / 256, 256, 0, c->stream>>>(K, d_S);
+    setup_kernel<<<K + std::max(2 * n_theta + 1, NT) / 256 + 1, 256, 0, c->stream>>>(K, n_theta, d_cl1, d_cl2, M, MT,
+                                                                                     cs, ln, win, d_S);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
     if (P > 0) {
