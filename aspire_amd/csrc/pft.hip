@@ -25,11 +25,12 @@
 // Four real products over a quarter of the pixels serve two rays: a quarter
 // of the multiplications of the sums as written.  The weights are never
 // stored: a lane forms its operand as one product of two table entries.
-// A mirrored ray is taken at the exact mirror of ray j's frequencies, which
-// differ from its own rounded ones in the last bit.  White noise, n = 129, n_r =
-// 65, worst error over max |pf| in extended precision: 2.3e-14 at the true polar
-// points and 3.2e-14 at the rounded frequencies (the sums as written with their
-// weights advanced by rotations: 3.5e-14 and 1.5e-14).
+// Two rays that share a quadrant point are taken at the mean of their rounded
+// frequencies, which differ in the last bits.  Worst error over max |pf| of
+// white noise in extended precision, n = 129 and n_r = 65: 1.6e-14 at the
+// rounded frequencies and 1.7e-14 at the true polar points (the sums as written
+// with their weights advanced by rotations: 1.5e-14 and 3.5e-14); rms 7.7e-15
+// and 9.4e-15 (6.1e-15 and 1.3e-14).
 //
 // CLM_PFT_NUFFT: the same sums by a type-2 non-uniform FFT, the method the
 // reference's nufft2 uses when a NUFFT library is installed
@@ -77,6 +78,8 @@ struct Geo {
 
 // tab[0][a*Mp + m] = cos(fx(m) a), tab[1] sin; then cos(fy(m) b) and
 // sin(fy(m) b), 4 nab rows each (zero for m >= M).  grid: (Mp/256, 8 nab).
+// The frequency of a point that serves two rays is the mean of the two rays'
+// rounded ones, f + df, and the phase keeps the product's rounding error.
 __global__ void tables_kernel(Geo g, double* tab) {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
     if (m >= g.Mp) return;
@@ -89,7 +92,14 @@ __global__ void tables_kernel(Geo g, double* tab) {
         const double omega0 = 2.0 * M_PI / (2.0 * g.n_r - 1.0);  // cryo_pft.m:49
         const double dtheta = 2.0 * M_PI / g.n_theta;             // cryo_pft.m:50
         const double f = is_x ? (k * omega0) * sin(j * dtheta) : (k * omega0) * cos(j * dtheta);
-        sincos(f * idx, &s, &c);
+        double df = 0.0;
+        const int jm = g.n_theta / 2 - j;  // the mirrored ray
+        if (j > 0 && j < jm) df = 0.5 * ((is_x ? (k * omega0) * sin(jm * dtheta) : -(k * omega0) * cos(jm * dtheta)) - f);
+        const double ph = f * idx, lo = fma(f, (double)idx, -ph) + df * idx;
+        double s0, c0;
+        sincos(ph, &s0, &c0);
+        s = fma(c0, lo, s0);
+        c = fma(-s0, lo, c0);
     }
     double* t = tab + (size_t)(is_x ? 0 : 2) * na * g.Mp + (size_t)idx * g.Mp + m;
     t[0] = c;
