@@ -145,11 +145,13 @@ constexpr bool pair_passes(size_t op_bytes, int Rp) { return op_bytes == 4 || Rp
 // Waves per SIMD the registers are held to: FP32 operands leave them idle with
 // two (each barrier and epilogue shows).  n_r = 44, 300 rays, 31375 pairs: three
 // waves 10.7 ms, 81% of the FP32 matrix rate; four 12.9, its spilled A prefetch
-// waits on every load.  Longer rays need the registers for B.
+// waits on every load.  Longer rays take the registers for B: spilled, they cost
+// the runtime 8192 waves' worth of private memory (65 MB at n_r = 65) and gained
+// nothing (7.84 against 7.88 ms for 150 images).
 template <typename OpT, int CT, int NK, bool EMIT>
 constexpr int pair_min_waves() {
     if (sizeof(OpT) != 4 || CT != 1 || EMIT) return 2;
-    return NK <= 8 ? 4 : NK <= 32 ? 3 : 2;
+    return NK <= 8 ? 4 : NK <= 24 ? 3 : 2;
 }
 
 // Persistent all-pairs kernel.  A workgroup takes a tile (one image k1 and up
@@ -363,8 +365,11 @@ __global__ __launch_bounds__(512, (pair_min_waves<OpT, CT, NK, EMIT>())) void pa
         };
         // FP32: one chunk holds this lane's fragments of the four k-steps 4q..4q+3
         auto quad = [&](const int4* buf, int half, int q) -> f32x4 {
-            const char* arow = (const char*)buf + lc * CPR * 16;
-            return *(const f32x4*)(arow + AT::phys(lc, half * (CPR / 2) + h * (NK / 4) + q) * 16);
+            int row = lc;
+            // long rays: addresses formed at each read, not kept in registers
+            if constexpr (NK >= 48) asm volatile("" : "+v"(row));
+            const char* arow = (const char*)buf + row * CPR * 16;
+            return *(const f32x4*)(arow + AT::phys(row, half * (CPR / 2) + h * (NK / 4) + q) * 16);
         };
         auto step = [&](int at, const int4* cur, int4* nxt) {
             if (at + 1 < g.NAT) {
@@ -498,7 +503,7 @@ __global__ __launch_bounds__(512, (pair_min_waves<OpT, CT, NK, EMIT>())) void pa
                 for (int ct = 0; ct < CT; ct++) epi(ct, g.NAT - 1);
                 keep_cells(g.NAT - 1);
             }
-            if (!pair_passes(sizeof(OpT), Rp) || pass == a.passes) break;
+            if (EMIT || !pair_passes(sizeof(OpT), Rp) || pass == a.passes) break;
             chunk++;
         }
         __syncthreads();

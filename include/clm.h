@@ -476,15 +476,17 @@ typedef struct clm_pft_params {
 } clm_pft_params;
 
 typedef struct clm_pft_stats {
-    float ms_tables;   /* exact: per-axis exponential tables; NUFFT:
-                          kernel weights of the polar points           */
-    float ms_stage;    /* exact: images to the pixel-major FP64 staging
-                          area; NUFFT: deconvolution onto the grids     */
+    float ms_tables;   /* exact: per-axis cosines and sines; NUFFT:
+                          deconvolution factors, kernel weights of the
+                          polar points                                  */
+    float ms_stage;    /* exact: images folded over both axes, FP64;
+                          NUFFT: norms, deconvolution onto the grids    */
     float ms_pft;      /* exact: the contraction (FP64 MFMA); NUFFT: the
                           interpolation at the polar points            */
     int32_t chunks;    /* image chunks (exact: at most 8192 images;
-                          NUFFT: at most 2048 images and 4 GiB of grid) */
-    float ms_fft;      /* NUFFT: the batched 2-D FFTs                   */
+                          NUFFT: at most 2048 images, and 4 GiB at a
+                          grid per image; two images share a grid)      */
+    float ms_fft;      /* NUFFT: the batched FFTs along both axes       */
     int32_t grid_side; /* NUFFT: oversampled grid side N (2,3,5-smooth,
                           >= 2n)                                        */
 } clm_pft_stats;
