@@ -502,7 +502,9 @@ def pft_bench(args):
     """cryo_pft of the K=5000 workload's images (n=129, n_r=65, n_theta=360,
     FP64) with clm_pft: images/s; the contraction kernel's FP64 MFMA roofline
     (algorithmic 4 flops per polar point, pixel and image: a complex weight
-    times a real pixel); the FP64 C oracle on a bounded image sample as the
+    times a real pixel; the pixels folded over both axes need about a quarter
+    of them, so frac can pass 1 and executed_frac is the matrix cores' share);
+    the FP64 C oracle on a bounded image sample as the
     CPU baseline and parity check; the same transform by torch (weights
     materialised, rocBLAS ZGEMM) for reference."""
     import torch
@@ -543,9 +545,10 @@ def pft_bench(args):
     tpath = os.path.join(ROOT, "profiles", "pft_kernel_k5000_traffic.json")
     if os.path.exists(tpath) and K == 5000:
         traffic = json.load(open(tpath))["hbm_bytes_per_launch"]
-    Mp = (M + 127) // 128 * 128
-    nup = (n + 3) // 4 * 4
-    Kp = (K + 63) // 64 * 64
+    # four real planes over a quarter of the pixels, tiles of 64 points x 64 images
+    Mq = (n_r * (T // 4 + 1) + 63) // 64 * 64
+    nh = n // 2 + 1
+    executed = 2.0 * 4 * Mq * ((nh + 3) // 4 * 4) * nh * ((K + 63) // 64 * 64)
     # torch (rocBLAS ZGEMM over materialised weights), same images
     torch.cuda.synchronize()
     t = time.perf_counter()
@@ -572,7 +575,8 @@ def pft_bench(args):
                       "n_r": n_r, "n_theta": T},
            "roofline": {"bound": "mfma", "achieved": achieved / 1e12, "peak": 78.6, "unit": "TFLOP/s",
                         "frac": achieved / 78.6e12, "traffic": traffic, "kernel": "pft_kernel", "kernel_ms": k_ms,
-                        "flops_per_image": W_img, "executed_flops": 4.0 * Mp * n * nup * Kp},
+                        "flops_per_image": W_img, "executed_flops": executed,
+                        "executed_frac": executed / (k_ms * 1e-3) / 78.6e12},
            "stats": st,
            "cpu_baseline": {"value": ns / cpu_sec, "unit": "images/s", "cores": nth, "kind": "port",
                             "sample": f"{ns} images of the workload, FP64 C oracle (OpenMP)"},
@@ -758,9 +762,10 @@ def estimate_shifts_dropin(st0, K, n_theta, max_shift=10, shift_step=0.5):
 def vote_bench(args):
     """S = cryo_syncmatrix_vote(clstack, 360) of the K=5000 workload's common
     lines (BF16 engine), on the device; the oracle on a seeded sample of pairs
-    (one thread) as the CPU baseline and parity sample.  The work is FP64
-    transcendental evaluation: the kernel evaluates 60 Gaussians per voting
-    triangle (the exponential count per second is reported)."""
+    (one thread) as the CPU baseline and parity sample.  The reference
+    evaluates 60 Gaussians per voting triangle (their number per second is
+    reported); the kernel forms them from two exponentials as an outer product on
+    the FP64 matrix cores."""
     import torch
 
     from aspire_amd import sim
@@ -819,11 +824,12 @@ def vote_bench(args):
 
 
 def vote_roofline(K, st):
-    """FP64 roofline of the vote at K=5000: its FP64 operations per vote
-    as rocprof counts them (ADD + MUL + 2 FMA + TRANS wave instructions x 64,
-    profiles/vote_kernel_k5000_f64.md: the reference's arithmetic, each
-    triangle evaluated once, 60 Gaussians of the histogram per triangle)
-    over the vote's own device time (HIP events around its kernels)."""
+    """FP64 roofline of the vote at K=5000: the FP64 operations of the
+    reference's arithmetic (each triangle evaluated once, 60 Gaussians of the
+    histogram per triangle, as rocprof counted them in kernels that did them:
+    ADD + MUL + 2 FMA + TRANS wave instructions x 64) over the vote's own device
+    time (HIP events around its kernels).  The outer-product histogram needs a
+    fraction of them, so frac can pass 1."""
     if K != 5000:
         return None
     flops = 6.9e13
@@ -832,9 +838,9 @@ def vote_roofline(K, st):
         return None
     achieved = flops / (ms * 1e-3)
     return {"bound": "fp64-valu", "achieved": achieved / 1e12, "peak": 78.6, "unit": "TFLOP/s",
-            "frac": achieved / 78.6e12, "traffic": None, "kernel": "vote (peak_kernel + rot_kernel)",
+            "frac": achieved / 78.6e12, "traffic": None, "kernel": "vote (peak_kernel + terms_kernel + rot_kernel)",
             "kernel_ms": ms, "flops_per_vote": flops,
-            "flops_basis": "FP64 operations counted by rocprof for this workload (each triangle once)"}
+            "flops_basis": "FP64 operations of the reference's arithmetic for this workload (each triangle once)"}
 
 
 def sync3n_bench(args):
@@ -844,9 +850,8 @@ def sync3n_bench(args):
     conjugated by J).  value = triangles/s of the scores kernel.  Roofline:
     FP64 vector; the reference's arithmetic is 297 flops per triangle (four
     3x3 products, four squared norms, three divisions, square roots and
-    subtractions), which the per-pair kernel evaluates three times (once per
-    side; rocprof counts 659 executed FP64 operations per triangle, with the
-    division and square-root sequences).  CPU baseline: the oracle's split
+    subtractions), and the per-pair kernel evaluates each triangle three
+    times (once per side), from one set of nine products each.  CPU baseline: the oracle's split
     of the triangle loop over threads (the reference's) on the first 600
     images; parity: the GPU against the one-thread oracle on those images."""
     import torch
@@ -929,8 +934,7 @@ def sync3n_bench(args):
            "signs_times_v": {"seconds": sec_v, "triangles_per_s": T / sec_v, "n_eigs": 4, "stats": stv},
            "roofline": {"bound": "fp64-valu", "achieved": achieved / 1e12, "peak": 78.6, "unit": "TFLOP/s",
                         "frac": achieved / 78.6e12, "traffic": traffic, "kernel": "tri_scores_kernel",
-                        "kernel_ms": st["ms_kernel"], "flops_per_triangle": 297,
-                        "executed_flops_per_triangle": 659},
+                        "kernel_ms": st["ms_kernel"], "flops_per_triangle": 297},
            "cpu_baseline": {"value": Ts / cpu_s, "unit": "triangles/s", "cores": int(nth), "kind": "port",
                             "sample": f"N={Ns} (first images), the oracle's threaded split (the reference's)"},
            "parity_sample": {"N": Ns, "hist_equal": bool(np.array_equal(hg, ho)),
