@@ -207,25 +207,33 @@ __global__ __launch_bounds__(512, (pair_min_waves<OpT, CT, NK, EMIT>())) void pa
     // k1 (which all stream its A-stack) meet in one XCD's L2.  A workgroup
     // drains its own XCD's queue, then helps the next ones.
     int cq = a.nq > 1 ? (int)(blockIdx.x % (unsigned)a.nq) : 0;
-    int left = a.nq > 1 ? a.nq : 1;
 
     for (;;) {
-        if (tid == 0) {
+        if (wv == 0) {
             int t = ntiles;
             if (a.nq > 1) {
-                while (left > 0) {
-                    const int u = a.qbeg[cq] + atomicAdd(a.counter + cq, 1);
+                for (;;) {
+                    int u = 0;
+                    if (lane == 0) u = a.qbeg[cq] + atomicAdd(a.counter + cq, 1);
+                    u = __builtin_amdgcn_readfirstlane(u);
                     if (u < a.qbeg[cq + 1]) {
                         t = u;
                         break;
                     }
-                    cq = cq + 1 == a.nq ? 0 : cq + 1;
-                    left--;
+                    // empty: look at all the queues at once.  The counts only grow, so
+                    // a queue that fails is not looked for again.
+                    const int q = (cq + 1 + lane) % a.nq;
+                    const bool some = lane < a.nq && a.qbeg[q] + __hip_atomic_load(a.counter + q, __ATOMIC_RELAXED,
+                                                                                   __HIP_MEMORY_SCOPE_AGENT) <
+                                                         a.qbeg[q + 1];
+                    const unsigned long long open = __ballot(some);
+                    if (!open) break;
+                    cq = (cq + 1 + __builtin_ctzll(open)) % a.nq;
                 }
             } else {
-                t = atomicAdd(a.counter, 1);
+                if (lane == 0) t = atomicAdd(a.counter, 1);
             }
-            s_i[0] = t;
+            if (lane == 0) s_i[0] = t;
         }
         if (tid >= 1 && tid < 32) s_i[tid] = 0;
         if (tid < 32) { s_unc[tid] = 0; s_pm[tid] = -INFINITY; }
