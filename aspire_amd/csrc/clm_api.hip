@@ -856,7 +856,14 @@ int launch_rescore(clm_ctx* c, const Plan& pl, unsigned grid, RescoreArgs a, int
         a.stat += 16 + GSTRIDE * pl.groups.size();
         a.stat_mask = NSTAT - 1;
     }
-    hipLaunchKernelGGL(rescore_kernel, dim3(grid), dim3(256), rescore_lds_bytes(a.mode, R), c->stream, a);
+    // a workgroup per pair while all of them run at once, four on a CU: the pair
+    // with the most cells then sets the time
+    const long long items = a.mode ? (long long)a.item_cap : (long long)a.n_items;
+    if (items <= 4LL * c->n_cu)
+        hipLaunchKernelGGL(rescore_kernel<true>, dim3((unsigned)std::max(items, 1LL)), dim3(256), rescore_lds_bytes(a.mode, R),
+                           c->stream, a);
+    else
+        hipLaunchKernelGGL(rescore_kernel<false>, dim3(grid), dim3(256), rescore_lds_bytes(a.mode, R), c->stream, a);
     HIPCHK(c, hipGetLastError());
     return CLM_OK;
 }

@@ -322,7 +322,9 @@ __host__ __device__ inline size_t rescore_lds_bytes(int mode, int R) {
 // Bound by the L1 accesses of the row loads where there are many pairs (3.1 ms
 // for 499,500 pairs with 6.8 cells each at n_r = 45; 3.4 with one candidate
 // per step in FP64, divisions to take a tie key apart and one counter for
-// all), by latency where there are few (54 us for 780 pairs, was 69).
+// all), by latency where there are few: with TEAM the four waves of a workgroup
+// share a pair's rows and candidates (780 pairs, 34 us; a wave each 53).
+template <bool TEAM>
 __global__ __launch_bounds__(256, 4) void rescore_kernel(RescoreArgs a) {
     extern __shared__ __align__(16) char s_rs[];
     const int lane = threadIdx.x & 63;
@@ -332,14 +334,19 @@ __global__ __launch_bounds__(256, 4) void rescore_kernel(RescoreArgs a) {
     const int ldt = a.Rmax | 1;
     double* const sterm = (double*)s_rs + (size_t)wave * RS_NB * ldt;
     long long* const skey = (long long*)((double*)s_rs + (size_t)4 * RS_NB * ldt) + wave * RS_NB;
-    float* const sval = (float*)((long long*)((double*)s_rs + (size_t)4 * RS_NB * ldt) + 4 * RS_NB) + (size_t)wave * nvmax;
+    float* const sval = (float*)((long long*)((double*)s_rs + (size_t)4 * RS_NB * ldt) + 4 * RS_NB) + (size_t)(TEAM ? 0 : wave) * nvmax;
+    // a team's bests, one per wave
+    __shared__ double s_tv[4];
+    __shared__ long long s_tk[4];
+    const bool lead = !TEAM || wave == 0;
     const int q = lane & 3, rl = lane >> 2;  // k-quarter, row within a set of 16
     const bool listed = a.mode != 0, emit = a.mode == 1;
     const long long n_items = listed ? (long long)min(*a.n_items_dev, a.item_cap) : a.n_items;
     // counts, summed over the workgroup's items and added once at the end
     __shared__ unsigned long long s_cnt[3][4];
     unsigned long long c_cell = 0, c_emit = 0, c_64 = 0;
-    for (long long item = (long long)blockIdx.x * W + wave; item < n_items; item += (long long)gridDim.x * W) {
+    for (long long item = TEAM ? (long long)blockIdx.x : (long long)blockIdx.x * W + wave; item < n_items;
+         item += TEAM ? (long long)gridDim.x : (long long)gridDim.x * W) {
         int stk, slot;
         if (!listed) {
             stk = a.stack0 + (a.nstacks > 1 ? find_stack(a.stacks + a.stack0, a.nstacks, item) : 0);
@@ -363,27 +370,27 @@ __global__ __launch_bounds__(256, 4) void rescore_kernel(RescoreArgs a) {
         int nrows;
         if (!emit) {
             if (rec.flags & F_EMPTY) {
-                if (lane == 0) write_result(sd, slot, 0.0, 0);
+                if (lead && lane == 0) write_result(sd, slot, 0.0, 0);
                 continue;
             }
             if (rec.flags & (F_UNCERTAIN | F_OVERFLOW)) {
-                if (lane == 0) { const int u = atomicAdd(a.unc_count, 1); a.unc_list[u] = SlotRef{stk, slot}; }
+                if (lead && lane == 0) { const int u = atomicAdd(a.unc_count, 1); a.unc_list[u] = SlotRef{stk, slot}; }
                 continue;
             }
             nrows = 16 * rec.ncells;
-            c_cell += (unsigned long long)rec.ncells;
+            if (lead) c_cell += (unsigned long long)rec.ncells;
         } else {
             if (er->overflow) {
-                if (lane == 0) { const int u = atomicAdd(a.fb_count, 1); a.fb_list[u] = SlotRef{stk, slot}; }
+                if (lead && lane == 0) { const int u = atomicAdd(a.fb_count, 1); a.fb_list[u] = SlotRef{stk, slot}; }
                 continue;
             }
             nrows = er->n;
-            c_emit += (unsigned long long)nrows;
+            if (lead) c_emit += (unsigned long long)nrows;
         }
         // ---- FP32 re-score
         float bv = -INFINITY;
         long long bk = 0x7fffffffffffffffLL;
-        for (int base = 0; base < nrows; base += 32) {
+        for (int base = TEAM ? 32 * wave : 0; base < nrows; base += TEAM ? 32 * W : 32) {
             int row[2], col[2], e[2], l1[2];
             const float4 *p[2], *bb[2], *ph[2];
             float X[2] = {0.f, 0.f}, Y[2] = {0.f, 0.f};
@@ -455,6 +462,16 @@ __global__ __launch_bounds__(256, 4) void rescore_kernel(RescoreArgs a) {
             const long long ok = __shfl_xor(bk, o, 64);
             if (better(ov, ok, bv, bk)) { bv = ov; bk = ok; }
         }
+        if constexpr (TEAM) {  // the team's best (a float's value is exact as a double)
+            if (lane == 0) {
+                s_tv[wave] = (double)bv;
+                s_tk[wave] = bk;
+            }
+            __syncthreads();
+            for (int w = 0; w < W; w++)
+                if (better((float)s_tv[w], s_tk[w], bv, bk)) { bv = (float)s_tv[w]; bk = s_tk[w]; }
+            __syncthreads();
+        }
         double fv = (double)bv;
         long long fk = bk;
         if (sd.fp64 && bv > -INFINITY) {
@@ -474,9 +491,9 @@ __global__ __launch_bounds__(256, 4) void rescore_kernel(RescoreArgs a) {
                 const bool on = ic < nv && sval[ic] >= lim;
                 const unsigned long long mask = __ballot(on);
                 const int n = __popcll(mask);
-                c_64 += (unsigned long long)n;
+                if (lead) c_64 += (unsigned long long)n;
                 const int pos = __popcll(mask & lanemask_lt());
-                for (int c0 = 0; c0 < n; c0 += RS_NB) {
+                for (int c0 = TEAM ? RS_NB * wave : 0; c0 < n; c0 += TEAM ? RS_NB * W : RS_NB) {
                     if (on && pos >= c0 && pos < c0 + RS_NB) {
                         int row, col;
                         cand_rc(cg, cmode, rec, er, ic >> 1, row, col);
@@ -521,10 +538,20 @@ __global__ __launch_bounds__(256, 4) void rescore_kernel(RescoreArgs a) {
                 const long long ok = __shfl_xor(k64, o, 64);
                 if (better64(ov, ok, b64, k64)) { b64 = ov; k64 = ok; }
             }
+            if constexpr (TEAM) {
+                if (lane == 0) {
+                    s_tv[wave] = b64;
+                    s_tk[wave] = k64;
+                }
+                __syncthreads();
+                for (int w = 0; w < W; w++)
+                    if (better64(s_tv[w], s_tk[w], b64, k64)) { b64 = s_tv[w]; k64 = s_tk[w]; }
+                __syncthreads();
+            }
             fv = b64;
             fk = k64;
         }
-        if (lane == 0) write_result(sd, slot, fv, fk);
+        if (lead && lane == 0) write_result(sd, slot, fv, fk);
         __builtin_amdgcn_wave_barrier();
     }
     if (lane == 0) {
