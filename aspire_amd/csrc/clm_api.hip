@@ -58,10 +58,13 @@ Variant choose_variant(int opk, int NCT, int Rp, int want_ct, int want_W, long l
     const int ncts = opk == OPK_F32 ? 2 : 3;
     // Column tiles of the busiest SIMD: a workgroup's waves go to the four SIMDs
     // in turn, so W waves cost as many as the next multiple of four, and the
-    // last round of workgroups counts whole.
-    auto cost = [&](int waves, int per_tile, int tiles_per_wave) {
+    // last round of workgroups counts whole.  A 16-bit column tile costs more
+    // the fewer share an A fragment: 1.5 times with two (0.655 us a pair against
+    // 0.321 with three and even loads, 41 shifts, n_r = 65), 2.2 with one.
+    auto cost = [&](int waves, int per_tile, int tiles_per_wave, int ct) {
         const long long per_round = (long long)per_tile * n_cu;
-        return (double)((npairs + per_round - 1) / per_round) * ((waves + 3) / 4) * tiles_per_wave;
+        const double w = opk == OPK_F32 || ct == 3 ? 1.0 : ct == 2 ? 1.5 : 2.2;
+        return w * (double)((npairs + per_round - 1) / per_round) * ((waves + 3) / 4) * tiles_per_wave;
     };
     for (int i = 0; i < ncts; i++) {
         const int ct = cts[i];
@@ -76,7 +79,7 @@ Variant choose_variant(int opk, int NCT, int Rp, int want_ct, int want_W, long l
         if (W < CPP || W % CPP || W > 8) continue;
         Variant v;
         v.ct = ct; v.W = W; v.CPP = CPP; v.NCTp = NCTp; v.ser = want_ser;
-        const double side = cost(W, W / CPP, ct), one = cost(sw, sw, NCTp);
+        const double side = cost(W, W / CPP, ct, ct), one = cost(sw, sw, NCTp, ct);
         const double waste = (double)NCTp / NCT;
         if (waste < best_waste - 1e-9) {
             best_waste = waste;
@@ -95,8 +98,9 @@ Variant choose_variant(int opk, int NCT, int Rp, int want_ct, int want_W, long l
     // tenth or more.  300 rays (five column tiles), five waves a pair put two
     // on one SIMD; FP32, 31375 pairs of n_r = 44 with one wave through the five:
     // 19.0 -> 10.7 ms; FP16, 124750 pairs of n_r = 45 with two waves of three tiles
-    // (one of padding): 25.6 -> 8.9 ms.  360 rays, BF16, 79800 pairs of n_r = 90: three
-    // waves a pair 16.7, one through the three 13.3 ms.
+    // (one of padding): 25.6 -> 8.9 ms.  BF16 rays of 90 points, one wave through the
+    // column groups: 360 rays, 79800 pairs, 16.7 -> 13.3 ms; 300 rays, 44850 pairs, 12.6
+    // -> 6.2 ms.
     return even_cost < 0.9 * best_cost ? even : best;
 }
 

@@ -373,11 +373,8 @@ __global__ __launch_bounds__(512, (pair_min_waves<OpT, CT, NK, EMIT>())) void pa
         };
         // FP32: one chunk holds this lane's fragments of the four k-steps 4q..4q+3
         auto quad = [&](const int4* buf, int half, int q) -> f32x4 {
-            int row = lc;
-            // long rays: addresses formed at each read, not kept in registers
-            if constexpr (NK >= 48) asm volatile("" : "+v"(row));
-            const char* arow = (const char*)buf + row * CPR * 16;
-            return *(const f32x4*)(arow + AT::phys(row, half * (CPR / 2) + h * (NK / 4) + q) * 16);
+            const char* arow = (const char*)buf + lc * CPR * 16;
+            return *(const f32x4*)(arow + AT::phys(lc, half * (CPR / 2) + h * (NK / 4) + q) * 16);
         };
         auto step = [&](int at, const int4* cur, int4* nxt) {
             if (at + 1 < g.NAT) {
