@@ -43,10 +43,14 @@
 //   a(x mod N, y mod N) = p(u, v) / (Phi(x) Phi(y)),  x = g(u), y = g(v)
 //   b = the unnormalized backward 2-D FFT of a (sum a e^{+2 pi i l x / N})
 //   pf(m) = sum_{t, r < NW} phi(2 (sx - lx - t)/NW) phi(2 (sy - ly - r)/NW) b(lx + t, ly + r)
-// Images are real, so two go through one grid, a = a_1 + i a_2: b at the points
-// m and, mirrored, -m gives b(m) = pf_1 + i pf_2 and conj b(-m) = pf_1 - i pf_2.
-// The window of -m is the window of m mirrored, with the same weights.  Half
-// the grids and transforms for the same number of grid reads.
+// Images are real, so b(-x, -y) = conj b(x, y) and the points' fx are in [0, pi):
+// an image keeps the columns x = 0..N/2 of its grid alone (real-to-complex
+// transforms along x), and a window's few columns beyond them are read from
+// their mirrors.  Half the grids and transforms of a complex grid per image, and
+// an image shares nothing with its neighbours in the stack: two images in one
+// complex grid cost about the same, and put the rounding of one's spectrum on the
+// other's (a point source, n = 359: 2.0e-14 of its own max |pf|, beside a
+// constant in one grid 6.0e-14).
 // Here sx = fx(m) N / (2 pi), lx = ceil(sx - NW/2) (sy, ly alike, indices mod
 // N) and Phi(x) = int phi(2s/NW) cos(2 pi s x / N) ds over |s| <= NW/2, the
 // kernel's Fourier transform (Gauss-Legendre quadrature).  The
@@ -54,7 +58,6 @@
 #include <hip/hip_runtime.h>
 #include <hipfft/hipfft.h>
 
-#include <climits>
 #include <cmath>
 #include <vector>
 
@@ -271,13 +274,13 @@ void pft_launch(hipStream_t st, const Geo& g, bool c128, const double* xt, const
 constexpr int NW = 16;                  // kernel width, grid points per axis
 constexpr double NBETA = 2.30 * NW;     // kernel shape for oversampling 2
 constexpr int NCHUNK = 2048;            // images per batch of FFTs (at most)
-constexpr int NIPW = 2;                 // grids (of two images) per direct interpolation workgroup
-constexpr int NBOXG = 4;                // grids per boxed interpolation workgroup
+constexpr int NIPW = 4;                 // images per direct interpolation workgroup
+constexpr int NBOXG = 8;                // images per boxed interpolation workgroup
 constexpr int BOXCAP = 1792;            // grid values of a box: 28 KB of LDS, five workgroups a CU
 
 struct NGeo {
     int n, n_r, n_theta, M;  // image side, rays, polar points M = n_r * n_theta/2
-    int N;                   // oversampled grid side
+    int N, H;                // oversampled grid side, columns kept of it (N/2 + 1)
     int x0;                  // g(0) = ceil(-n/2): pixel u sits at x = x0 + u
     int Kc;                  // images in this chunk
 };
@@ -319,113 +322,72 @@ __global__ __launch_bounds__(64) void dec_kernel(NGeo g, const double* __restric
     if (threadIdx.x == 0) dec[blockIdx.x] = 0.5 * NW * acc;
 }
 
-// The two images of a grid share its rounding, so each is brought to a norm
-// near 1 by a power of two first (exact), and an image that holds an infinity
-// or a NaN is kept out of the grid and becomes NaN at its own points alone
-// (as an image of zeros becomes zero).
-// part[i][s] = (sum of squares, largest |p|) of slice s of image i.
-constexpr int NSLICE = 32768;  // pixels per slice
-constexpr int NOT_FINITE = INT_MIN, ALL_ZERO = INT_MIN + 1;
-template <typename T>
-__global__ __launch_bounds__(256) void norm_kernel(NGeo g, const T* __restrict__ img, long long k0,
-                                                   double2* __restrict__ part) {
-    __shared__ double2 s_w[4];
-    const int px = g.n * g.n, end = min(px, ((int)blockIdx.x + 1) * NSLICE);
-    const T* p = img + (size_t)(k0 + blockIdx.y) * px;
-    double ss = 0.0, mx = 0.0;
-#pragma unroll 4
-    for (int q = blockIdx.x * NSLICE + threadIdx.x; q < end; q += 256) {
-        const double v = (double)p[q];
-        ss += v * v;
-        mx = fmax(mx, fabs(v));
-    }
-    for (int s = 32; s; s >>= 1) {
-        ss += __shfl_xor(ss, s);
-        mx = fmax(mx, __shfl_xor(mx, s));
-    }
-    if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = make_double2(ss, mx);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < 4; w++) {
-            ss += s_w[w].x;
-            mx = fmax(mx, s_w[w].y);
-        }
-        part[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = make_double2(ss, mx);
-    }
-}
-
-// Exponent e of an image's norm, or NOT_FINITE or ALL_ZERO.  Squares that left the range
-// of a double are replaced by the largest |p|.
-__global__ void exponent_kernel(NGeo g, const double2* __restrict__ part, int slices, int* __restrict__ ex) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= g.Kc) return;
-    double ss = 0.0, mx = 0.0;
-    for (int s = 0; s < slices; s++) {
-        const double2 v = part[(size_t)i * slices + s];
-        ss += v.x;
-        mx = fmax(mx, v.y);
-    }
-    int e;
-    if (ss != ss || mx > 1.7976931348623157e308) e = NOT_FINITE;
-    else if (ss > 1e-290 && ss <= 1.7976931348623157e308) e = ilogb(sqrt(ss));
-    else e = mx > 0.0 ? ilogb(mx) : ALL_ZERO;
-    ex[i] = e;
-}
-
-// Rows of the chunk's grids that hold pixels, a[i/2][v][x mod N], image i in
-// the real (i even) or imaginary part: 2^-ex[i] p(u, v, k0 + i) / (dec[u]
-// dec[v]) where a pixel sits, zero elsewhere.
+// Rows of the chunk's grids that hold pixels, a[i][v][x mod N]:
+// p(u, v, k0 + i) / (dec[u] dec[v]) where a pixel sits, zero elsewhere.
 template <typename T>
 __global__ void deconv_kernel(NGeo g, const T* __restrict__ img, long long k0, const double* __restrict__ dec,
-                              const int* __restrict__ ex, double2* __restrict__ a) {
+                              double* __restrict__ a) {
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const long long nN = (long long)g.n * g.N;
-    if (q >= nN * ((g.Kc + 1) / 2)) return;
-    const int i = 2 * (int)(q / nN);
+    if (q >= nN * g.Kc) return;
+    const int i = (int)(q / nN);
     const int r = (int)(q % nN);
     const int v = r / g.N, lx = r - v * g.N;
     const int xmax = g.x0 + g.n - 1;  // pixel offsets x0..xmax; N >= 2n keeps x and x - N apart
     const int x = lx <= xmax ? lx : lx - g.N;
-    double re = 0.0, im = 0.0;
+    double val = 0.0;
     if (x >= g.x0) {
         const int u = x - g.x0;
-        const size_t at = ((size_t)(k0 + i) * g.n + v) * g.n + u;
-        const double d = dec[u] * dec[v];
-        const int er = ex[i], ei = i + 1 < g.Kc ? ex[i + 1] : NOT_FINITE;
-        if (er > ALL_ZERO) re = ldexp((double)img[at], -er) / d;
-        if (ei > ALL_ZERO) im = ldexp((double)img[at + (size_t)g.n * g.n], -ei) / d;
+        val = (double)img[((size_t)(k0 + i) * g.n + v) * g.n + u] / (dec[u] * dec[v]);
     }
-    a[q] = make_double2(re, im);
+    a[q] = val;
 }
 
-// The rows' transforms over x, turned to b[i/2][x][y mod N] (y contiguous)
-// with zeros in the rows that held no pixel, for the transforms over y.  Those
-// rows (half of them and more) are neither transformed over x nor read, and b
-// is left turned: the interpolation reads it with its axes exchanged.  Tiles of
-// 32 x 32 through LDS.  For 50 grids of 720 x 720: 72 us (transforms over x) + 109
-// (this, 620 MB) + 146 (over y), where a 2-D plan takes 600: two whole passes
-// of transforms and two of transposes.
+// The rows' transforms over x, turned to b[i][x][y mod N] (x <= N/2, y
+// contiguous) with zeros in the rows that held no pixel, for the transforms over
+// y.  Those rows (half of them and more) are neither transformed over x nor read,
+// and b is left turned: the interpolation reads it with its axes exchanged.  The
+// real-to-complex transform has the sign of e^{-2 pi i l x / N}; its conjugate is
+// taken here.  Tiles of 32 x 32 through LDS.
 __global__ __launch_bounds__(256) void turn_kernel(NGeo g, const double2* __restrict__ a, double2* __restrict__ b) {
     __shared__ double2 s_t[32][33];
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
     const int x0 = blockIdx.x * 32, y0 = blockIdx.y * 32;
     const int xmax = g.x0 + g.n - 1;
-    a += (size_t)blockIdx.z * g.n * g.N;
-    b += (size_t)blockIdx.z * g.N * g.N;
+    a += (size_t)blockIdx.z * g.n * g.H;
+    b += (size_t)blockIdx.z * g.H * g.N;
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         const int ly = y0 + ty + 8 * r;
         const int y = ly <= xmax ? ly : ly - g.N;
         double2 v = make_double2(0.0, 0.0);
-        if (ly < g.N && y >= g.x0 && x0 + tx < g.N) v = a[(size_t)(y - g.x0) * g.N + x0 + tx];
+        if (ly < g.N && y >= g.x0 && x0 + tx < g.H) v = a[(size_t)(y - g.x0) * g.H + x0 + tx];
+        v.y = -v.y;
         s_t[ty + 8 * r][tx] = v;
     }
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         const int x = x0 + ty + 8 * r;
-        if (x < g.N && y0 + tx < g.N) b[(size_t)x * g.N + y0 + tx] = s_t[tx][ty + 8 * r];
+        if (x < g.H && y0 + tx < g.N) b[(size_t)x * g.N + y0 + tx] = s_t[tx][ty + 8 * r];
     }
+}
+
+// Where grid value (x, y mod N) of an image is kept, and whether its conjugate
+// is: x is in [-NW/2, N/2 + NW/2], and columns outside 0..N/2 are mirrors.
+struct Cell {
+    int at;
+    bool conj;
+};
+__device__ inline Cell cell_of(const NGeo& g, int x, int y) {
+    y %= g.N;
+    if (y < 0) y += g.N;
+    const bool mir = x < 0 || x >= g.H;
+    if (mir) {
+        x = x < 0 ? -x : g.N - x;
+        y = y ? g.N - y : 0;
+    }
+    return Cell{x * g.N + y, mir};
 }
 
 // Sum over the 16 lanes of each row (quad_perm [1,0,3,2], [2,3,0,1],
@@ -448,110 +410,64 @@ __device__ inline double row16_sum(double x) {
 __device__ inline void put_pf(double2* o, double re, double im) { *o = make_double2(re, im); }
 __device__ inline void put_pf(float2* o, double re, double im) { *o = make_float2((float)re, (float)im); }
 
-// Image i + t of a grid at a point from the grid's sums there (re, im) and at
-// the mirrored point (rm, imm).  Two images: b = re + i im, conj b(-m) = rm -
-// i imm; a lone one: b.
-template <typename OutT>
-__device__ inline void store_point(const NGeo& g, OutT* __restrict__ pf, const int* __restrict__ ex, long long k0,
-                                   int i, int t, bool two, int j, int k, double re, double im, double rm,
-                                   double imm) {
-    double x = re, y = im;
-    if (two) {
-        x = t == 0 ? 0.5 * (re + rm) : 0.5 * (im + imm);
-        y = t == 0 ? 0.5 * (im - imm) : 0.5 * (rm - re);
-    }
-    const int e = ex[i + t];
-    x = e > ALL_ZERO ? ldexp(x, e) : e == ALL_ZERO ? 0.0 : NAN;
-    y = e > ALL_ZERO ? ldexp(y, e) : e == ALL_ZERO ? 0.0 : NAN;
-    const size_t col = (size_t)(k0 + i + t) * g.n_theta;
-    put_pf(pf + (col + j) * g.n_r + k, x, y);
-    put_pf(pf + (col + j + g.n_theta / 2) * g.n_r + k, x, -y);
-}
-
 // pf of the chunk's images at the polar points.  Workgroup: 16 points (4
-// per wave, 16 lanes each; lane t = y offset of the window) x NIPW grids of
-// two images; each lane walks the NW rows of the point's window and of the
-// mirrored one in order, then the point's 16 lanes are summed.  pf(k, j) and its
-// conjugate pf(k, j + n_theta/2) (cryo_pft.m:75).
+// per wave, 16 lanes each; lane t = y offset of the window) x NIPW images; each
+// lane walks the NW columns of the point's window in order, then the point's 16
+// lanes are summed.  pf(k, j) and its conjugate pf(k, j + n_theta/2)
+// (cryo_pft.m:75).
 template <typename OutT>
 __global__ __launch_bounds__(256) void interp_kernel(NGeo g, const double2* __restrict__ b,
                                                      const int2* __restrict__ base, const double* __restrict__ wt,
-                                                     const int* __restrict__ ex, OutT* __restrict__ pf,
-                                                     long long k0) {
-    __shared__ double s_wy[16][NW];
+                                                     OutT* __restrict__ pf, long long k0) {
+    __shared__ double s_wx[16][NW];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int t = lane & 15, ps = wave * 4 + (lane >> 4);
     const int m = blockIdx.x * 16 + ps;
     const bool act = m < g.M;
-    int cx = 0, ry0 = 0, mx = 0;
-    double wx = 0.0;
+    int2 bs = make_int2(0, 0);
+    double wy = 0.0;
     if (act) {
-        const int2 bs = base[m];
-        wx = wt[(size_t)m * 2 * NW + t];
-        s_wy[ps][t] = wt[(size_t)m * 2 * NW + NW + t];
-        cx = (bs.x + t) % g.N;
-        if (cx < 0) cx += g.N;
-        mx = cx ? g.N - cx : 0;
-        ry0 = bs.y % g.N;
-        if (ry0 < 0) ry0 += g.N;
+        bs = base[m];
+        wy = wt[(size_t)m * 2 * NW + t];
+        s_wx[ps][t] = wt[(size_t)m * 2 * NW + NW + t];
     }
     __syncthreads();
     const int L = g.n_theta / 2;
     const int k = act ? m % g.n_r : 0, j = act ? m / g.n_r : 0;
-    const long long NN = (long long)g.N * g.N;
+    const size_t HN = (size_t)g.H * g.N;
     for (int ii = 0; ii < NIPW; ii++) {
-        const int i = 2 * (blockIdx.y * NIPW + ii);
+        const int i = blockIdx.y * NIPW + ii;
         if (i >= g.Kc) break;  // the same for the whole workgroup
-        const double2* bi = b + (size_t)(i / 2) * NN;
-        double re = 0.0, im = 0.0, rm = 0.0, imm = 0.0;  // at the point, at the mirrored point
-        const bool two = i + 1 < g.Kc;
-        if (act && two) {
-            int ry = ry0;
+        const double2* bi = b + i * HN;
+        double re = 0.0, im = 0.0;
+        if (act) {
 #pragma unroll 4
             for (int r = 0; r < NW; r++) {
-                const double w = s_wy[ps][r] * wx;
-                const int my = ry ? g.N - ry : 0;
-                const double2 v = bi[(size_t)ry * g.N + cx], n = bi[(size_t)my * g.N + mx];
+                const double w = s_wx[ps][r] * wy;
+                const Cell c = cell_of(g, bs.y + r, bs.x + t);
+                const double2 v = bi[c.at];
                 re = fma(w, v.x, re);
-                im = fma(w, v.y, im);
-                rm = fma(w, n.x, rm);
-                imm = fma(w, n.y, imm);
-                ry = ry + 1 == g.N ? 0 : ry + 1;
-            }
-        } else if (act) {
-            int ry = ry0;
-#pragma unroll 4
-            for (int r = 0; r < NW; r++) {
-                const double w = s_wy[ps][r] * wx;
-                const double2 v = bi[(size_t)ry * g.N + cx];
-                re = fma(w, v.x, re);
-                im = fma(w, v.y, im);
-                ry = ry + 1 == g.N ? 0 : ry + 1;
+                im = fma(c.conj ? -w : w, v.y, im);
             }
         }
         re = row16_sum(re);
         im = row16_sum(im);
-        if (two) {
-            rm = row16_sum(rm);
-            imm = row16_sum(imm);
-        }
-        if (act && t < (two ? 2 : 1)) store_point(g, pf, ex, k0, i, t, two, j, k, re, im, rm, imm);
+        if (act && t < 2)
+            put_pf(pf + ((size_t)(k0 + i) * g.n_theta + j + t * L) * g.n_r + k, re, t ? -im : im);
     }
 }
 
 // The same sums, bit for bit, with the windows read from LDS: a workgroup's 16
 // points are neighbours on one ray, so their windows lie in one box of the
-// grid, which is read once (and once mirrored) instead of 16 times.  The next
-// box is on its way into registers while this one is summed; a lane keeps its
-// 16 weights for all NBOXG grids.  The direct form reads 512 grid values a
-// point through the vector L1 and is bound there: 13.3 GB at 21 TB/s, 625 us for
-// 100 images, n = 359, 180 x 180 points.  This one takes 410 us; LDS is busy 60%
-// and the vector units 63% of it.
+// grid, which is read once instead of 16 times.  The next image's box is on its
+// way into registers while this one is summed; a lane keeps its 16 weights for
+// all NBOXG images.  The direct form reads 256 grid values a point and image
+// through the vector L1 and is bound there.
 template <typename OutT>
 __global__ __launch_bounds__(256) void interp_box_kernel(NGeo g, const d2* __restrict__ b,
                                                          const int2* __restrict__ base,
-                                                         const double* __restrict__ wt, const int* __restrict__ ex,
-                                                         OutT* __restrict__ pf, long long k0, int nkb) {
+                                                         const double* __restrict__ wt, OutT* __restrict__ pf,
+                                                         long long k0, int nkb) {
     __shared__ d2 s_box[BOXCAP];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int t = lane & 15, ps = wave * 4 + (lane >> 4);
@@ -560,50 +476,49 @@ __global__ __launch_bounds__(256) void interp_box_kernel(NGeo g, const d2* __res
     const bool act = k < g.n_r;
     // the windows' first indices are monotone along a ray, so its ends bound the box
     const int2 b0 = base[j * g.n_r + kb], b1 = base[j * g.n_r + kl];
-    const int x0 = min(b0.x, b1.x), y0 = min(b0.y, b1.y);
+    const int y0 = min(b0.x, b1.x), x0 = min(b0.y, b1.y);
     const int W = abs(b1.x - b0.x) + NW, H = abs(b1.y - b0.y) + NW;
     const int cells = min(W * H, BOXCAP);
     const int m = j * g.n_r + min(k, kl);  // lanes past the ray's end repeat its last point
     const int2 bs = base[m];
-    const double wx = wt[(size_t)m * 2 * NW + t];
+    const double wy = wt[(size_t)m * 2 * NW + t];
     double w[NW];
 #pragma unroll
-    for (int r = 0; r < NW; r++) w[r] = wt[(size_t)m * 2 * NW + NW + r] * wx;
-    const int at = (bs.y - y0) * W + bs.x - x0 + t;
+    for (int r = 0; r < NW; r++) w[r] = wt[(size_t)m * 2 * NW + NW + r] * wy;
+    const int at = (bs.y - x0) * W + bs.x - y0 + t;
     constexpr int NC = (BOXCAP + 255) / 256;  // cells per thread
-    unsigned off[NC], mir[NC];  // bytes into a grid (below 2^32: N <= 4096)
+    unsigned off[NC];                         // bytes into a grid (below 2^32: N <= 4096)
+    unsigned conj = 0;                        // bit q: cell q is a mirror
 #pragma unroll
     for (int q = 0; q < NC; q++) {
         const int c = min((int)threadIdx.x + q * 256, cells - 1);
         const int r = c / W;
-        int y = (y0 + r) % g.N, x = (x0 + c - r * W) % g.N;
-        if (y < 0) y += g.N;
-        if (x < 0) x += g.N;
-        off[q] = (y * g.N + x) * sizeof(d2);
-        mir[q] = ((y ? g.N - y : 0) * g.N + (x ? g.N - x : 0)) * sizeof(d2);
+        const Cell o = cell_of(g, x0 + r, y0 + c - r * W);
+        off[q] = o.at * (unsigned)sizeof(d2);
+        conj |= (unsigned)o.conj << q;
     }
-    const long long NN = (long long)g.N * g.N;
-    const int gr0 = blockIdx.y * NBOXG, gr1 = min(gr0 + NBOXG, (g.Kc + 1) / 2);
-    const char* bc = (const char*)(b + (size_t)gr0 * NN);
+    const size_t HN = (size_t)g.H * g.N;
+    const int i0 = blockIdx.y * NBOXG, i1 = min(i0 + NBOXG, g.Kc);
+    const char* bc = (const char*)(b + i0 * HN);
+    const int L = g.n_theta / 2;
     d2 nx[NC];
 #pragma unroll
     for (int q = 0; q < NC; q++)
         if (q * 256 < cells) nx[q] = *(const d2*)(bc + off[q]);
-    // phases: a grid's box, then its mirrored box (not for a lone image)
-    const int phases = 2 * (gr1 - gr0) - (2 * gr1 > g.Kc ? 1 : 0);
-    double r0 = 0.0, i0 = 0.0;
-    for (int ph = 0; ph < phases; ph++) {
+    for (int i = i0; i < i1; i++) {
         __syncthreads();  // the last box is no longer read
 #pragma unroll
         for (int q = 0; q < NC; q++)
-            if ((int)threadIdx.x + q * 256 < cells) s_box[threadIdx.x + q * 256] = nx[q];
+            if ((int)threadIdx.x + q * 256 < cells) {
+                if (conj >> q & 1) nx[q].y = -nx[q].y;
+                s_box[threadIdx.x + q * 256] = nx[q];
+            }
         __syncthreads();
-        if (ph + 1 < phases) {
-            const bool mirrored = (ph & 1) == 0;
-            if (!mirrored) bc += NN * sizeof(d2);
+        if (i + 1 < i1) {
+            bc += HN * sizeof(d2);
 #pragma unroll
             for (int q = 0; q < NC; q++)
-                if (q * 256 < cells) nx[q] = *(const d2*)(bc + (mirrored ? mir[q] : off[q]));
+                if (q * 256 < cells) nx[q] = *(const d2*)(bc + off[q]);
         }
         double re = 0.0, im = 0.0;
 #pragma unroll
@@ -614,18 +529,8 @@ __global__ __launch_bounds__(256) void interp_box_kernel(NGeo g, const d2* __res
         }
         re = row16_sum(re);
         im = row16_sum(im);
-        const bool two = (ph & 1) || ph + 1 < phases;
-        if ((ph & 1) || !two) {
-            const int i = 2 * (gr0 + ph / 2);
-            if (!two) {
-                r0 = re;
-                i0 = im;
-            }
-            if (act && t < (two ? 2 : 1)) store_point(g, pf, ex, k0, i, t, two, j, k, r0, i0, re, im);
-        } else {
-            r0 = re;
-            i0 = im;
-        }
+        if (act && t < 2)
+            put_pf(pf + ((size_t)(k0 + i) * g.n_theta + j + t * L) * g.n_r + k, re, t ? -im : im);
     }
 }
 
@@ -780,15 +685,15 @@ int smooth_at_least(int n) {
 
 // Plan of `batch` contiguous transforms of N points; the context keeps the
 // FFT_PLANS last used (two a shape), most recent first.
-hipfftHandle fft_plan(clm_ctx* c, int N, int batch, int* rc) {
+hipfftHandle fft_plan(clm_ctx* c, hipfftType type, int N, int batch, int* rc) {
     constexpr int S = clm_ctx::FFT_PLANS;
     int s = 0;
-    while (s < S && !(c->fft_plan[s] && c->fft_side[s] == N && c->fft_batch[s] == batch)) s++;
+    while (s < S && !(c->fft_plan[s] && c->fft_type[s] == (int)type && c->fft_side[s] == N && c->fft_batch[s] == batch)) s++;
     hipfftHandle h = nullptr;
     if (s < S) {
         h = (hipfftHandle)c->fft_plan[s];
     } else {
-        hipfftResult r = hipfftPlan1d(&h, N, HIPFFT_Z2Z, batch);
+        hipfftResult r = hipfftPlan1d(&h, N, type, batch);
         if (r == HIPFFT_SUCCESS) r = hipfftSetStream(h, c->stream);
         if (r != HIPFFT_SUCCESS) {
             if (h) (void)hipfftDestroy(h);
@@ -800,10 +705,12 @@ hipfftHandle fft_plan(clm_ctx* c, int N, int batch, int* rc) {
     }
     for (; s > 0; s--) {
         c->fft_plan[s] = c->fft_plan[s - 1];
+        c->fft_type[s] = c->fft_type[s - 1];
         c->fft_side[s] = c->fft_side[s - 1];
         c->fft_batch[s] = c->fft_batch[s - 1];
     }
     c->fft_plan[0] = (void*)h;
+    c->fft_type[0] = (int)type;
     c->fft_side[0] = N;
     c->fft_batch[0] = batch;
     return h;
@@ -817,13 +724,13 @@ int nufft_run(clm_ctx* c, const clm_pft_params* p, const void* d_img, void* d_pf
     g.n_theta = p->n_theta;
     g.M = p->n_r * (p->n_theta / 2);
     g.N = smooth_at_least(std::max(2 * p->n, 2 * NW));
+    g.H = g.N / 2 + 1;
     g.x0 = (int)std::ceil(-0.5 * p->n);
     const int K = p->K;
     const size_t NN = (size_t)g.N * g.N;
     // images per batch: at most NCHUNK, and grids of at most 4 GiB
     const int kc = (int)std::max<long long>(1, std::min<long long>({(long long)K, (long long)NCHUNK,
                                                                      (4LL << 30) / (long long)(NN * sizeof(double2))}));
-    const int slices = (g.n * g.n + NSLICE - 1) / NSLICE;
     // boxed interpolation where the box of 16 points of a ray fits: its sides
     // are at most 15 steps of N / (2 n_r - 1) times the ray's |sin| and |cos|,
     // plus 18, and their product is largest on the diagonal.  That is where n_r
@@ -831,12 +738,12 @@ int nufft_run(clm_ctx* c, const clm_pft_params* p, const void* d_img, void* d_pf
     const double side = 15.0 * g.N / (2.0 * g.n_r - 1.0) * M_SQRT1_2 + NW + 2;
     const bool boxed = side * side <= BOXCAP;
     int rc;
-    if ((rc = ensure(c, c->pft_grid, (size_t)((kc + 1) / 2) * NN * sizeof(double2))) ||
-        (rc = ensure(c, c->pft_xt, (size_t)((kc + 1) / 2) * g.n * g.N * sizeof(double2))) ||
+    // the grids' half columns (before them, the real rows), the rows' transforms
+    if ((rc = ensure(c, c->pft_grid, (size_t)kc * g.H * g.N * sizeof(double2))) ||
+        (rc = ensure(c, c->pft_xt, (size_t)kc * g.n * g.H * sizeof(double2))) ||
         (rc = ensure(c, c->pft_base, (size_t)g.M * sizeof(int2))) ||
         (rc = ensure(c, c->pft_wt, (size_t)g.M * 2 * NW * sizeof(double))) ||
-        (rc = ensure(c, c->pft_dec, (size_t)(g.n + 2 * NQ + 1) * sizeof(double) +
-                                        (size_t)kc * (slices * sizeof(double2) + sizeof(int)))))
+        (rc = ensure(c, c->pft_dec, (size_t)(g.n + 2 * NQ) * sizeof(double))))
         return rc;
     hipEvent_t* ev = c->ev;
     HIPCHK(c, hipEventRecord(ev[0], c->stream));
@@ -844,8 +751,6 @@ int nufft_run(clm_ctx* c, const clm_pft_params* p, const void* d_img, void* d_pf
     const std::vector<double>& nodes = kernel_nodes();
     double* dec = (double*)c->pft_dec.p;
     double* dnodes = dec + g.n;
-    double2* part = (double2*)(dec + ((g.n + 1) & ~1) + 2 * NQ);  // on 16 bytes
-    int* ex = (int*)(part + (size_t)kc * slices);
     HIPCHK(c, hipMemcpyAsync(dnodes, nodes.data(), nodes.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
     dec_kernel<<<g.n, 64, 0, c->stream>>>(g, dnodes, dnodes + NQ, dec);
     HIPCHK(c, hipGetLastError());
@@ -856,52 +761,46 @@ int nufft_run(clm_ctx* c, const clm_pft_params* p, const void* d_img, void* d_pf
     int chunks = 0;
     double2* grid = (double2*)c->pft_grid.p;
     double2* rows = (double2*)c->pft_xt.p;
+    double* real = (double*)c->pft_grid.p;  // n rows of N reals fit in H rows of N complex values
     for (long long k0 = 0; k0 < K; k0 += kc) {
         g.Kc = (int)((K - k0) < kc ? (K - k0) : kc);
-        const int ngrid = (g.Kc + 1) / 2;  // two images per grid
-        hipfftHandle plan_x = fft_plan(c, g.N, g.n * ngrid, &rc);
-        hipfftHandle plan_y = plan_x ? fft_plan(c, g.N, g.N * ngrid, &rc) : nullptr;
+        hipfftHandle plan_x = fft_plan(c, HIPFFT_D2Z, g.N, g.n * g.Kc, &rc);
+        hipfftHandle plan_y = plan_x ? fft_plan(c, HIPFFT_Z2Z, g.N, g.H * g.Kc, &rc) : nullptr;
         if (!plan_y) return rc;
         HIPCHK(c, hipEventRecord(ev[2], c->stream));
-        const long long nq = (long long)g.n * g.N * ngrid;
-        const dim3 ngrd(slices, g.Kc);
-        const unsigned dgrd = (unsigned)((nq + 255) / 256), egrd = (g.Kc + 63) / 64;
-        if (p->img_dtype == CLM_R64) {
-            norm_kernel<double><<<ngrd, 256, 0, c->stream>>>(g, (const double*)d_img, k0, part);
-            exponent_kernel<<<egrd, 64, 0, c->stream>>>(g, part, slices, ex);
-            deconv_kernel<double><<<dgrd, 256, 0, c->stream>>>(g, (const double*)d_img, k0, dec, ex, rows);
-        } else {
-            norm_kernel<float><<<ngrd, 256, 0, c->stream>>>(g, (const float*)d_img, k0, part);
-            exponent_kernel<<<egrd, 64, 0, c->stream>>>(g, part, slices, ex);
-            deconv_kernel<float><<<dgrd, 256, 0, c->stream>>>(g, (const float*)d_img, k0, dec, ex, rows);
-        }
+        const long long nq = (long long)g.n * g.N * g.Kc;
+        const unsigned dgrd = (unsigned)((nq + 255) / 256);
+        if (p->img_dtype == CLM_R64)
+            deconv_kernel<double><<<dgrd, 256, 0, c->stream>>>(g, (const double*)d_img, k0, dec, real);
+        else
+            deconv_kernel<float><<<dgrd, 256, 0, c->stream>>>(g, (const float*)d_img, k0, dec, real);
         HIPCHK(c, hipGetLastError());
         HIPCHK(c, hipEventRecord(ev[3], c->stream));
-        hipfftDoubleComplex *fx = (hipfftDoubleComplex*)rows, *fy = (hipfftDoubleComplex*)grid;
-        hipfftResult fr = hipfftExecZ2Z(plan_x, fx, fx, HIPFFT_BACKWARD);
+        hipfftDoubleComplex* fy = (hipfftDoubleComplex*)grid;
+        hipfftResult fr = hipfftExecD2Z(plan_x, real, (hipfftDoubleComplex*)rows);
         if (fr == HIPFFT_SUCCESS) {
-            const dim3 tgrd((g.N + 31) / 32, (g.N + 31) / 32, ngrid);
+            const dim3 tgrd((g.H + 31) / 32, (g.N + 31) / 32, g.Kc);
             turn_kernel<<<tgrd, 256, 0, c->stream>>>(g, rows, grid);
             HIPCHK(c, hipGetLastError());
             fr = hipfftExecZ2Z(plan_y, fy, fy, HIPFFT_BACKWARD);
         }
-        if (fr != HIPFFT_SUCCESS) return fail(c, CLM_E_HIP, "hipfftExecZ2Z failed (hipfftResult %d)", (int)fr);
+        if (fr != HIPFFT_SUCCESS) return fail(c, CLM_E_HIP, "hipFFT transform failed (hipfftResult %d)", (int)fr);
         HIPCHK(c, hipEventRecord(ev[4], c->stream));
         const int2* base = (const int2*)c->pft_base.p;
         const double* wt = (const double*)c->pft_wt.p;
         if (boxed) {
             const int nkb = (g.n_r + 15) / 16;
-            const dim3 igrid((g.n_theta / 2) * nkb, (ngrid + NBOXG - 1) / NBOXG);
+            const dim3 igrid((g.n_theta / 2) * nkb, (g.Kc + NBOXG - 1) / NBOXG);
             if (p->pf_dtype == CLM_C128)
-                interp_box_kernel<double2><<<igrid, 256, 0, c->stream>>>(g, (const d2*)grid, base, wt, ex, (double2*)d_pf, k0, nkb);
+                interp_box_kernel<double2><<<igrid, 256, 0, c->stream>>>(g, (const d2*)grid, base, wt, (double2*)d_pf, k0, nkb);
             else
-                interp_box_kernel<float2><<<igrid, 256, 0, c->stream>>>(g, (const d2*)grid, base, wt, ex, (float2*)d_pf, k0, nkb);
+                interp_box_kernel<float2><<<igrid, 256, 0, c->stream>>>(g, (const d2*)grid, base, wt, (float2*)d_pf, k0, nkb);
         } else {
-            const dim3 igrid((g.M + 15) / 16, (ngrid + NIPW - 1) / NIPW);
+            const dim3 igrid((g.M + 15) / 16, (g.Kc + NIPW - 1) / NIPW);
             if (p->pf_dtype == CLM_C128)
-                interp_kernel<double2><<<igrid, 256, 0, c->stream>>>(g, grid, base, wt, ex, (double2*)d_pf, k0);
+                interp_kernel<double2><<<igrid, 256, 0, c->stream>>>(g, grid, base, wt, (double2*)d_pf, k0);
             else
-                interp_kernel<float2><<<igrid, 256, 0, c->stream>>>(g, grid, base, wt, ex, (float2*)d_pf, k0);
+                interp_kernel<float2><<<igrid, 256, 0, c->stream>>>(g, grid, base, wt, (float2*)d_pf, k0);
         }
         HIPCHK(c, hipGetLastError());
         HIPCHK(c, hipEventRecord(ev[5], c->stream));
@@ -940,7 +839,7 @@ void pft_release(clm_ctx* c) {
     for (int s = 0; s < clm_ctx::FFT_PLANS; s++) {
         if (c->fft_plan[s]) (void)hipfftDestroy((hipfftHandle)c->fft_plan[s]);
         c->fft_plan[s] = nullptr;
-        c->fft_side[s] = c->fft_batch[s] = 0;
+        c->fft_type[s] = c->fft_side[s] = c->fft_batch[s] = 0;
     }
 }
 }  // namespace clmh
