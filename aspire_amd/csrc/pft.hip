@@ -83,8 +83,11 @@ struct Geo {
 // sin(fy(m) b), 4 nab rows each (zero for m >= M).  grid: (Mp/256, 8 nab).
 // The frequency of a point that serves two rays is the mean of the two rays'
 // rounded ones, f + df, and the phase keeps the product's rounding error.
-__global__ void tables_kernel(Geo g, double* tab) {
+// bad[i], i < K, is cleared.
+__global__ void tables_kernel(Geo g, double* tab, int* bad, int K) {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
+    if (blockIdx.y == 0)
+        for (long long i = m; i < K; i += gridDim.x * blockDim.x) bad[i] = 0;
     if (m >= g.Mp) return;
     const int na = 4 * g.nab;
     const bool is_x = (int)blockIdx.y < na;
@@ -115,9 +118,10 @@ __global__ void tables_kernel(Geo g, double* tab) {
 // planes ee, oo, oe (odd in u), eo; zero past nh and past the last image.
 // One workgroup folds FA columns a of the two rows +-b of 16 images: the rows
 // are read along u (contiguous) into LDS and written along the images.
+// bad[i] = 1: the image holds an infinity or a NaN.
 template <typename T>
 __global__ __launch_bounds__(256) void fold_kernel(Geo g, const T* __restrict__ img, long long k0,
-                                                   double* __restrict__ xt) {
+                                                   double* __restrict__ xt, int* __restrict__ bad) {
     __shared__ double s_p[4][16][FA + 1];  // p(+a,+b), p(-a,+b), p(+a,-b), p(-a,-b), zero where not a pixel
     const int a0 = blockIdx.x * FA, b = blockIdx.y, ct = blockIdx.z;
     const int tid = threadIdx.x;
@@ -128,7 +132,9 @@ __global__ __launch_bounds__(256) void fold_kernel(Geo g, const T* __restrict__ 
         const int u = q & 1 ? g.c - a : g.c + a, v = q & 2 ? g.c - b : g.c + b;
         const bool ok = u >= 0 && u < g.n && v >= 0 && v < g.n && 16 * ct + i < g.Kc && !((q & 1) && a == 0) &&
                         !((q & 2) && b == 0);
-        s_p[q][i][da] = ok ? (double)img[((size_t)(k0 + 16 * ct + i) * g.n + v) * g.n + u] : 0.0;
+        const double p = ok ? (double)img[((size_t)(k0 + 16 * ct + i) * g.n + v) * g.n + u] : 0.0;
+        s_p[q][i][da] = p;
+        if (!isfinite(p)) bad[k0 + 16 * ct + i] = 1;
     }
     __syncthreads();
     for (int x = tid; x < 16 * FA; x += 256) {
@@ -260,6 +266,54 @@ __global__ __launch_bounds__(256, 2) void pft_kernel(Geo g, const double* __rest
     }
 }
 
+// The folded sums of an image that holds an infinity or a NaN mix it into
+// planes that cancel or vanish; the sums as written carry it to every point with
+// its weight's sign.  One workgroup per image, which returns at once if the image
+// is finite; else the sums over its non-finite pixels (which decide every
+// value) in place of the folded ones.
+template <typename T, typename OutT>
+__global__ __launch_bounds__(256) void non_finite_kernel(Geo g, const T* __restrict__ img, long long k0,
+                                                         const int* __restrict__ bad, OutT* __restrict__ pf) {
+    constexpr int NL = 1024;  // pixels looked through at a time
+    __shared__ int s_list[NL];
+    __shared__ int s_n;
+    const size_t i = k0 + blockIdx.x;
+    if (!bad[i]) return;
+    const int px = g.n * g.n, L = g.n_theta / 2, M = g.n_r * L;
+    const double omega0 = 2.0 * M_PI / (2.0 * g.n_r - 1.0), dtheta = 2.0 * M_PI / g.n_theta;
+    const T* p = img + i * px;
+    bool first = true;
+    for (int q0 = 0; q0 < px; q0 += NL) {
+        if (threadIdx.x == 0) s_n = 0;
+        __syncthreads();
+        for (int q = q0 + threadIdx.x; q < min(q0 + NL, px); q += 256)
+            if (!isfinite((double)p[q])) s_list[atomicAdd(&s_n, 1)] = q;
+        __syncthreads();
+        const int cnt = s_n;
+        for (int m = threadIdx.x; m < M && cnt; m += 256) {
+            const int k = m % g.n_r, j = m / g.n_r;
+            const double fx = (k * omega0) * sin(j * dtheta), fy = (k * omega0) * cos(j * dtheta);
+            double re = 0.0, im = 0.0;
+            for (int c = 0; c < cnt; c++) {
+                const int q = s_list[c], v = q / g.n, u = q - v * g.n;
+                double sn, cs;
+                sincos(fx * (u - g.c) + fy * (v - g.c), &sn, &cs);
+                re += cs * (double)p[q];
+                im += sn * (double)p[q];
+            }
+            const size_t a = (i * g.n_theta + j) * g.n_r + k, b = a + (size_t)L * g.n_r;
+            if (!first) {
+                re += pf[a].x;
+                im += pf[a].y;
+            }
+            put<OutT>(pf, a, re, im);
+            put<OutT>(pf, b, re, -im);
+        }
+        if (cnt) first = false;
+        __syncthreads();
+    }
+}
+
 template <int RT, int CT>
 void pft_launch(hipStream_t st, const Geo& g, bool c128, const double* xt, const double* tab, void* pf, long long k0) {
     const int nmb = (g.M + 16 * RT - 1) / (16 * RT), ntiles = nmb * ((g.nct + CT - 1) / CT);
@@ -268,6 +322,13 @@ void pft_launch(hipStream_t st, const Geo& g, bool c128, const double* xt, const
         pft_kernel<double2, RT, CT><<<8 * per, 256, 0, st>>>(g, xt, tab, (double2*)pf, k0, nmb, ntiles, per);
     else
         pft_kernel<float2, RT, CT><<<8 * per, 256, 0, st>>>(g, xt, tab, (float2*)pf, k0, nmb, ntiles, per);
+}
+
+template <typename T>
+void non_finite_launch(hipStream_t st, const Geo& g, bool c128, const T* img, long long k0, const int* bad,
+                       void* pf) {
+    if (c128) non_finite_kernel<T, double2><<<g.Kc, 256, 0, st>>>(g, img, k0, bad, (double2*)pf);
+    else non_finite_kernel<T, float2><<<g.Kc, 256, 0, st>>>(g, img, k0, bad, (float2*)pf);
 }
 
 // ------------------------------------------------------------ type-2 NUFFT
@@ -572,14 +633,16 @@ int pft_run(clm_ctx* c, const clm_pft_params* p, const void* d_img, void* d_pf, 
     const int K = p->K;
     const int kc = K < KCHUNK ? K : KCHUNK;
     int rc;
-    if ((rc = ensure(c, c->pft_ax, (size_t)16 * g.nab * g.Mp * sizeof(double))) ||
+    const size_t ntab = (size_t)16 * g.nab * g.Mp;
+    if ((rc = ensure(c, c->pft_ax, ntab * sizeof(double) + (size_t)K * sizeof(int))) ||
         (rc = ensure(c, c->pft_xt, (size_t)((kc + 15) / 16) * 4 * g.nab * g.nh * 64 * sizeof(double))))
         return rc;
     hipEvent_t* ev = c->ev;
     double* tab = (double*)c->pft_ax.p;
+    int* bad = (int*)(tab + ntab);
     double* xt = (double*)c->pft_xt.p;
     HIPCHK(c, hipEventRecord(ev[0], c->stream));
-    tables_kernel<<<dim3((g.Mp + 255) / 256, 8 * g.nab), 256, 0, c->stream>>>(g, tab);
+    tables_kernel<<<dim3((g.Mp + 255) / 256, 8 * g.nab), 256, 0, c->stream>>>(g, tab, bad, K);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipEventRecord(ev[1], c->stream));
     float ms_stage = 0.f, ms_pft = 0.f;
@@ -590,9 +653,9 @@ int pft_run(clm_ctx* c, const clm_pft_params* p, const void* d_img, void* d_pf, 
         dim3 fgrid((4 * g.nab + FA - 1) / FA, g.nh, g.nct);
         HIPCHK(c, hipEventRecord(ev[2], c->stream));
         if (p->img_dtype == CLM_R64)
-            fold_kernel<double><<<fgrid, 256, 0, c->stream>>>(g, (const double*)d_img, k0, xt);
+            fold_kernel<double><<<fgrid, 256, 0, c->stream>>>(g, (const double*)d_img, k0, xt, bad);
         else
-            fold_kernel<float><<<fgrid, 256, 0, c->stream>>>(g, (const float*)d_img, k0, xt);
+            fold_kernel<float><<<fgrid, 256, 0, c->stream>>>(g, (const float*)d_img, k0, xt, bad);
         HIPCHK(c, hipGetLastError());
         HIPCHK(c, hipEventRecord(ev[3], c->stream));
         // the tile whose busiest CU has the fewest cycles: 64 per MFMA, and
@@ -613,6 +676,9 @@ int pft_run(clm_ctx* c, const clm_pft_params* p, const void* d_img, void* d_pf, 
         else if (best == 1) pft_launch<2, 4>(c->stream, g, c128, xt, tab, d_pf, k0);
         else if (best == 2) pft_launch<1, 4>(c->stream, g, c128, xt, tab, d_pf, k0);
         else pft_launch<1, 1>(c->stream, g, c128, xt, tab, d_pf, k0);
+        HIPCHK(c, hipGetLastError());
+        if (p->img_dtype == CLM_R64) non_finite_launch(c->stream, g, c128, (const double*)d_img, k0, bad, d_pf);
+        else non_finite_launch(c->stream, g, c128, (const float*)d_img, k0, bad, d_pf);
         HIPCHK(c, hipGetLastError());
         HIPCHK(c, hipEventRecord(ev[4], c->stream));
         HIPCHK(c, hipEventSynchronize(ev[4]));
