@@ -1834,7 +1834,7 @@ void clm_destroy(clm_ctx* c) {
                     &c->w_list, &c->w_plist, &c->w_tiles, &c->w_counts, &c->w_shiftv};
     for (DevBuf* b : wb) release(*b);
     pft_release(c);
-    DevBuf* pb[] = {&c->pft_ax, &c->pft_xt, &c->pft_img, &c->pft_out,
+    DevBuf* pb[] = {&c->pft_ax, &c->pft_ray, &c->pft_xt, &c->pft_img, &c->pft_out,
                     &c->pft_grid, &c->pft_base, &c->pft_wt, &c->pft_dec,
                     &c->ls_pack, &c->ls_u, &c->ls_part, &c->ls_vec, &c->ls_tab, &c->ls_state, &c->ls_tiles,
                     &c->es_rot, &c->es_x,

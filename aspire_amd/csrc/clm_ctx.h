@@ -63,6 +63,8 @@ struct clm_ctx {
     // deconvolution factors, and its hipFFT plans (opaque handles) with their
     // kind, transform length and batch
     clmh::DevBuf pft_ax, pft_xt, pft_img, pft_out;
+    clmh::DevBuf pft_ray;  // the rays' sines and cosines, for pft_ray_T rays
+    int pft_ray_T = 0;
     clmh::DevBuf pft_grid, pft_base, pft_wt, pft_dec;
     static constexpr int FFT_PLANS = 4;
     void* fft_plan[FFT_PLANS] = {};

@@ -25,12 +25,15 @@
 // Four real products over a quarter of the pixels serve two rays: a quarter
 // of the multiplications of the sums as written.  The weights are never
 // stored: a lane forms its operand as one product of two table entries.
-// Two rays that share a quadrant point are taken at the mean of their rounded
-// frequencies, which differ in the last bits.  Worst error over max |pf| of
-// white noise in extended precision, n = 129 and n_r = 65: 1.6e-14 at the
-// rounded frequencies and 1.7e-14 at the true polar points (the sums as written
-// with their weights advanced by rotations: 1.5e-14 and 3.5e-14); rms 7.7e-15
-// and 9.4e-15 (6.1e-15 and 1.3e-14).
+// Two rays that share a quadrant point have rounded frequencies that differ in
+// the last bits.  Ray j's are taken for the sums; for the mirror ray the
+// differences times the sums' derivatives are added (shift_kernel), a
+// contraction of the same shape whose values are 1e-14 of pf's, so that
+// operands of 11 bits leave less than 1e-16.  Error over max |pf| of white noise
+// in extended precision, n = 129 and n_r = 65: 2.8e-15 at worst, 7.5e-16 rms; with
+// the mean of the two frequencies for both rays 1.2e-14 and 2.4e-15; the sums as
+// written with phases rounded to a double, or weights advanced by rotations,
+// 1.5e-14 and 6.1e-15.
 //
 // CLM_PFT_NUFFT: the same sums by a type-2 non-uniform FFT, the method the
 // reference's nufft2 uses when a NUFFT library is installed
@@ -67,6 +70,9 @@ namespace pft {
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 typedef double d2 __attribute__((ext_vector_type(2)));
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 
 constexpr int KCHUNK = 8192;  // images per staged chunk
 constexpr int FA = 32;        // folded columns per staging workgroup
@@ -76,32 +82,34 @@ struct Geo {
     int M, Mp;       // quadrant points n_r * (n_theta/4 + 1), rows of the tables (padded for the row tiles)
     int c;           // pixel index of the origin: g(c) = 0
     int nh, nab;     // folded side floor(n/2) + 1, blocks of 4 of it
+    int nb8;         // blocks of 8 of the folded side
     int Kc, nct;     // images in this chunk, column tiles of 16
 };
 
 // tab[0][a*Mp + m] = cos(fx(m) a), tab[1] sin; then cos(fy(m) b) and
 // sin(fy(m) b), 4 nab rows each (zero for m >= M).  grid: (Mp/256, 8 nab).
-// The frequency of a point that serves two rays is the mean of the two rays'
-// rounded ones, f + df, and the phase keeps the product's rounding error.
-// bad[i], i < K, is cleared.
-__global__ void tables_kernel(Geo g, double* tab, int* bad, int K) {
+// ray: sin(j dtheta), then cos(j dtheta), j < n_theta/2, as cryo_pft.m:52-58 has
+// them.  The phase keeps the product's rounding error.
+// dx[a*Mp + m] = (cos(fx a), d a), (sin, d a) for the shift from fx to the
+// mirror ray's frequency fx + d: (X, X') of shift_kernel, X' = 2^DSCALE d dX/dfx;
+// along y eight b to a point, Y then Y': dy[((kind*nb8 + b/8)*Mp + m)*16 + b%8].
+// Null where they are not used.
+constexpr int DSCALE = 44;
+__global__ void tables_kernel(Geo g, const double* __restrict__ ray, double* tab, h2* dx, _Float16* dy) {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (blockIdx.y == 0)
-        for (long long i = m; i < K; i += gridDim.x * blockDim.x) bad[i] = 0;
     if (m >= g.Mp) return;
-    const int na = 4 * g.nab;
+    const int na = 4 * g.nab, L = g.n_theta / 2;
     const bool is_x = (int)blockIdx.y < na;
     const int idx = is_x ? blockIdx.y : blockIdx.y - na;
-    double s = 0.0, c = 0.0;
+    double s = 0.0, c = 0.0, d = 0.0;
     if (m < g.M) {
         const int k = m % g.n_r, j = m / g.n_r;
-        const double omega0 = 2.0 * M_PI / (2.0 * g.n_r - 1.0);  // cryo_pft.m:49
-        const double dtheta = 2.0 * M_PI / g.n_theta;             // cryo_pft.m:50
-        const double f = is_x ? (k * omega0) * sin(j * dtheta) : (k * omega0) * cos(j * dtheta);
-        double df = 0.0;
-        const int jm = g.n_theta / 2 - j;  // the mirrored ray
-        if (j > 0 && j < jm) df = 0.5 * ((is_x ? (k * omega0) * sin(jm * dtheta) : -(k * omega0) * cos(jm * dtheta)) - f);
-        const double ph = f * idx, lo = fma(f, (double)idx, -ph) + df * idx;
+        const int jm = L - j;  // the mirrored ray
+        const double r = k * (2.0 * M_PI / (2.0 * g.n_r - 1.0));  // cryo_pft.m:49
+        const double* t = is_x ? ray : ray + L;
+        const double f = r * t[j];
+        if (j > 0 && j < jm) d = (is_x ? r * t[jm] : -r * t[jm]) - f;
+        const double ph = f * idx, lo = fma(f, (double)idx, -ph);
         double s0, c0;
         sincos(ph, &s0, &c0);
         s = fma(c0, lo, s0);
@@ -110,6 +118,22 @@ __global__ void tables_kernel(Geo g, double* tab, int* bad, int K) {
     double* t = tab + (size_t)(is_x ? 0 : 2) * na * g.Mp + (size_t)idx * g.Mp + m;
     t[0] = c;
     t[(size_t)na * g.Mp] = s;
+    if (!dx) return;
+    d = ldexp(d, DSCALE) * idx;
+    const h2 vc = {(_Float16)c, (_Float16)(-d * s)}, vs = {(_Float16)s, (_Float16)(d * c)};
+    if (is_x) {
+        dx[(size_t)idx * g.Mp + m] = vc;
+        dx[(size_t)(na + idx) * g.Mp + m] = vs;
+        return;
+    }
+    const size_t kind = (size_t)g.nb8 * g.Mp * 16;
+    _Float16* y = dy + ((size_t)(idx / 8) * g.Mp + m) * 16 + idx % 8;
+    y[0] = vc.x;
+    y[8] = vc.y;
+    y[kind] = vs.x;
+    y[kind + 8] = vs.y;
+    if (idx + 4 >= na && idx + 4 < 8 * g.nb8)  // past the last four rows
+        y[4] = y[12] = y[kind + 4] = y[kind + 12] = (_Float16)0.f;
 }
 
 // Folded images, one 512-byte block per (column tile of 16 images, plane,
@@ -118,14 +142,19 @@ __global__ void tables_kernel(Geo g, double* tab, int* bad, int K) {
 // planes ee, oo, oe (odd in u), eo; zero past nh and past the last image.
 // One workgroup folds FA columns a of the two rows +-b of 16 images: the rows
 // are read along u (contiguous) into LDS and written along the images.
-// bad[i] = 1: the image holds an infinity or a NaN.
+// part[(ct*nh + b)*gridDim.x + blockIdx.x][16]: the high word of the largest |p|
+// the workgroup has seen of each image.
 template <typename T>
 __global__ __launch_bounds__(256) void fold_kernel(Geo g, const T* __restrict__ img, long long k0,
-                                                   double* __restrict__ xt, int* __restrict__ bad) {
+                                                   double* __restrict__ xt, unsigned* __restrict__ part) {
     __shared__ double s_p[4][16][FA + 1];  // p(+a,+b), p(-a,+b), p(+a,-b), p(-a,-b), zero where not a pixel
     const int a0 = blockIdx.x * FA, b = blockIdx.y, ct = blockIdx.z;
     const int tid = threadIdx.x;
-    for (int x = tid; x < 4 * 16 * FA; x += 256) {
+    unsigned hi[2] = {0, 0};  // of images tid/FA and tid/FA + 8
+    static_assert(FA == 32, "half waves");
+#pragma unroll
+    for (int s = 0; s < 4 * 16 * FA / 256; s++) {
+        const int x = tid + 256 * s;
         const int da = x % FA, i = (x / FA) % 16, q = x / (16 * FA);
         const int a = a0 + da;
         // the axes' own pixels count once
@@ -134,7 +163,12 @@ __global__ __launch_bounds__(256) void fold_kernel(Geo g, const T* __restrict__ 
                         !((q & 2) && b == 0);
         const double p = ok ? (double)img[((size_t)(k0 + 16 * ct + i) * g.n + v) * g.n + u] : 0.0;
         s_p[q][i][da] = p;
-        if (!isfinite(p)) bad[k0 + 16 * ct + i] = 1;
+        hi[s & 1] = max(hi[s & 1], (unsigned)(__double_as_longlong(p) >> 32) & 0x7fffffffu);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        for (int o = FA / 2; o; o >>= 1) hi[h] = max(hi[h], (unsigned)__shfl_xor((int)hi[h], o, FA));
+        if (tid % FA == 0) part[(((size_t)ct * g.nh + b) * gridDim.x + blockIdx.x) * 16 + tid / FA + 8 * h] = hi[h];
     }
     __syncthreads();
     for (int x = tid; x < 16 * FA; x += 256) {
@@ -153,6 +187,27 @@ __global__ __launch_bounds__(256) void fold_kernel(Geo g, const T* __restrict__ 
     }
 }
 
+// top[i]: the high word of image i's largest |p| (NOT_FINITE and above: it holds
+// an infinity or a NaN), over the cnt workgroups that folded it (one maximum an
+// image and workgroup by atomics took as long as the folding: an image tile's 16
+// words are one line).  One workgroup per column tile.
+constexpr unsigned NOT_FINITE = 0x7ff00000u;
+__global__ __launch_bounds__(256) void top_kernel(Geo g, const unsigned* __restrict__ part, int cnt,
+                                                  unsigned* __restrict__ top) {
+    __shared__ unsigned s_m[256];
+    const unsigned* p = part + (size_t)blockIdx.x * cnt * 16;
+    unsigned m = 0;
+#pragma unroll 4
+    for (int q = threadIdx.x; q < 16 * cnt; q += 256) m = max(m, p[q]);
+    s_m[threadIdx.x] = m;
+    __syncthreads();
+    if (threadIdx.x < 16) {
+        for (int q = 1; q < 16; q++) m = max(m, s_m[threadIdx.x + 16 * q]);
+        top[16 * blockIdx.x + threadIdx.x] = m;
+    }
+}
+__device__ inline int top_exponent(unsigned top) { return (int)(top >> 20) - 1023; }
+
 template <typename OutT>
 __device__ inline void put(OutT* pf, size_t at, double re, double im);
 template <>
@@ -162,6 +217,131 @@ __device__ inline void put<double2>(double2* pf, size_t at, double re, double im
 template <>
 __device__ inline void put<float2>(float2* pf, size_t at, double re, double im) {
     pf[at] = make_float2((float)re, (float)im);
+}
+
+// The folded images times 2^-e, e the exponent of the image's largest |p|, in
+// FP16 and in the operand order of the 16 x 16 x 32 MFMA:
+//   xh[(((ct*4 + plane)*nab + a/4)*nb8 + b/8)*64 + (a%4)*16 + image%16][b%8],
+// zero past nh.  One workgroup per (4 values of a, plane, column tile).
+__global__ __launch_bounds__(256) void narrow_kernel(Geo g, const double* __restrict__ xt,
+                                                     const unsigned* __restrict__ top, h8* __restrict__ xh) {
+    const size_t blk = ((size_t)blockIdx.z * 4 + blockIdx.y) * g.nab + blockIdx.x;
+    const int lane = threadIdx.x & 63;
+    const int e = top_exponent(top[16 * blockIdx.z + (lane & 15)]);
+    const double* x = xt + blk * g.nh * 64 + lane;
+    for (int bb = threadIdx.x >> 6; bb < g.nb8; bb += 4) {
+        h8 v;
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            const int b = 8 * bb + q;
+            v[q] = (_Float16)(b < g.nh ? (float)ldexp(x[(size_t)b * 64], -e) : 0.f);
+        }
+        xh[(blk * g.nb8 + bb) * 64 + lane] = v;
+    }
+}
+
+// What the mirror rays' sums change by from ray j's frequencies to their own,
+// times 2^(DSCALE - e): shift[i*Mp + m].  With (X, X') and (Y, Y') of the tables,
+// the plane's weights change by X' Y + X Y'.  Tiles, waves and planes as in
+// pft_kernel; a lane forms its eight weights of a row tile (one a, eight b) by
+// packed FP16 operations from one X pair and eight Y pairs that it keeps over the
+// loop of a; the next PD values' operands are on their way meanwhile.
+// 243 us for 1000 images of 129 x 129, n_r = 65, n_theta = 360 (the sums take
+// 3.24 ms), 1.0 PFLOP/s.  Bound: the operands' loads; tiles of 8 x 4 have two thirds
+// of them and took 212 us, but leave fewer images without work for every CU.
+template <int RT, int CT, int PD>
+__global__ __launch_bounds__(256, 2) void shift_kernel(Geo g, const h8* __restrict__ xh, const h2* __restrict__ dx,
+                                                       const _Float16* __restrict__ dy, float2* __restrict__ shift,
+                                                       int nmb, int ntiles, int per_xcd) {
+    __shared__ float s_s[4][16][16 * CT + 1];
+    const int t = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+    if (t >= ntiles) return;
+    const int mb = t % nmb, kb = t / nmb;
+    const int lane = threadIdx.x & 63;
+    const int plane = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int r16 = lane & 15, kq = lane >> 4;
+    const int m0 = mb * 16 * RT + r16;
+    const h2* px = dx + (size_t)((plane == 1 || plane == 2) * 4 * g.nab + kq) * g.Mp + m0;
+    const h8* py = (const h8*)(dy + ((size_t)(plane & 1) * g.nb8 * g.Mp + m0) * 16);
+    const h8* bp[CT];
+#pragma unroll
+    for (int c = 0; c < CT; c++) {
+        const int ct = min(kb * CT + c, g.nct - 1);  // past the last tile: that tile again, not stored
+        bp[c] = xh + ((size_t)ct * 4 + plane) * g.nab * g.nb8 * 64 + lane;
+    }
+    f4 acc[RT][CT];
+#pragma unroll
+    for (int r = 0; r < RT; r++)
+#pragma unroll
+        for (int c = 0; c < CT; c++) acc[r][c] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int bb = 0; bb < g.nb8; bb++) {
+        h8 y[RT], yd[RT], b[PD][CT];
+        h2 x[PD][RT];
+        auto load = [&](int ab0, h2 (&x)[PD][RT], h8 (&b)[PD][CT]) {
+#pragma unroll
+            for (int d = 0; d < PD; d++) {
+                const int ab = min(ab0 + d, g.nab - 1);
+#pragma unroll
+                for (int r = 0; r < RT; r++) x[d][r] = px[(size_t)4 * ab * g.Mp + 16 * r];
+#pragma unroll
+                for (int c = 0; c < CT; c++) b[d][c] = bp[c][((size_t)ab * g.nb8 + bb) * 64];
+            }
+        };
+#pragma unroll
+        for (int r = 0; r < RT; r++) {
+            y[r] = py[((size_t)bb * g.Mp + 16 * r) * 2];
+            yd[r] = py[((size_t)bb * g.Mp + 16 * r) * 2 + 1];
+        }
+        load(0, x, b);
+        for (int ab = 0; ab < g.nab; ab += PD) {
+            h2 xn[PD][RT];
+            h8 bn[PD][CT];
+            load(ab + PD, xn, bn);
+#pragma unroll
+            for (int d = 0; d < PD; d++) {
+                if (ab + d >= g.nab) break;
+#pragma unroll
+                for (int r = 0; r < RT; r++) {
+                    const _Float16 u = x[d][r].x, v = x[d][r].y;
+                    const h8 w = __builtin_elementwise_fma(h8{u, u, u, u, u, u, u, u}, yd[r], h8{v, v, v, v, v, v, v, v} * y[r]);
+#pragma unroll
+                    for (int c = 0; c < CT; c++)
+                        acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, b[d][c], acc[r][c], 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int d = 0; d < PD; d++) {
+#pragma unroll
+                for (int r = 0; r < RT; r++) x[d][r] = xn[d][r];
+#pragma unroll
+                for (int c = 0; c < CT; c++) b[d][c] = bn[d][c];
+            }
+        }
+    }
+    // D tile of the FP32 16x16 MFMAs: lane l, element e holds row 4*(l/16) + e
+#pragma unroll
+    for (int r = 0; r < RT; r++) {
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < CT; c++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) s_s[plane][4 * kq + e][16 * c + r16] = acc[r][c][e];
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < CT; q++) {
+            const int row = threadIdx.x & 15, col = (threadIdx.x >> 4) + 16 * q;
+            const int m = (mb * RT + r) * 16 + row, i = kb * 16 * CT + col;
+            if (m < g.M && i < g.Kc)
+                shift[(size_t)i * g.Mp + m] = make_float2(s_s[0][row][col] + s_s[1][row][col], s_s[2][row][col] - s_s[3][row][col]);
+        }
+    }
+}
+
+template <int RT, int CT, int PD>
+void shift_launch(hipStream_t st, const Geo& g, const h8* xh, const h2* dx, const _Float16* dy, float2* shift) {
+    const int nmb = (g.M + 16 * RT - 1) / (16 * RT), ntiles = nmb * ((g.nct + CT - 1) / CT);
+    const int per = (ntiles + 7) / 8;
+    shift_kernel<RT, CT, PD><<<8 * per, 256, 0, st>>>(g, xh, dx, dy, shift, nmb, ntiles, per);
 }
 
 // One workgroup: 16 RT quadrant points x 16 CT images; wave w contracts plane
@@ -182,7 +362,9 @@ __device__ inline void put<float2>(float2* pf, size_t at, double re, double im) 
 // cycles on the busiest CU (few images or points).
 template <typename OutT, int RT, int CT>
 __global__ __launch_bounds__(256, 2) void pft_kernel(Geo g, const double* __restrict__ xt,
-                                                     const double* __restrict__ tab, OutT* __restrict__ pf,
+                                                     const double* __restrict__ tab,
+                                                     const float2* __restrict__ shift,
+                                                     const unsigned* __restrict__ top, OutT* __restrict__ pf,
                                                      long long k0, int nmb, int ntiles, int per_xcd) {
     __shared__ double s_s[4][16][16 * CT + 1];
     const int t = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
@@ -259,8 +441,15 @@ __global__ __launch_bounds__(256, 2) void pft_kernel(Geo g, const double* __rest
             put<OutT>(pf, (ray + j) * g.n_r + k, cc - ss, sc + cs);
             put<OutT>(pf, (ray + j + L) * g.n_r + k, cc - ss, -(sc + cs));
             if (j > 0 && 2 * j < L) {
-                put<OutT>(pf, (ray + L - j) * g.n_r + k, cc + ss, sc - cs);
-                put<OutT>(pf, (ray + 2 * L - j) * g.n_r + k, cc + ss, -(sc - cs));
+                double re = cc + ss, im = sc - cs;
+                if (shift) {
+                    const float2 d = shift[(size_t)i * g.Mp + m];
+                    const int e = top_exponent(top[i]) - DSCALE;
+                    re += ldexp((double)d.x, e);
+                    im += ldexp((double)d.y, e);
+                }
+                put<OutT>(pf, (ray + L - j) * g.n_r + k, re, im);
+                put<OutT>(pf, (ray + 2 * L - j) * g.n_r + k, re, -im);
             }
         }
     }
@@ -273,12 +462,12 @@ __global__ __launch_bounds__(256, 2) void pft_kernel(Geo g, const double* __rest
 // value) in place of the folded ones.
 template <typename T, typename OutT>
 __global__ __launch_bounds__(256) void non_finite_kernel(Geo g, const T* __restrict__ img, long long k0,
-                                                         const int* __restrict__ bad, OutT* __restrict__ pf) {
+                                                         const unsigned* __restrict__ top, OutT* __restrict__ pf) {
     constexpr int NL = 1024;  // pixels looked through at a time
     __shared__ int s_list[NL];
     __shared__ int s_n;
     const size_t i = k0 + blockIdx.x;
-    if (!bad[i]) return;
+    if (top[blockIdx.x] < NOT_FINITE) return;
     const int px = g.n * g.n, L = g.n_theta / 2, M = g.n_r * L;
     const double omega0 = 2.0 * M_PI / (2.0 * g.n_r - 1.0), dtheta = 2.0 * M_PI / g.n_theta;
     const T* p = img + i * px;
@@ -315,20 +504,21 @@ __global__ __launch_bounds__(256) void non_finite_kernel(Geo g, const T* __restr
 }
 
 template <int RT, int CT>
-void pft_launch(hipStream_t st, const Geo& g, bool c128, const double* xt, const double* tab, void* pf, long long k0) {
+void pft_launch(hipStream_t st, const Geo& g, bool c128, const double* xt, const double* tab, const float2* shift,
+                const unsigned* top, void* pf, long long k0) {
     const int nmb = (g.M + 16 * RT - 1) / (16 * RT), ntiles = nmb * ((g.nct + CT - 1) / CT);
     const int per = (ntiles + 7) / 8;
     if (c128)
-        pft_kernel<double2, RT, CT><<<8 * per, 256, 0, st>>>(g, xt, tab, (double2*)pf, k0, nmb, ntiles, per);
+        pft_kernel<double2, RT, CT><<<8 * per, 256, 0, st>>>(g, xt, tab, shift, top, (double2*)pf, k0, nmb, ntiles, per);
     else
-        pft_kernel<float2, RT, CT><<<8 * per, 256, 0, st>>>(g, xt, tab, (float2*)pf, k0, nmb, ntiles, per);
+        pft_kernel<float2, RT, CT><<<8 * per, 256, 0, st>>>(g, xt, tab, shift, top, (float2*)pf, k0, nmb, ntiles, per);
 }
 
 template <typename T>
-void non_finite_launch(hipStream_t st, const Geo& g, bool c128, const T* img, long long k0, const int* bad,
+void non_finite_launch(hipStream_t st, const Geo& g, bool c128, const T* img, long long k0, const unsigned* top,
                        void* pf) {
-    if (c128) non_finite_kernel<T, double2><<<g.Kc, 256, 0, st>>>(g, img, k0, bad, (double2*)pf);
-    else non_finite_kernel<T, float2><<<g.Kc, 256, 0, st>>>(g, img, k0, bad, (float2*)pf);
+    if (c128) non_finite_kernel<T, double2><<<g.Kc, 256, 0, st>>>(g, img, k0, top, (double2*)pf);
+    else non_finite_kernel<T, float2><<<g.Kc, 256, 0, st>>>(g, img, k0, top, (float2*)pf);
 }
 
 // ------------------------------------------------------------ type-2 NUFFT
@@ -633,16 +823,45 @@ int pft_run(clm_ctx* c, const clm_pft_params* p, const void* d_img, void* d_pf, 
     const int K = p->K;
     const int kc = K < KCHUNK ? K : KCHUNK;
     int rc;
-    const size_t ntab = (size_t)16 * g.nab * g.Mp;
-    if ((rc = ensure(c, c->pft_ax, ntab * sizeof(double) + (size_t)K * sizeof(int))) ||
-        (rc = ensure(c, c->pft_xt, (size_t)((kc + 15) / 16) * 4 * g.nab * g.nh * 64 * sizeof(double))))
+    g.nb8 = (g.nh + 7) / 8;
+    // the mirror rays' shifts: 3e-14, nothing to a result in single precision
+    const bool c128 = p->pf_dtype == CLM_C128, shifted = c128 && p->n_theta > 4;
+    const int nct = (kc + 15) / 16, nfold = (4 * g.nab + FA - 1) / FA;
+    const size_t ntab = (size_t)16 * g.nab * g.Mp, nxt = (size_t)nct * 4 * g.nab * g.nh * 64;
+    const size_t npart = (size_t)nct * g.nh * nfold * 16;  // then 16 nct for top
+    const size_t ndx = shifted ? (size_t)8 * g.nab * g.Mp : 0, ndy = shifted ? (size_t)32 * g.nb8 * g.Mp : 0;
+    const size_t nxh = shifted ? (size_t)nct * 4 * g.nab * g.nb8 * 64 : 0, nsh = shifted ? (size_t)kc * g.Mp : 0;
+    if ((rc = ensure(c, c->pft_ax, ntab * sizeof(double) + ndx * sizeof(h2) + ndy * sizeof(_Float16))) ||
+        (rc = ensure(c, c->pft_xt, nxt * sizeof(double) + nxh * sizeof(h8) + nsh * sizeof(float2) +
+                                       (npart + 16 * nct) * sizeof(unsigned))))
         return rc;
+    const int L = g.n_theta / 2;
+    if (c->pft_ray_T != g.n_theta) {
+        // the rays' sines and cosines, as clm_pft_freqs returns them
+        std::vector<double> h(2 * (size_t)L);
+        const double dtheta = 2.0 * M_PI / g.n_theta;  // cryo_pft.m:50
+        for (int j = 0; j < L; j++) {
+            h[j] = sin(j * dtheta);
+            h[L + j] = cos(j * dtheta);
+        }
+        c->pft_ray_T = 0;
+        if ((rc = ensure(c, c->pft_ray, h.size() * sizeof(double)))) return rc;
+        HIPCHK(c, hipMemcpyAsync(c->pft_ray.p, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
+        HIPCHK(c, hipStreamSynchronize(c->stream));  // h is released on return
+        c->pft_ray_T = g.n_theta;
+    }
     hipEvent_t* ev = c->ev;
     double* tab = (double*)c->pft_ax.p;
-    int* bad = (int*)(tab + ntab);
+    h2* dx = shifted ? (h2*)(tab + ntab) : nullptr;
+    _Float16* dy = (_Float16*)(dx + ndx);
     double* xt = (double*)c->pft_xt.p;
+    h8* xh = (h8*)(xt + nxt);
+    float2* shift = shifted ? (float2*)(xh + nxh) : nullptr;
+    unsigned* part = (unsigned*)((float2*)(xh + nxh) + nsh);
+    unsigned* top = part + npart;
     HIPCHK(c, hipEventRecord(ev[0], c->stream));
-    tables_kernel<<<dim3((g.Mp + 255) / 256, 8 * g.nab), 256, 0, c->stream>>>(g, tab, bad, K);
+    tables_kernel<<<dim3((g.Mp + 255) / 256, 8 * g.nab), 256, 0, c->stream>>>(
+        g, (const double*)c->pft_ray.p, tab, dx, dy);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipEventRecord(ev[1], c->stream));
     float ms_stage = 0.f, ms_pft = 0.f;
@@ -650,17 +869,26 @@ int pft_run(clm_ctx* c, const clm_pft_params* p, const void* d_img, void* d_pf, 
     for (long long k0 = 0; k0 < K; k0 += KCHUNK) {
         g.Kc = (int)((K - k0) < KCHUNK ? (K - k0) : KCHUNK);
         g.nct = (g.Kc + 15) / 16;
-        dim3 fgrid((4 * g.nab + FA - 1) / FA, g.nh, g.nct);
+        const dim3 fgrid(nfold, g.nh, g.nct);
         HIPCHK(c, hipEventRecord(ev[2], c->stream));
         if (p->img_dtype == CLM_R64)
-            fold_kernel<double><<<fgrid, 256, 0, c->stream>>>(g, (const double*)d_img, k0, xt, bad);
+            fold_kernel<double><<<fgrid, 256, 0, c->stream>>>(g, (const double*)d_img, k0, xt, part);
         else
-            fold_kernel<float><<<fgrid, 256, 0, c->stream>>>(g, (const float*)d_img, k0, xt, bad);
+            fold_kernel<float><<<fgrid, 256, 0, c->stream>>>(g, (const float*)d_img, k0, xt, part);
         HIPCHK(c, hipGetLastError());
+        top_kernel<<<g.nct, 256, 0, c->stream>>>(g, part, g.nh * nfold, top);
         HIPCHK(c, hipEventRecord(ev[3], c->stream));
+        if (shifted) {
+            narrow_kernel<<<dim3(g.nab, 4, g.nct), 256, 0, c->stream>>>(g, xt, top, xh);
+            // small tiles while three a CU hold all of them (one image: 25 us
+            // against 51; 100: 72 against 57)
+            const long long small = (long long)((g.M + 31) / 32) * g.nct;
+            if (small <= 3LL * c->n_cu) shift_launch<2, 1, 4>(c->stream, g, xh, dx, dy, shift);
+            else shift_launch<4, 4, 2>(c->stream, g, xh, dx, dy, shift);
+            HIPCHK(c, hipGetLastError());
+        }
         // the tile whose busiest CU has the fewest cycles: 64 per MFMA, and
         // about 24 per operand load of a step
-        const bool c128 = p->pf_dtype == CLM_C128;
         const int rts[] = {4, 2, 1, 1}, cts[] = {4, 4, 4, 1};
         int best = 0;
         double cost = 0;
@@ -672,13 +900,13 @@ int pft_run(clm_ctx* c, const clm_pft_params* p, const void* d_img, void* d_pf, 
                 best = q;
             }
         }
-        if (best == 0) pft_launch<4, 4>(c->stream, g, c128, xt, tab, d_pf, k0);
-        else if (best == 1) pft_launch<2, 4>(c->stream, g, c128, xt, tab, d_pf, k0);
-        else if (best == 2) pft_launch<1, 4>(c->stream, g, c128, xt, tab, d_pf, k0);
-        else pft_launch<1, 1>(c->stream, g, c128, xt, tab, d_pf, k0);
+        if (best == 0) pft_launch<4, 4>(c->stream, g, c128, xt, tab, shift, top, d_pf, k0);
+        else if (best == 1) pft_launch<2, 4>(c->stream, g, c128, xt, tab, shift, top, d_pf, k0);
+        else if (best == 2) pft_launch<1, 4>(c->stream, g, c128, xt, tab, shift, top, d_pf, k0);
+        else pft_launch<1, 1>(c->stream, g, c128, xt, tab, shift, top, d_pf, k0);
         HIPCHK(c, hipGetLastError());
-        if (p->img_dtype == CLM_R64) non_finite_launch(c->stream, g, c128, (const double*)d_img, k0, bad, d_pf);
-        else non_finite_launch(c->stream, g, c128, (const float*)d_img, k0, bad, d_pf);
+        if (p->img_dtype == CLM_R64) non_finite_launch(c->stream, g, c128, (const double*)d_img, k0, top, d_pf);
+        else non_finite_launch(c->stream, g, c128, (const float*)d_img, k0, top, d_pf);
         HIPCHK(c, hipGetLastError());
         HIPCHK(c, hipEventRecord(ev[4], c->stream));
         HIPCHK(c, hipEventSynchronize(ev[4]));
