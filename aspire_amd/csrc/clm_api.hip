@@ -302,6 +302,7 @@ struct Plan {
     std::vector<Group> groups;
     std::vector<int> order;      // table index -> job index
     std::vector<StackDev> table;
+    std::vector<char> consts;    // host copy of the table and the stacks' constants, in flight until the job waits
     int sb_base = 0;             // first per-stack buffer set of the context used
     long long tw_max = 0;        // largest group refined by a twin (pairs)
     long long P = 0;
@@ -489,7 +490,8 @@ int prepare(clm_ctx* c, Plan& pl, int n, const clm_params* ps, const clm_stack_i
     pl.table.assign(nt, StackDev{});
     // the table and every stack's constants in one buffer and one copy: the
     // copies of a small job cost more than its kernels
-    std::vector<char> consts((size_t)nt * sizeof(StackDev));
+    std::vector<char>& consts = pl.consts;
+    consts.assign((size_t)nt * sizeof(StackDev), 0);
     std::vector<size_t> off((size_t)nt * 5, 0);
     auto place = [&](const void* v, size_t bytes) {
         const size_t at = (consts.size() + 255) & ~(size_t)255;
@@ -594,8 +596,6 @@ int prepare(clm_ctx* c, Plan& pl, int n, const clm_params* ps, const clm_stack_i
             base += pl.table[ti].npairs;
         }
     }
-    std::memcpy(consts.data(), pl.table.data(), (size_t)nt * sizeof(StackDev));
-    if ((rc = upload(c, c->table, consts))) return rc;
     // shared buffers: counters, lists, pass-2 tiles
     if ((rc = ensure(c, c->ctr, ctr_words(c, pl) * sizeof(unsigned long long)))) return rc;
     if ((rc = ensure(c, c->ulist, (size_t)std::max<long long>(ubase, 1) * sizeof(SlotRef)))) return rc;
@@ -679,7 +679,9 @@ int prepare(clm_ctx* c, Plan& pl, int n, const clm_params* ps, const clm_stack_i
             if (tc.key == key) G.tc = &tc;
         if (!G.tc) return fail(c, CLM_E_UNSUP, "tile cache too small for %zu groups", pl.groups.size());
     }
-    return CLM_OK;
+    // last, so that a plan that fails here leaves no copy of its memory in flight
+    if (nt) std::memcpy(consts.data(), pl.table.data(), (size_t)nt * sizeof(StackDev));
+    return upload(c, c->table, consts);
 }
 
 // Per-stack preprocessing (lines, filter, normalization, operand planes) and
@@ -1509,7 +1511,10 @@ int run_subset(clm_ctx* c, const clm_params* p, const uint8_t* d_sel, const clm_
         return fail(c, CLM_E_HIP, "subset tile shape changed");
     begin_stats(pl, st);
     if (st) st->pairs = nsel;
-    if (nsel == 0) return CLM_OK;
+    if (nsel == 0) {
+        HIPCHK(c, hipStreamSynchronize(c->stream));  // the plan's constants are released on return
+        return CLM_OK;
+    }
     if ((rc = run_plan(c, pl, true, st))) return rc;
     timed_stats(c, st);
     return CLM_OK;
