@@ -618,8 +618,11 @@ extern "C" int clm_sync3n_pairs_probabilities(clm_ctx* c, int32_t N, const doubl
         a.lk[3] = (1 - P2) * A;
         // products of the likelihoods where no factor over- or underflows:
         // the exponential's argument at most 0, the arbitrary model present,
-        // and u^df (u >= 2^-53 or 0) far from the smallest number
-        if (a.lform && x0 < 1 && a.lk[1] <= 16 && a.lk[3] >= 1e-100 && a.lk[3] <= 1e100 && a.lk[2] <= 1e100)
+        // and its least factor far from the smallest number: c_a, or with b < a
+        // c_a u^df, u >= 2^-53 or 0 (and c_b may vanish)
+        const double least = eb < ea ? std::ldexp(a.lk[3], -53 * 16) : a.lk[3];
+        if (a.lform && x0 < 1 && a.lk[1] <= 16 && a.lk[3] >= 1e-100 && least >= 1e-290 && a.lk[3] <= 1e100 &&
+            a.lk[2] <= 1e100)
             a.lform = 2;
     }
     a.ind = d_ln_f_ind;
