@@ -260,7 +260,7 @@ struct StackJob {
     Setup s;
     int opk = 0, exact = 0, use64 = 0;
     Variant v;
-    int lag = 0;
+    int lag = 0;                     // the lagged schedule is wanted
     long long P = 0;
     int group = -1;
     const double* lsh = nullptr;     // per-line pre-shift [K][L] (windowed search) or null
@@ -277,7 +277,9 @@ struct StackJob {
 
 // Stacks that share one pair-kernel instantiation (or the FP64 kernel).
 struct Group {
-    int opk = 0, exact = 0, ct = 0, Rp = 0, sym = 0, W = 0, CPP = 0, lag = 0;
+    int opk = 0, exact = 0, ct = 0, Rp = 0, sym = 0, W = 0, CPP = 0;
+    int lag = 0;                // lagged schedule: of W waves (an even number only)
+    int lag1 = 0;               // and of the first pass's
     int ser = 0;                // first pass: waves of a workgroup, a pair each (0: CPP waves a pair)
     int sel = 0;                // one stack of selected pairs (device-built tiles and list)
     int filt = 0;               // (FP64 groups) map_filter_radius of its stacks
@@ -371,7 +373,7 @@ int plan_stack(clm_ctx* c, const clm_params* p, StackJob& j) {
     g.NROWS = g.NE * g.L;
     g.NAT = (g.NROWS + 31) / 32;
     if ((long long)g.NROWS * g.Lp > 0xffffffffLL) return fail(c, CLM_E_UNSUP, "map too large");
-    j.lag = ((j.v.ser || j.v.W % 2 == 0) && want_lag && !(p->reserved & 1)) ? 1 : 0;
+    j.lag = want_lag && !(p->reserved & 1) ? 1 : 0;
     return CLM_OK;
 }
 
@@ -406,15 +408,15 @@ int prepare(clm_ctx* c, Plan& pl, int n, const clm_params* ps, const clm_stack_i
         StackJob& j = pl.jobs[i];
         if (j.P == 0) continue;
         const Geom& g = j.s.g;
-        const int lag = j.lag;
         if (j.sel_list) j.v.ser = 0;  // the selected pairs may be few
+        const int lag = j.lag && j.v.W % 2 == 0, lag1 = j.v.ser ? j.lag : lag;
         const int norefine = (j.p.reserved & 2) ? 1 : 0;
         int gi = -1;
         for (size_t q = 0; q < pl.groups.size() && !j.sel_list; q++) {
             const Group& G = pl.groups[q];
             if (!G.sel && G.exact == j.exact && G.filt == j.filt && G.norefine == norefine &&
                 (j.exact || (G.opk == j.opk && G.ct == j.v.ct && G.Rp == g.Rp && G.sym == g.sym && G.W == j.v.W &&
-                             G.CPP == j.v.CPP && G.ser == j.v.ser && G.lag == lag))) {
+                             G.CPP == j.v.CPP && G.ser == j.v.ser && G.lag == lag && G.lag1 == lag1))) {
                 gi = (int)q;
                 break;
             }
@@ -422,7 +424,7 @@ int prepare(clm_ctx* c, Plan& pl, int n, const clm_params* ps, const clm_stack_i
         if (gi < 0) {
             Group G;
             G.opk = j.opk; G.exact = j.exact; G.ct = j.v.ct; G.Rp = g.Rp; G.sym = g.sym;
-            G.W = j.v.W; G.CPP = j.v.CPP; G.ser = j.v.ser; G.lag = lag;
+            G.W = j.v.W; G.CPP = j.v.CPP; G.ser = j.v.ser; G.lag = lag; G.lag1 = lag1;
             G.sel = j.sel_list != nullptr;
             G.norefine = norefine;
             G.filt = j.filt;
@@ -445,7 +447,7 @@ int prepare(clm_ctx* c, Plan& pl, int n, const clm_params* ps, const clm_stack_i
         if (!v32.ct) continue;
         Group T;
         T.opk = OPK_F32; T.ct = v32.ct; T.Rp = pl.groups[gi].Rp; T.sym = pl.groups[gi].sym;
-        T.W = v32.W; T.CPP = v32.CPP; T.lag = (v32.W % 2 == 0) ? 1 : 0;
+        T.W = v32.W; T.CPP = v32.CPP; T.lag = T.lag1 = (v32.W % 2 == 0) ? 1 : 0;
         T.sel = 1;
         T.twin_of = (int)gi;
         for (int i : pl.groups[gi].members) {
@@ -975,7 +977,7 @@ int enqueue_job(clm_ctx* c, const Plan& pl, bool timed, int phases = PHASE_ALL) 
         pa.erecs = nullptr;
         pa.CPP = G.ser ? 1 : G.CPP;
         pa.passes = G.ser ? G.CPP : 1;
-        pa.lag = G.lag;
+        pa.lag = G.lag1;
         pa.prio = (pl.jobs[G.members[0]].p.reserved & 4) ? 0 : 1;
         long long max_tiles;
         if (G.sel) {
@@ -1583,7 +1585,7 @@ int autotune(clm_ctx* c, const clm_params* p, const void* d_pf, int sample_pairs
             pa.nq = 1;
             pa.CPP = G.ser ? 1 : G.CPP;
             pa.passes = G.ser ? G.CPP : 1;
-            pa.lag = G.lag;
+            pa.lag = G.lag1;
             pa.prio = (p->reserved & 4) ? 0 : 1;
             const unsigned grid = (unsigned)std::min<long long>((long long)c->n_cu * G.occ1, (long long)ntiles);
             if (grid >= (unsigned)NQ) {  // the same XCD queues as the measured job
@@ -1602,11 +1604,11 @@ int autotune(clm_ctx* c, const clm_params* p, const void* d_pf, int sample_pairs
                 ms = event_ms(c->ev[4], c->ev[5]);
             }
             const double per = (double)ms / (double)taken;
-            if (out && n < max_out) out[n] = clm_tune_entry{q.variant, G.lag, (double)ms, (int64_t)taken};
+            if (out && n < max_out) out[n] = clm_tune_entry{q.variant, G.lag1, (double)ms, (int64_t)taken};
             n++;
             if (per < best) {
                 best = per;
-                best_v = make_int4(cw.first, cw.second, G.lag, 0);
+                best_v = make_int4(cw.first, cw.second, G.lag1, 0);
             }
         }
     }
