@@ -366,7 +366,7 @@ int plan_stack(clm_ctx* c, const clm_params* p, StackJob& j) {
         for (const auto& e : c->tuned)
             if (e.first == key) { want_ct = e.second.x; want_W = e.second.y; want_lag = e.second.z; }
     }
-    j.v = choose_variant(j.opk, NCT, g.Rp, want_ct, want_W, j.P, c->n_cu);
+    j.v = choose_variant(j.opk, NCT, g.Rp, want_ct, want_W, c->least_padding ? 0 : j.P, c->n_cu);
     if (!j.v.ct) return fail(c, CLM_E_UNSUP, "no kernel variant for L=%d (variant %d)", g.L, p->variant);
     g.NCT = j.v.NCTp;
     g.Lp = 32 * j.v.NCTp;
@@ -1673,6 +1673,7 @@ struct NoAllocScope {
         c->arena = (char*)c->scratch;
         c->arena_cap = c->scratch_cap;
         c->arena_off = 0;
+        c->arena_short = false;
     }
     ~NoAllocScope() {
         c->arena = nullptr;
@@ -1881,8 +1882,20 @@ int clm_clmatrix_device_noalloc(clm_ctx* c, const clm_params* p, const void* d_p
                                                                                 : hipErrorInvalidDevice));
     HIPCHK(c, hipSetDevice(c->device));
     const clm_stack_io io{d_pf, d_cl1, d_cl2, d_jidx, d_corr, d_shift1d};
-    NoAllocScope scope(c);
-    return run_job(c, 1, p, &io, false, st);
+    int rc;
+    {
+        NoAllocScope scope(c);
+        rc = run_job(c, 1, p, &io, false, st);
+    }
+    // no room: nothing has run, and a split that pads the columns less may fit
+    // (120 points, 150 rays, FP16: 643 images against 630)
+    if (rc == CLM_E_UNSUP && c->arena_short) {
+        c->least_padding = true;
+        NoAllocScope scope(c);
+        rc = run_job(c, 1, p, &io, false, st);
+        c->least_padding = false;
+    }
+    return rc;
 }
 
 int clm_clmatrix_windowed(clm_ctx* c, const clm_params* p, const void* d_pf, const float* d_prop, double window,

@@ -98,6 +98,8 @@ struct clm_ctx {
     size_t scratch_cap = 0;
     char* arena = nullptr;
     size_t arena_cap = 0, arena_off = 0;
+    bool arena_short = false;    // the region was too small for the call
+    bool least_padding = false;  // search: the kernel variant of least column padding
 };
 
 namespace clmh {
@@ -129,11 +131,13 @@ inline int ensure(clm_ctx* c, DevBuf& b, size_t bytes) {
     if (c->arena) {
         // allocation-free call: carve from the scratch array, never hipMalloc/hipFree
         const size_t off = (c->arena_off + 255) & ~(size_t)255;
-        if (off > c->arena_cap || bytes > c->arena_cap - off)
+        if (off > c->arena_cap || bytes > c->arena_cap - off) {
+            c->arena_short = true;
             return fail(c, CLM_E_UNSUP,
                         "allocation-free call: the shape needs more device memory than the %zu-byte scratch "
                         "array (%zu bytes carved, %zu more requested)",
                         c->arena_cap, off, bytes);
+        }
         b.p = c->arena + off;
         b.n = bytes;
         c->arena_off = off + bytes;
