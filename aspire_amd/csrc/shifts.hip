@@ -339,14 +339,11 @@ constexpr int VE = 64, NG = 16;
 // the tiles in its column block, each in block order over the g-th of NG
 // slices of the blocks.  (A'u)[i] = (..((g0 + g1) + g2) ..) + g(NG-1).
 __device__ inline double atu_part(int K, const double* rowp, const double* colp, int i, int g) {
-    const int k = i >> 1, n2 = 2 * K;
-    const int kb = k / TR, cbk = k / TC;
+    const int n2 = 2 * K;
     const int ncb = (K + TC - 1) / TC, nkb = (K + TR - 1) / TR;
     // the partials of tiles that do not exist are zero (cleared before the
     // solve, never written), so every block is added: +0 changes no sum
     // that starts at +0, and the loads need no branch
-    (void)kb;
-    (void)cbk;
     double t = 0.0;
     const double* rp = rowp + (size_t)(g * ncb / NG) * n2 + i;
 #pragma unroll 4
@@ -481,11 +478,13 @@ __global__ __launch_bounds__(VE * NG) void step_kernel(int K, int ntiles, const 
         // workgroup reads the state any more): it does the scalar step
         int last = 0;
         if (threadIdx.x == 0) {
-            // the partial norm goes past the caches and is there before the
-            // count is raised; a release would write back the whole L2
+            // The order of the two is the hardware's, not the memory model's (whose
+            // release would write back the whole L2): an agent-scope store goes
+            // through to memory, stores count in vmcnt until they are there, and the
+            // asm block, which no memory access crosses, waits for it before the
+            // count is raised.  The last workgroup's loads go past its caches.
             __hip_atomic_store(part + blockIdx.x, sq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __builtin_amdgcn_s_waitcnt(0);
-            asm volatile("" ::: "memory");
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             const unsigned n = __hip_atomic_fetch_add(&S->arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             last = n + 1 == gridDim.x;
         }
