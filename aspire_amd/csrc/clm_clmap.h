@@ -221,6 +221,7 @@ __global__ __launch_bounds__(256, 2) void clmap64_kernel(Search64Args a) {
     double* s_rv = s_w + 2 * CF_MAXW;
     long long* s_rk = (long long*)(s_rv + 4);
     int* s_lost = (int*)(s_rk + 4);
+    int* s_stop = s_lost + 4;  // a wave has stopped (CandList)
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, kq = lane >> 4;
@@ -236,6 +237,7 @@ __global__ __launch_bounds__(256, 2) void clmap64_kernel(Search64Args a) {
         const double2* P1 = sd.P64 + (size_t)k1 * L * R;
         const double2* P2 = sd.P64 + (size_t)k2 * L * R;
         __syncthreads();
+        if (tid == 0) *s_stop = 0;
         if (tid < w) {
             s_w[tid] = 2.0 * sd.wts[tid * w + d];  // 2: a map entry is twice its sum
             s_w[CF_MAXW + tid] = sd.wts[d * w + tid] / sd.wts[d * w + d];
@@ -253,7 +255,8 @@ __global__ __launch_bounds__(256, 2) void clmap64_kernel(Search64Args a) {
         const int U = S * NO * NO;
         const int u0 = (int)((long long)blockIdx.y * U / a.x.sj), u1 = (int)((long long)(blockIdx.y + 1) * U / a.x.sj);
         const int KS = (R + 3) / 4;
-        for (int u = u0; u < u1; u++) {
+        int stop = 0;
+        for (int u = u0; u < u1 && !stop; u++) {
             const int j = u / (NO * NO), tr = (u / NO) % NO, tc = u % NO;
             const int row0 = tr * OT, col0 = tc * OT;
             const double2* ph = sd.ph64 + (size_t)j * R;
@@ -323,6 +326,9 @@ __global__ __launch_bounds__(256, 2) void clmap64_kernel(Search64Args a) {
                 }
             }
             __syncthreads();
+            // the units before this one's: all waves read it between two barriers
+            // that a wave of this unit writes it after
+            const int stopped = *s_stop;
             // rows (half, i) dealt to the waves, a lane per column; the taps
             // outermost, so that 32 reads are in flight
             double sum[32];
@@ -348,6 +354,7 @@ __global__ __launch_bounds__(256, 2) void clmap64_kernel(Search64Args a) {
                     sum[x] = fma(wt, s_T[(size_t)((x >> 4) * CF_T + i + y) * CF_LD + lane], sum[x]);
                 }
             }
+            stop = __builtin_amdgcn_readfirstlane(stopped);
             const bool okc = lane < OT && col0 + lane < L;
             const int rows = min(OT, L - row0);
             double m = -INFINITY;
@@ -365,6 +372,7 @@ __global__ __launch_bounds__(256, 2) void clmap64_kernel(Search64Args a) {
                 const int h = x >> 4, i = 4 * (x & 15) + wave;
                 if (i < rows) cl.keep(okc, sum[x], tie_key(j, h * L + col0 + lane, row0 + i), lane);
             }
+            if (lane == 0 && cl.stopped()) *s_stop = 1;
         }
         // the workgroup's maximum, then the candidates within the margin of it
         // with the oracle's arithmetic

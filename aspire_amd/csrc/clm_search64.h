@@ -25,6 +25,11 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 
 constexpr int S64_ROWS = 64;   // rows l1 staged at a time
 constexpr int S64_LIST = 64;   // candidates kept per wave
+// Sets of up to 64 candidates that found no room in a wave's list, after which
+// the wave stops: its pair is one of ties everywhere and goes to the exhaustive
+// kernels (4950 pairs of radially symmetric images: 44.4 ms there alone, 52.3
+// after a whole search, 44.3 so; filtered 17.4, 19.6, 18.2).
+constexpr int S64_STOP = 64;
 
 struct Search64Args {
     Exact64Args x;            // items, shift ranges (over units, see below), sv/sk
@@ -37,14 +42,13 @@ struct CandList {
     double* v;       // LDS, S64_LIST each
     long long* k;
     double mg, wm, thr;  // margin, maximum, keep threshold
-    int n;
-    bool lost;
+    int n, lost;  // entries; sets that did not all fit
     __device__ inline void reset(double margin) {
         mg = margin;
         wm = thr = -INFINITY;
-        n = 0;
-        lost = false;
+        n = lost = 0;
     }
+    __device__ inline bool stopped() const { return lost > S64_STOP; }
     // Raise the threshold for a new maximum (wave-uniform).
     __device__ inline void raise(double m) {
         wm = fmax(wm, m);
@@ -78,16 +82,16 @@ struct CandList {
                 k[pos] = key;
             }
         }
-        if (n + cnt > S64_LIST) lost = true;
+        if (n + cnt > S64_LIST) lost++;
         n = min(n + cnt, S64_LIST);
         __builtin_amdgcn_wave_barrier();
     }
     // The workgroup's maximum M; true if a list lost entries that the margin
-    // may hold.  Called by the four waves of the workgroup.
+    // may hold, or a wave has stopped.  Called by the four waves of the workgroup.
     __device__ inline bool finish(double* s_rv, int* s_lost, int wave, int lane, double& M) {
         if (lane == 0) {
             s_rv[wave] = wm;
-            s_lost[wave] = lost;
+            s_lost[wave] = stopped() ? 2 : lost != 0;
         }
         __syncthreads();
         M = s_rv[0];
@@ -95,7 +99,7 @@ struct CandList {
         for (int w = 1; w < 4; w++) M = fmax(M, s_rv[w]);
         bool over = false;
 #pragma unroll
-        for (int w = 0; w < 4; w++) over = over || (s_lost[w] && s_rv[w] >= M - mg);
+        for (int w = 0; w < 4; w++) over = over || s_lost[w] == 2 || (s_lost[w] && s_rv[w] >= M - mg);
         __syncthreads();
         return over;
     }
@@ -210,7 +214,7 @@ __global__ __launch_bounds__(256, (KS * CT * 4 + CT * 16 <= 200 ? 2 : 1)) void s
                     }
                     __syncthreads();
                 }
-                if (!work) continue;
+                if (!work || cl.stopped()) continue;
                 // conj(P1) .* ph = conj(P1 .* conj(ph)): the rows of the second
                 // half of an asymmetric grid take conjugate phases here and the
                 // imaginary part's sign below
