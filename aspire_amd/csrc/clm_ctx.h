@@ -61,14 +61,14 @@ struct clm_ctx {
     // polar Fourier transform: per-axis tables, folded images, host-form buffers;
     // the NUFFT method's oversampled grids, windows, kernel weights and
     // deconvolution factors, and its hipFFT plans (opaque handles) with their
-    // kind, transform length and batch
+    // transform length and batch
     clmh::DevBuf pft_ax, pft_xt, pft_img, pft_out;
     clmh::DevBuf pft_ray;  // the rays' sines and cosines, for pft_ray_T rays
     int pft_ray_T = 0;
     clmh::DevBuf pft_grid, pft_base, pft_wt, pft_dec;
     static constexpr int FFT_PLANS = 4;
     void* fft_plan[FFT_PLANS] = {};
-    int fft_type[FFT_PLANS] = {}, fft_side[FFT_PLANS] = {}, fft_batch[FFT_PLANS] = {};
+    int fft_side[FFT_PLANS] = {}, fft_batch[FFT_PLANS] = {};
     // shift least squares: packed lines, u, per-tile sums, 2K vectors and the tiles' partial
     // A'u sums, tables, scalar state, pair tiles
     clmh::DevBuf ls_pack, ls_u, ls_part, ls_vec, ls_tab, ls_state, ls_tiles;

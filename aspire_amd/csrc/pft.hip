@@ -47,13 +47,14 @@
 //   b = the unnormalized backward 2-D FFT of a (sum a e^{+2 pi i l x / N})
 //   pf(m) = sum_{t, r < NW} phi(2 (sx - lx - t)/NW) phi(2 (sy - ly - r)/NW) b(lx + t, ly + r)
 // Images are real, so b(-x, -y) = conj b(x, y) and the points' fx are in [0, pi):
-// an image keeps the columns x = 0..N/2 of its grid alone (real-to-complex
-// transforms along x), and a window's few columns beyond them are read from
-// their mirrors.  Half the grids and transforms of a complex grid per image, and
-// an image shares nothing with its neighbours in the stack: two images in one
-// complex grid cost about the same, and put the rounding of one's spectrum on the
-// other's (a point source, n = 359: 2.0e-14 of its own max |pf|, beside a
-// constant in one grid 6.0e-14).
+// an image keeps the columns x = 0..N/2 of its grid alone, and a window's few
+// columns beyond them are read from their mirrors.  Along x two rows of an image
+// go through one complex transform and are taken apart as they are turned.  Half
+// the grids and transforms of a complex grid per image, and an image shares
+// nothing with its neighbours in the stack: two images in one complex grid cost
+// the same, and put the rounding of one's spectrum on the other's (a point
+// source, n = 359: 2.0e-14 of its own max |pf|, beside a constant in one grid
+// 6.0e-14).
 // Here sx = fx(m) N / (2 pi), lx = ceil(sx - NW/2) (sy, ly alike, indices mod
 // N) and Phi(x) = int phi(2s/NW) cos(2 pi s x / N) ds over |s| <= NW/2, the
 // kernel's Fourier transform (Gauss-Legendre quadrature).  The
@@ -532,6 +533,7 @@ constexpr int BOXCAP = 1792;            // grid values of a box: 28 KB of LDS, f
 struct NGeo {
     int n, n_r, n_theta, M;  // image side, rays, polar points M = n_r * n_theta/2
     int N, H;                // oversampled grid side, columns kept of it (N/2 + 1)
+    int np;                  // pairs of pixel rows, (n + 1)/2
     int x0;                  // g(0) = ceil(-n/2): pixel u sits at x = x0 + u
     int Kc;                  // images in this chunk
 };
@@ -573,54 +575,62 @@ __global__ __launch_bounds__(64) void dec_kernel(NGeo g, const double* __restric
     if (threadIdx.x == 0) dec[blockIdx.x] = 0.5 * NW * acc;
 }
 
-// Rows of the chunk's grids that hold pixels, a[i][v][x mod N]:
-// p(u, v, k0 + i) / (dec[u] dec[v]) where a pixel sits, zero elsewhere.
+// Rows of the chunk's grids that hold pixels, two to a complex row, a[i][v/2][x mod
+// N]: p(u, v, k0 + i) / (dec[u] dec[v]) where a pixel sits, zero elsewhere, in the
+// real part for even v and the imaginary part for odd.
 template <typename T>
 __global__ void deconv_kernel(NGeo g, const T* __restrict__ img, long long k0, const double* __restrict__ dec,
-                              double* __restrict__ a) {
+                              double2* __restrict__ a) {
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long nN = (long long)g.n * g.N;
-    if (q >= nN * g.Kc) return;
-    const int i = (int)(q / nN);
-    const int r = (int)(q % nN);
-    const int v = r / g.N, lx = r - v * g.N;
+    const long long pN = (long long)g.np * g.N;
+    if (q >= pN * g.Kc) return;
+    const int i = (int)(q / pN);
+    const int r = (int)(q % pN);
+    const int v = 2 * (r / g.N), lx = r - (v / 2) * g.N;
     const int xmax = g.x0 + g.n - 1;  // pixel offsets x0..xmax; N >= 2n keeps x and x - N apart
     const int x = lx <= xmax ? lx : lx - g.N;
-    double val = 0.0;
+    double2 val = make_double2(0.0, 0.0);
     if (x >= g.x0) {
         const int u = x - g.x0;
-        val = (double)img[((size_t)(k0 + i) * g.n + v) * g.n + u] / (dec[u] * dec[v]);
+        const size_t at = ((size_t)(k0 + i) * g.n + v) * g.n + u;
+        val.x = (double)img[at] / (dec[u] * dec[v]);
+        if (v + 1 < g.n) val.y = (double)img[at + g.n] / (dec[u] * dec[v + 1]);
     }
     a[q] = val;
 }
 
-// The rows' transforms over x, turned to b[i][x][y mod N] (x <= N/2, y
-// contiguous) with zeros in the rows that held no pixel, for the transforms over
-// y.  Those rows (half of them and more) are neither transformed over x nor read,
-// and b is left turned: the interpolation reads it with its axes exchanged.  The
-// real-to-complex transform has the sign of e^{-2 pi i l x / N}; its conjugate is
-// taken here.  Tiles of 32 x 32 through LDS.
+// The rows' transforms over x, taken apart (z(x) = row_v(x) + i row_{v+1}(x), both
+// Hermitian) and turned to b[i][x][y mod N] (x <= N/2, y contiguous) with zeros in
+// the rows that held no pixel, for the transforms over y.  Those rows (half of them
+// and more) are neither transformed over x nor read, and b is left turned: the
+// interpolation reads it with its axes exchanged.  Tiles of 32 x 32 through LDS.
+// For 100 images, N = 720: 71 us (transforms over x) + 112 (this, 620 MB) + 147
+// (over y).  Real-to-complex transforms along x took 70, but a second kernel
+// compiled at the first use of each size (2.3 s against 1.2, n = 150).
 __global__ __launch_bounds__(256) void turn_kernel(NGeo g, const double2* __restrict__ a, double2* __restrict__ b) {
     __shared__ double2 s_t[32][33];
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
     const int x0 = blockIdx.x * 32, y0 = blockIdx.y * 32;
     const int xmax = g.x0 + g.n - 1;
-    a += (size_t)blockIdx.z * g.n * g.H;
+    const int x = x0 + tx, xm = x ? g.N - x : 0;
+    a += (size_t)blockIdx.z * g.np * g.N;
     b += (size_t)blockIdx.z * g.H * g.N;
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         const int ly = y0 + ty + 8 * r;
-        const int y = ly <= xmax ? ly : ly - g.N;
-        double2 v = make_double2(0.0, 0.0);
-        if (ly < g.N && y >= g.x0 && x0 + tx < g.H) v = a[(size_t)(y - g.x0) * g.H + x0 + tx];
-        v.y = -v.y;
-        s_t[ty + 8 * r][tx] = v;
+        const int v = (ly <= xmax ? ly : ly - g.N) - g.x0;
+        double2 o = make_double2(0.0, 0.0);
+        if (ly < g.N && v >= 0 && x < g.H) {
+            const double2 z = a[(size_t)(v >> 1) * g.N + x], m = a[(size_t)(v >> 1) * g.N + xm];
+            o = v & 1 ? make_double2(0.5 * (z.y + m.y), 0.5 * (m.x - z.x)) : make_double2(0.5 * (z.x + m.x), 0.5 * (z.y - m.y));
+        }
+        s_t[ty + 8 * r][tx] = o;
     }
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-        const int x = x0 + ty + 8 * r;
-        if (x < g.H && y0 + tx < g.N) b[(size_t)x * g.N + y0 + tx] = s_t[tx][ty + 8 * r];
+        const int xr = x0 + ty + 8 * r;
+        if (xr < g.H && y0 + tx < g.N) b[(size_t)xr * g.N + y0 + tx] = s_t[tx][ty + 8 * r];
     }
 }
 
@@ -713,7 +723,8 @@ __global__ __launch_bounds__(256) void interp_kernel(NGeo g, const double2* __re
 // grid, which is read once instead of 16 times.  The next image's box is on its
 // way into registers while this one is summed; a lane keeps its 16 weights for
 // all NBOXG images.  The direct form reads 256 grid values a point and image
-// through the vector L1 and is bound there.
+// through the vector L1 and is bound there.  390 us for 100 images, n = 359, 180 x
+// 180 points; LDS and the vector units are each busy about 60% of it.
 template <typename OutT>
 __global__ __launch_bounds__(256) void interp_box_kernel(NGeo g, const d2* __restrict__ b,
                                                          const int2* __restrict__ base,
@@ -979,15 +990,15 @@ int smooth_at_least(int n) {
 
 // Plan of `batch` contiguous transforms of N points; the context keeps the
 // FFT_PLANS last used (two a shape), most recent first.
-hipfftHandle fft_plan(clm_ctx* c, hipfftType type, int N, int batch, int* rc) {
+hipfftHandle fft_plan(clm_ctx* c, int N, int batch, int* rc) {
     constexpr int S = clm_ctx::FFT_PLANS;
     int s = 0;
-    while (s < S && !(c->fft_plan[s] && c->fft_type[s] == (int)type && c->fft_side[s] == N && c->fft_batch[s] == batch)) s++;
+    while (s < S && !(c->fft_plan[s] && c->fft_side[s] == N && c->fft_batch[s] == batch)) s++;
     hipfftHandle h = nullptr;
     if (s < S) {
         h = (hipfftHandle)c->fft_plan[s];
     } else {
-        hipfftResult r = hipfftPlan1d(&h, N, type, batch);
+        hipfftResult r = hipfftPlan1d(&h, N, HIPFFT_Z2Z, batch);
         if (r == HIPFFT_SUCCESS) r = hipfftSetStream(h, c->stream);
         if (r != HIPFFT_SUCCESS) {
             if (h) (void)hipfftDestroy(h);
@@ -999,12 +1010,10 @@ hipfftHandle fft_plan(clm_ctx* c, hipfftType type, int N, int batch, int* rc) {
     }
     for (; s > 0; s--) {
         c->fft_plan[s] = c->fft_plan[s - 1];
-        c->fft_type[s] = c->fft_type[s - 1];
         c->fft_side[s] = c->fft_side[s - 1];
         c->fft_batch[s] = c->fft_batch[s - 1];
     }
     c->fft_plan[0] = (void*)h;
-    c->fft_type[0] = (int)type;
     c->fft_side[0] = N;
     c->fft_batch[0] = batch;
     return h;
@@ -1019,6 +1028,7 @@ int nufft_run(clm_ctx* c, const clm_pft_params* p, const void* d_img, void* d_pf
     g.M = p->n_r * (p->n_theta / 2);
     g.N = smooth_at_least(std::max(2 * p->n, 2 * NW));
     g.H = g.N / 2 + 1;
+    g.np = (p->n + 1) / 2;
     g.x0 = (int)std::ceil(-0.5 * p->n);
     const int K = p->K;
     const size_t NN = (size_t)g.N * g.N;
@@ -1032,9 +1042,9 @@ int nufft_run(clm_ctx* c, const clm_pft_params* p, const void* d_img, void* d_pf
     const double side = 15.0 * g.N / (2.0 * g.n_r - 1.0) * M_SQRT1_2 + NW + 2;
     const bool boxed = side * side <= BOXCAP;
     int rc;
-    // the grids' half columns (before them, the real rows), the rows' transforms
+    // the grids' half columns, the pairs of rows
     if ((rc = ensure(c, c->pft_grid, (size_t)kc * g.H * g.N * sizeof(double2))) ||
-        (rc = ensure(c, c->pft_xt, (size_t)kc * g.n * g.H * sizeof(double2))) ||
+        (rc = ensure(c, c->pft_xt, (size_t)kc * g.np * g.N * sizeof(double2))) ||
         (rc = ensure(c, c->pft_base, (size_t)g.M * sizeof(int2))) ||
         (rc = ensure(c, c->pft_wt, (size_t)g.M * 2 * NW * sizeof(double))) ||
         (rc = ensure(c, c->pft_dec, (size_t)(g.n + 2 * NQ) * sizeof(double))))
@@ -1055,23 +1065,22 @@ int nufft_run(clm_ctx* c, const clm_pft_params* p, const void* d_img, void* d_pf
     int chunks = 0;
     double2* grid = (double2*)c->pft_grid.p;
     double2* rows = (double2*)c->pft_xt.p;
-    double* real = (double*)c->pft_grid.p;  // n rows of N reals fit in H rows of N complex values
     for (long long k0 = 0; k0 < K; k0 += kc) {
         g.Kc = (int)((K - k0) < kc ? (K - k0) : kc);
-        hipfftHandle plan_x = fft_plan(c, HIPFFT_D2Z, g.N, g.n * g.Kc, &rc);
-        hipfftHandle plan_y = plan_x ? fft_plan(c, HIPFFT_Z2Z, g.N, g.H * g.Kc, &rc) : nullptr;
+        hipfftHandle plan_x = fft_plan(c, g.N, g.np * g.Kc, &rc);
+        hipfftHandle plan_y = plan_x ? fft_plan(c, g.N, g.H * g.Kc, &rc) : nullptr;
         if (!plan_y) return rc;
         HIPCHK(c, hipEventRecord(ev[2], c->stream));
-        const long long nq = (long long)g.n * g.N * g.Kc;
+        const long long nq = (long long)g.np * g.N * g.Kc;
         const unsigned dgrd = (unsigned)((nq + 255) / 256);
         if (p->img_dtype == CLM_R64)
-            deconv_kernel<double><<<dgrd, 256, 0, c->stream>>>(g, (const double*)d_img, k0, dec, real);
+            deconv_kernel<double><<<dgrd, 256, 0, c->stream>>>(g, (const double*)d_img, k0, dec, rows);
         else
-            deconv_kernel<float><<<dgrd, 256, 0, c->stream>>>(g, (const float*)d_img, k0, dec, real);
+            deconv_kernel<float><<<dgrd, 256, 0, c->stream>>>(g, (const float*)d_img, k0, dec, rows);
         HIPCHK(c, hipGetLastError());
         HIPCHK(c, hipEventRecord(ev[3], c->stream));
-        hipfftDoubleComplex* fy = (hipfftDoubleComplex*)grid;
-        hipfftResult fr = hipfftExecD2Z(plan_x, real, (hipfftDoubleComplex*)rows);
+        hipfftDoubleComplex *fx = (hipfftDoubleComplex*)rows, *fy = (hipfftDoubleComplex*)grid;
+        hipfftResult fr = hipfftExecZ2Z(plan_x, fx, fx, HIPFFT_BACKWARD);
         if (fr == HIPFFT_SUCCESS) {
             const dim3 tgrd((g.H + 31) / 32, (g.N + 31) / 32, g.Kc);
             turn_kernel<<<tgrd, 256, 0, c->stream>>>(g, rows, grid);
@@ -1133,7 +1142,7 @@ void pft_release(clm_ctx* c) {
     for (int s = 0; s < clm_ctx::FFT_PLANS; s++) {
         if (c->fft_plan[s]) (void)hipfftDestroy((hipfftHandle)c->fft_plan[s]);
         c->fft_plan[s] = nullptr;
-        c->fft_type[s] = c->fft_side[s] = c->fft_batch[s] = 0;
+        c->fft_side[s] = c->fft_batch[s] = 0;
     }
 }
 }  // namespace clmh
