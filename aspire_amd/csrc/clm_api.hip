@@ -44,8 +44,29 @@ int pad_R(int R) {
 // a CU (by registers), the 16-bit operands one or two.
 int serial_waves(int opk) { return opk == OPK_F32 ? 4 : 8; }
 
-// npairs: pairs of the first pass, or 0 where they are few or unknown.
-Variant choose_variant(int opk, int NCT, int Rp, int want_ct, int want_W, long long npairs, int n_cu) {
+// Workgroups a first pass of K images has with `per` pairs each (those of a tile
+// share their first image).
+long long pass_tiles(long long K, int per) {
+    long long n = 0;
+    for (long long k = 1; k < K; k++) n += (k + per - 1) / per;
+    return n;
+}
+
+// Cost of a column tile by how many share an A fragment, against three (16 bits)
+// or two (FP32) with even loads.  16 bits, 360 rays, 13 shifts, ten thousand pairs
+// and more: two 1.1 to 1.3; one 1.3 to 1.4 with rays of 16 and 32 points, 2.2 and
+// 2.0 with 48 and 64; longer rays have no three, and one costs 1.4 (96 points) and
+// 1.0 (128) times two.  With few pairs one is dearer on short rays: 72 rays of 16
+// points, 2775 pairs, 36.7 us where the even loads are one's and 24.9 with two; FP32,
+// 1225 pairs, 42 and 31.
+double tile_weight(int opk, int ct, int Rp) {
+    if (opk == OPK_F32) return ct == 1 && Rp <= 32 ? 1.3 : 1.0;
+    if (ct > 1) return ct == 3 ? 1.0 : 1.2;
+    return Rp <= 32 ? 1.6 : Rp <= 64 ? 2.2 : Rp <= 96 ? 1.7 : 1.25;
+}
+
+// K: images of the first pass, or 0 where its pairs are few or unknown.
+Variant choose_variant(int opk, int NCT, int Rp, int want_ct, int want_W, long long K, int n_cu) {
     Variant best, even;
     double best_waste = 1e9, best_cost = 0, even_cost = 0;
     const bool passes = pair_passes(opk == OPK_F32 ? 4 : 2, Rp);
@@ -57,14 +78,20 @@ Variant choose_variant(int opk, int NCT, int Rp, int want_ct, int want_W, long l
     const int* cts = opk == OPK_F32 ? cts_f32 : cts_mfma16;
     const int ncts = opk == OPK_F32 ? 2 : 3;
     // Column tiles of the busiest SIMD: a workgroup's waves go to the four SIMDs
-    // in turn, so W waves cost as many as the next multiple of four, and the
-    // last round of workgroups counts whole.  A 16-bit column tile costs more
-    // the fewer share an A fragment: 1.5 times with two (0.655 us a pair against
-    // 0.321 with three and even loads, 41 shifts, n_r = 65), 2.2 with one.
+    // in turn, so W waves cost as many as the next multiple of four, and rounds of
+    // workgroups that fill the chip take turns.  A last round that leaves a wave
+    // alone on its SIMD has nothing to run beside its epilogues: a quarter more.
+    // FP32 rays of 128 points lose 15% to the passes (420 rays, 33670 pairs, as even
+    // either way: 39.3 ms against 37.9).
     auto cost = [&](int waves, int per_tile, int tiles_per_wave, int ct) {
-        const long long per_round = (long long)per_tile * n_cu;
-        const double w = opk == OPK_F32 || ct == 3 ? 1.0 : ct == 2 ? 1.5 : 2.2;
-        return w * (double)((npairs + per_round - 1) / per_round) * ((waves + 3) / 4) * tiles_per_wave;
+        if (!K) return 0.0;
+        const int simd = (waves + 3) / 4;
+        const int room = opk == OPK_F32 && ct == 1 ? (Rp <= 16 ? 4 : Rp <= 48 ? 3 : 2) : 2;  // waves a SIMD holds
+        const int wgs = std::max(1, room / simd);
+        const long long n = pass_tiles(K, per_tile), full = n / ((long long)n_cu * wgs);
+        const double last = (double)((n - full * n_cu * wgs + n_cu - 1) / n_cu * simd);
+        const double pass = opk == OPK_F32 && Rp > 96 && tiles_per_wave > ct ? 1.15 : 1.0;
+        return pass * tile_weight(opk, ct, Rp) * tiles_per_wave * ((double)full * wgs * simd + (last > 0 ? std::max(last, 1.25) : 0.0));
     };
     for (int i = 0; i < ncts; i++) {
         const int ct = cts[i];
@@ -93,15 +120,24 @@ Variant choose_variant(int opk, int NCT, int Rp, int want_ct, int want_W, long l
             even.ser = ser ? sw : 0;
         }
     }
-    if (want_W || want_ct || !npairs || !best.ct) return best;
+    if (want_W || want_ct || !K || !best.ct) return best;
     // The least padding, unless another split loads the SIMDs more evenly by a
     // tenth or more.  300 rays (five column tiles), five waves a pair put two
     // on one SIMD; FP32, 31375 pairs of n_r = 44 with one wave through the five:
     // 19.0 -> 10.7 ms; FP16, 124750 pairs of n_r = 45 with two waves of three tiles
     // (one of padding): 25.6 -> 8.9 ms.  BF16 rays of 90 points, one wave through the
     // column groups: 360 rays, 79800 pairs, 16.7 -> 13.3 ms; 300 rays, 44850 pairs, 12.6
-    // -> 6.2 ms.
-    return even_cost < 0.9 * best_cost ? even : best;
+    // -> 6.2 ms.  With fewer than sixteen pairs a compute unit the count of tiles says
+    // less: by a quarter or more there (FP16, 360 rays of 16 points, 990 pairs, a split
+    // that counts 0.8: 54.7 -> 64.4 us), and FP32 with fewer than four not at all (120
+    // rays of 16 points, 990 pairs, counted 0.7: 11% slower).  Over 2860 shapes (36 to
+    // 480 rays of 16 to 119 points, 10 to 350 images, FP32, FP16 and BF16) the choice
+    // takes 0.92 of the least padding's time in the geometric mean, and none takes
+    // over 3% and 3 us longer.
+    const long long pairs = K * (K - 1) / 2;
+    if (opk == OPK_F32 && pairs < 4LL * n_cu) return best;
+    const double gain = pairs < 16LL * n_cu ? 0.75 : 0.9;
+    return even_cost < gain * best_cost ? even : best;
 }
 
 PairFn pick_pair_kernel(int opk, int ct, int Rp, bool sym, bool emit) {
@@ -366,7 +402,7 @@ int plan_stack(clm_ctx* c, const clm_params* p, StackJob& j) {
         for (const auto& e : c->tuned)
             if (e.first == key) { want_ct = e.second.x; want_W = e.second.y; want_lag = e.second.z; }
     }
-    j.v = choose_variant(j.opk, NCT, g.Rp, want_ct, want_W, c->least_padding ? 0 : j.P, c->n_cu);
+    j.v = choose_variant(j.opk, NCT, g.Rp, want_ct, want_W, c->least_padding ? 0 : K, c->n_cu);
     if (!j.v.ct) return fail(c, CLM_E_UNSUP, "no kernel variant for L=%d (variant %d)", g.L, p->variant);
     g.NCT = j.v.NCTp;
     g.Lp = 32 * j.v.NCTp;

@@ -40,3 +40,27 @@ print(json.dumps(r))
     assert out["both1"][0]["lag"] == 0 and out["subset1"][0]["lag"] == 0
     if n_theta == 300 and not (prec == "fp16" and n_r == 17):
         assert out["both0"][0]["passes"] > 1 and out["subset0"][0]["passes"] == 1
+
+
+# (precision, rays, points, images) -> the first pass's variant: column tiles per
+# wave * 100 + waves, + 50 for waves that take the column groups in turn
+CHOICES = [
+    # the least padding, where a split of more even loads measured slower
+    (("fp32", 420, 120, 90), 107), (("fp16", 150, 120, 90), 106), (("bf16", 180, 120, 90), 106),
+    (("fp32", 300, 17, 90), 105), (("fp32", 120, 17, 45), 204), (("fp16", 360, 17, 45), 308),
+    # more even loads, where they measured faster
+    (("fp32", 300, 44, 251), 154), (("fp16", 300, 45, 500), 308), (("bf16", 360, 91, 400), 258),
+    (("bf16", 300, 91, 300), 258),
+]
+
+
+def test_split_of_the_first_pass(tmp_path):
+    out = hip_stub.run(f"""
+h = context()
+r = []
+for prec, n_theta, n_r, K in {[c[0] for c in CHOICES]!r}:
+    rc, st = search(h, params(K, n_r, n_theta, prec))
+    r.append([rc, st.variant])
+print(json.dumps(r))
+""", tmp_path)
+    assert out == [[0, v] for _, v in CHOICES]
