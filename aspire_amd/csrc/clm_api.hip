@@ -65,8 +65,11 @@ double tile_weight(int opk, int ct, int Rp) {
     return Rp <= 32 ? 1.6 : Rp <= 64 ? 2.2 : Rp <= 96 ? 1.7 : 1.25;
 }
 
-// K: images of the first pass, or 0 where its pairs are few or unknown.
-Variant choose_variant(int opk, int NCT, int Rp, int want_ct, int want_W, long long K, int n_cu) {
+// K: images of the first pass, or 0 where its pairs are few or unknown.  least: the
+// split that needs least memory, which is the least padding with the most pairs a
+// tile (FP32, 300 rays of 16 points, no shifts: 1376 images in the allocation-free
+// call's array against 1365 with a tile a pair).
+Variant choose_variant(int opk, int NCT, int Rp, int want_ct, int want_W, long long K, int n_cu, bool least = false) {
     Variant best, even;
     double best_waste = 1e9, best_cost = 0, even_cost = 0;
     const bool passes = pair_passes(opk == OPK_F32 ? 4 : 2, Rp);
@@ -121,6 +124,10 @@ Variant choose_variant(int opk, int NCT, int Rp, int want_ct, int want_W, long l
         }
     }
     if (want_W || want_ct || !K || !best.ct) return best;
+    if (least) {
+        if (passes && best.CPP > 1) best.ser = sw;
+        return best;
+    }
     // The least padding, unless another split loads the SIMDs more evenly by a
     // tenth or more.  300 rays (five column tiles), five waves a pair put two
     // on one SIMD; FP32, 31375 pairs of n_r = 44 with one wave through the five:
@@ -402,7 +409,7 @@ int plan_stack(clm_ctx* c, const clm_params* p, StackJob& j) {
         for (const auto& e : c->tuned)
             if (e.first == key) { want_ct = e.second.x; want_W = e.second.y; want_lag = e.second.z; }
     }
-    j.v = choose_variant(j.opk, NCT, g.Rp, want_ct, want_W, c->least_padding ? 0 : K, c->n_cu);
+    j.v = choose_variant(j.opk, NCT, g.Rp, want_ct, want_W, K, c->n_cu, c->least_padding);
     if (!j.v.ct) return fail(c, CLM_E_UNSUP, "no kernel variant for L=%d (variant %d)", g.L, p->variant);
     g.NCT = j.v.NCTp;
     g.Lp = 32 * j.v.NCTp;

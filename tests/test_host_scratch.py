@@ -10,7 +10,8 @@ from tests import hip_stub
 # n_r, n_theta, max_shift (step 0.5), precision, images that fit with the least padding
 CASES = [(120, 150, 0.0, "fp16", 643), (120, 180, 6.0, "bf16", 127), (90, 180, 0.0, "fp16", 739),
          (65, 420, 0.0, "bf16", 527), (45, 300, 6.0, "fp16", 187), (17, 420, 6.0, "fp16", 333),
-         (17, 300, 0.0, "fp32", 1353), (65, 360, 0.0, "fp32", 693)]
+         (17, 300, 0.0, "fp32", 1353), (65, 360, 0.0, "fp32", 693),
+         (17, 300, 0.0, "fp32", 1376), (17, 420, 6.0, "fp32", 467)]
 
 
 @pytest.mark.parametrize("n_r,n_theta,ms,prec,K", CASES)
