@@ -47,31 +47,62 @@ int serial_waves(int opk) { return opk == OPK_F32 ? 4 : 8; }
 // Workgroups a first pass of K images has with `per` pairs each (those of a tile
 // share their first image).
 long long pass_tiles(long long K, int per) {
-    long long n = 0;
-    for (long long k = 1; k < K; k++) n += (k + per - 1) / per;
-    return n;
+    const long long n = K > 0 ? K - 1 : 0, q = n / per, r = n % per;  // sum of ceil(k / per), k = 1..n
+    return per * (q * (q + 1) / 2) + r * (q + 1);
 }
 
-// Cost of a column tile by how many share an A fragment, against three (16 bits)
-// or two (FP32) with even loads.  16 bits, 360 rays, 13 shifts, ten thousand pairs
-// and more: two 1.1 to 1.3; one 1.3 to 1.4 with rays of 16 and 32 points, 2.2 and
-// 2.0 with 48 and 64; longer rays have no three, and one costs 1.4 (96 points) and
-// 1.0 (128) times two.  With few pairs one is dearer on short rays: 72 rays of 16
-// points, 2775 pairs, 36.7 us where the even loads are one's and 24.9 with two; FP32,
-// 1225 pairs, 42 and 31.
-double tile_weight(int opk, int ct, int Rp) {
-    if (opk == OPK_F32) return ct == 1 && Rp <= 32 ? 1.3 : 1.0;
-    if (ct > 1) return ct == 3 ? 1.0 : 1.2;
-    return Rp <= 32 ? 1.6 : Rp <= 64 ? 2.2 : Rp <= 96 ? 1.7 : 1.25;
+// us that a SIMD with two waves spends on one A-tile (32 rows) of one column tile: these
+// and pass_us's constants are the least squares over every split of 3276 shapes (72 to 480
+// rays of 16 to 119 points, 10 to 420 images, 1, 5 and 41 shifts; 11% rms).
+// FP32: by the k-steps, a tenth less where two tiles share an A fragment; with the
+// column groups in turn 4% less (one pair's epilogue beside another's), 14% more where
+// B's registers leave no room (128 points).  16 bits: by the tiles that share a
+// fragment; the jump from 32 to 48 points with one is where a wave's next fragments no
+// longer come in time.
+double tile_us(int opk, int ct, int Rp, bool ser) {
+    if (opk == OPK_F32) return 0.0345 * Rp * (ct == 2 ? 0.9 : 1.0) * (ser ? Rp > 96 ? 1.14 : 0.96 : 1.0);
+    static const double us[6][3] = {{0.19, 0.17, 0.12}, {0.20, 0.18, 0.14}, {0.39, 0.20, 0.155},
+                                    {0.42, 0.24, 0.20}, {0.49, 0.315, 0.0}, {0.50, 0.50, 0.0}};
+    const int i = Rp <= 64 ? Rp / 16 - 1 : Rp <= 96 ? 4 : 5;
+    return us[i][ct - 1] * (ser ? 0.87 : 1.0);
 }
 
-// K: images of the first pass, or 0 where its pairs are few or unknown.  least: the
-// split that needs least memory, which is the least padding with the most pairs a
+// us of a first pass of K images with NAT A-tiles: `waves` a workgroup, `per` pairs a
+// tile, `cols` column tiles a wave.  Workgroups of a CU share its SIMDs (wave w goes to
+// SIMD w % 4, so W waves cost as many as the next multiple of four), and the busiest CU
+// sets the time: whole rounds of the workgroups that it holds, then what is left.  After
+// a whole round those that finish first take what is left, two of one CU as likely as
+// one of each.  A wave alone on its SIMD has nothing beside its epilogues.  Per column
+// tile B is read (0.015 us a point); a tile's own start and end take 1.1 us; where
+// the waves of a pair hand their maxima round on short rays, 2, and 4.5 with several
+// FP32 workgroups on a CU (72 rays of 16 points, 1485 pairs, FP32: two waves a pair
+// 51 us, a pair a wave 34).
+double pass_us(int opk, int ct, int Rp, bool ser, int waves, int per, int cols, int NAT, long long K, int n_cu) {
+    const bool f32 = opk == OPK_F32;
+    const int simd = (waves + 3) / 4;
+    const int room = f32 && ct == 1 ? (Rp <= 16 ? 4 : Rp <= 48 ? 3 : 2) : 2;  // waves that a SIMD holds
+    const long long wgs = std::max(1, room / simd), n = (pass_tiles(K, per) + n_cu - 1) / n_cu, full = n / wgs;
+    long long rest = n - full * wgs;
+    if (full && rest) rest = std::min(wgs, rest + 1);
+    const bool shared = Rp <= 32 && ct == 1 && !ser && per < waves;
+    const double ends = !shared ? 1.1 : !f32 ? 2.0 : simd == 1 && n > 1 ? 4.5 : 1.1;
+    auto busy = [&](long long w) {  // SIMD time of w waves side by side
+        return (double)w * (f32 ? w == 1 ? (Rp > 96 ? 1.3 : 1.17) : w > 2 ? 0.95 : 1.0 : 1.0);
+    };
+    const double wave = cols * (NAT * tile_us(opk, ct, Rp, ser) + 0.015 * Rp) + ends;
+    return 10.0 + wave * (full * busy(simd * wgs) + (rest ? busy(simd * rest) : 0.0));
+}
+
+// K: images of the first pass, or 0 where its pairs are few or unknown.  sel: of
+// selected pairs, whose lists may be too short for the column groups in turn.  least:
+// the split that needs least memory, which is the least padding with the most pairs a
 // tile (FP32, 300 rays of 16 points, no shifts: 1376 images in the allocation-free
 // call's array against 1365 with a tile a pair).
-Variant choose_variant(int opk, int NCT, int Rp, int want_ct, int want_W, long long K, int n_cu, bool least = false) {
-    Variant best, even;
-    double best_waste = 1e9, best_cost = 0, even_cost = 0;
+Variant choose_variant(int opk, int NCT, const Geom& g, int want_ct, int want_W, long long K, int n_cu,
+                       bool sel = false, bool least = false) {
+    Variant best, fast;
+    const int Rp = g.Rp;
+    double best_waste = 1e9, best_us = 0, fast_us = 0;
     const bool passes = pair_passes(opk == OPK_F32 ? 4 : 2, Rp);
     const int sw = serial_waves(opk);
     const int want_ser = want_W > SER_ID ? want_W - SER_ID : 0;
@@ -80,22 +111,6 @@ Variant choose_variant(int opk, int NCT, int Rp, int want_ct, int want_W, long l
     const int cts_f32[] = {2, 1};
     const int* cts = opk == OPK_F32 ? cts_f32 : cts_mfma16;
     const int ncts = opk == OPK_F32 ? 2 : 3;
-    // Column tiles of the busiest SIMD: a workgroup's waves go to the four SIMDs
-    // in turn, so W waves cost as many as the next multiple of four, and rounds of
-    // workgroups that fill the chip take turns.  A last round that leaves a wave
-    // alone on its SIMD has nothing to run beside its epilogues: a quarter more.
-    // FP32 rays of 128 points lose 15% to the passes (420 rays, 33670 pairs, as even
-    // either way: 39.3 ms against 37.9).
-    auto cost = [&](int waves, int per_tile, int tiles_per_wave, int ct) {
-        if (!K) return 0.0;
-        const int simd = (waves + 3) / 4;
-        const int room = opk == OPK_F32 && ct == 1 ? (Rp <= 16 ? 4 : Rp <= 48 ? 3 : 2) : 2;  // waves a SIMD holds
-        const int wgs = std::max(1, room / simd);
-        const long long n = pass_tiles(K, per_tile), full = n / ((long long)n_cu * wgs);
-        const double last = (double)((n - full * n_cu * wgs + n_cu - 1) / n_cu * simd);
-        const double pass = opk == OPK_F32 && Rp > 96 && tiles_per_wave > ct ? 1.15 : 1.0;
-        return pass * tile_weight(opk, ct, Rp) * tiles_per_wave * ((double)full * wgs * simd + (last > 0 ? std::max(last, 1.25) : 0.0));
-    };
     for (int i = 0; i < ncts; i++) {
         const int ct = cts[i];
         if (want_ct && ct != want_ct) continue;
@@ -109,18 +124,19 @@ Variant choose_variant(int opk, int NCT, int Rp, int want_ct, int want_W, long l
         if (W < CPP || W % CPP || W > 8) continue;
         Variant v;
         v.ct = ct; v.W = W; v.CPP = CPP; v.NCTp = NCTp; v.ser = want_ser;
-        const double side = cost(W, W / CPP, ct, ct), one = cost(sw, sw, NCTp, ct);
         const double waste = (double)NCTp / NCT;
+        const double side = pass_us(opk, ct, Rp, false, W, W / CPP, ct, g.NAT, K, n_cu);
         if (waste < best_waste - 1e-9) {
             best_waste = waste;
             best = v;
-            best_cost = side;
+            best_us = side;
         }
-        const bool ser = passes && CPP > 1 && one < side;
-        if (!even.ct || (ser ? one : side) < even_cost) {
-            even_cost = ser ? one : side;
-            even = v;
-            even.ser = ser ? sw : 0;
+        const double turns = pass_us(opk, ct, Rp, true, sw, sw, NCTp, g.NAT, K, n_cu);
+        const bool ser = passes && !sel && CPP > 1 && turns < side;
+        if (!fast.ct || (ser ? turns : side) < fast_us) {
+            fast_us = ser ? turns : side;
+            fast = v;
+            fast.ser = ser ? sw : 0;
         }
     }
     if (want_W || want_ct || !K || !best.ct) return best;
@@ -128,23 +144,16 @@ Variant choose_variant(int opk, int NCT, int Rp, int want_ct, int want_W, long l
         if (passes && best.CPP > 1) best.ser = sw;
         return best;
     }
-    // The least padding, unless another split loads the SIMDs more evenly by a
-    // tenth or more.  300 rays (five column tiles), five waves a pair put two
-    // on one SIMD; FP32, 31375 pairs of n_r = 44 with one wave through the five:
-    // 19.0 -> 10.7 ms; FP16, 124750 pairs of n_r = 45 with two waves of three tiles
-    // (one of padding): 25.6 -> 8.9 ms.  BF16 rays of 90 points, one wave through the
-    // column groups: 360 rays, 79800 pairs, 16.7 -> 13.3 ms; 300 rays, 44850 pairs, 12.6
-    // -> 6.2 ms.  With fewer than sixteen pairs a compute unit the count of tiles says
-    // less: by a quarter or more there (FP16, 360 rays of 16 points, 990 pairs, a split
-    // that counts 0.8: 54.7 -> 64.4 us), and FP32 with fewer than four not at all (120
-    // rays of 16 points, 990 pairs, counted 0.7: 11% slower).  Over 2860 shapes (36 to
-    // 480 rays of 16 to 119 points, 10 to 350 images, FP32, FP16 and BF16) the choice
-    // takes 0.92 of the least padding's time in the geometric mean, and none takes
-    // over 3% and 3 us longer.
-    const long long pairs = K * (K - 1) / 2;
-    if (opk == OPK_F32 && pairs < 4LL * n_cu) return best;
-    const double gain = pairs < 16LL * n_cu ? 0.75 : 0.9;
-    return even_cost < gain * best_cost ? even : best;
+    // The least padding, unless another split counts 8% and 2 us less.  300 rays (five
+    // column tiles), five waves a pair put two on one SIMD; FP32, 31375 pairs of n_r = 44
+    // with one wave through the five: 19.0 -> 10.7 ms; FP16, 124750 pairs of n_r = 45 with
+    // two waves of three tiles (one of padding): 25.6 -> 8.9 ms.  BF16 rays of 90 points,
+    // one wave through the column groups: 360 rays, 79800 pairs, 16.7 -> 13.3 ms; 300
+    // rays, 44850 pairs, 12.6 -> 6.2 ms.  Over 3320 shapes that the counts were not fitted
+    // to (90 to 500 rays of 24 to 109 points, 15 to 210 images, 1 to 25 shifts; FP32,
+    // FP16, BF16) the choice differs from the least padding in 1163, takes 0.73 of its
+    // time there in the geometric mean, and at most 8% more.
+    return fast_us < 0.92 * best_us && fast_us < best_us - 2.0 ? fast : best;
 }
 
 PairFn pick_pair_kernel(int opk, int ct, int Rp, bool sym, bool emit) {
@@ -409,12 +418,12 @@ int plan_stack(clm_ctx* c, const clm_params* p, StackJob& j) {
         for (const auto& e : c->tuned)
             if (e.first == key) { want_ct = e.second.x; want_W = e.second.y; want_lag = e.second.z; }
     }
-    j.v = choose_variant(j.opk, NCT, g.Rp, want_ct, want_W, K, c->n_cu, c->least_padding);
+    g.NROWS = g.NE * g.L;
+    g.NAT = (g.NROWS + 31) / 32;
+    j.v = choose_variant(j.opk, NCT, g, want_ct, want_W, K, c->n_cu, j.sel_list != nullptr, c->least_padding);
     if (!j.v.ct) return fail(c, CLM_E_UNSUP, "no kernel variant for L=%d (variant %d)", g.L, p->variant);
     g.NCT = j.v.NCTp;
     g.Lp = 32 * j.v.NCTp;
-    g.NROWS = g.NE * g.L;
-    g.NAT = (g.NROWS + 31) / 32;
     if ((long long)g.NROWS * g.Lp > 0xffffffffLL) return fail(c, CLM_E_UNSUP, "map too large");
     j.lag = want_lag && !(p->reserved & 1) ? 1 : 0;
     return CLM_OK;
@@ -486,7 +495,7 @@ int prepare(clm_ctx* c, Plan& pl, int n, const clm_params* ps, const clm_stack_i
     for (size_t gi = 0; gi < n_orig_groups && twins; gi++) {
         if (pl.groups[gi].exact || pl.groups[gi].opk == OPK_F32 || pl.groups[gi].norefine) continue;
         const StackJob& j0 = pl.jobs[pl.groups[gi].members[0]];
-        const Variant v32 = choose_variant(OPK_F32, (j0.s.g.L + 31) / 32, j0.s.g.Rp, 0, 0, 0, c->n_cu);
+        const Variant v32 = choose_variant(OPK_F32, (j0.s.g.L + 31) / 32, j0.s.g, 0, 0, 0, c->n_cu);
         if (!v32.ct) continue;
         Group T;
         T.opk = OPK_F32; T.ct = v32.ct; T.Rp = pl.groups[gi].Rp; T.sym = pl.groups[gi].sym;

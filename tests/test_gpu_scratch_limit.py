@@ -10,7 +10,7 @@ from tests.test_zz_no_alloc import run, same
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("K,n_r,n_theta,ms,prec", [(739, 90, 180, 0.0, "fp16"), (187, 45, 300, 6.0, "fp16")])
+@pytest.mark.parametrize("K,n_r,n_theta,ms,prec", [(510, 90, 300, 0.0, "fp16"), (187, 45, 300, 6.0, "fp16")])
 def test_at_the_limit(K, n_r, n_theta, ms, prec):
     import torch
 

@@ -42,15 +42,19 @@ print(json.dumps(r))
         assert out["both0"][0]["passes"] > 1 and out["subset0"][0]["passes"] == 1
 
 
-# (precision, rays, points, images) -> the first pass's variant: column tiles per
-# wave * 100 + waves, + 50 for waves that take the column groups in turn
+# (precision, rays, points, images) of five shifts -> the first pass's variant, any
+# within 3% of the fastest measured: column tiles per wave * 100 + waves, + 50 for
+# waves that take the column groups in turn
 CHOICES = [
-    # the least padding, where a split of more even loads measured slower
-    (("fp32", 420, 120, 90), 107), (("fp16", 150, 120, 90), 106), (("bf16", 180, 120, 90), 106),
-    (("fp32", 300, 17, 90), 105), (("fp32", 120, 17, 45), 204), (("fp16", 360, 17, 45), 308),
-    # more even loads, where they measured faster
-    (("fp32", 300, 44, 251), 154), (("fp16", 300, 45, 500), 308), (("bf16", 360, 91, 400), 258),
-    (("bf16", 300, 91, 300), 258),
+    # the least padding, where splits of more even loads are slower
+    (("fp32", 420, 120, 90), {107}), (("fp16", 150, 120, 90), {106}), (("bf16", 180, 120, 90), {106}),
+    (("fp32", 120, 17, 45), {204}), (("fp16", 360, 17, 45), {308}),
+    # more even loads, where they are faster
+    (("fp32", 300, 44, 251), {154}), (("fp16", 300, 45, 500), {308}), (("bf16", 360, 91, 400), {258}),
+    (("bf16", 300, 91, 300), {258}), (("fp32", 300, 17, 90), {154}),
+    # few pairs a compute unit
+    (("bf16", 420, 90, 80), {208, 258}), (("fp16", 300, 90, 65), {206}), (("fp32", 360, 33, 12), {106}),
+    (("fp32", 300, 45, 40), {154}),
 ]
 
 
@@ -63,4 +67,5 @@ for prec, n_theta, n_r, K in {[c[0] for c in CHOICES]!r}:
     r.append([rc, st.variant])
 print(json.dumps(r))
 """, tmp_path)
-    assert out == [[0, v] for _, v in CHOICES]
+    for (shape, want), (rc, got) in zip(CHOICES, out):
+        assert rc == 0 and got in want, (shape, got)
