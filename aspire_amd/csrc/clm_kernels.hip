@@ -40,8 +40,11 @@ namespace clm {
 // stride of a whole line apart, took 784 and 1830 us.
 constexpr int PREP_T = 256;
 
-// Lines per workgroup: as many as keep the terms and rays of a workgroup
-// within 40 KB of LDS, so that four workgroups share a CU.
+// Lines per workgroup.  Sixteen read whole cache lines, eight leave room in LDS for
+// twice the workgroups, whose two serial sums per line hide each other.  K = 1000,
+// complex128, us with 16 and 8 lines: n_r = 33 97 and 122, 45 118 and 141, 65 193 and
+// 183, 66 216 and 200, 79 228 and 214, 90 299 and 229, 97 319 and 258.  The line
+// lies where 16 need 34 KB of LDS; between 46 and 66 points it is within 8% either way.
 __host__ __device__ inline int prep_lines(int n_r) { return n_r <= 66 ? 16 : 8; }
 // per line: 2 n_r - 1 terms (the row padded to an odd number of doubles, for
 // the banks of the threads that walk the rows) and R complex values

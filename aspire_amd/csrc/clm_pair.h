@@ -138,8 +138,9 @@ __device__ inline float wave_max_dpp(float v) {
 __host__ __device__ inline size_t pair_lds_bytes(int W) { return 384 + (size_t)W * WCAP * 8; }
 
 // Whether a kernel can take a pair's column chunks one after another.  The
-// 16-bit kernels of shorter rays have even loads without (and the loop costs
-// them 4%: 583 to 605 ms for 2000 images, 41 shifts, n_r = 65).
+// 16-bit kernels of shorter rays hold three column tiles a wave, which evens most
+// loads out, and the loop costs them 4% where it is not used (one shape measured:
+// 583 to 605 ms for 2000 images, 41 shifts, n_r = 65).
 constexpr bool pair_passes(size_t op_bytes, int Rp) { return op_bytes == 4 || Rp > 64; }
 
 // Waves per SIMD the registers are held to: FP32 operands leave them idle with

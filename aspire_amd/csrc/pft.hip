@@ -248,8 +248,10 @@ __global__ __launch_bounds__(256) void narrow_kernel(Geo g, const double* __rest
 // packed FP16 operations from one X pair and eight Y pairs that it keeps over the
 // loop of a; the next PD values' operands are on their way meanwhile.
 // 243 us for 1000 images of 129 x 129, n_r = 65, n_theta = 360 (the sums take
-// 3.24 ms), 1.0 PFLOP/s.  Bound: the operands' loads; tiles of 8 x 4 have two thirds
-// of them and took 212 us, but leave fewer images without work for every CU.
+// 3.24 ms), 1.0 PFLOP/s.  Bound: the weights' vector instructions (the vector units
+// are busy 50% of the cycles, the matrix cores 48%, in turn); tiles of 8 x 4 form
+// each weight for twice the MFMAs' share and took 212 us, but leave fewer images
+// without work for every CU.
 template <int RT, int CT, int PD>
 __global__ __launch_bounds__(256, 2) void shift_kernel(Geo g, const h8* __restrict__ xh, const h2* __restrict__ dx,
                                                        const _Float16* __restrict__ dy, float2* __restrict__ shift,
@@ -356,8 +358,8 @@ void shift_launch(hipStream_t st, const Geo& g, const h8* xh, const h2* dx, cons
 // The 1-D grid gives each XCD (dispatch goes round-robin over 8) a contiguous
 // range of tiles, points fastest, so that its workgroups stream the same
 // images through its L2.
-// Bound: FP64 MFMA.  3.33 ms for 1000 images of 129 x 129, n_r = 65,
-// n_theta = 360: 63 TFLOP/s of the folded work (a large FP64 matrix product
+// Bound: FP64 MFMA (busy 86% of the cycles).  3.24 ms for 1000 images of 129 x 129,
+// n_r = 65, n_theta = 360: 65 TFLOP/s of the folded work (a large FP64 matrix product
 // reaches 72 here).  The unfolded contraction, 3.9 times the work, took 13.7 ms
 // at 57 TFLOP/s.  Smaller tiles than 4 x 4 only where they leave fewer MFMA
 // cycles on the busiest CU (few images or points).
@@ -604,8 +606,8 @@ __global__ void deconv_kernel(NGeo g, const T* __restrict__ img, long long k0, c
 // the rows that held no pixel, for the transforms over y.  Those rows (half of them
 // and more) are neither transformed over x nor read, and b is left turned: the
 // interpolation reads it with its axes exchanged.  Tiles of 32 x 32 through LDS.
-// For 100 images, N = 720: 71 us (transforms over x) + 112 (this, 620 MB) + 147
-// (over y).  Real-to-complex transforms along x took 70, but a second kernel
+// For 100 images, N = 720: 62 us (transforms over x) + 115 (this, 663 MB: HBM bound)
+// + 147 (over y).  Real-to-complex transforms along x took 70, but a second kernel
 // compiled at the first use of each size (2.3 s against 1.2, n = 150).
 __global__ __launch_bounds__(256) void turn_kernel(NGeo g, const double2* __restrict__ a, double2* __restrict__ b) {
     __shared__ double2 s_t[32][33];
@@ -723,8 +725,9 @@ __global__ __launch_bounds__(256) void interp_kernel(NGeo g, const double2* __re
 // grid, which is read once instead of 16 times.  The next image's box is on its
 // way into registers while this one is summed; a lane keeps its 16 weights for
 // all NBOXG images.  The direct form reads 256 grid values a point and image
-// through the vector L1 and is bound there.  390 us for 100 images, n = 359, 180 x
-// 180 points; LDS and the vector units are each busy about 60% of it.
+// through the vector L1 and is bound there.  383 us for 100 images, n = 359, 180 x
+// 180 points: the vector units are busy 69% of it and LDS 65% (a fifth of that on
+// bank conflicts).
 template <typename OutT>
 __global__ __launch_bounds__(256) void interp_box_kernel(NGeo g, const d2* __restrict__ b,
                                                          const int2* __restrict__ base,

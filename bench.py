@@ -503,8 +503,10 @@ def pft_bench(args):
     FP64) with clm_pft: images/s; the contraction kernel's FP64 MFMA roofline
     (algorithmic 4 flops per polar point, pixel and image: a complex weight
     times a real pixel; the pixels folded over both axes need about a quarter
-    of them, so frac can pass 1 and executed_frac is the matrix cores' share);
-    the FP64 C oracle on a bounded image sample as the
+    of them, so frac can pass 1 and executed_frac is the FP64 matrix cores'
+    share of the stage: kernel_ms also covers the mirror rays' change of
+    frequency, whose FP16 products are not counted, and the look for infinities
+    and NaN); the FP64 C oracle on a bounded image sample as the
     CPU baseline and parity check; the same transform by torch (weights
     materialised, rocBLAS ZGEMM) for reference."""
     import torch

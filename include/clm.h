@@ -481,12 +481,15 @@ typedef struct clm_pft_stats {
                           polar points                                  */
     float ms_stage;    /* exact: images folded over both axes, FP64;
                           NUFFT: deconvolution onto the grids           */
-    float ms_pft;      /* exact: the contraction (FP64 MFMA); NUFFT: the
-                          interpolation at the polar points            */
+    float ms_pft;      /* exact: the contraction (FP64 MFMA), with the
+                          mirror rays' change of frequency and the
+                          images that hold infinities or NaN; NUFFT:
+                          the interpolation at the polar points        */
     int32_t chunks;    /* image chunks (exact: at most 8192 images;
                           NUFFT: at most 2048 images, and 4 GiB of
                           whole grids, of which half is kept)           */
-    float ms_fft;      /* NUFFT: the batched FFTs along both axes       */
+    float ms_fft;      /* NUFFT: the batched FFTs along both axes and the
+                          transpose between them                       */
     int32_t grid_side; /* NUFFT: oversampled grid side N (2,3,5-smooth,
                           >= 2n)                                        */
 } clm_pft_stats;
